@@ -29,6 +29,10 @@ extern "C" {
 /* element types of activation / weight buffers */
 enum { LLMC_BF16 = 0, LLMC_F16 = 1, LLMC_F32 = 2 };
 
+/* stored scale codes that llmc_quantize reads in place of a numeric scale dtype: e4m3 bytes (read as fp32 values)
+ * and E8M0 exponents (2^(e-127), rounded to the input's 16-bit dtype, to bf16 for fp32 input) */
+enum { LLMC_E4M3 = 3, LLMC_E8M0 = 4 };
+
 /* element formats of the quantised value */
 enum {
   LLMC_FMT_INT = 0,  /* signed integer, num_bits in [2,8], round-half-even       */
@@ -73,6 +77,13 @@ int llmc_hessian_accumulate(float* H, int64_t ldh, const void* X, int64_t ldx,
                             int64_t T, int64_t K, int32_t x_dtype, float alpha,
                             int32_t flags, void* workspace, int64_t workspace_bytes,
                             void* stream);
+
+/* llmc_hessian_accumulate that also adds `add` to the fp32 device value *count (the hook's num_samples; NULL: no
+ * count), in the same launch where the 16-bit kernels run. */
+int llmc_hessian_accumulate_counted(float* H, int64_t ldh, const void* X, int64_t ldx,
+                                    int64_t T, int64_t K, int32_t x_dtype, float alpha,
+                                    int32_t flags, float* count, float add, void* workspace,
+                                    int64_t workspace_bytes, void* stream);
 
 /* Grouped form for the per-expert Hessians of an MoE layer (the 128 x 3 accumulate_hessian calls
  * that LinearExperts2D.forward triggers per batch, modeling/moe/linear_experts.py:235-268): n
@@ -196,13 +207,21 @@ int llmc_imatrix_observe_blocks(const void* x, int32_t dtype, int64_t R, int64_t
  * product, rounded again), returned as fp32 [1].
  * llmc_calculate_qparams replaces CT calculate_qparams as called from
  * observers/base.py:114-119: n (min,max) pairs -> scale (scale_out_dtype; fp32
- * e4m3-grid values for LLMC_SCALE_NVFP4), int8 zero points (NULL when symmetric),
- * and optionally the stored scale code (e4m3 byte for NVFP4, E8M0 byte for MXFP4).
+ * e4m3-grid values for LLMC_SCALE_NVFP4), int8 zero points (zeros when symmetric),
+ * and the stored scale code (e4m3 byte for NVFP4, E8M0 byte for MXFP4).  Each output
+ * may be NULL where it is not wanted, but not scale and code both.
  */
 int llmc_absmax_accumulate(const void* min_vals, const void* max_vals, int64_t n, int32_t dtype,
                            float* absmax_inout, void* stream);
 int llmc_generate_gparam(const float* absmax, int32_t stats_dtype, float* global_scale_out,
                          void* stream);
+/* Both steps over the arrays of a fused group without a zero-initialised cell: one call per (min, max) array on one
+ * stream and one workspace (llmc_global_scale_workspace_bytes), `first` set on the first, `last` on the last, whose
+ * global_scale_out receives the result for statistics of out_stats_dtype. */
+int64_t llmc_global_scale_workspace_bytes(void);
+int llmc_global_scale(const void* min_vals, const void* max_vals, int64_t n, int32_t dtype, int32_t first,
+                      int32_t last, int32_t out_stats_dtype, float* global_scale_out, void* workspace,
+                      int64_t workspace_bytes, void* stream);
 int llmc_calculate_qparams(const void* min_vals, const void* max_vals, int64_t n,
                            int32_t stats_dtype, int32_t fmt, int32_t num_bits, int32_t symmetric,
                            int32_t scale_mode, const float* global_scale, void* scale_out,
@@ -231,10 +250,27 @@ int llmc_quantize(const void* x, int32_t x_dtype, int64_t R, int64_t K, int64_t 
                   int64_t row_div, int64_t scale_row_stride, int64_t col_div, int32_t out_mode,
                   void* out, int32_t out_dtype, int64_t ldo, void* stream);
 
+/* llmc_quantize of a checkpoint weight: the launch also writes the int64 pair (R, K) to shape_out (the weight_shape
+ * tensor stored beside packed weights; NULL: not wanted). */
+int llmc_quantize_shaped(const void* x, int32_t x_dtype, int64_t R, int64_t K, int64_t ldx,
+                         const void* scale, int32_t scale_dtype, const int8_t* zero_point,
+                         const int32_t* g_idx, const float* global_scale, int32_t fmt, int32_t num_bits,
+                         int64_t row_div, int64_t scale_row_stride, int64_t col_div, int32_t out_mode,
+                         void* out, int32_t out_dtype, int64_t ldo, int64_t* shape_out, void* stream);
+
+/* Dynamic group quantisation (CT compute_dynamic_scales_and_zp + fake_quantize with strategy "group" or
+ * "tensor_group", symmetric, reached through forward_quantize): each run of `group` columns gets the scale of its own
+ * largest magnitude (llmc_calculate_qparams' rule for scale_mode; NVFP4 under global_scale) and is fake-quantised
+ * with it, in one pass.  16-bit input (bf16 for MXFP4), group a power of two in [16, 1024] that divides K, ints of 4
+ * or 8 bits, 16-byte aligned rows; x_dtype output. */
+int llmc_dynamic_group_quantize(const void* x, int32_t x_dtype, int64_t N, int64_t K, int64_t ldx, int64_t group,
+                                int32_t fmt, int32_t num_bits, int32_t scale_mode, const float* global_scale,
+                                void* out, int64_t ldo, void* stream);
+
 /* Dynamic per-token quantisation (CT compute_dynamic_scales_and_zp + fake_quantize,
  * strategy "token", reached through forward_quantize, calibration.py:178-183):
  * per row absmax -> scale = absmax/(range/2) in the row dtype -> quantise.
- * out_mode FAKEQUANT (row dtype) or CODES (bytes). scale_out: [N] in the row dtype. */
+ * out_mode FAKEQUANT (row dtype) or CODES (bytes). scale_out: [N] in the row dtype, or NULL. */
 int llmc_dynamic_per_token_quantize(const void* x, int32_t x_dtype, int64_t N, int64_t K,
                                     int64_t ldx, int32_t fmt, int32_t num_bits, int32_t out_mode,
                                     void* out, int64_t ldo, void* scale_out, void* stream);

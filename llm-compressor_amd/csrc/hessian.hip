@@ -235,7 +235,10 @@ struct GroupArgs {
 struct NoGroup {
   static constexpr bool grouped = false;
   static constexpr bool segmented = false;
+  float* count;  // the hook's sample count, raised by `add` beside the product (NULL: none): a launch of its own
+  float add;     // took 5 us of a 70 us call
 };
+__global__ void add_count_kernel(float* count, float add) { *count += add; }
 // One problem whose token rows lie in up to SEG_MAX separate buffers of seg_tokens rows each (a
 // multiple of the slab depth, so no slab straddles two buffers; the last one may hold fewer): the
 // calibration batches as the forward hook received them, without first copying them together.
@@ -258,6 +261,8 @@ __global__ __launch_bounds__(256) void hessian_syrk_kernel(float* __restrict__ H
     if (Tfull <= 0) return;
     H = grp.H[blockIdx.y];
     Xfull = grp.X[blockIdx.y];
+  } else if constexpr (!GRP::segmented) {
+    if (grp.count && blockIdx.x == 0 && threadIdx.x == 0) *grp.count += grp.add;
   }
   constexpr int RT = BT / 32;  // token rows per thread per panel
   constexpr int GI = BT / 8;   // 8-feature groups per panel
@@ -685,7 +690,7 @@ __global__ void zero_u32_kernel(unsigned* p, int n) {
 
 template <int BT, int DT>
 int launch(const Choice& c, float* H, int64_t ldh, const void* X, int64_t ldx, int64_t T, int64_t K, float alpha,
-           int flags, float* ws, unsigned* pace, hipStream_t st, const SegArgs* segs = nullptr) {
+           int flags, float* ws, unsigned* pace, hipStream_t st, const SegArgs* segs = nullptr, NoGroup single = {}) {
   const int nb = (int)((K + BT - 1) / BT);
   const bool aligned = segs || ((K % 8 == 0) && (ldx % 8 == 0) && (((uintptr_t)X & 15) == 0));
   const int sym = (flags & LLMC_HESSIAN_ASSUME_SYMMETRIC) ? 1 : 0;
@@ -717,7 +722,7 @@ int launch(const Choice& c, float* H, int64_t ldh, const void* X, int64_t ldx, i
                        (int)K, alpha, sym, nb, c.plan, ws, *segs, pace);
   } else {
     hipLaunchKernelGGL(kern, dim3(c.grid), dim3(256), smem, st, H, ldh, (const uint16_t*)X, ldx, (int)T,
-                       (int)K, alpha, sym, nb, c.plan, ws, NoGroup{}, pace);
+                       (int)K, alpha, sym, nb, c.plan, ws, single, pace);
   }
   LLMC_LAUNCH_STATUS();
   if (c.nsplit_tiles > 0) {
@@ -742,9 +747,20 @@ extern "C" int64_t llmc_hessian_workspace_bytes(int64_t T, int64_t K) {
 extern "C" int llmc_hessian_accumulate(float* H, int64_t ldh, const void* X, int64_t ldx, int64_t T,
                                        int64_t K, int32_t x_dtype, float alpha, int32_t flags,
                                        void* workspace, int64_t workspace_bytes, void* stream) {
+  return llmc_hessian_accumulate_counted(H, ldh, X, ldx, T, K, x_dtype, alpha, flags, nullptr, 0.f, workspace,
+                                         workspace_bytes, stream);
+}
+
+extern "C" int llmc_hessian_accumulate_counted(float* H, int64_t ldh, const void* X, int64_t ldx, int64_t T,
+                                               int64_t K, int32_t x_dtype, float alpha, int32_t flags, float* count,
+                                               float add, void* workspace, int64_t workspace_bytes, void* stream) {
   LLMC_CHECK_ARG(H != nullptr, 1);
   LLMC_CHECK_ARG(K > 0 && K < (1 << 30) && ldh >= K, 2);
   LLMC_CHECK_ARG(T >= 0 && T < (1ll << 31), 5);
+  if (count && (T == 0 || x_dtype == LLMC_F32)) {
+    hipLaunchKernelGGL(add_count_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream, count, add);
+    LLMC_LAUNCH_STATUS();
+  }
   if (T == 0) return 0;
   LLMC_CHECK_ARG(X != nullptr, 3);
   LLMC_CHECK_ARG(ldx >= K, 4);
@@ -781,11 +797,12 @@ extern "C" int llmc_hessian_accumulate(float* H, int64_t ldh, const void* X, int
   const Choice c = choose(T, K, pace_room ? avail - PACE_BYTES : avail);
   unsigned* pace = pace_room ? (unsigned*)workspace : nullptr;
   float* ws = (float*)((char*)workspace + (pace_room ? PACE_BYTES : 0));
+  const NoGroup one = {count, add};
   if (x_dtype == LLMC_BF16)
-    return c.bt == 256 ? launch<256, LLMC_BF16>(c, H, ldh, X, ldx, T, K, alpha, flags, ws, pace, st)
-                       : launch<128, LLMC_BF16>(c, H, ldh, X, ldx, T, K, alpha, flags, ws, pace, st);
-  return c.bt == 256 ? launch<256, LLMC_F16>(c, H, ldh, X, ldx, T, K, alpha, flags, ws, pace, st)
-                     : launch<128, LLMC_F16>(c, H, ldh, X, ldx, T, K, alpha, flags, ws, pace, st);
+    return c.bt == 256 ? launch<256, LLMC_BF16>(c, H, ldh, X, ldx, T, K, alpha, flags, ws, pace, st, nullptr, one)
+                       : launch<128, LLMC_BF16>(c, H, ldh, X, ldx, T, K, alpha, flags, ws, pace, st, nullptr, one);
+  return c.bt == 256 ? launch<256, LLMC_F16>(c, H, ldh, X, ldx, T, K, alpha, flags, ws, pace, st, nullptr, one)
+                     : launch<128, LLMC_F16>(c, H, ldh, X, ldx, T, K, alpha, flags, ws, pace, st, nullptr, one);
 }
 
 extern "C" int llmc_hessian_accumulate_segments(float* H, int64_t ldh, const void* const* X, int32_t n_seg,
