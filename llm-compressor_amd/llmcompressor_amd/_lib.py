@@ -10,6 +10,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libllmc_amd.so")
+BIND_PATH = os.path.join(_HERE, "libllmc_torch.so")  # the native half of torch_ops.py
 CSRC_DIR = os.path.join(os.path.dirname(_HERE), "csrc")
 
 _lib = None
@@ -27,6 +28,11 @@ def build(jobs: int = 8) -> str:
     global _lib
     _lib = None
     return LIB_PATH
+
+
+def missing_native(*_args, **_kwargs):
+    raise LibraryMissing(f"{BIND_PATH} is not built; run `python -c 'import __graft_entry__ as g; g.build()'` "
+                         "(there is no fallback path)")
 
 
 def lib() -> ctypes.CDLL:
@@ -61,6 +67,12 @@ SIGNATURES = {
     "llmc_sparsegpt_sparsify": [_P, _I32, _I64, _I64, _I64, _P, _I64, _P, ctypes.c_double, _I32, _I32, _I32, _I32, _I32,
                                 _P, _I64, _P, _P, _I64, _P],
     "llmc_hessian_accumulate_segments": [_P, _I64, _P, _I32, _I64, _I64, _I64, _I64, _I32, _F32, _I32, _P, _I64, _P],
+    "llmc_hessian_accumulate_counted": [_P, _I64, _P, _I64, _I64, _I64, _I32, _F32, _I32, _P, _F32, _P, _I64, _P],
+    "llmc_global_scale_workspace_bytes": [],
+    "llmc_global_scale": [_P, _P, _I64, _I32, _I32, _I32, _I32, _P, _P, _I64, _P],
+    "llmc_dynamic_group_quantize": [_P, _I32, _I64, _I64, _I64, _I64, _I32, _I32, _I32, _P, _P, _I64, _P],
+    "llmc_quantize_shaped": [_P, _I32, _I64, _I64, _I64, _P, _I32, _P, _P, _P, _I32, _I32, _I64, _I64, _I64, _I32, _P,
+                             _I32, _I64, _P, _P],
     "llmc_hessian_accumulate": [_P, _I64, _P, _I64, _I64, _I64, _I32, _F32, _I32, _P, _I64, _P],
     "llmc_minmax_groups": [_P, _I32, _I64, _I64, _I64, _I64, _P, _P, _P, _I64, _P],
     "llmc_minmax_blocks": [_P, _I32, _I64, _I64, _I64, _I32, _I32, _P, _P, _P],
@@ -106,6 +118,7 @@ SIGNATURES["llmc_grouped_linear"] = [_P, _I32, _I64, _P, _I64, _I32, _I32, _P, _
 RESTYPES = {
     "llmc_hessian_workspace_bytes": ctypes.c_int64,
     "llmc_minmax_workspace_bytes": ctypes.c_int64,
+    "llmc_global_scale_workspace_bytes": ctypes.c_int64,
     "llmc_gptq_hinv_workspace_bytes": ctypes.c_int64,
     "llmc_mse_workspace_bytes": ctypes.c_int64,
     "llmc_gptq_quantize_workspace_bytes": ctypes.c_int64,

@@ -29,7 +29,7 @@ from ..quantization import (
     QuantizationType,
     is_module_quantized,
 )
-from ..quantization.lifecycle import effective_scale, kernel_format, scale_indexing
+from ..quantization.lifecycle import kernel_format, scale_indexing
 
 __all__ = ["infer_format", "resolve_format", "compress_module", "decompress_weight", "compress_model_state_dict",
            "save_pretrained_compressed", "quantization_config_dict", "CompressionFormat"]
@@ -97,15 +97,25 @@ def resolve_format(scheme: QuantizationScheme, override=None) -> str:
     return fmt
 
 
-def _run(weight, scale, zp, args: QuantizationArgs, mode, g_idx=None, global_scale=None):
+def _run(weight, scale, zp, args: QuantizationArgs, mode, g_idx=None, global_scale=None, shaped=False):
+    """The codes of ``weight``; with ``shaped`` also the int64 tensor of its shape, written by the same launch."""
     fmt, bits = kernel_format(args)
     R, K = weight.shape
     row_div, srow, col_div = scale_indexing(args, R, K)
-    es = effective_scale(scale, args, weight.dtype)
     zpa = None if args.symmetric or zp is None else zp.to(torch.int8)
     if g_idx is not None and bool((g_idx < 0).any()):
         g_idx = None
-    return llmc.quant_pack(weight.contiguous(), es, zpa, fmt, bits, row_div, srow, col_div, mode, g_idx, global_scale)
+    op = llmc.quant_pack_shaped if shaped else llmc.quant_pack
+    return op(weight.contiguous(), scale, zpa, fmt, bits, row_div, srow, col_div, mode, g_idx, global_scale)
+
+
+def _tensor_of(module: torch.nn.Module, name: str) -> Optional[torch.Tensor]:
+    """``module.<name>`` without the failing attribute lookups (a microsecond each) for the names it does not have."""
+    d = module.__dict__
+    for where in (d["_parameters"], d["_buffers"], d):
+        if name in where:
+            return where[name]
+    return getattr(module, name, None) if hasattr(type(module), name) else None
 
 
 def compress_module(module: torch.nn.Module, fmt: Optional[str] = None) -> Dict[str, torch.Tensor]:
@@ -115,16 +125,15 @@ def compress_module(module: torch.nn.Module, fmt: Optional[str] = None) -> Dict[
     fmt = fmt or infer_format(scheme)
     weight = module.weight.data
     scale = module.weight_scale.data
-    zp = getattr(module, "weight_zero_point", None)
+    zp = _tensor_of(module, "weight_zero_point")
     zp = None if zp is None else zp.data
-    gs = getattr(module, "weight_global_scale", None)
+    gs = _tensor_of(module, "weight_global_scale")
     gs = None if gs is None else gs.data.to(torch.float32)
-    g_idx = getattr(module, "weight_g_idx", None)
+    g_idx = _tensor_of(module, "weight_g_idx")
     g_idx = None if g_idx is None else g_idx.data
     out: Dict[str, torch.Tensor] = {}
     if fmt == CompressionFormat.pack_quantized:
-        out["weight_packed"] = _run(weight, scale, zp, args, ops.OUT_PACKED, g_idx)
-        out["weight_shape"] = torch.tensor(list(weight.shape), dtype=torch.int64, device=weight.device)
+        out["weight_packed"], out["weight_shape"] = _run(weight, scale, zp, args, ops.OUT_PACKED, g_idx, shaped=True)
         out["weight_scale"] = scale
         if not args.symmetric and zp is not None and args.strategy not in (QuantizationStrategy.GROUP,
                                                                            QuantizationStrategy.CHANNEL):
@@ -156,7 +165,7 @@ def compress_module(module: torch.nn.Module, fmt: Optional[str] = None) -> Dict[
     else:
         raise ValueError(f"unsupported compression format {fmt}")
     for name in ("input_scale", "input_zero_point", "input_global_scale", "output_scale", "output_zero_point"):
-        t = getattr(module, name, None)
+        t = _tensor_of(module, name)
         if t is None:
             continue
         if name.endswith("zero_point"):  # zero points of symmetric arguments are all zero and are not stored
@@ -164,8 +173,9 @@ def compress_module(module: torch.nn.Module, fmt: Optional[str] = None) -> Dict[
             if act is None or act.symmetric:
                 continue
         out[name] = t.data
-    if getattr(module, "bias", None) is not None:
-        out["bias"] = module.bias.data
+    bias = _tensor_of(module, "bias")
+    if bias is not None:
+        out["bias"] = bias.data
     return out
 
 

@@ -36,21 +36,25 @@ def make_empty_hessian(module: torch.nn.Module, device: torch.device | None = No
 def accumulate_hessian(inp: torch.Tensor, module: torch.nn.Module, H: torch.Tensor | None,
                        num_samples: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     """H += 2 X^T X in place; num_samples += batch entries (not tokens)."""
-    inp = inp.to(device=H.device)
-    if len(inp.shape) == 2:
-        inp = inp.unsqueeze(0)
-    elif len(inp.shape) > 3:
-        inp = inp.reshape(inp.shape[0], -1, inp.shape[-1])
-    num_added = inp.shape[0]
+    if inp.device != H.device:
+        inp = inp.to(device=H.device)
+    num_added = 1 if inp.ndim == 2 else inp.shape[0]
     if isinstance(module, torch.nn.Conv2d):
+        if inp.ndim == 2:
+            inp = inp.unsqueeze(0)
+        elif inp.ndim > 3:
+            inp = inp.reshape(inp.shape[0], -1, inp.shape[-1])
         unfold = torch.nn.Unfold(module.kernel_size, dilation=module.dilation, padding=module.padding,
                                  stride=module.stride)
         inp = unfold(inp).permute([1, 0, 2]).flatten(1).t()
-    else:  # Linear / Conv1D: rows are tokens
-        inp = inp.reshape((-1, inp.shape[-1]))
+    # Linear / Conv1D: rows are tokens
+    if (isinstance(num_samples, torch.Tensor) and num_samples.dtype == torch.float32 and num_samples.numel() == 1
+            and num_samples.device == H.device):
+        ops.hessian_accumulate_(H, inp, count=num_samples, samples=num_added)
+        return H, num_samples
     num_samples += num_added
-    if inp.shape[0] > 0:
-        llmc.hessian_accum_(H, inp.contiguous(), 2.0, True)
+    if inp.numel() > 0:
+        ops.hessian_accumulate_(H, inp)
     return H, num_samples
 
 

@@ -81,7 +81,7 @@ class HessianStagingMixin:
         st = self._staged.get(module)
         if st is None or st[1] == 0:
             return
-        llmc.hessian_accum_(self._hessians[module], st[0].narrow(0, 0, st[1]), 2.0, True)
+        ops.hessian_accumulate_(self._hessians[module], st[0].narrow(0, 0, st[1]))
         self._num_samples[module] += st[2]
         st[1] = 0
         st[2] = 0

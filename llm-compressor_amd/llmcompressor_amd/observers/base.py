@@ -8,6 +8,7 @@ global_scale}``, ``get_global_scale``, ``delete_statistics``, ``Observer.registe
 """
 from __future__ import annotations
 
+import functools
 from typing import Dict, List, Optional, Tuple, TypedDict
 
 import torch
@@ -15,12 +16,27 @@ import torch
 from .. import ops
 from ..torch_ops import llmc
 from ..quantization import QuantizationArgs, QuantizationStrategy, calculate_qparams, generate_gparam
+from ..quantization.lifecycle import kernel_format, scale_mode
 from .fusion import FusionHandler
 from .helpers import flatten_for_calibration
 
 __all__ = ["Observer", "MinMaxTuple", "QParamsDict"]
 
 MinMaxTuple = Tuple[torch.Tensor, torch.Tensor]
+
+
+def _without_grad(fn):
+    """``torch.no_grad()`` around ``fn``, entered only where gradients are on (calibration runs without them, and
+    entering it again takes 2 us)."""
+
+    @functools.wraps(fn)
+    def wrapped(*args, **kwargs):
+        if torch.is_grad_enabled():
+            with torch.no_grad():
+                return fn(*args, **kwargs)
+        return fn(*args, **kwargs)
+
+    return wrapped
 
 
 class QParamsDict(TypedDict, total=False):
@@ -39,7 +55,7 @@ def _observed_layout(value: torch.Tensor, base_name: str, args: QuantizationArgs
     s = args.strategy
     if base_name == "weight":
         w = value if value.is_contiguous() else value.contiguous()
-        w2 = w.reshape(-1, w.shape[-1])
+        w2 = w if w.ndim == 2 else w.reshape(-1, w.shape[-1])
         if s == S.TENSOR:
             return ("groups", w2.reshape(1, -1), w2.numel()), (1,)
         if s == S.CHANNEL:
@@ -122,7 +138,8 @@ class Observer(torch.nn.Module):
 
     @property
     def has_statistics(self) -> bool:
-        return all(hasattr(self, a) for a in self._stats_attrs)
+        own = self.__dict__  # a failing lookup through Module.__getattr__ costs as much as the launch's arguments
+        return all(a in own or hasattr(self, a) for a in self._stats_attrs)
 
     @property
     def is_weight_obs(self) -> bool:
@@ -138,14 +155,15 @@ class Observer(torch.nn.Module):
             mn, mx = llmc.minmax_observe_blocks(t, *p)
         else:
             mn, mx = llmc.minmax_observe_strided(t, *p)
-        return mn.reshape(shape), mx.reshape(shape)
+        return (mn, mx) if mn.shape == shape else (mn.reshape(shape), mx.reshape(shape))
 
     def compute_min_max(self, value: torch.Tensor) -> MinMaxTuple:
         return self._min_max_kernel(value)
 
     def update_statistics(self, min_vals: torch.Tensor, max_vals: torch.Tensor) -> None:
         """Fold a fresh (min, max) into the running statistics (memoryless: replace)."""
-        self.min_vals, self.max_vals = min_vals, max_vals
+        own = self.__dict__  # plain tensors: nothing for Module.__setattr__ to register
+        own["min_vals"], own["max_vals"] = min_vals, max_vals
 
     def update_statistics_from_observed(self, observed: torch.Tensor) -> None:
         """Reference entry point: ``observed`` is already flattened to (num_observations, *qparam_shape, group)."""
@@ -173,7 +191,7 @@ class Observer(torch.nn.Module):
         all_stats = self.fusion_handler.get_fused_statistics()
         return generate_gparam([(s["min_vals"], s["max_vals"]) for s in all_stats])
 
-    @torch.no_grad()
+    @_without_grad
     def get_qparams(self) -> QParamsDict:
         assert self.has_statistics, "No statistics available. Call observer(value) first."
         global_scale = self.get_global_scale()
@@ -183,7 +201,41 @@ class Observer(torch.nn.Module):
         self.delete_statistics()
         return {"scale": scale, "zero_point": zero_point, "global_scale": global_scale}
 
-    @torch.no_grad()
+    @_without_grad
+    def qparams_into(self, scale: torch.Tensor, zero_point: Optional[torch.Tensor],
+                     global_scale: Optional[torch.Tensor]) -> bool:
+        """``get_qparams`` written straight into a module's parameters (device tensors; the scale parameter may hold
+        stored codes), without the temporaries and copies in between.  False, with nothing done, where the
+        parameters' shapes or dtypes ask for the conversions of the general path."""
+        if type(self).get_qparams is not Observer.get_qparams or type(self).get_global_scale is not Observer.get_global_scale:
+            return False
+        args, mn, mx = self.args, self.min_vals, self.max_vals
+        grouped = args.strategy == QuantizationStrategy.TENSOR_GROUP
+        mode = scale_mode(args, grouped)
+        if mode == ops.SCALE_PLAIN:
+            fits = scale.dtype == mn.dtype
+        elif mode == ops.SCALE_NVFP4:
+            fits = scale.dtype in (torch.float8_e4m3fn, torch.float32)
+        else:
+            fits = scale.dtype == torch.uint8 and mn.dtype == torch.bfloat16
+        if not (fits and scale.is_cuda and scale.shape == mn.shape and scale.is_contiguous()):
+            return False
+        if zero_point is not None and not (
+                zero_point.device == scale.device and zero_point.shape == mn.shape and zero_point.is_contiguous()
+                and (zero_point.dtype == torch.int8 or (args.symmetric and zero_point.element_size() == 1))):
+            return False
+        if grouped:
+            if global_scale is None or global_scale.dtype != torch.float32 or global_scale.shape != (1,):
+                return False
+            stats = self.fusion_handler.get_fused_statistics()
+            llmc.global_scale_into_([s["min_vals"] for s in stats], [s["max_vals"] for s in stats], global_scale)
+        fmt, bits = kernel_format(args)
+        llmc.qparams_into_(mn, mx, scale, zero_point, fmt, bits, bool(args.symmetric), mode,
+                           global_scale if mode == ops.SCALE_NVFP4 else None)
+        self.delete_statistics()
+        return True
+
+    @_without_grad
     def forward(self, observed: torch.Tensor) -> "Observer":
         if observed.numel() == 0:
             return self
@@ -191,7 +243,8 @@ class Observer(torch.nn.Module):
             return self
         mn, mx = self.compute_min_max(observed)
         self.update_statistics(mn, mx)
-        self.fusion_handler.get_fused_statistics()
+        if self.fusion_handler.is_fused:
+            self.fusion_handler.get_fused_statistics()
         return self
 
     def sync_activation_stats(self) -> list:
@@ -202,8 +255,11 @@ class Observer(torch.nn.Module):
         if check_fused:
             self.fusion_handler.maybe_delete_statistics()
         else:
+            own = self.__dict__
             for attr in self._stats_attrs:
-                if hasattr(self, attr):
+                if attr in own:
+                    del own[attr]
+                elif hasattr(self, attr):
                     delattr(self, attr)
 
     def get_statistics(self) -> dict[str, torch.Tensor]:

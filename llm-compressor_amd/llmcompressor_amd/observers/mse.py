@@ -48,7 +48,7 @@ class MemorylessMSEObserver(Observer):
             mn, mx = llmc.mse_observe_blocks(t, p[0], p[1], fmt, bits, self.args.symmetric, mode, **kw)
         else:
             mn, mx = llmc.mse_observe_strided(t, *p, fmt, bits, self.args.symmetric, mode, **kw)
-        return mn.reshape(shape), mx.reshape(shape)
+        return (mn, mx) if mn.shape == shape else (mn.reshape(shape), mx.reshape(shape))
 
     def _rows(self, rows2d):
         fmt, bits = kernel_format(self.args)

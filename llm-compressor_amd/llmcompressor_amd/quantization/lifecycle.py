@@ -204,14 +204,27 @@ def _run_quantize(x, scale, zero_point, args: QuantizationArgs, out_mode, g_idx=
     row_div, srow, col_div = scale_indexing(args, rows, cols)
     if args.strategy == QuantizationStrategy.TENSOR and scale.numel() != 1:
         raise ValueError("tensor strategy expects a single scale")
-    es = effective_scale(scale, args, x.dtype)
     zp = None
     if zero_point is not None and not args.symmetric:
         zp = zero_point.to(torch.int8)
-    out = llmc.quant_pack(x2, es, zp, fmt, bits, row_div, srow, col_div, out_mode, g_idx, global_scale)
+    out = llmc.quant_pack(x2, scale, zp, fmt, bits, row_div, srow, col_div, out_mode, g_idx, global_scale)
     if out_mode == ops.OUT_PACKED:
         return out
     return out.reshape(shape)
+
+
+def _fused_group_mode(x2: torch.Tensor, args: QuantizationArgs, global_scale) -> Optional[int]:
+    """The scale mode of llmc_dynamic_group_quantize when it takes these arguments, else None: symmetric groups of a
+    power of two between 16 and 1024 columns of 16-bit values, integers of 4 or 8 bits."""
+    g = args.group_size
+    if not args.symmetric or g < 16 or g > 1024 or g & (g - 1) or x2.data_ptr() % 16:
+        return None
+    if args.type == QuantizationType.INT and args.num_bits not in (4, 8):
+        return None
+    mode = scale_mode(args, global_scale is not None)
+    if x2.dtype != torch.bfloat16 and (x2.dtype != torch.float16 or mode == ops.SCALE_MXFP4):
+        return None
+    return mode
 
 
 def fake_quantize(x, scale, zero_point, args: QuantizationArgs, g_idx=None, global_scale=None):
@@ -230,11 +243,10 @@ def forward_quantize(module: Module, value: torch.Tensor, base_name: str, args: 
         return value
     if args.dynamic is True and args.strategy == QuantizationStrategy.TOKEN:
         fmt, bits = kernel_format(args)
+        if args.symmetric and bits == 8:  # the fused kernel: row absmax, scale and fake-quant in one pass
+            return llmc.dynamic_token_quantize(value, fmt, bits)
         x2, shape = _as_2d(value)
         x2 = x2.contiguous()
-        if args.symmetric and bits == 8:  # the fused kernel: row absmax, scale and fake-quant in one pass
-            out, _ = llmc.fp8_dynamic_per_token(x2, fmt, bits)
-            return out.reshape(shape)
         # other widths and asymmetric ranges: row min/max, qparams and fake-quant as separate kernels
         mn, mx = llmc.minmax_observe(x2, x2.shape[1])
         scale, zp = calculate_qparams(mn, mx, args)
@@ -251,6 +263,11 @@ def forward_quantize(module: Module, value: torch.Tensor, base_name: str, args: 
             if cols % args.group_size != 0:
                 raise ValueError(f"dynamic group quantization: last dimension {cols} is not a multiple of the "
                                  f"group size {args.group_size}")
+            mode = _fused_group_mode(x2, args, gs)
+            if mode is not None:  # group absmax, scale and fake-quant in one pass
+                fmt, bits = kernel_format(args)
+                return llmc.dynamic_group_quantize(value, args.group_size, fmt, bits, mode,
+                                                   gs if mode == ops.SCALE_NVFP4 else None)
             mn, mx = llmc.minmax_observe(x2, args.group_size)
         elif args.strategy == QuantizationStrategy.TENSOR:
             # one group holding every element: the split reduction of the row kernels fills the chip

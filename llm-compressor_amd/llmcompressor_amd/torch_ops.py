@@ -1,7 +1,9 @@
 """``torch.ops.llmc.*``: the C ABI of ``libllmc_amd.so`` registered with the torch dispatcher.
 
-Every op is a thin shim: the registered implementation (``ops.py``) extracts ``data_ptr``, sizes, strides and
-the current HIP stream from its tensor arguments and calls one plain ``extern "C"`` function of the library.
+Every op is a thin shim: the registered implementation extracts ``data_ptr``, sizes, strides and the current HIP
+stream from its tensor arguments and calls one plain ``extern "C"`` function of the library.  The ops of the short
+calls (observers, scales, quantise / pack, one Hessian batch) are implemented natively in ``csrc/torch_bind.cpp``,
+whose host time per call is a third of the interpreter's; the others are the functions of ``ops.py``.
 The ops are registered for the CUDA (= HIP on ROCm) dispatch key only.  There is no CPU implementation on
 purpose: a call with host tensors fails in the dispatcher ("could not run 'llmc::...' with arguments from the
 'CPU' backend") instead of silently computing somewhere else.
@@ -16,10 +18,12 @@ Seams of the reference that the ops stand behind (src/llmcompressor/...):
 """
 from __future__ import annotations
 
-from typing import List, Optional
+import os
+from typing import List
 
 import torch
 
+from . import _lib
 from . import ops as _impl
 
 NAMESPACE = "llmc"
@@ -30,18 +34,18 @@ _cuda = torch.library.Library(NAMESPACE, "IMPL", "CUDA")
 OP_NAMES: List[str] = []
 
 
-def _register(schema: str, fn) -> None:
+def _register(schema: str, fn=None) -> None:
+    """Define an op; without ``fn`` its implementation is in the native library."""
     name = schema.split("(", 1)[0]
     _defs.define(schema)
-    _cuda.impl(name, fn)
+    if fn is None and not os.path.exists(_lib.BIND_PATH):
+        fn = _lib.missing_native
+    if fn is not None:
+        _cuda.impl(name, fn)
     OP_NAMES.append(name)
 
 
 # ---- GPTQ Hessian --------------------------------------------------------------------------------------------
-
-def _hessian_accum_(H, X, alpha=2.0, assume_symmetric=True):
-    _impl.hessian_accumulate_(H, X, alpha=alpha, assume_symmetric=assume_symmetric)
-
 
 def _hessian_accum_segments_(H, Xs, alpha=2.0, assume_symmetric=True):
     _impl.hessian_accumulate_segments_(H, list(Xs), alpha=alpha, assume_symmetric=assume_symmetric)
@@ -51,7 +55,10 @@ def _hessian_accum_grouped_(Hs, Xs, alpha=2.0, assume_symmetric=True):
     _impl.hessian_accumulate_grouped_(list(Hs), list(Xs), alpha=alpha, assume_symmetric=assume_symmetric)
 
 
-_register("hessian_accum_(Tensor(a!) H, Tensor X, float alpha=2.0, bool assume_symmetric=True) -> ()", _hessian_accum_)
+_register("hessian_accum_(Tensor(a!) H, Tensor X, float alpha=2.0, bool assume_symmetric=True, "
+          "bool use_workspace=True) -> ()")
+_register("hessian_accum_counted_(Tensor(a!) H, Tensor X, Tensor(b!) count, float samples, float alpha=2.0, "
+          "bool assume_symmetric=True, bool use_workspace=True) -> ()")
 _register("hessian_accum_segments_(Tensor(a!) H, Tensor[] Xs, float alpha=2.0, bool assume_symmetric=True) -> ()",
           _hessian_accum_segments_)
 _register("hessian_accum_grouped_(Tensor(a!)[] Hs, Tensor[] Xs, float alpha=2.0, bool assume_symmetric=True) -> ()",
@@ -110,36 +117,6 @@ _register("sparsegpt_sparsify(Tensor W, Tensor Hinv, float sparsity, int prune_n
 
 # ---- observers ---------------------------------------------------------------------------------------------------
 
-def _minmax_observe(W, group):
-    return _impl.minmax_groups(W, group)
-
-
-def _minmax_observe_blocks(W, block_h, block_w):
-    return _impl.minmax_blocks(W, block_h, block_w)
-
-
-def _minmax_observe_strided(x, n0, n1, group, stride0, stride1):
-    return _impl.minmax_strided(x, n0, n1, group, stride0, stride1)
-
-
-def _mse_observe(W, group, fmt, num_bits, symmetric, scale_mode=0, maxshrink=0.20, patience=5, grid=100.0, norm=2.4,
-                 expand=1.0):
-    return _impl.mse_observe_groups(W, group, fmt, num_bits, symmetric, scale_mode, maxshrink=maxshrink,
-                                    patience=patience, grid=grid, norm=norm, expand=expand)
-
-
-def _mse_observe_blocks(W, block_h, block_w, fmt, num_bits, symmetric, scale_mode=0, maxshrink=0.20, patience=5,
-                        grid=100.0, norm=2.4, expand=1.0):
-    return _impl.mse_observe_blocks(W, block_h, block_w, fmt, num_bits, symmetric, scale_mode, maxshrink=maxshrink,
-                                    patience=patience, grid=grid, norm=norm, expand=expand)
-
-
-def _mse_observe_strided(x, n0, n1, group, stride0, stride1, fmt, num_bits, symmetric, scale_mode=0, maxshrink=0.20,
-                         patience=5, grid=100.0, norm=2.4, expand=1.0):
-    return _impl.mse_observe_strided(x, n0, n1, group, stride0, stride1, fmt, num_bits, symmetric, scale_mode,
-                                     maxshrink=maxshrink, patience=patience, grid=grid, norm=norm, expand=expand)
-
-
 def _sumsq_accum_(total, x):
     _impl.sumsq_accumulate_(total, x)
 
@@ -170,14 +147,13 @@ _SEARCH = ("int fmt, int num_bits, bool symmetric, int scale_mode=0, float maxsh
            "float grid=100.0, float norm=2.4, float expand=1.0) -> (Tensor min, Tensor max)")
 _ISEARCH = ("float maxshrink=0.95, int patience=5, float grid=20.0, float norm=3.0, float expand=1.0) "
             "-> (Tensor min, Tensor max)")
-_register("minmax_observe(Tensor W, int group) -> (Tensor min, Tensor max)", _minmax_observe)
-_register("minmax_observe_blocks(Tensor W, int block_h, int block_w) -> (Tensor min, Tensor max)", _minmax_observe_blocks)
+_register("minmax_observe(Tensor W, int group) -> (Tensor min, Tensor max)")
+_register("minmax_observe_blocks(Tensor W, int block_h, int block_w) -> (Tensor min, Tensor max)")
 _register("minmax_observe_strided(Tensor x, int n0, int n1, int group, int stride0, int stride1) "
-          "-> (Tensor min, Tensor max)", _minmax_observe_strided)
-_register("mse_observe(Tensor W, int group, " + _SEARCH, _mse_observe)
-_register("mse_observe_blocks(Tensor W, int block_h, int block_w, " + _SEARCH, _mse_observe_blocks)
-_register("mse_observe_strided(Tensor x, int n0, int n1, int group, int stride0, int stride1, " + _SEARCH,
-          _mse_observe_strided)
+          "-> (Tensor min, Tensor max)")
+_register("mse_observe(Tensor W, int group, " + _SEARCH)
+_register("mse_observe_blocks(Tensor W, int block_h, int block_w, " + _SEARCH)
+_register("mse_observe_strided(Tensor x, int n0, int n1, int group, int stride0, int stride1, " + _SEARCH)
 _register("sumsq_accum_(Tensor(a!) total, Tensor x) -> ()", _sumsq_accum_)
 _register("sumsq_accum_noalloc_(Tensor(a!) total, Tensor x) -> ()", _sumsq_accum_noalloc_)
 _register("imatrix_observe(Tensor W, int group, int fmt, int num_bits, bool symmetric, int scale_mode=0, "
@@ -190,32 +166,32 @@ _register("imatrix_observe_strided(Tensor x, int n0, int n1, int group, int stri
 
 # ---- qparams, quantise, pack ---------------------------------------------------------------------------------------
 
-def _global_scale(mins, maxs):
-    return _impl.global_scale_from_stats(list(zip(mins, maxs)))
-
-
-def _qparams(min_vals, max_vals, fmt, num_bits, symmetric, scale_mode=0, global_scale=None, want_codes=False):
-    return _impl.calculate_qparams(min_vals, max_vals, fmt, num_bits, symmetric, scale_mode, global_scale, want_codes)
-
-
-def _quant_pack(x, scale, zero_point, fmt, num_bits, row_div, scale_row_stride, col_div, out_mode=0, g_idx=None,
-                global_scale=None, out_dtype=None):
-    return _impl.quantize(x, scale, zero_point, fmt, num_bits, row_div, scale_row_stride, col_div, out_mode=out_mode,
-                          g_idx=g_idx, global_scale=global_scale, out_dtype=out_dtype)
-
-
-def _fp8_dynamic_per_token(X, fmt=1, num_bits=8, out_mode=0):
-    return _impl.dynamic_per_token_quantize(X, fmt, num_bits, out_mode)
-
-
-_register("global_scale(Tensor[] mins, Tensor[] maxs) -> Tensor", _global_scale)
+_register("global_scale(Tensor[] mins, Tensor[] maxs) -> Tensor")
+_register("global_scale_into_(Tensor[] mins, Tensor[] maxs, Tensor(a!) out) -> ()")
 _register("qparams(Tensor min_vals, Tensor max_vals, int fmt, int num_bits, bool symmetric, int scale_mode=0, "
-          "Tensor? global_scale=None, bool want_codes=False) -> (Tensor scale, Tensor zero_point, Tensor? scale_code)",
-          _qparams)
-_register("quant_pack(Tensor x, Tensor scale, Tensor? zero_point, int fmt, int num_bits, int row_div, "
-          "int scale_row_stride, int col_div, int out_mode=0, Tensor? g_idx=None, Tensor? global_scale=None, "
-          "ScalarType? out_dtype=None) -> Tensor", _quant_pack)
-_register("fp8_dynamic_per_token(Tensor X, int fmt=1, int num_bits=8, int out_mode=0) -> (Tensor out, Tensor scale)",
-          _fp8_dynamic_per_token)
+          "Tensor? global_scale=None, bool want_codes=False) -> (Tensor scale, Tensor zero_point, Tensor? scale_code)")
+_register("qparams_into_(Tensor min_vals, Tensor max_vals, Tensor(a!) scale, Tensor(b!)? zero_point, int fmt, "
+          "int num_bits, bool symmetric, int scale_mode=0, Tensor? global_scale=None) -> ()")
+_QUANT = ("Tensor x, Tensor scale, Tensor? zero_point, int fmt, int num_bits, int row_div, int scale_row_stride, "
+          "int col_div, int out_mode=0, Tensor? g_idx=None, Tensor? global_scale=None")
+_register("quant_pack(" + _QUANT + ", ScalarType? out_dtype=None) -> Tensor")
+_register("quant_pack_shaped(" + _QUANT + ") -> (Tensor out, Tensor shape)")
+_register("fp8_dynamic_per_token(Tensor X, int fmt=1, int num_bits=8, int out_mode=0) -> (Tensor out, Tensor scale)")
+_register("dynamic_token_quantize(Tensor x, int fmt, int num_bits) -> Tensor")
+_register("dynamic_group_quantize(Tensor x, int group, int fmt, int num_bits, int scale_mode=0, "
+          "Tensor? global_scale=None) -> Tensor")
 
-llmc = getattr(torch.ops, NAMESPACE)
+if os.path.exists(_lib.BIND_PATH):
+    torch.ops.load_library(_lib.BIND_PATH)
+
+
+class _Ops:
+    """The ops by name, each as its one overload: a packet looks its overload up at every call."""
+
+    def __init__(self):
+        packets = getattr(torch.ops, NAMESPACE)
+        for name in OP_NAMES:
+            setattr(self, name, getattr(packets, name).default)
+
+
+llmc = _Ops()

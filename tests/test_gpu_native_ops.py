@@ -1,0 +1,125 @@
+"""GPU: the one-pass and whole-matrix kernels at the sizes where their indexing can go wrong -- one column chunk, rows
+that are no multiple of 16 columns, the boundaries between the row kernels, ragged blocks, tails of a workgroup --
+against the oracle, or against the separate kernels (themselves tested against it) that they stand in for."""
+import pytest
+import torch
+
+from oracle import qformat as F
+
+pytestmark = pytest.mark.gpu
+
+BIG = 1 << 40
+
+
+def _llmc():
+    from llmcompressor_amd.torch_ops import llmc
+
+    return llmc
+
+
+def _values(rows, cols, dtype=torch.bfloat16, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(rows, cols, generator=g) * torch.logspace(-2, 1, cols)
+    x[rows // 2] = 0.0
+    return x.to(dtype)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 8), (3, 24), (257, 40), (5, 16), (700, 264), (64, 4104), (2, 13320)])
+@pytest.mark.parametrize("scheme", ["int8", "int4", "fp8"])
+def test_rows_of_eight_column_chunks(rows, cols, scheme):
+    """Per-channel codes, packed words and fake-quantised values where K is a multiple of 8, and of 16 or not."""
+    from llmcompressor_amd import ops
+
+    args = F.QArgs(num_bits=8 if scheme != "int4" else 4, type="float" if scheme == "fp8" else "int", strategy="channel")
+    x = _values(rows, cols)
+    scale, zp = F.calculate_qparams(x.amin(1, keepdim=True), x.amax(1, keepdim=True), args)
+    fmt = ops.FMT_FP8 if scheme == "fp8" else ops.FMT_INT
+    for mode, want in ((ops.OUT_FAKEQUANT, F.fake_quantize(x, scale, zp, args)),
+                       (ops.OUT_CODES, F.quantize(x, scale, zp, args, dtype=torch.float8_e4m3fn if scheme == "fp8" else torch.int8))):
+        got = _llmc().quant_pack(x.cuda(), scale.cuda(), None, fmt, args.num_bits, 1, 1, BIG, mode).cpu()
+        assert torch.equal(got.view(torch.uint8), want.to(got.dtype).view(torch.uint8))
+    if scheme != "fp8":
+        from oracle import pack as P
+
+        got, shape = _llmc().quant_pack_shaped(x.cuda(), scale.cuda(), None, fmt, args.num_bits, 1, 1, BIG, ops.OUT_PACKED)
+        assert shape.tolist() == [rows, cols]
+        assert torch.equal(got.cpu(), P.pack_to_int32(F.quantize(x, scale, zp, args, dtype=torch.int8), args.num_bits))
+
+
+@pytest.mark.parametrize("rows,cols,group", [(1, 16, 16), (3, 64, 32), (9, 128, 128), (130, 1024, 1024), (33, 3168, 32),
+                                             (7, 2432, 128), (1, 14336, 128)])
+@pytest.mark.parametrize("kind", ["fp8", "int8", "mxfp4", "nvfp4"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_dynamic_groups_in_one_pass_equal_the_three_kernels(rows, cols, group, kind, dtype):
+    from llmcompressor_amd import ops
+
+    llmc = _llmc()
+    fmt, bits, mode = {"fp8": (ops.FMT_FP8, 8, ops.SCALE_PLAIN), "int8": (ops.FMT_INT, 8, ops.SCALE_PLAIN),
+                       "mxfp4": (ops.FMT_FP4, 4, ops.SCALE_MXFP4), "nvfp4": (ops.FMT_FP4, 4, ops.SCALE_NVFP4)}[kind]
+    x = _values(rows, cols, dtype).cuda()
+    gs = torch.tensor([37.0], device="cuda") if kind == "nvfp4" else None
+    if kind == "mxfp4" and dtype is torch.float16:
+        with pytest.raises(ValueError):
+            llmc.dynamic_group_quantize(x, group, fmt, bits, mode, gs)
+        return
+    mn, mx = llmc.minmax_observe(x, group)
+    scale, _, codes = llmc.qparams(mn, mx, fmt, bits, True, mode, gs, kind == "mxfp4")
+    want = llmc.quant_pack(x, codes if kind == "mxfp4" else scale, None, fmt, bits, 1, cols // group, group,
+                           ops.OUT_FAKEQUANT, None, gs)
+    got = llmc.dynamic_group_quantize(x.view(1, rows, cols), group, fmt, bits, mode, gs)
+    assert got.shape == (1, rows, cols) and torch.equal(got[0], want)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 8), (1, 4096), (3, 8192), (2, 8200), (1030, 1032), (5, 16384), (2, 16392),
+                                       (1, 65536), (4, 100)])
+@pytest.mark.parametrize("kind", ["float", "int"])
+def test_dynamic_tokens_at_the_row_kernels_boundaries(rows, cols, kind):
+    x = _values(rows, cols)
+    args = F.QArgs(num_bits=8, type=kind, strategy="token", dynamic=True)
+    want, _ = F.forward_quantize_dynamic(x.unsqueeze(0), args)
+    got = _llmc().dynamic_token_quantize(x.cuda(), 1 if kind == "float" else 0, 8)
+    assert torch.equal(got.cpu(), want[0])
+
+
+@pytest.mark.parametrize("rows,cols,bh,bw", [(1, 8, 128, 128), (128, 128, 128, 128), (130, 264, 128, 128), (5, 20, 2, 3),
+                                             (300, 1000, 64, 24)])
+def test_block_min_max_on_ragged_edges(rows, cols, bh, bw):
+    x = _values(rows, cols).abs() + 1  # the zero padding of an edge block is its minimum
+    mn, mx = _llmc().minmax_observe_blocks(x.cuda(), bh, bw)
+    p = torch.nn.functional.pad(x, (0, -cols % bw, 0, -rows % bh))
+    p = p.view(p.shape[0] // bh, bh, p.shape[1] // bw, bw)
+    assert torch.equal(mn.cpu(), p.amin((1, 3))) and torch.equal(mx.cpu(), p.amax((1, 3)))
+
+
+@pytest.mark.parametrize("sizes", [(1,), (7,), (131072,), (131080,), (300001, 5), (5, 300001), (5, 9, 200000)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_global_scale_over_arrays_of_any_size(sizes, dtype):
+    g = torch.Generator().manual_seed(len(sizes))
+    stats = []
+    for i, n in enumerate(sizes):
+        mn, mx = -torch.rand(n, generator=g), torch.rand(n, generator=g)
+        (mn if i % 2 else mx)[n - 1] = (-40.0 if i % 2 else 40.0) - i  # the largest magnitude is the last value
+        stats.append((mn.to(dtype), mx.to(dtype)))
+    got = _llmc().global_scale([m.cuda() for m, _ in stats], [m.cuda() for _, m in stats])
+    top = max(max(-mn.min().item(), mx.max().item()) for mn, mx in stats)
+    want = (torch.tensor([top], dtype=dtype).reciprocal() * 2688.0).float()
+    assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.parametrize("scheme", ["W4A16", "W4A16_ASYM", "W8A8", "FP8_BLOCK", "NVFP4A16", "MXFP4A16"])
+def test_parameters_written_in_place_equal_the_observers_own_answer(scheme):
+    from llmcompressor_amd.modifiers.quantization.calibration import initialize_observer, observe, update_qparams
+    from llmcompressor_amd.quantization import initialize_module_for_quantization, preset_name_to_scheme
+
+    module = torch.nn.Linear(512, 96, bias=False, dtype=torch.bfloat16, device="cuda")
+    initialize_module_for_quantization(module, preset_name_to_scheme(scheme, ["Linear"]))
+    initialize_observer(module, "weight")
+    observe(module, "weight")
+    want = module.weight_observer.get_qparams()
+    observe(module, "weight")
+    update_qparams(module, "weight")
+    assert not module.weight_observer.has_statistics
+    for name in ("scale", "zero_point", "global_scale"):
+        if want[name] is not None:
+            got = getattr(module, f"weight_{name}").data
+            assert torch.equal(got.float(), want[name].float()), name
