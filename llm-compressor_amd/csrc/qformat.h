@@ -128,6 +128,19 @@ __device__ __forceinline__ float round16_finite(float f) {
   return (float)(_Float16)f;
 }
 
+// the same from two values packed in the 16-bit type DT; this form saturates at +-6 by itself
+template <int DT>
+__device__ __forceinline__ uint32_t hw_e2m1_pair16(uint32_t w) {
+  if (DT == LLMC_BF16) {
+    bf16x2_t v;
+    __builtin_memcpy(&v, &w, 4);
+    return __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(0u, v, 1.0f, 0) & 0xffu;
+  }
+  f16x2_t v;
+  __builtin_memcpy(&v, &w, 4);
+  return __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(0u, v, 1.0f, 0) & 0xffu;
+}
+
 // ---- division by a value shared by many elements.  The steps are those of the correctly
 // rounded fp32 division sequence (reciprocal with one Newton step, quotient with two residual
 // corrections) with the divisor's part hoisted; they give the IEEE quotient whenever nothing
@@ -195,6 +208,40 @@ __device__ __forceinline__ bool bf16_scale_plain(float s) {
   const float a = fabsf(s);
   return a > 0x1p-30f && a < 0x1p30f;
 }
+
+// ---- x / s rounded to the 16-bit dtype of both, without a guard per element: DT(quot16(x, d)) == DT(x / s) where
+// ValueRange::plain() holds for x and scale_plain() for s.  bf16: the multiply above.  f16 (11-bit significands X, S in
+// [1024, 2047]): the quotient cannot be a rounding midpoint unless that midpoint has fewer bits, in which case it is an
+// fp32 value and the correction below hits it exactly; from every other midpoint it lies at least 2^-23 (relative)
+// away (|2^k X - M S| >= 1 over 2^k X < 2^23), and one residual correction leaves less than that: half an fp32 ulp
+// (2^-24) of the last operation and about 2^-46 of the residual's.
+template <int DT>
+__device__ __forceinline__ float quot16(float x, const FastDiv& d) {
+  const float q = x * d.y;
+  if (DT == LLMC_BF16) return q;
+  return fmaf(fmaf(-d.s, q, x), d.y, q);
+}
+template <int DT>
+__device__ __forceinline__ bool scale_plain(float s) {
+  if (DT == LLMC_BF16) return bf16_scale_plain(s);
+  return s > 0.f && s < 0x1p16f;  // any positive finite f16 value
+}
+// the magnitudes of the values a lane has seen, as 16-bit patterns
+template <int DT>
+struct ValueRange {
+  Bf16Range r = bf16_range_init();
+  __device__ __forceinline__ void add(const uint4& v) {
+    bf16_range_add(r, v.x);
+    bf16_range_add(r, v.y);
+    bf16_range_add(r, v.z);
+    bf16_range_add(r, v.w);
+  }
+  __device__ __forceinline__ void add(uint32_t w) { bf16_range_add(r, w); }
+  __device__ __forceinline__ bool plain() const {
+    if (DT == LLMC_BF16) return bf16_inputs_plain(r);
+    return max((uint32_t)r.mx.x, (uint32_t)r.mx.y) < 0x7c00u;  // f16: finite
+  }
+};
 
 struct QFormat {
   int fmt;   // LLMC_FMT_*
