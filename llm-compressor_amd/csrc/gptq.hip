@@ -12,38 +12,27 @@
 #include <vector>
 
 #include "gemm_f32.h"
+#include "gptq_group.h"
 #include "qformat.h"
 
 namespace {
 
-constexpr int GB = 128;       // widest column block held on chip
-constexpr int GROUP = 4;      // column blocks whose updates of the far columns are applied together
 constexpr int TEAM = 16;      // lanes per row
 constexpr int CPL = GB / TEAM;  // columns per lane (8)
 constexpr int ROWS_PER_WG = 256 / TEAM;
-
-// One problem of a grouped call (llmc_gptq_quantize_grouped); the kernels pick theirs by a grid index and
-// find its work buffers at a fixed stride behind those of problem 0.
-struct GptqItem {
-  const void* weight;
-  const void* scale;
-  const int8_t* zp;
-  const float* gscale;
-  const int32_t* g_idx;
-  void* out;
-};
 
 template <int WDT>
 __global__ __launch_bounds__(256) void gptq_prepare_w_kernel(const void* __restrict__ w, int64_t ldw, int R,
                                                              int K, const int32_t* __restrict__ perm,
                                                              const uint8_t* __restrict__ dead,
-                                                             float* __restrict__ Wf,
+                                                             float* __restrict__ Wf, int64_t ldf,
+                                                             int64_t w_stride = 0,
                                                              const GptqItem* __restrict__ items = nullptr) {
   if (items) {  // grouped: problem blockIdx.z, perm / dead rows of [n,K] arrays
     w = items[blockIdx.z].weight;
     if (perm) perm += (int64_t)blockIdx.z * K;
     if (dead) dead += (int64_t)blockIdx.z * K;
-    Wf += (int64_t)blockIdx.z * R * K;
+    Wf += (int64_t)blockIdx.z * w_stride;
   }
   const int c = blockIdx.x * 256 + threadIdx.x;
   const int r = blockIdx.y;
@@ -51,7 +40,7 @@ __global__ __launch_bounds__(256) void gptq_prepare_w_kernel(const void* __restr
   const int src = perm ? perm[c] : c;
   float v = load_as_f32<WDT>(w, (int64_t)r * ldw + src);
   if (dead && dead[c]) v = 0.f;
-  Wf[(int64_t)r * K + c] = v;
+  Wf[(int64_t)r * ldf + c] = v;
 }
 
 // Row-at-a-time forms of the column gather / scatter for a permuted column order (activation ordering): one
@@ -63,14 +52,15 @@ template <int WDT>
 __global__ __launch_bounds__(1024) void gptq_prepare_w_rows_kernel(const void* __restrict__ w, int64_t ldw, int R,
                                                                   int K, const int32_t* __restrict__ perm,
                                                                   const uint8_t* __restrict__ dead,
-                                                                  float* __restrict__ Wf,
+                                                                  float* __restrict__ Wf, int64_t ldf,
+                                                                  int64_t w_stride,
                                                                   const GptqItem* __restrict__ items) {
   extern __shared__ float rowbuf[];
   if (items) {
     w = items[blockIdx.y].weight;
     perm += (int64_t)blockIdx.y * K;
     if (dead) dead += (int64_t)blockIdx.y * K;
-    Wf += (int64_t)blockIdx.y * R * K;
+    Wf += (int64_t)blockIdx.y * w_stride;
   }
   const int r = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;  // 256 threads, 1024 for rows above 8192 values
   constexpr int BATCH = 8;
@@ -91,12 +81,13 @@ __global__ __launch_bounds__(1024) void gptq_prepare_w_rows_kernel(const void* _
   for (int c = tid; c < K; c += nt) {
     float v = rowbuf[perm[c]];
     if (dead && dead[c]) v = 0.f;
-    Wf[(int64_t)r * K + c] = v;
+    Wf[(int64_t)r * ldf + c] = v;
   }
 }
 
 template <int WDT>
-__global__ __launch_bounds__(1024) void gptq_finalize_rows_kernel(const float* __restrict__ Wf, int R, int K,
+__global__ __launch_bounds__(1024) void gptq_finalize_rows_kernel(const float* __restrict__ Wf, int64_t ldf,
+                                                                 int64_t w_stride, int R, int K,
                                                                  const int32_t* __restrict__ perm,
                                                                  void* __restrict__ out, int64_t ldo,
                                                                  const GptqItem* __restrict__ items) {
@@ -104,7 +95,7 @@ __global__ __launch_bounds__(1024) void gptq_finalize_rows_kernel(const float* _
   if (items) {
     out = items[blockIdx.y].out;
     perm += (int64_t)blockIdx.y * K;
-    Wf += (int64_t)blockIdx.y * R * K;
+    Wf += (int64_t)blockIdx.y * w_stride;
   }
   const int r = blockIdx.x, tid = threadIdx.x, nt = blockDim.x;  // 256 threads, 1024 for rows above 8192 values
   constexpr int BATCH = 8;
@@ -115,7 +106,7 @@ __global__ __launch_bounds__(1024) void gptq_finalize_rows_kernel(const float* _
     for (int b = 0; b < BATCH; ++b) {
       const int c = c0 + b * nt + tid;
       const int cc = c < K ? c : K - 1;
-      v[b] = Wf[(int64_t)r * K + cc];
+      v[b] = Wf[(int64_t)r * ldf + cc];
       dst[b] = perm[cc];
     }
 #pragma unroll
@@ -177,307 +168,6 @@ __device__ __forceinline__ void load_u_block(float* __restrict__ Hs, const float
       const int i = (it0 + b) * (256 / GB) + tid / GB;
       Hs[(it0 + b) * 256 + tid] = (c >= i && c < count) ? v[b] : 0.f;
     }
-  }
-}
-
-struct GptqBlockParams {
-  float* Wf;        // [R,K] fp32 work copy (permuted columns)
-  int R, K;
-  const float* U;   // inverse-Hessian upper factor
-  int64_t ldu;
-  int i1, count;    // block = columns [i1, i1+count)
-  const void* scale;
-  int scale_dt;
-  const int8_t* zp;
-  const float* gscale;
-  const int32_t* g_idx;  // group of each (permuted) column, or NULL
-  int64_t row_div, srow;
-  int fmt, bits;
-  int sd;           // dtype the dequantised value is formed in
-  float* E;         // scaled errors of this block, row stride ldE
-  int ldE;
-  float* loss_rows; // [R]
-  // grouped call: problem blockIdx.y takes scale / zp / gscale / g_idx from items and its Wf, U, E and
-  // loss rows at these strides (in elements)
-  const GptqItem* items;
-  int64_t u_stride;
-};
-
-// Layout of the quantiser's block kernel: a row is spread over a team of QTEAM lanes (one DPP quad), each
-// holding QCPL columns of the block in registers as QNCH runs of QG neighbouring columns; run j of lane t
-// covers columns j*QCW + t*QG .. +QG-1.  The lane that owns a run quantises its QG columns by itself (the
-// serial chain of a row never crosses lanes inside a run), then the QG scaled errors are broadcast to the team
-// once and every lane applies them, in column order, to the runs that are still open.
-// Two team sizes are built.  Four lanes per row (one DPP quad, 32 columns per lane, 64 rows per workgroup) is the
-// layout for many rows: few waves, each doing as little redundant work as possible.  Sixteen lanes per row (8
-// columns per lane, 16 rows per workgroup) spreads a problem of a few thousand rows over every CU, one wave per
-// SIMD, and each wave applies a run's errors to two runs per lane instead of eight: the per-block time is bound
-// by one wave's instruction issue, so it falls with the instruction count.  Both apply the same operations to
-// every element in the same order, so they give the same bits.
-constexpr int QG = 4;              // neighbouring columns per run
-template <int TEAM>
-struct QLayout {
-  static constexpr int QTEAM = TEAM;
-  static constexpr int QCPL = GB / TEAM;   // columns per lane
-  static constexpr int QNCH = QCPL / QG;   // runs per lane
-  static constexpr int QCW = TEAM * QG;    // columns per round of the team
-  static constexpr int ROWS_PER_WG = 256 / TEAM;
-};
-// rows (of all problems of a launch) up to which the sixteen-lane layout is used
-constexpr int64_t Q_WIDE_TEAM_MAX_ROWS = 8192;
-
-// ---- divisions of the column loop.  x / s goes through the hoisted reciprocal y of s (see make_fastdiv():
-// the steps of the correctly rounded division with the divisor's part taken out).  The short form gives the
-// IEEE quotient while |q| stays in [2^-40, 2^100) or both x and q are zero; `worst` collects, without a
-// branch, how far outside that window any quotient of a run fell, and the caller redoes the run with plain
-// divisions when it did.  A divisor outside make_fastdiv()'s range has a NaN reciprocal, which lands outside
-// the window as well.
-constexpr uint32_t QDIV_LO = 0x2b800000u;  // bits of 2^-40
-constexpr uint32_t QDIV_SPAN = 0x71800000u - QDIV_LO;  // up to 2^100
-__device__ __forceinline__ float shared_reciprocal(float s) {
-  const FastDiv d = make_fastdiv(s);
-  return d.ok ? d.y : __builtin_nanf("");
-}
-template <bool EXACT>
-__device__ __forceinline__ float run_div(float x, float s, float y, uint32_t& worst) {
-  if (EXACT) return x / s;
-  float q = x * y;
-  float r = fmaf(-s, q, x);
-  q = fmaf(r, y, q);
-  r = fmaf(-s, q, x);
-  q = fmaf(r, y, q);
-  const uint32_t qb = __float_as_uint(q) & 0x7fffffffu, xb = __float_as_uint(x) & 0x7fffffffu;
-  const uint32_t t = (qb | xb) == 0u ? QDIV_LO : qb;
-  worst = max(worst, t - QDIV_LO);
-  return q;
-}
-
-template <int SD>
-__device__ __forceinline__ float round_sd(float x) {
-  if (SD == LLMC_BF16) return round16_finite<LLMC_BF16>(x);
-  if (SD == LLMC_F16) return round16_finite<LLMC_F16>(x);
-  return x;
-}
-
-struct QRun {
-  float4 q, e;  // dequantised values and scaled errors of the run's QG columns
-};
-
-// One run of QG neighbouring columns of one row, start to finish inside a lane: column m is quantised, its
-// scaled error err = (w - q) / d is applied to the columns of the run behind it (one fused multiply-subtract
-// per element; the reference rounds the outer product before it subtracts, the fused form keeps the product
-// exact), and so on.  u0..u2 are rows 0..2 of the run's QG x QG diagonal block of U.
-template <int FMT, int SD, bool HAS_ZP, bool EXACT>
-__device__ __forceinline__ QRun gptq_run(float4 w, float4 s, float4 y, float4 z, float4 d, float4 dy,
-                                         float4 u0, float4 u1, float4 u2, const QFormat& f, uint32_t& worst) {
-  QRun o;
-  auto column = [&](float wv, float sc, float yc, float zp, float dc, float dyc, float& q, float& err) {
-    // quantize_value() with the quotient formed by run_div()
-    float v = run_div<EXACT>(wv, sc, yc, worst);
-    v = HAS_ZP ? v + zp : v + 0.0f;
-    const float qc = round_to_grid(v, f);
-    float dq = qc;
-    if (HAS_ZP) dq = round_sd<SD>(dq - zp);
-    q = round_sd<SD>(dq * sc);
-    err = run_div<EXACT>(__fsub_rn(wv, q), dc, dyc, worst);
-  };
-  column(w.x, s.x, y.x, z.x, d.x, dy.x, o.q.x, o.e.x);
-  w.y = fmaf(-o.e.x, u0.y, w.y);
-  w.z = fmaf(-o.e.x, u0.z, w.z);
-  w.w = fmaf(-o.e.x, u0.w, w.w);
-  column(w.y, s.y, y.y, z.y, d.y, dy.y, o.q.y, o.e.y);
-  w.z = fmaf(-o.e.y, u1.z, w.z);
-  w.w = fmaf(-o.e.y, u1.w, w.w);
-  column(w.z, s.z, y.z, z.z, d.z, dy.z, o.q.z, o.e.z);
-  w.w = fmaf(-o.e.z, u2.w, w.w);
-  column(w.w, s.w, y.w, z.w, d.w, dy.w, o.q.w, o.e.w);
-  return o;
-}
-static_assert(QG == 4, "gptq_run() is written out for runs of four columns");
-
-// the rare way round: plain divisions, kept out of line
-template <int FMT, int SD, bool HAS_ZP>
-__device__ __noinline__ QRun gptq_run_exact(float4 w, float4 s, float4 z, float4 d, float4 u0, float4 u1,
-                                            float4 u2, int bits) {
-  const QFormat f = make_qformat(FMT, bits);
-  uint32_t unused = 0;
-  return gptq_run<FMT, SD, HAS_ZP, true>(w, s, s, z, d, d, u0, u1, u2, f, unused);
-}
-
-// the registers of one lane: QCPL columns of one row, their scales, the scales' reciprocals, zero points
-template <bool HAS_ZP, int TEAM>
-struct QLane {
-  static constexpr int QNCH = QLayout<TEAM>::QNCH;
-  float4 w[QNCH], sv[QNCH], yv[QNCH], zv[HAS_ZP ? QNCH : 1];
-};
-
-// Round J of the team: for each lane in turn, its run J is quantised and the errors applied to everything
-// that is still open.  Columns at or past `count` hold w = 0, scale 1, d = 1 and zero rows of U: they
-// quantise to zero with zero error, so only the stores look at `count`.
-template <int J, int FMT, int SD, bool HAS_ZP, int TEAM>
-__device__ __forceinline__ void gptq_round(QLane<HAS_ZP, TEAM>& r, const float* __restrict__ Hs,
-                                           const float* __restrict__ Dd, const float* __restrict__ Dy, int tl,
-                                           int count, bool live, float* __restrict__ wrow,
-                                           float* __restrict__ erow, const QFormat& f, int bits, float& loss) {
-  constexpr int QTEAM = TEAM, QNCH = QLayout<TEAM>::QNCH, QCW = QLayout<TEAM>::QCW;
-#pragma unroll 1
-  for (int li = 0; li < QTEAM; ++li) {
-    const int i0 = J * QCW + li * QG;  // first column of this run
-    if (i0 >= count) break;            // uniform across the workgroup
-    const float* diag = Hs + i0 * GB + i0;
-    const float4 d = *(const float4*)&Dd[i0], dy = *(const float4*)&Dy[i0];
-    const float4 u0 = *(const float4*)&diag[0], u1 = *(const float4*)&diag[GB], u2 = *(const float4*)&diag[2 * GB];
-    const float4 z = r.zv[HAS_ZP ? J : 0];
-    const bool own = tl == li;
-    // every lane runs the chain on its own run J; only the owner's is due, the others' results are dropped
-    uint32_t worst = 0;
-    QRun o = gptq_run<FMT, SD, HAS_ZP, false>(r.w[J], r.sv[J], r.yv[J], z, d, dy, u0, u1, u2, f, worst);
-    if (own && worst >= QDIV_SPAN) o = gptq_run_exact<FMT, SD, HAS_ZP>(r.w[J], r.sv[J], z, d, u0, u1, u2, bits);
-    if (own && live) {
-      if (i0 + 0 < count) wrow[i0 + 0] = o.q.x;
-      if (i0 + 1 < count) wrow[i0 + 1] = o.q.y;
-      if (i0 + 2 < count) wrow[i0 + 2] = o.q.z;
-      if (i0 + 3 < count) wrow[i0 + 3] = o.q.w;
-      erow[i0 + 0] = o.e.x;
-      erow[i0 + 1] = o.e.y;
-      erow[i0 + 2] = o.e.z;
-      erow[i0 + 3] = o.e.w;
-    }
-    const float eb[QG] = {__shfl(o.e.x, li, QTEAM), __shfl(o.e.y, li, QTEAM), __shfl(o.e.z, li, QTEAM),
-                          __shfl(o.e.w, li, QTEAM)};
-#pragma unroll
-    for (int m = 0; m < QG; ++m) {
-      loss += eb[m] * eb[m];  // (w-q)^2 / d^2
-      // this round's run: lanes before the owner see zeros of U, the owner is already done
-      const float eff = own ? 0.f : eb[m];
-      const float* hrow = Hs + (i0 + m) * GB + tl * QG;
-      const float4 h = *(const float4*)&hrow[J * QCW];
-      r.w[J].x = fmaf(-eff, h.x, r.w[J].x);
-      r.w[J].y = fmaf(-eff, h.y, r.w[J].y);
-      r.w[J].z = fmaf(-eff, h.z, r.w[J].z);
-      r.w[J].w = fmaf(-eff, h.w, r.w[J].w);
-#pragma unroll
-      for (int j2 = J + 1; j2 < QNCH; ++j2) {
-        const float4 g = *(const float4*)&hrow[j2 * QCW];
-        r.w[j2].x = fmaf(-eb[m], g.x, r.w[j2].x);
-        r.w[j2].y = fmaf(-eb[m], g.y, r.w[j2].y);
-        r.w[j2].z = fmaf(-eb[m], g.z, r.w[j2].z);
-        r.w[j2].w = fmaf(-eb[m], g.w, r.w[j2].w);
-      }
-    }
-  }
-}
-
-// the block's weights, scales and zero points of one lane; SDT = dtype of the stored scales
-template <int SDT, bool HAS_ZP, int TEAM>
-__device__ __forceinline__ void gptq_load_lane(QLane<HAS_ZP, TEAM>& r, const GptqBlockParams& p, int row, int tl,
-                                               bool live) {
-  constexpr int QCPL = QLayout<TEAM>::QCPL, QNCH = QLayout<TEAM>::QNCH, QCW = QLayout<TEAM>::QCW;
-  const int rowc = live ? row : p.R - 1;  // every load stays inside the arrays; dead lanes are blanked below
-  const float* wsrc = p.Wf + (int64_t)rowc * p.K + p.i1;
-  const int64_t sbase = ((int64_t)rowc / p.row_div) * p.srow;
-  const float gs = p.gscale ? p.gscale[0] : 1.f;
-  float w[QCPL], s[QCPL], zp[QCPL];
-  int gi[QCPL];
-  // three sweeps, each with all its loads in flight: group numbers, then what they index
-#pragma unroll
-  for (int e = 0; e < QCPL; ++e) gi[e] = 0;
-  if (p.g_idx) {
-#pragma unroll
-    for (int e = 0; e < QCPL; ++e) {
-      const int cb = (e / QG) * QCW + tl * QG + (e % QG);
-      gi[e] = p.g_idx[p.i1 + (cb < p.count ? cb : p.count - 1)];
-    }
-  }
-#pragma unroll
-  for (int e = 0; e < QCPL; ++e) {
-    const int cb = (e / QG) * QCW + tl * QG + (e % QG);
-    w[e] = wsrc[cb < p.count ? cb : p.count - 1];
-    s[e] = load_as_f32<SDT>(p.scale, sbase + gi[e]);
-    zp[e] = HAS_ZP ? (float)p.zp[sbase + gi[e]] : 0.f;
-  }
-#pragma unroll
-  for (int e = 0; e < QCPL; ++e) {
-    const int cb = (e / QG) * QCW + tl * QG + (e % QG);
-    if (p.gscale) s[e] = s[e] / gs;
-    if (!live || cb >= p.count) {
-      w[e] = 0.f;
-      s[e] = 1.f;
-      zp[e] = 0.f;
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < QNCH; ++j) {
-    r.w[j] = make_float4(w[j * QG], w[j * QG + 1], w[j * QG + 2], w[j * QG + 3]);
-    r.sv[j] = make_float4(s[j * QG], s[j * QG + 1], s[j * QG + 2], s[j * QG + 3]);
-    r.yv[j] = make_float4(shared_reciprocal(s[j * QG]), shared_reciprocal(s[j * QG + 1]),
-                          shared_reciprocal(s[j * QG + 2]), shared_reciprocal(s[j * QG + 3]));
-    if (HAS_ZP) r.zv[j] = make_float4(zp[j * QG], zp[j * QG + 1], zp[j * QG + 2], zp[j * QG + 3]);
-  }
-  if (!HAS_ZP) r.zv[0] = make_float4(0.f, 0.f, 0.f, 0.f);
-}
-
-template <int FMT, int SD, bool HAS_ZP, int TEAM>
-__global__ __launch_bounds__(256) void gptq_block_kernel(GptqBlockParams p) {
-  constexpr int QTEAM = TEAM, QNCH = QLayout<TEAM>::QNCH, QCW = QLayout<TEAM>::QCW;
-  constexpr int Q_ROWS_PER_WG = QLayout<TEAM>::ROWS_PER_WG;
-  // [GB][GB] slice of U, zero outside the upper triangle; then its diagonal and the diagonal's reciprocals
-  extern __shared__ __attribute__((aligned(16))) float Hs[];
-  float* Dd = Hs + GB * GB;
-  float* Dy = Dd + GB;
-  if (p.items) {
-    const GptqItem it = p.items[blockIdx.y];
-    p.scale = it.scale; p.zp = it.zp; p.gscale = it.gscale; p.g_idx = it.g_idx;
-    p.Wf += (int64_t)blockIdx.y * p.R * p.K;
-    p.U += (int64_t)blockIdx.y * p.u_stride;
-    p.E += (int64_t)blockIdx.y * p.R * p.ldE;
-    p.loss_rows += (int64_t)blockIdx.y * p.R;
-  }
-  const int tid = threadIdx.x;
-  const int count = p.count;
-  load_u_block(Hs, p.U, p.ldu, p.i1, count, tid);
-  if (tid < GB) {
-    const float d = tid < count ? p.U[(int64_t)(p.i1 + tid) * p.ldu + p.i1 + tid] : 1.f;
-    Dd[tid] = d;
-    Dy[tid] = shared_reciprocal(d);
-  }
-  const int tl = tid % QTEAM;
-  const int row = blockIdx.x * Q_ROWS_PER_WG + tid / QTEAM;
-  const bool live = row < p.R;
-  const QFormat f = make_qformat(FMT, p.bits);  // the format is a compile-time constant here
-  float* wrow = p.Wf + (int64_t)row * p.K + p.i1;
-  float* erow = p.E + (int64_t)row * p.ldE;
-
-  QLane<HAS_ZP, TEAM> r;
-  if (p.scale_dt == LLMC_BF16)
-    gptq_load_lane<LLMC_BF16, HAS_ZP, TEAM>(r, p, row, tl, live);
-  else if (p.scale_dt == LLMC_F16)
-    gptq_load_lane<LLMC_F16, HAS_ZP, TEAM>(r, p, row, tl, live);
-  else
-    gptq_load_lane<LLMC_F32, HAS_ZP, TEAM>(r, p, row, tl, live);
-  __syncthreads();
-
-  float loss = 0.f;
-#define LLMC_ROUND(J)                                                                                          \
-  if constexpr (J < QNCH) {                                                                                    \
-    if (J * QCW < count)                                                                                       \
-      gptq_round<J, FMT, SD, HAS_ZP, TEAM>(r, Hs, Dd, Dy, tl, count, live, wrow, erow, f, p.bits, loss);       \
-  }
-  LLMC_ROUND(0) LLMC_ROUND(1) LLMC_ROUND(2) LLMC_ROUND(3)
-  LLMC_ROUND(4) LLMC_ROUND(5) LLMC_ROUND(6) LLMC_ROUND(7)
-#undef LLMC_ROUND
-  static_assert(QNCH <= 8, "one LLMC_ROUND per run of a lane");
-
-  if (live) {
-    // the runs that were never reached carry no error into the trailing products
-#pragma unroll
-    for (int j = 0; j < QNCH; ++j) {
-      if (j * QCW >= count) {
-#pragma unroll
-        for (int m = 0; m < QG; ++m) erow[j * QCW + tl * QG + m] = 0.f;
-      }
-    }
-    if (tl == 0) p.loss_rows[row] += loss * 0.5f;
   }
 }
 
@@ -551,20 +241,21 @@ __global__ __launch_bounds__(256) void gptq_group_update_kernel(GroupUpdate g) {
 
 
 template <int WDT>
-__global__ __launch_bounds__(256) void gptq_finalize_kernel(const float* __restrict__ Wf, int R, int K,
+__global__ __launch_bounds__(256) void gptq_finalize_kernel(const float* __restrict__ Wf, int64_t ldf,
+                                                            int64_t w_stride, int R, int K,
                                                             const int32_t* __restrict__ perm,
                                                             void* __restrict__ out, int64_t ldo,
                                                             const GptqItem* __restrict__ items = nullptr) {
   if (items) {
     out = items[blockIdx.z].out;
     if (perm) perm += (int64_t)blockIdx.z * K;
-    Wf += (int64_t)blockIdx.z * R * K;
+    Wf += (int64_t)blockIdx.z * w_stride;
   }
   const int c = blockIdx.x * 256 + threadIdx.x;
   const int r = blockIdx.y;
   if (c >= K) return;
   const int dst = perm ? perm[c] : c;
-  store_from_f32<WDT>(out, (int64_t)r * ldo + dst, Wf[(int64_t)r * K + c]);
+  store_from_f32<WDT>(out, (int64_t)r * ldo + dst, Wf[(int64_t)r * ldf + c]);
 }
 
 __global__ __launch_bounds__(256) void sum_rows_kernel(const float* __restrict__ v, int n, float* out) {
@@ -1030,7 +721,7 @@ extern "C" int llmc_sparsegpt_sparsify(const void* weight, int32_t w_dtype, int6
   dim3 grid2((unsigned)((K + 255) / 256), (unsigned)R);
 #define LLMC_PREP(DT) \
   hipLaunchKernelGGL((gptq_prepare_w_kernel<DT>), grid2, dim3(256), 0, st, weight, ldw, (int)R, (int)K, \
-                     (const int32_t*)nullptr, dead, Wf)
+                     (const int32_t*)nullptr, dead, Wf, K)
   if (w_dtype == LLMC_BF16) LLMC_PREP(LLMC_BF16);
   else if (w_dtype == LLMC_F16) LLMC_PREP(LLMC_F16);
   else LLMC_PREP(LLMC_F32);
@@ -1118,7 +809,7 @@ extern "C" int llmc_sparsegpt_sparsify(const void* weight, int32_t w_dtype, int6
   }
 
 #define LLMC_FIN(DT) \
-  hipLaunchKernelGGL((gptq_finalize_kernel<DT>), grid2, dim3(256), 0, st, Wf, (int)R, (int)K, \
+  hipLaunchKernelGGL((gptq_finalize_kernel<DT>), grid2, dim3(256), 0, st, Wf, K, (int64_t)0, (int)R, (int)K, \
                      (const int32_t*)nullptr, out_weight, ldo)
   if (w_dtype == LLMC_BF16) LLMC_FIN(LLMC_BF16);
   else if (w_dtype == LLMC_F16) LLMC_FIN(LLMC_F16);
@@ -1132,60 +823,87 @@ extern "C" int llmc_sparsegpt_sparsify(const void* weight, int32_t w_dtype, int6
   return 0;
 }
 
-// The quantiser's blocked column loop for n problems of one shape (n = 1: the single call), lazy updates on
-// two levels.  After a block is quantised its scaled errors E_b update only the columns left in its group of
-// GROUP blocks (what the next block needs); the columns beyond the group get the whole group's errors in one
-// rank-(GROUP*bs) product.  Same sums as updating everything after every block, regrouped -- but the big part
-// of W is read and written a quarter as often, which is what bounds a rank-128 update.
-static int gptq_column_loop(void (*kern)(GptqBlockParams), GptqBlockParams p, int smem, unsigned wgs, int n, int64_t R,
-                            int64_t K, int bs, float* E, const float* U, int64_t ldu, int64_t u_stride, float* Wf,
-                            int form, char* extra, hipStream_t st) {
-  const int ldE = GROUP * GB;
-  p.ldE = ldE;
+// ---- the quantiser's work buffers ------------------------------------------------------------------------------
+// The work copy of W has rows and columns up to multiples of 128 (and E the rows), so that the products with them are
+// whole tiles of the split product whatever the weight's shape: a ragged weight's far updates would otherwise all
+// go to the element-wise edges of the fp32 kernel (39 ms for 4135 x 13072 as a whole).  What the padding holds is
+// never read back: rows are independent, and columns past K have nothing behind them.
+inline int64_t work_rows(int64_t R) { return (R + 127) / 128 * 128; }
+inline int64_t work_cols(int64_t K) { return (K + 127) / 128 * 128; }
+
+struct GptqWork {
+  float *Wf, *E, *loss_rows;
+  char* extra;
+  int64_t w_stride, e_stride;  // per problem, in floats
+};
+inline int64_t gptq_work_bytes(int64_t n, int64_t R, int64_t K, int form) {
+  return align256(n * work_rows(R) * work_cols(K) * 4) + align256(n * work_rows(R) * Q_LDE * 4) + align256(n * R * 4) +
+         left_extra_bytes(n, work_rows(R), K, form);
+}
+inline GptqWork gptq_work(char* p, int64_t n, int64_t R, int64_t K) {
+  GptqWork w;
+  w.w_stride = work_rows(R) * work_cols(K);
+  w.e_stride = work_rows(R) * Q_LDE;
+  w.Wf = (float*)p; p += align256(n * w.w_stride * 4);
+  w.E = (float*)p; p += align256(n * w.e_stride * 4);
+  w.loss_rows = (float*)p; p += align256(n * R * 4);
+  w.extra = p;
+  return w;
+}
+
+// The quantiser's blocked column loop for n problems of one shape (n = 1: the single call), lazy updates on two
+// levels: the group's kernel applies errors inside its GROUP blocks, the columns beyond the group get the whole group's
+// errors in one rank-(GROUP*bs) product (the big part of W is read and written a quarter as often as with one
+// product per block).
+//
+// Rows per workgroup: 16 while that is at most one workgroup per CU (4096 rows in all), 32 beyond: a pass of the chip
+// over the group takes 45 us with 16 rows each and 63 us with 32 (see gptq_group.h).  Both give the same bits.
+constexpr int64_t Q_FEW_ROWS = 16 * 256;
+static int gptq_column_loop(GptqGroupParams p, bool has_zp, int n, int64_t R, int64_t K, int bs,
+                            const GptqWork& w, int form, hipStream_t st) {
+  const int64_t Rp = work_rows(R), ldw = work_cols(K);
+  const GptqGroupKernels kernels =
+      p.fmt == LLMC_FMT_INT ? llmc_gptq_group_kernels_int(p.sd, has_zp) : llmc_gptq_group_kernels_fp(p.fmt, p.sd, has_zp);
+  const int team = (int64_t)n * R > Q_FEW_ROWS ? 8 : 16;
+  const GptqGroupKernel kern = team == 8 ? kernels.many : kernels.few;
+  const int rows = q_rows(team), smem = q_smem(team, has_zp);
+  const hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  if (e != hipSuccess) return 1000 + (int)e;
+  p.Wf = w.Wf; p.ldw = ldw; p.w_stride = w.w_stride; p.E = w.E; p.e_stride = w.e_stride; p.loss_rows = w.loss_rows;
+  p.R = (int)R; p.bs = bs;
   const int64_t gw = (int64_t)GROUP * bs;
   const bool left = form == LLMC_FACTOR_GROUPS;  // the callers have checked gw == 512 and K % 128 == 0
-  auto product = [&](const float* A, int64_t k0, int64_t kc, int64_t c0, int64_t c1) {
-    GemmF32 g = {};
-    g.A = A; g.lda = ldE; g.B = U + k0 * ldu + c0; g.ldb = ldu; g.C = Wf + c0; g.ldc = K;
-    g.M = (int)R; g.N = (int)(c1 - c0); g.Kc = (int)kc; g.alpha = -1.f; g.beta = 1.f;
-    g.batch = 1; g.batch2 = n; g.stride2_a = R * (int64_t)ldE; g.stride2_b = u_stride; g.stride2_c = R * K;
-    return llmc_gemm_f32(g, st);
-  };
   for (int64_t g0 = 0, gend = 0; g0 < K; g0 = gend) {
     gend = left ? left_group_end(g0, K) : ((g0 + gw) < K ? g0 + gw : K);
     if (left && (g0 > 0 || gend < K)) {  // the only group of a narrow weight needs neither D nor a sum
-      const int rc = left_begin_group(n, R, K, g0, U, ldu, u_stride, Wf, extra, st);
+      const int rc = left_begin_group(n, Rp, K, g0, p.U, p.ldu, p.u_stride, w.Wf, w.extra, st);
       if (rc) return rc;
     }
-    for (int64_t i1 = g0; i1 < gend; i1 += bs) {
-      const int count = (int)((gend - i1) < bs ? (gend - i1) : bs);
-      p.i1 = (int)i1;
-      p.count = count;
-      p.E = E + (i1 - g0);
-      hipLaunchKernelGGL(kern, dim3(wgs, (unsigned)n), dim3(256), smem, st, p);
-      LLMC_LAUNCH_STATUS();
-      const int64_t i2 = i1 + count;
-      if (i2 < gend) {
-        int rc = launch_group_update(p.E, ldE, U, ldu, u_stride, Wf, R, K, n, i1, count, i2, gend, st);
-        if (rc < 0) rc = product(p.E, i1, count, i2, gend);
-        if (rc) return rc;
-      }
-    }
-    if (gend < K) {
-      if (left) {
-        const int rc = left_end_group(n, R, K, g0, Wf, extra, st);
-        if (rc) return rc;
-      } else {
-        const int rc = product(E, g0, gend - g0, gend, K);
-        if (rc) return rc;
-      }
+    p.g0 = (int)g0;
+    p.gend = (int)gend;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((R + rows - 1) / rows), (unsigned)n), dim3(Q_THREADS), smem, st, p);
+    LLMC_LAUNCH_STATUS();
+    if (gend == K) break;
+    if (left) {
+      const int rc = left_end_group(n, Rp, K, g0, w.Wf, w.extra, st);
+      if (rc) return rc;
+    } else {
+      // up to the work copy's last column where the tiles are aligned: the rows of U that are read are above row
+      // gend < K, so 127 columns past K are still inside its memory
+      const int64_t c1 = gend % 128 == 0 && K >= 128 ? ldw : K;
+      GemmF32 g = {};
+      g.A = w.E; g.lda = Q_LDE; g.B = p.U + g0 * p.ldu + gend; g.ldb = p.ldu; g.C = w.Wf + gend; g.ldc = ldw;
+      g.M = (int)Rp; g.N = (int)(c1 - gend); g.Kc = (int)(gend - g0); g.alpha = 1.f; g.beta = 1.f;  // E is negated
+      g.batch = 1; g.batch2 = n; g.stride2_a = w.e_stride; g.stride2_b = p.u_stride; g.stride2_c = w.w_stride;
+      const int rc = llmc_gemm_f32(g, st);
+      if (rc) return rc;
     }
   }
   return 0;
 }
 
 extern "C" int64_t llmc_gptq_quantize_workspace_bytes(int64_t R, int64_t K, int32_t form) {
-  return align256(R * K * 4) + align256(R * GROUP * GB * 4) + align256(R * 4) + left_extra_bytes(1, R, K, form);
+  return gptq_work_bytes(1, R, K, form);
 }
 
 extern "C" int llmc_gptq_quantize(const void* weight, int32_t w_dtype, int64_t R, int64_t K, int64_t ldw,
@@ -1217,10 +935,8 @@ extern "C" int llmc_gptq_quantize(const void* weight, int32_t w_dtype, int64_t R
   // regroups fp32 sums); widths above what fits on chip run as 128-wide blocks
   const int bs = blocksize > GB ? GB : blocksize;
 
-  float* Wf = (float*)workspace;
-  float* E = (float*)((char*)workspace + align256(R * K * 4));
-  float* loss_rows = (float*)((char*)E + align256(R * GROUP * GB * 4));
-  char* extra = (char*)loss_rows + align256(R * 4);
+  const GptqWork work = gptq_work((char*)workspace, 1, R, K);
+  const int64_t ldf = work_cols(K);
 
   dim3 grid2((unsigned)((K + 255) / 256), (unsigned)R);
   const bool by_rows = perm != nullptr && K <= ROW_STAGE_MAX;  // permuted columns: gather and scatter a row in LDS
@@ -1229,53 +945,26 @@ extern "C" int llmc_gptq_quantize(const void* weight, int32_t w_dtype, int64_t R
     const int arc = allow_row_stage(gptq_prepare_w_rows_kernel<DT>, (int)K);                                        \
     if (arc) return arc;                                                                                            \
     hipLaunchKernelGGL((gptq_prepare_w_rows_kernel<DT>), dim3((unsigned)R), dim3(K > 8192 ? 1024 : 256), (size_t)K * 4, st, weight, ldw, \
-                       (int)R, (int)K, perm, dead, Wf, (const GptqItem*)nullptr);                                   \
+                       (int)R, (int)K, perm, dead, work.Wf, ldf, (int64_t)0, (const GptqItem*)nullptr);             \
   } else {                                                                                                          \
     hipLaunchKernelGGL((gptq_prepare_w_kernel<DT>), grid2, dim3(256), 0, st, weight, ldw, (int)R, (int)K, perm, dead, \
-                       Wf);                                                                                         \
+                       work.Wf, ldf);                                                                               \
   }
   if (w_dtype == LLMC_BF16) LLMC_PREP(LLMC_BF16)
   else if (w_dtype == LLMC_F16) LLMC_PREP(LLMC_F16)
   else LLMC_PREP(LLMC_F32)
 #undef LLMC_PREP
   LLMC_LAUNCH_STATUS();
-  hipLaunchKernelGGL(zero_f32_kernel, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, st, loss_rows, R);
-  LLMC_LAUNCH_STATUS();
-
-  GptqBlockParams p;
-  p.Wf = Wf; p.R = (int)R; p.K = (int)K; p.U = U; p.ldu = ldu;
+  GptqGroupParams p;
+  p.U = U; p.ldu = ldu;
   p.scale = scale; p.scale_dt = scale_dtype; p.zp = zero_point; p.gscale = global_scale; p.g_idx = g_idx;
   p.row_div = row_div; p.srow = scale_row_stride;
   p.fmt = fmt; p.bits = fmt == LLMC_FMT_INT ? num_bits : (fmt == LLMC_FMT_FP8 ? 8 : 4);
   p.sd = global_scale ? LLMC_F32 : scale_dtype;
-  p.E = E; p.loss_rows = loss_rows;
   p.items = nullptr; p.u_stride = 0;
 
-  const int smem = (GB * GB + 2 * GB) * 4;
-  void (*kern)(GptqBlockParams) = nullptr;
-  const bool hz = zero_point != nullptr;
-  const bool wide_team = R <= Q_WIDE_TEAM_MAX_ROWS;
-#define LLMC_PICK(F, S)                                                                                  \
-  if (p.fmt == F && p.sd == S)                                                                           \
-    kern = wide_team ? (hz ? gptq_block_kernel<F, S, true, 16> : gptq_block_kernel<F, S, false, 16>)     \
-                     : (hz ? gptq_block_kernel<F, S, true, 4> : gptq_block_kernel<F, S, false, 4>);
-  LLMC_PICK(LLMC_FMT_INT, LLMC_BF16)
-  LLMC_PICK(LLMC_FMT_INT, LLMC_F16)
-  LLMC_PICK(LLMC_FMT_INT, LLMC_F32)
-  LLMC_PICK(LLMC_FMT_FP8, LLMC_BF16)
-  LLMC_PICK(LLMC_FMT_FP8, LLMC_F16)
-  LLMC_PICK(LLMC_FMT_FP8, LLMC_F32)
-  LLMC_PICK(LLMC_FMT_FP4, LLMC_BF16)
-  LLMC_PICK(LLMC_FMT_FP4, LLMC_F16)
-  LLMC_PICK(LLMC_FMT_FP4, LLMC_F32)
-#undef LLMC_PICK
-  if (kern == nullptr) return -17;
-  hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-  if (e != hipSuccess) return 1000 + (int)e;
-  const int rows_per_wg = wide_team ? QLayout<16>::ROWS_PER_WG : QLayout<4>::ROWS_PER_WG;
-  const unsigned wgs = (unsigned)((R + rows_per_wg - 1) / rows_per_wg);
   {
-    const int rc = gptq_column_loop(kern, p, smem, wgs, 1, R, K, bs, E, U, ldu, 0, Wf, form, extra, st);
+    const int rc = gptq_column_loop(p, zero_point != nullptr, 1, R, K, bs, work, form, st);
     if (rc) return rc;
   }
 
@@ -1283,10 +972,11 @@ extern "C" int llmc_gptq_quantize(const void* weight, int32_t w_dtype, int64_t R
   if (by_rows) {                                                                                                    \
     const int arc = allow_row_stage(gptq_finalize_rows_kernel<DT>, (int)K);                                         \
     if (arc) return arc;                                                                                            \
-    hipLaunchKernelGGL((gptq_finalize_rows_kernel<DT>), dim3((unsigned)R), dim3(K > 8192 ? 1024 : 256), (size_t)K * 4, st, Wf, (int)R,   \
-                       (int)K, perm, out_weight, ldo, (const GptqItem*)nullptr);                                    \
+    hipLaunchKernelGGL((gptq_finalize_rows_kernel<DT>), dim3((unsigned)R), dim3(K > 8192 ? 1024 : 256), (size_t)K * 4, st, work.Wf,    \
+                       ldf, (int64_t)0, (int)R, (int)K, perm, out_weight, ldo, (const GptqItem*)nullptr);                                    \
   } else {                                                                                                          \
-    hipLaunchKernelGGL((gptq_finalize_kernel<DT>), grid2, dim3(256), 0, st, Wf, (int)R, (int)K, perm, out_weight, ldo); \
+    hipLaunchKernelGGL((gptq_finalize_kernel<DT>), grid2, dim3(256), 0, st, work.Wf, ldf, (int64_t)0, (int)R, (int)K, \
+                       perm, out_weight, ldo);                                                                      \
   }
   if (w_dtype == LLMC_BF16) LLMC_FIN(LLMC_BF16)
   else if (w_dtype == LLMC_F16) LLMC_FIN(LLMC_F16)
@@ -1294,7 +984,7 @@ extern "C" int llmc_gptq_quantize(const void* weight, int32_t w_dtype, int64_t R
 #undef LLMC_FIN
   LLMC_LAUNCH_STATUS();
   if (loss_out) {
-    hipLaunchKernelGGL(sum_rows_kernel, dim3(1), dim3(256), 0, st, loss_rows, (int)R, loss_out);
+    hipLaunchKernelGGL(sum_rows_kernel, dim3(1), dim3(256), 0, st, work.loss_rows, (int)R, loss_out);
     LLMC_LAUNCH_STATUS();
   }
   return 0;
@@ -1305,8 +995,7 @@ extern "C" int llmc_gptq_quantize(const void* weight, int32_t w_dtype, int64_t R
 // the serial chain of column blocks is as long as one problem's while each launch carries n times the rows.
 
 extern "C" int64_t llmc_gptq_quantize_grouped_workspace_bytes(int64_t n, int64_t R, int64_t K, int32_t form) {
-  return align256(n * (int64_t)sizeof(GptqItem)) + align256(n * R * K * 4) + align256(n * R * GROUP * GB * 4) +
-         align256(n * R * 4) + left_extra_bytes(n, R, K, form);
+  return align256(n * (int64_t)sizeof(GptqItem)) + gptq_work_bytes(n, R, K, form);
 }
 
 extern "C" int llmc_gptq_quantize_grouped(const void* const* weight, int32_t w_dtype, int32_t n, int64_t R, int64_t K,
@@ -1341,10 +1030,8 @@ extern "C" int llmc_gptq_quantize_grouped(const void* const* weight, int32_t w_d
 
   char* wp = (char*)workspace;
   GptqItem* items = (GptqItem*)wp; wp += align256(n * (int64_t)sizeof(GptqItem));
-  float* Wf = (float*)wp; wp += align256(n * R * K * 4);
-  float* E = (float*)wp; wp += align256(n * R * GROUP * GB * 4);
-  float* loss_rows = (float*)wp; wp += align256(n * R * 4);
-  char* extra = wp;
+  const GptqWork work = gptq_work(wp, n, R, K);
+  const int64_t ldf = work_cols(K);
   std::vector<GptqItem> host(n);
   for (int b = 0; b < n; ++b) {
     LLMC_CHECK_ARG(weight[b] != nullptr && scale[b] != nullptr && out_weight[b] != nullptr, 1);
@@ -1367,53 +1054,27 @@ extern "C" int llmc_gptq_quantize_grouped(const void* const* weight, int32_t w_d
     const int arc = allow_row_stage(gptq_prepare_w_rows_kernel<DT>, (int)K);                                    \
     if (arc) return arc;                                                                                        \
     hipLaunchKernelGGL((gptq_prepare_w_rows_kernel<DT>), dim3((unsigned)R, (unsigned)n), dim3(K > 8192 ? 1024 : 256), (size_t)K * 4, \
-                       st, (const void*)nullptr, ldw, (int)R, (int)K, perm, dead, Wf, (const GptqItem*)items);  \
+                       st, (const void*)nullptr, ldw, (int)R, (int)K, perm, dead, work.Wf, ldf, work.w_stride,  \
+                       (const GptqItem*)items);                                                                 \
   } else {                                                                                                      \
     hipLaunchKernelGGL((gptq_prepare_w_kernel<DT>), grid3, dim3(256), 0, st, (const void*)nullptr, ldw, (int)R, \
-                       (int)K, perm, dead, Wf, (const GptqItem*)items);                                         \
+                       (int)K, perm, dead, work.Wf, ldf, work.w_stride, (const GptqItem*)items);                \
   }
   if (w_dtype == LLMC_BF16) LLMC_PREP(LLMC_BF16)
   else if (w_dtype == LLMC_F16) LLMC_PREP(LLMC_F16)
   else LLMC_PREP(LLMC_F32)
 #undef LLMC_PREP
   LLMC_LAUNCH_STATUS();
-  hipLaunchKernelGGL(zero_f32_kernel, dim3((unsigned)((n * R + 255) / 256)), dim3(256), 0, st, loss_rows, n * R);
-  LLMC_LAUNCH_STATUS();
-
-  GptqBlockParams p;
-  p.Wf = Wf; p.R = (int)R; p.K = (int)K; p.U = U; p.ldu = ldu;
+  GptqGroupParams p;
+  p.U = U; p.ldu = ldu;
   p.scale = nullptr; p.scale_dt = scale_dtype; p.zp = nullptr; p.gscale = nullptr; p.g_idx = nullptr;
   p.row_div = row_div; p.srow = scale_row_stride;
   p.fmt = fmt; p.bits = fmt == LLMC_FMT_INT ? num_bits : (fmt == LLMC_FMT_FP8 ? 8 : 4);
   p.sd = global_scale ? LLMC_F32 : scale_dtype;
-  p.E = E; p.loss_rows = loss_rows;
   p.items = items; p.u_stride = u_stride;
 
-  const int smem = (GB * GB + 2 * GB) * 4;
-  void (*kern)(GptqBlockParams) = nullptr;
-  const bool hz = zero_point != nullptr;
-  const bool wide_team = (int64_t)n * R <= Q_WIDE_TEAM_MAX_ROWS;
-#define LLMC_PICK(F, S)                                                                                  \
-  if (p.fmt == F && p.sd == S)                                                                           \
-    kern = wide_team ? (hz ? gptq_block_kernel<F, S, true, 16> : gptq_block_kernel<F, S, false, 16>)     \
-                     : (hz ? gptq_block_kernel<F, S, true, 4> : gptq_block_kernel<F, S, false, 4>);
-  LLMC_PICK(LLMC_FMT_INT, LLMC_BF16)
-  LLMC_PICK(LLMC_FMT_INT, LLMC_F16)
-  LLMC_PICK(LLMC_FMT_INT, LLMC_F32)
-  LLMC_PICK(LLMC_FMT_FP8, LLMC_BF16)
-  LLMC_PICK(LLMC_FMT_FP8, LLMC_F16)
-  LLMC_PICK(LLMC_FMT_FP8, LLMC_F32)
-  LLMC_PICK(LLMC_FMT_FP4, LLMC_BF16)
-  LLMC_PICK(LLMC_FMT_FP4, LLMC_F16)
-  LLMC_PICK(LLMC_FMT_FP4, LLMC_F32)
-#undef LLMC_PICK
-  if (kern == nullptr) return -19;
-  hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-  if (e != hipSuccess) return 1000 + (int)e;
-  const int rows_per_wg = wide_team ? QLayout<16>::ROWS_PER_WG : QLayout<4>::ROWS_PER_WG;
-  const unsigned wgs = (unsigned)((R + rows_per_wg - 1) / rows_per_wg);
   {
-    const int rc = gptq_column_loop(kern, p, smem, wgs, n, R, K, bs, E, U, ldu, u_stride, Wf, form, extra, st);
+    const int rc = gptq_column_loop(p, zero_point != nullptr, n, R, K, bs, work, form, st);
     if (rc) return rc;
   }
 
@@ -1422,9 +1083,11 @@ extern "C" int llmc_gptq_quantize_grouped(const void* const* weight, int32_t w_d
     const int arc = allow_row_stage(gptq_finalize_rows_kernel<DT>, (int)K);                                     \
     if (arc) return arc;                                                                                        \
     hipLaunchKernelGGL((gptq_finalize_rows_kernel<DT>), dim3((unsigned)R, (unsigned)n), dim3(K > 8192 ? 1024 : 256), (size_t)K * 4,  \
-                       st, Wf, (int)R, (int)K, perm, (void*)nullptr, ldo, (const GptqItem*)items);              \
+                       st, work.Wf, ldf, work.w_stride, (int)R, (int)K, perm, (void*)nullptr, ldo,              \
+                       (const GptqItem*)items);                                                                 \
   } else {                                                                                                      \
-    hipLaunchKernelGGL((gptq_finalize_kernel<DT>), grid3, dim3(256), 0, st, Wf, (int)R, (int)K, perm,           \
+    hipLaunchKernelGGL((gptq_finalize_kernel<DT>), grid3, dim3(256), 0, st, work.Wf, ldf, work.w_stride, (int)R, \
+                       (int)K, perm,                                                                            \
                        (void*)nullptr, ldo, (const GptqItem*)items);                                            \
   }
   if (w_dtype == LLMC_BF16) LLMC_FIN(LLMC_BF16)
@@ -1433,7 +1096,7 @@ extern "C" int llmc_gptq_quantize_grouped(const void* const* weight, int32_t w_d
 #undef LLMC_FIN
   LLMC_LAUNCH_STATUS();
   if (loss_out) {
-    hipLaunchKernelGGL(sum_rows_kernel, dim3((unsigned)n), dim3(256), 0, st, loss_rows, (int)R, loss_out);
+    hipLaunchKernelGGL(sum_rows_kernel, dim3((unsigned)n), dim3(256), 0, st, work.loss_rows, (int)R, loss_out);
     LLMC_LAUNCH_STATUS();
   }
   return 0;

@@ -1,0 +1,721 @@
+// The quantiser's column loop inside one group of column blocks (up to 512 columns): kernels and their parameters.
+// Launched once per group by gptq.hip, instantiated in gptq_group_int.hip and gptq_group_fp.hip.
+//
+// What bounds it: rows are independent, but every column of a row depends on the one before it, so a wave works
+// through 128 dependent steps per block.  A wave issues an independent vector instruction every 5.5 cycles here and a
+// dependent one every 9, and a SIMD completes one every 4 however many waves it holds.  Both kernels are therefore
+// laid out for few instructions on that chain:
+//   * a row belongs to a team of 16 or 8 lanes, each holding runs of 4 neighbouring columns in registers.  In every
+//     turn each lane evaluates its own run with its own column constants.  Only the lane whose turn it is has final
+//     values; a lane's later evaluations repeat its own, because the LDS copy of U holds zeros below the diagonal and
+//     in the 4 x 4 diagonal blocks, so nothing is taken off a finished run.  Nothing is selected, stored or branched on
+//     inside a turn; after the last turn of a run every lane holds its columns' values and errors;
+//   * a turn's four errors reach the team as DPP operands (an immediate lane number, hence the unrolled turns), without
+//     a pass through LDS;
+//   * a division is two operations (two_step_div below); a wave that meets a divisor or a value outside the range
+//     where that holds repeats its block with plain divisions.
+// Before block b is quantised, the group's earlier errors are taken off its columns on the matrix cores,
+// W[:, b] - E U[:, b], as 16 x 16 tiles accumulated by v_mfma_f32_16x16x4_f32 in fp32.
+//
+// A workgroup is four waves that run the chain, one per SIMD, and four that prepare the next block meanwhile: its slice
+// of U, its scales and the part of its tiles that does not wait for the current block.
+//   16 lanes per row (16 rows per workgroup): the shortest chain, for weights that the chip takes in one pass.
+//   A 4096-row group takes 46 us (as four block launches and three update launches: 124 us).
+//   8 lanes per row (32 rows per workgroup): a turn has a quarter more instructions for twice the rows.  24576 rows:
+//   196 us per group (before: 314 us).
+// Both apply the same operations to every element in the same order, so they give the same bits.
+#pragma once
+#include "common.h"
+#include "qformat.h"
+
+constexpr int GB = 128;       // widest column block held on chip
+constexpr int GROUP = 4;      // column blocks whose updates of the far columns are applied together
+constexpr int Q_LDE = GROUP * GB;      // row stride of the scaled errors in memory
+
+// One problem of a grouped call (llmc_gptq_quantize_grouped); the kernels pick theirs by a grid index and
+// find its work buffers at a fixed stride behind those of problem 0.
+struct GptqItem {
+  const void* weight;
+  const void* scale;
+  const int8_t* zp;
+  const float* gscale;
+  const int32_t* g_idx;
+  void* out;
+};
+
+struct GptqGroupParams {
+  float* Wf;        // [rows up to a multiple of 128, ldw] fp32 work copy (permuted columns)
+  int64_t ldw;
+  int R;
+  const float* U;   // inverse-Hessian upper factor
+  int64_t ldu;
+  int g0, gend, bs; // columns [g0, gend) in blocks of bs
+  const void* scale;
+  int scale_dt;
+  const int8_t* zp;
+  const float* gscale;
+  const int32_t* g_idx;  // group of each (permuted) column, or NULL
+  int64_t row_div, srow;
+  int fmt, bits;
+  int sd;           // dtype the dequantised value is formed in
+  float* E;         // scaled errors of the group, negated, row stride Q_LDE
+  float* loss_rows; // [R], written by the first group and added to by the others
+  // grouped call: problem blockIdx.y takes scale / zp / gscale / g_idx from items and its Wf, U, E and
+  // loss rows at these strides (in elements)
+  const GptqItem* items;
+  int64_t u_stride, w_stride, e_stride;
+};
+
+typedef void (*GptqGroupKernel)(GptqGroupParams);
+struct GptqGroupKernels {
+  GptqGroupKernel few, many;  // 16 and 8 lanes per row
+};
+// by element format; fmt / sd as in GptqGroupParams
+GptqGroupKernels llmc_gptq_group_kernels_int(int sd, bool has_zp);
+GptqGroupKernels llmc_gptq_group_kernels_fp(int fmt, int sd, bool has_zp);
+
+constexpr int QG = 4;                           // neighbouring columns per run
+constexpr int Q_UHALF = GB / 2;
+constexpr int Q_U = Q_UHALF * GB + Q_UHALF * Q_UHALF;  // LDS slice of U: rows 0..63 whole, rows 64..127 from column 64 on
+constexpr int Q_D = GB / QG * 16;               // LDS column constants: four float4 per quad of columns
+constexpr int Q_LDS_W = GB + 4;                 // LDS row stride of a block's values
+constexpr int Q_LDS_E = (GROUP - 1) * GB + 4;   // LDS row stride of the group's errors
+constexpr int Q_THREADS = 512;
+constexpr int q_rows(int team) { return 256 / team; }
+constexpr int q_smem(int team, bool has_zp) {
+  return (Q_U + Q_D + q_rows(team) * ((has_zp ? 3 : 2) * Q_LDS_W + Q_LDS_E)) * 4;
+}
+
+#ifdef LLMC_GPTQ_GROUP_KERNELS
+namespace {
+
+// x / s in two operations from yh = 1/s rounded (hardware estimate and one Newton step) and yl = (1/s - yh) rounded:
+// RN(x * yh + RN(x * yl)).  The sum before the last rounding is within 2^-46 (relative) of x / s, so the result is the
+// IEEE quotient except where x / s lies within 2^-22 of an ulp of a midpoint between two floats, where it is the
+// other neighbour: an error of at most 0.5000003 ulp against 0.5.  Holds while s is in [2^-100, 2^100] and x is finite;
+// outside, the reciprocal is NaN (or the result is not finite) and the caller falls back to plain divisions.  The
+// addend +0 of the low product turns a -0 quotient into +0, as adding a zero point of zero does.
+__device__ __forceinline__ void two_step_reciprocal(const float s, float& yh, float& yl) {
+  const float a = fabsf(s), y0 = __builtin_amdgcn_rcpf(s), y = fmaf(fmaf(-s, y0, 1.0f), y0, y0);
+  const bool ok = a >= 0x1p-100f && a <= 0x1p100f;
+  yl = fmaf(-s, y, 1.0f) * y;
+  yh = ok ? y : __builtin_nanf("");
+}
+__device__ __forceinline__ float two_step_div(float x, float yh, float yl) { return fmaf(x, yh, fmaf(x, yl, 0.0f)); }
+
+template <int SD>
+__device__ __forceinline__ float round_sd(float x) {
+  if (SD == LLMC_BF16) return round16_finite<LLMC_BF16>(x);
+  if (SD == LLMC_F16) return round16_finite<LLMC_F16>(x);
+  return x;
+}
+
+// clamp and round a quotient onto the element grid (round_to_grid() with the conversion instructions)
+template <int FMT, bool EXACT>
+__device__ __forceinline__ float grid_value(float v, float qmin, float qmax) {
+  v = EXACT ? fminf(fmaxf(v, qmin), qmax) : __builtin_amdgcn_fmed3f(v, qmin, qmax);
+  if (FMT == LLMC_FMT_INT) return rintf(v);
+  if (FMT == LLMC_FMT_FP8) return hw_e4m3_pair_decode(hw_e4m3_pair(v, v)).x;
+  return hw_e2m1_pair_decode(hw_e2m1_pair(v, v)).x;
+}
+
+// a lane's run: 4 columns of one row, and everything about those columns that its evaluation needs
+struct QRun {
+  float w[QG], s[QG], yh[QG], yl[QG], z[QG];  // values, scales, their reciprocals, zero points
+  float dh[QG], dl[QG];                       // minus reciprocals of U's diagonal; with EXACT dh holds the diagonal
+  float u01, u02, u03, u12, u13, u23;         // the 4 x 4 diagonal block of U above its diagonal
+};
+struct QResult {
+  float q[QG], e[QG];  // dequantised values and negated scaled errors
+};
+// sum of (w - q)^2 / d^2 over a run
+__device__ __forceinline__ float run_loss(const QResult& o) {
+  return fmaf(o.e[3], o.e[3], fmaf(o.e[2], o.e[2], fmaf(o.e[1], o.e[1], o.e[0] * o.e[0])));
+}
+
+// One run, start to finish inside a lane: column m is quantised, its scaled error err = (w - q) / d (kept negated, so that
+// every update is one in-place multiply-add) is applied to
+// the columns of the run behind it (one fused multiply-subtract per element; the reference rounds the outer product
+// before it subtracts, the fused form keeps the product exact), and so on.
+template <int FMT, int SD, bool HAS_ZP, bool EXACT>
+__device__ __forceinline__ void gptq_run(const QRun& r, QResult& o, float qmin, float qmax) {
+  float w1 = r.w[1], w2 = r.w[2], w3 = r.w[3];
+  auto column = [&](float wv, int m) {
+    float v = EXACT ? wv / r.s[m] + 0.0f : two_step_div(wv, r.yh[m], r.yl[m]);
+    if (HAS_ZP) v = v + r.z[m];
+    float dq = grid_value<FMT, EXACT>(v, qmin, qmax);
+    if (HAS_ZP) dq = round_sd<SD>(dq - r.z[m]);
+    o.q[m] = round_sd<SD>(dq * r.s[m]);
+    const float x = __fsub_rn(wv, o.q[m]);
+    o.e[m] = EXACT ? -(x / r.dh[m]) : two_step_div(x, r.dh[m], r.dl[m]);
+    return o.e[m];
+  };
+  const float e0 = column(r.w[0], 0);
+  w1 = fmaf(e0, r.u01, w1);
+  w2 = fmaf(e0, r.u02, w2);
+  w3 = fmaf(e0, r.u03, w3);
+  const float e1 = column(w1, 1);
+  w2 = fmaf(e1, r.u12, w2);
+  w3 = fmaf(e1, r.u13, w3);
+  const float e2 = column(w2, 2);
+  w3 = fmaf(e2, r.u23, w3);
+  column(w3, 3);
+}
+static_assert(QG == 4, "gptq_run() is written out for runs of four columns");
+
+// lane LI's value in every lane of the team: a row of 16 lanes (row_newbcast), or each half of it by its own
+template <int TEAM, int LI>
+__device__ __forceinline__ float team_value(float v) {
+  const int x = __float_as_int(v);
+  const int lo = __builtin_amdgcn_mov_dpp(x, 0x150 + LI, 0xf, 0xf, true);
+  return __int_as_float(TEAM == 16 ? lo : __builtin_amdgcn_update_dpp(lo, x, 0x158 + (LI & 7), 0xf, 0xc, false));
+}
+
+__device__ __forceinline__ void add_row(float (&w)[QG], float e, const float4& u) {
+  w[0] = fmaf(e, u.x, w[0]);
+  w[1] = fmaf(e, u.y, w[1]);
+  w[2] = fmaf(e, u.z, w[2]);
+  w[3] = fmaf(e, u.w, w[3]);
+}
+// row i of the LDS slice of U at column c (c >= 64 where i >= 64)
+__device__ __forceinline__ float4 u_row(const float* __restrict__ Us, int i, int c) {
+  return *(const float4*)(i < Q_UHALF ? Us + i * GB + c : Us + Q_UHALF * GB + (i - Q_UHALF) * Q_UHALF + c - Q_UHALF);
+}
+
+// keeps the loads of one phase out of the phase before it (registers)
+__device__ __forceinline__ void phase_end() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// the values are final here: without it their updates are put off, and the rows of U they take kept, to the end
+__device__ __forceinline__ void settle(float (&w)[QG]) {
+  asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
+}
+
+// Run J of lane t covers columns 4 TEAM J + 4 t .. + 3.
+// Turn LI of run J, what it takes off the lanes' run J, and the turns after it.  What the turns of run J take off the later
+// runs is applied one turn later (`ep`: the errors of the turn before), in the gaps of the evaluation's dependent chain.
+// The rows of U are asked for before the evaluation; a turn is one scheduling region, which bounds the registers.
+template <int TEAM, int J, int LI, int FMT, int SD, bool HAS_ZP>
+__device__ __forceinline__ void gptq_turns(QRun& run, float (&w)[32 / TEAM][QG], QResult& o, float (&ep)[QG],
+                                           const float* __restrict__ Us, int tl, float qmin, float qmax) {
+  constexpr int NRUN = 32 / TEAM, SPAN = TEAM * QG;
+  constexpr bool LAST = LI == TEAM - 1;
+  float4 h[QG], g[QG][NRUN];
+#pragma unroll
+  for (int m = 0; m < QG; ++m) {
+    if (!LAST) h[m] = u_row(Us, J * SPAN + LI * QG + m, J * SPAN + tl * QG);
+    if (LI > 0) {
+#pragma unroll
+      for (int k = J + 1; k < NRUN; ++k) g[m][k] = u_row(Us, J * SPAN + (LI - 1) * QG + m, k * SPAN + tl * QG);
+    }
+  }
+  gptq_run<FMT, SD, HAS_ZP, false>(run, o, qmin, qmax);
+#pragma unroll
+  for (int m = 0; m < QG; ++m) {
+    if (LI > 0) {
+#pragma unroll
+      for (int k = J + 1; k < NRUN; ++k) add_row(w[k], ep[m], g[m][k]);
+    }
+    ep[m] = team_value<TEAM, LI>(o.e[m]);
+    if (!LAST) add_row(run.w, ep[m], h[m]);
+  }
+  if (LAST) {
+#pragma unroll
+    for (int m = 0; m < QG; ++m)
+#pragma unroll
+      for (int k = J + 1; k < NRUN; ++k) add_row(w[k], ep[m], u_row(Us, J * SPAN + LI * QG + m, k * SPAN + tl * QG));
+  }
+#pragma unroll
+  for (int k = J + 1; k < NRUN; ++k) settle(w[k]);
+  phase_end();
+  if constexpr (!LAST) gptq_turns<TEAM, J, LI + 1, FMT, SD, HAS_ZP>(run, w, o, ep, Us, tl, qmin, qmax);
+}
+
+// The turns of one run as a loop, operation for operation the same: formats without unrolled turns, and (EXACT) the rare
+// way round with plain divisions.
+template <int TEAM, int J, int FMT, int SD, bool HAS_ZP, bool EXACT>
+__device__ __forceinline__ void gptq_turns_rolled(QRun& run, float (&w)[32 / TEAM][QG], QResult& o,
+                                                  const float* __restrict__ Us, int tl, int count, float qmin, float qmax) {
+  constexpr int NRUN = 32 / TEAM, SPAN = TEAM * QG;
+#pragma unroll 1
+  for (int li = 0; li < TEAM; ++li) {
+    // columns at or past `count` hold w = 0, scale 1, d = 1 and zeros of U: nothing comes of their turns
+    if (J * SPAN + li * QG >= count) break;
+    gptq_run<FMT, SD, HAS_ZP, EXACT>(run, o, qmin, qmax);
+    // a finished run meets zeros of U; the test keeps an error that is not finite away from it
+    const bool open = tl > li;
+#pragma unroll
+    for (int m = 0; m < QG; ++m) {
+      const float e = __shfl(o.e[m], li, TEAM);
+      const int i = J * SPAN + li * QG + m;
+      if (open) add_row(run.w, e, u_row(Us, i, J * SPAN + tl * QG));
+#pragma unroll
+      for (int k = J + 1; k < NRUN; ++k) add_row(w[k], e, u_row(Us, i, k * SPAN + tl * QG));
+    }
+  }
+}
+
+// base[row_off + off] with the base and the row offset uniform: a scalar address and one 32-bit lane offset (in elements;
+// the offsets stay within 128 rows of at most 65536 values)
+template <typename T>
+__device__ __forceinline__ T load_at(const float* __restrict__ base, int64_t row_off, uint32_t off) {
+  return *(const T*)((const char*)(base + row_off) + (off << 2));
+}
+
+// ---- the block's slice of U: entries above the 4 x 4 diagonal blocks, zeros elsewhere and past `count` --------------
+// NQ quads per thread f = tid + n * nt.  Whole aligned blocks: fetch() issues the loads, put() stores them; others are
+// copied by put() alone.
+__device__ __forceinline__ void put_u(float* __restrict__ Us, int f, float4 v, int count) {
+  const int i = f >> 5, c = (f & 31) * 4;
+  const bool keep = c > (i & ~3) && i < count;
+  v.x = keep && c + 0 < count ? v.x : 0.f;
+  v.y = keep && c + 1 < count ? v.y : 0.f;
+  v.z = keep && c + 2 < count ? v.z : 0.f;
+  v.w = keep && c + 3 < count ? v.w : 0.f;
+  if (i < Q_UHALF)
+    *(float4*)&Us[i * GB + c] = v;
+  else if (c >= Q_UHALF)
+    *(float4*)&Us[Q_UHALF * GB + (i - Q_UHALF) * Q_UHALF + c - Q_UHALF] = v;
+}
+template <int NQ, int NT>
+struct USlice {
+  float4 v[NQ];
+  __device__ __forceinline__ void fetch(const float* __restrict__ base, int64_t ldu, bool whole, int tid) {
+    if (!whole) return;
+#pragma unroll
+    for (int n = 0; n < NQ; ++n)
+      v[n] = load_at<float4>(base, n * (NT / 32) * ldu, (uint32_t)(tid >> 5) * (uint32_t)ldu + (tid & 31) * 4);
+  }
+  __device__ __forceinline__ void put(float* __restrict__ Us, const float* __restrict__ base, int64_t ldu, int count,
+                                      bool whole, int tid) const {
+    if (whole) {
+#pragma unroll
+      for (int n = 0; n < NQ; ++n) put_u(Us, tid + n * NT, v[n], GB);
+      return;
+    }
+#pragma unroll 1
+    for (int n = 0; n < NQ; ++n) {
+      const int f = tid + n * NT, i = f >> 5, c = (f & 31) * 4;
+      const float* src = base + (int64_t)(i < count ? i : count - 1) * ldu;
+      put_u(Us, f, make_float4(src[c + 0 < count ? c + 0 : count - 1], src[c + 1 < count ? c + 1 : count - 1],
+                               src[c + 2 < count ? c + 2 : count - 1], src[c + 3 < count ? c + 3 : count - 1]), count);
+    }
+  }
+};
+
+// column constants of a block, for thread i < 128 (column i): Ds[comp][quad] float4 with comp 0 = -1/d high parts, 1 = low
+// parts, 2 = u01 u02 u03 u12, 3 = u13 u23
+struct DColumn {
+  float u[QG];  // U[i][4 (i/4) .. + 3]; only entries from the diagonal on are used
+  __device__ __forceinline__ void fetch(const float* __restrict__ base, int64_t ldu, int count, int i) {
+    const float* src = base + (int64_t)(i < count ? i : count - 1) * ldu;
+#pragma unroll
+    for (int k = 0; k < QG; ++k) {
+      const int c = (i & ~3) + k;
+      u[k] = src[c < count ? c : count - 1];
+    }
+  }
+  __device__ __forceinline__ void put(float* __restrict__ Ds, int count, int i) const {
+    const int quad = i >> 2, m = i & 3;
+    float v[QG];
+#pragma unroll
+    for (int k = 0; k < QG; ++k) v[k] = i < count && (i & ~3) + k < count ? u[k] : 0.f;
+    const float d = m == 0 ? v[0] : (m == 1 ? v[1] : (m == 2 ? v[2] : v[3]));
+    float dh, dl;
+    two_step_reciprocal(i < count ? d : 1.f, dh, dl);
+    float* q = Ds + quad * 4;
+    constexpr int COMP = GB / QG * 4;
+    q[m] = -dh;
+    q[COMP + m] = -dl;
+    if (m == 0) {
+      q[2 * COMP + 0] = v[1];
+      q[2 * COMP + 1] = v[2];
+      q[2 * COMP + 2] = v[3];
+    } else if (m == 1) {
+      q[2 * COMP + 3] = v[2];
+      q[3 * COMP + 0] = v[3];
+    } else if (m == 2) {
+      q[3 * COMP + 1] = v[3];
+    }
+  }
+};
+__device__ __forceinline__ void load_d(QRun& r, const float* __restrict__ Ds, int quad) {
+  constexpr int COMP = GB / QG * 4;
+  const float4 a = *(const float4*)(Ds + quad * 4), b = *(const float4*)(Ds + COMP + quad * 4);
+  const float4 c = *(const float4*)(Ds + 2 * COMP + quad * 4), d = *(const float4*)(Ds + 3 * COMP + quad * 4);
+  r.dh[0] = a.x; r.dh[1] = a.y; r.dh[2] = a.z; r.dh[3] = a.w;
+  r.dl[0] = b.x; r.dl[1] = b.y; r.dl[2] = b.z; r.dl[3] = b.w;
+  r.u01 = c.x; r.u02 = c.y; r.u03 = c.z; r.u12 = c.w; r.u13 = d.x; r.u23 = d.y;
+}
+
+template <int N>
+__device__ __forceinline__ void load_scales(float (&s)[N], const void* p, int dt, int64_t base, const int (&gi)[N]) {
+  if (dt == LLMC_BF16) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) s[e] = load_as_f32<LLMC_BF16>(p, base + gi[e]);
+  } else if (dt == LLMC_F16) {
+#pragma unroll
+    for (int e = 0; e < N; ++e) s[e] = load_as_f32<LLMC_F16>(p, base + gi[e]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < N; ++e) s[e] = load_as_f32<LLMC_F32>(p, base + gi[e]);
+  }
+}
+// a value the compiler knows nothing about: what is computed from it is not kept in registers from one block to the next
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// ---- tiles of W[:, block] - E U[:, block] --------------------------------------------------------------------------
+// A wave's NR x 2 tiles of 16 x 16: rows 16 t + .. of the workgroup, columns col0 / col1 (of the lane) of the block.
+// The inner index runs over earlier blocks of the group, 64 at a time and never across a block's end; lane group
+// q = lane / 16 contributes indices 16 q .. 16 q + 15 of a chunk, one per matrix instruction.
+constexpr int KS = 64, KL = KS / 4;
+struct BChunk {
+  float b0[KL], b1[KL];
+  __device__ __forceinline__ void fetch(const float* __restrict__ src, int64_t ldu, int len, int col0, int col1, int q) {
+    if (len == KS) {
+      const uint32_t o = (uint32_t)(KL * q) * (uint32_t)ldu;
+#pragma unroll
+      for (int j = 0; j < KL; ++j) {
+        b0[j] = load_at<float>(src, j * ldu, o + (uint32_t)col0);
+        b1[j] = load_at<float>(src, j * ldu, o + (uint32_t)col1);
+      }
+      return;
+    }
+#pragma unroll
+    for (int j = 0; j < KL; ++j) {
+      const uint32_t o = (uint32_t)(KL * q + j < len ? KL * q + j : len - 1) * (uint32_t)ldu;
+      b0[j] = load_at<float>(src, 0, o + (uint32_t)col0);
+      b1[j] = load_at<float>(src, 0, o + (uint32_t)col1);
+    }
+  }
+};
+template <int NR>
+struct Tiles {
+  f32x4_t acc[NR][2];
+  __device__ __forceinline__ void load(const float* __restrict__ W, int64_t ldw, int col0, int col1, int q) {
+#pragma unroll
+    for (int t = 0; t < NR; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        acc[t][0][i] = load_at<float>(W, (t * 16 + i) * ldw, (uint32_t)(4 * q) * (uint32_t)ldw + (uint32_t)col0);
+        acc[t][1][i] = load_at<float>(W, (t * 16 + i) * ldw, (uint32_t)(4 * q) * (uint32_t)ldw + (uint32_t)col1);
+      }
+  }
+  // E: the workgroup's rows at the chunk's first column
+  __device__ __forceinline__ void multiply(const BChunk& b, const float* __restrict__ E, int lde, bool vec, int len, int c,
+                                           int q) {
+#pragma unroll
+    for (int t = 0; t < NR; ++t) {
+      const float* src = E + (t * 16 + c) * lde + KL * q;
+      float a[KL];
+      if (vec) {
+#pragma unroll
+        for (int j = 0; j < KL; j += 4) {
+          const float4 v = *(const float4*)(src + j);
+          a[j] = v.x; a[j + 1] = v.y; a[j + 2] = v.z; a[j + 3] = v.w;
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < KL; ++j) a[j] = src[KL * q + j < len ? j : 0];
+      }
+      if (len < KS) {
+#pragma unroll
+        for (int j = 0; j < KL; ++j) a[j] = KL * q + j < len ? a[j] : 0.f;
+      }
+#pragma unroll
+      for (int j = 0; j < KL; ++j) {
+        acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b.b0[j], acc[t][0], 0, 0, 0);
+        acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b.b1[j], acc[t][1], 0, 0, 0);
+      }
+    }
+  }
+  // inner indices 0 .. kc - 1 (whole blocks of bs)
+  __device__ __forceinline__ void accumulate(const float* __restrict__ U, int64_t ldu, const float* __restrict__ E, int lde,
+                                             int kc, int bs, int col0, int col1, int c, int q) {
+    if (kc <= 0) return;
+    BChunk cur, nxt;
+    int k = 0, left = bs, len = left < KS ? left : KS;
+    cur.fetch(U, ldu, len, col0, col1, q);
+#pragma unroll 1
+    while (true) {
+      int kn = k + len, ln = left - len;
+      if (ln == 0) ln = bs;
+      const bool more = kn < kc;
+      const int nlen = ln < KS ? ln : KS;
+      if (more) nxt.fetch(U + (int64_t)kn * ldu, ldu, nlen, col0, col1, q);
+      multiply(cur, E + k, lde, (k & 3) == 0 && len == KS, len, c, q);
+      if (!more) break;
+      cur = nxt;
+      k = kn;
+      left = ln;
+      len = nlen;
+    }
+  }
+};
+
+// UNROLL: the turns unrolled (formats in common use) or as a loop
+template <int TEAM, int FMT, int SD, bool HAS_ZP, bool UNROLL>
+__global__ __launch_bounds__(Q_THREADS) void gptq_group_kernel(GptqGroupParams p) {
+  constexpr int ROWS = q_rows(TEAM), NRUN = 32 / TEAM, SPAN = TEAM * QG;
+  constexpr int NR = ROWS / 16;  // tile rows
+  extern __shared__ __attribute__((aligned(16))) float qsmem[];
+  float* const Us = qsmem;                       // slice of U of this block
+  float* const Ds = Us + Q_U;                    // its column constants
+  float* const Es = Ds + Q_D;                    // the group's errors
+  float* const Ws = Es + ROWS * Q_LDS_E;         // the block's values after the group's earlier errors
+  float* const Ss = Ws + ROWS * Q_LDS_W;         // scales
+  float* const Zs = Ss + ROWS * Q_LDS_W;         // zero points (HAS_ZP only)
+  if (p.items) {
+    const GptqItem it = p.items[blockIdx.y];
+    p.scale = it.scale; p.zp = it.zp; p.gscale = it.gscale; p.g_idx = it.g_idx;
+    p.Wf += (int64_t)blockIdx.y * p.w_stride;
+    p.U += (int64_t)blockIdx.y * p.u_stride;
+    p.E += (int64_t)blockIdx.y * p.e_stride;
+    p.loss_rows += (int64_t)blockIdx.y * p.R;
+  }
+  const int row0 = blockIdx.x * ROWS;
+  const bool vec_u = (p.ldu & 3) == 0 && (p.bs & 3) == 0 && ((uintptr_t)p.U & 15) == 0;
+
+  // Barriers, in the order in which both roles pass them: "ready" (a block's slice, scales and values are in LDS), "read"
+  // (the chain has the scales and values in registers), and, unless it was the last block, "errors" (its errors are
+  // in LDS, and the chain is done with the slice).
+  if (threadIdx.x >= 256) {  // ---- helpers: whole waves
+#pragma unroll 1
+    for (int i2 = p.g0;;) {
+      const int count = p.gend - i2 < p.bs ? p.gend - i2 : p.bs;
+      const int kc = i2 - p.g0, last = kc - p.bs;  // the block before starts at column `last` of the group
+      const int tid = opaque(threadIdx.x - 256), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+      const int tl = tid % TEAM, team = tid / TEAM, row = row0 + team;
+      const bool live = row < p.R;
+      const float* const base = p.U + (int64_t)i2 * p.ldu + i2;
+      const bool whole = vec_u && count == GB;
+      USlice<16, 256> u;
+      u.fetch(base, p.ldu, whole, tid);
+      DColumn d;
+      if (tid < GB) d.fetch(base, p.ldu, count, tid);
+      {
+        // scales and zero points for the columns and the row of the chain's lane of the same number
+        constexpr int N = NRUN * QG;
+        const int64_t sbase = ((int64_t)(live ? row : p.R - 1) / p.row_div) * p.srow;
+        int gi[N];
+        float s[N], z[N];
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+          const int c = (e / QG) * SPAN + tl * QG + (e % QG);
+          gi[e] = p.g_idx ? p.g_idx[i2 + (c < count ? c : count - 1)] : 0;
+        }
+        load_scales(s, p.scale, p.scale_dt, sbase, gi);
+#pragma unroll
+        for (int e = 0; e < N; ++e) z[e] = HAS_ZP ? (float)p.zp[sbase + gi[e]] : 0.f;
+        const float gs = p.gscale ? p.gscale[0] : 1.f;
+#pragma unroll
+        for (int J = 0; J < NRUN; ++J) {
+#pragma unroll
+          for (int m = 0; m < QG; ++m) {
+            const int e = QG * J + m;
+            if (p.gscale) s[e] = s[e] / gs;
+            const bool in = live && J * SPAN + tl * QG + m < count;
+            s[e] = in ? s[e] : 1.f;
+            z[e] = in ? z[e] : 0.f;
+          }
+          const int o = team * Q_LDS_W + J * SPAN + tl * QG;
+          *(float4*)&Ss[o] = make_float4(s[4 * J], s[4 * J + 1], s[4 * J + 2], s[4 * J + 3]);
+          if (HAS_ZP) *(float4*)&Zs[o] = make_float4(z[4 * J], z[4 * J + 1], z[4 * J + 2], z[4 * J + 3]);
+        }
+      }
+      phase_end();
+      if (kc > 0) {
+        const int c = lane & 15, q = lane >> 4;
+        const int ct0 = wave * 16 + c, ct1 = ct0 + Q_UHALF;
+        const int col0 = ct0 < count ? ct0 : count - 1, col1 = ct1 < count ? ct1 : count - 1;
+        const float* const Uc = p.U + (int64_t)p.g0 * p.ldu + i2;
+        Tiles<NR> tiles;
+        tiles.load(p.Wf + (int64_t)row0 * p.ldw + i2, p.ldw, col0, col1, q);
+        tiles.accumulate(Uc, p.ldu, Es, Q_LDS_E, last, p.bs, col0, col1, c, q);
+        phase_end();
+        // rows of U for the errors of the block before, in flight until they are there
+        const int len0 = p.bs < KS ? p.bs : KS, len1 = p.bs - len0;
+        BChunk b0, b1;
+        b0.fetch(Uc + (int64_t)last * p.ldu, p.ldu, len0, col0, col1, q);
+        if (len1 > 0) b1.fetch(Uc + (int64_t)(last + KS) * p.ldu, p.ldu, len1, col0, col1, q);
+        __syncthreads();  // errors
+        tiles.multiply(b0, Es + last, Q_LDS_E, (last & 3) == 0 && len0 == KS, len0, c, q);
+        if (len1 > 0) tiles.multiply(b1, Es + last + KS, Q_LDS_E, (last & 3) == 0 && len1 == KS, len1, c, q);
+#pragma unroll
+        for (int t = 0; t < NR; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            Ws[(t * 16 + 4 * q + i) * Q_LDS_W + ct0] = tiles.acc[t][0][i];
+            Ws[(t * 16 + 4 * q + i) * Q_LDS_W + ct1] = tiles.acc[t][1][i];
+          }
+      }
+      u.put(Us, base, p.ldu, count, whole, tid);
+      if (tid < GB) d.put(Ds, count, tid);
+      __syncthreads();  // ready
+      __syncthreads();  // read
+      i2 += count;
+      if (i2 >= p.gend) return;
+    }
+  }
+
+  // ---- the chain
+  const QFormat f = make_qformat(FMT, p.bits);   // the format is a compile-time constant here
+  const bool vec_w = (p.bs & 3) == 0;
+  float loss = 0.f;
+#pragma unroll 1
+  for (int i1 = p.g0; i1 < p.gend; i1 += p.bs) {
+    const int count = p.gend - i1 < p.bs ? p.gend - i1 : p.bs;
+    const int kc = i1 - p.g0;
+    const bool more = i1 + count < p.gend;
+    const int tid = opaque(threadIdx.x), tl = tid % TEAM, team = tid / TEAM, row = row0 + team;
+    const bool live = row < p.R;
+    float* const wrow = p.Wf + (int64_t)row * p.ldw;
+    float* const erow = p.E + (int64_t)row * Q_LDE;
+    __syncthreads();  // ready
+    float w[NRUN][QG], s[NRUN][QG], z[NRUN][QG];
+    auto load_w = [&]() {
+#pragma unroll
+      for (int J = 0; J < NRUN; ++J) {
+        const int c = J * SPAN + tl * QG;
+        float4 v;
+        if (kc > 0)
+          v = *(const float4*)&Ws[team * Q_LDS_W + c];
+        else if (vec_w)
+          v = *(const float4*)&wrow[i1 + (c < count ? c : 0)];
+        else
+          v = make_float4(wrow[i1 + (c < count ? c : 0)], wrow[i1 + (c + 1 < count ? c + 1 : 0)],
+                          wrow[i1 + (c + 2 < count ? c + 2 : 0)], wrow[i1 + (c + 3 < count ? c + 3 : 0)]);
+        w[J][0] = live && c + 0 < count ? v.x : 0.f;
+        w[J][1] = live && c + 1 < count ? v.y : 0.f;
+        w[J][2] = live && c + 2 < count ? v.z : 0.f;
+        w[J][3] = live && c + 3 < count ? v.w : 0.f;
+      }
+    };
+    load_w();
+#pragma unroll
+    for (int J = 0; J < NRUN; ++J) {
+      const int o = team * Q_LDS_W + J * SPAN + tl * QG;
+      const float4 a = *(const float4*)&Ss[o];
+      const float4 b = HAS_ZP ? *(const float4*)&Zs[o] : make_float4(0.f, 0.f, 0.f, 0.f);
+      s[J][0] = a.x; s[J][1] = a.y; s[J][2] = a.z; s[J][3] = a.w;
+      z[J][0] = b.x; z[J][1] = b.y; z[J][2] = b.z; z[J][3] = b.w;
+    }
+    __syncthreads();  // read
+    __builtin_amdgcn_s_setprio(3);  // the helper on the same SIMD takes what this wave leaves
+
+    QResult o[NRUN];
+#pragma unroll
+    for (int J = 0; J < NRUN; ++J)
+#pragma unroll
+      for (int m = 0; m < QG; ++m) o[J].q[m] = o[J].e[m] = 0.f;
+    bool bad = false;
+    auto run_step = [&](auto tag, auto exact_tag) {
+      constexpr int J = decltype(tag)::value;
+      constexpr bool EXACT = decltype(exact_tag)::value;
+      if (J * SPAN >= count) return;  // uniform
+      QRun r;
+      load_d(r, Ds, J * TEAM + tl);
+#pragma unroll
+      for (int m = 0; m < QG; ++m) {
+        r.w[m] = w[J][m];
+        r.s[m] = s[J][m];
+        r.z[m] = z[J][m];
+        two_step_reciprocal(r.s[m], r.yh[m], r.yl[m]);
+        bad = bad | (r.yh[m] != r.yh[m]);
+        if (EXACT) {
+          const int c = J * SPAN + tl * QG + m;
+          r.dh[m] = c < count ? p.U[(int64_t)(i1 + c) * p.ldu + i1 + c] : 1.f;
+        }
+      }
+      if constexpr (UNROLL && !EXACT) {
+        float ep[QG];
+        gptq_turns<TEAM, J, 0, FMT, SD, HAS_ZP>(r, w, o[J], ep, Us, tl, f.qmin, f.qmax);
+      } else {
+        gptq_turns_rolled<TEAM, J, FMT, SD, HAS_ZP, EXACT>(r, w, o[J], Us, tl, count, f.qmin, f.qmax);
+      }
+    };
+    auto all_runs = [&](auto exact_tag) {
+      run_step(std::integral_constant<int, 0>{}, exact_tag);
+      run_step(std::integral_constant<int, 1>{}, exact_tag);
+      if constexpr (NRUN > 2) {
+        run_step(std::integral_constant<int, 2>{}, exact_tag);
+        run_step(std::integral_constant<int, 3>{}, exact_tag);
+      }
+      static_assert(NRUN == 2 || NRUN == 4, "one step per run of a lane");
+    };
+    all_runs(std::false_type{});
+    float total = 0.f;
+#pragma unroll
+    for (int J = 0; J < NRUN; ++J) total += run_loss(o[J]);
+    if (__any(bad || !(total < 0x1p100f))) {
+      load_w();
+      all_runs(std::true_type{});
+    }
+    __builtin_amdgcn_s_setprio(0);
+    if (more) {
+#pragma unroll
+      for (int J = 0; J < NRUN; ++J) {
+        const int c = J * SPAN + tl * QG;
+        if (vec_w && c + QG <= count) {
+          *(float4*)&Es[team * Q_LDS_E + kc + c] = make_float4(o[J].e[0], o[J].e[1], o[J].e[2], o[J].e[3]);
+        } else {
+#pragma unroll
+          for (int m = 0; m < QG; ++m)
+            if (c + m < count) Es[team * Q_LDS_E + kc + c + m] = o[J].e[m];
+        }
+      }
+      __syncthreads();  // errors
+    }
+    // the row's loss in an order that does not depend on the team: lane t adds up the runs of 4 columns number t, t + 8,
+    // t + 16, t + 24 of every block
+#pragma unroll
+    for (int J = 0; J < NRUN; ++J) {
+      const float part = run_loss(o[J]);
+      if (TEAM == 8) {
+        loss += part;
+      } else {
+        loss += __shfl(part, tl & 7, 16);
+        loss += __shfl(part, 8 + (tl & 7), 16);
+      }
+    }
+    if (live) {
+#pragma unroll
+      for (int J = 0; J < NRUN; ++J) {
+        const int c = J * SPAN + tl * QG;
+        if (vec_w && c + QG <= count) {
+          *(float4*)&wrow[i1 + c] = make_float4(o[J].q[0], o[J].q[1], o[J].q[2], o[J].q[3]);
+          *(float4*)&erow[kc + c] = make_float4(o[J].e[0], o[J].e[1], o[J].e[2], o[J].e[3]);
+        } else {
+#pragma unroll
+          for (int m = 0; m < QG; ++m)
+            if (c + m < count) {
+              wrow[i1 + c + m] = o[J].q[m];
+              erow[kc + c + m] = o[J].e[m];
+            }
+        }
+      }
+    }
+  }
+  loss += __shfl_xor(loss, 1, 8);
+  loss += __shfl_xor(loss, 2, 8);
+  loss += __shfl_xor(loss, 4, 8);
+  const int row = row0 + (int)threadIdx.x / TEAM;
+  if (row < p.R && threadIdx.x % TEAM == 0) p.loss_rows[row] = (p.g0 == 0 ? 0.f : p.loss_rows[row]) + loss * 0.5f;
+}
+
+template <int FMT, int SD, bool HAS_ZP>
+GptqGroupKernels unrolled_kernels() {
+  return {gptq_group_kernel<16, FMT, SD, HAS_ZP, true>, gptq_group_kernel<8, FMT, SD, HAS_ZP, true>};
+}
+template <int FMT, int SD, bool HAS_ZP>
+GptqGroupKernels rolled_kernels() {
+  return {gptq_group_kernel<16, FMT, SD, HAS_ZP, false>, gptq_group_kernel<8, FMT, SD, HAS_ZP, false>};
+}
+
+}  // namespace
+#endif

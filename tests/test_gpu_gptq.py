@@ -744,3 +744,57 @@ def test_factor_forms_agree_over_shapes_and_formats(R, K, fmt_name, bits, group,
             # q * scale was rounded to bf16: the quotient is an integer to within 2^-8 of its magnitude
             assert torch.all((q - q.round()).abs() <= 0.005 * q.abs() + 1e-6)
             assert q.round().min() >= grid.min() and q.round().max() <= grid.max()
+
+
+def _column_loop(W, U, scale_cols, zp_cols, grid, sd):
+    """The column loop written out in fp32: scales and zero points per element, ``grid`` rounds a quotient."""
+    W = W.float().clone()
+    loss = torch.zeros((), device=W.device)
+    for i in range(W.shape[1]):
+        s, z = scale_cols[:, i], zp_cols[:, i]
+        q = ((grid(W[:, i] / s + z) - z).to(sd).float() * s).to(sd).float()
+        err = (W[:, i] - q) / U[i, i]
+        loss += (err * err).sum() / 2
+        W[:, i] = q
+        W[:, i + 1:] -= err[:, None] * U[i, i + 1:]
+    return W, loss
+
+
+@pytest.mark.parametrize("R,K,blocksize", [(1, 1, 128), (15, 129, 128), (16, 256, 128), (17, 516, 128), (33, 700, 37),
+                                           (16, 640, 64), (4096, 132, 128), (4097, 260, 128)])
+@pytest.mark.parametrize("case", ["int4_bf16", "int4_zp_f16", "int8_f32", "fp8_bf16", "fp4_f32_global", "fp4_f16"])
+def test_gptq_column_loop_at_tile_edges(R, K, blocksize, case):
+    """Partial blocks and groups, block widths that leave every access unaligned, a last workgroup of one row, and
+    weights on both sides of the line between 16 and 8 lanes per row, for formats with unrolled turns and with loops."""
+    from llmcompressor_amd import ops
+
+    torch.manual_seed(R + K)
+    W = (torch.randn(R, K, device="cuda") * 0.02).bfloat16()
+    U = torch.triu(torch.randn(K, K, device="cuda") * 0.05, 1) + torch.diag(torch.rand(K, device="cuda") + 0.5)
+    U_in = U + torch.tril(torch.full((K, K), float("nan"), device="cuda"), -1)  # what is below must not be read
+    sd = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[case.split("_")[-1].replace("global", "f32")]
+    qmax = 127.0 if "int8" in case else 448.0 if "fp8" in case else 6.0 if "fp4" in case else 7.0
+    scale = ((torch.rand(R, 1, device="cuda") + 0.5) * 0.05 / qmax).to(sd)
+    zp = torch.randint(-5, 5, (R, 1), dtype=torch.int8, device="cuda") if "zp" in case else None
+    gs = torch.tensor([3.7], device="cuda") if "global" in case else None
+    if "int" in case:
+        fmt, bits, grid = ops.FMT_INT, 8 if "int8" in case else 4, lambda v: torch.round(v.clamp(-qmax - 1, qmax))
+    elif "fp8" in case:
+        fmt, bits, grid = ops.FMT_FP8, 8, lambda v: v.clamp(-qmax, qmax).to(torch.float8_e4m3fn).float()
+    else:
+        points = torch.tensor([0, .5, 1, 1.5, 2, 3, 4, 6.], device="cuda")
+
+        def grid(v):
+            a = v.abs().clamp(max=6.0)
+            r = torch.where(a < 2, torch.round(a * 2) / 2, torch.where(a < 4, torch.round(a), torch.round(a / 2) * 2))
+            assert torch.isin(r, points).all()
+            return torch.copysign(r, v)
+        fmt, bits = ops.FMT_FP4, 4
+    s = scale.float() / gs if gs is not None else scale.float()
+    expected, loss_e = _column_loop(W, U, s.expand(R, K), (zp.float() if zp is not None else torch.zeros_like(s)).expand(R, K),
+                                    grid, torch.float32 if gs is not None else sd)
+    got, loss = ops.gptq_quantize(W, U_in, scale, zp, fmt, bits, 1, 1, global_scale=gs, blocksize=blocksize)
+    # another order of the sums moves a value across a rounding boundary now and then, and what follows with it
+    same = (got == expected.to(W.dtype)).float().mean().item()
+    assert same > 0.985, same
+    assert abs(loss.item() - loss_e.item()) <= 0.01 * loss_e.item() + 1e-9
