@@ -6,8 +6,8 @@
 // below 2^-24 of |a||b|, the rounding of an fp32 product, so the result is as accurate as the fp32 matrix
 // instruction's while the 16-bit matrix pipe runs 16 times its rate (six products: 2.6x the fp32 peak).
 //
-// One workgroup owns a 256 x 256 tile of C (eight waves of 64 x 128) or a 128 x 128 one (four waves of
-// 64 x 64).  A k-step is 16 deep.  Per k-step the workgroup fetches the fp32 slabs of both operands
+// One workgroup owns a 256 x 256 tile of C (eight waves of 64 x 128), a 128 x 128 one (four waves of
+// 64 x 64) or, further down, a 64 x 64 one.  A k-step is 16 deep in the larger two.  Per k-step the workgroup fetches the fp32 slabs of both operands
 // (tile edge x 16 each) into registers two steps ahead of their use, splits them into the three
 // planes in the same step and stores them to one of three LDS stages k-contiguous (a row of a plane is 16 bf16
 // = 32 bytes = two 16-byte chunks, the chunk index XOR-ed with bit 3 of the row: a 16-byte read is served
@@ -324,6 +324,164 @@ int launch_x3(const GemmF32& g, hipStream_t st) {
   return e == hipSuccess ? 0 : 1000 + (int)e;
 }
 
+// ---- 64 x 64 tiles, for products that larger tiles cannot spread over the chip: the levels of the triangular inverse
+// below 1024 columns, updates of narrow panels, weights of few rows.  These are bound by latency: a k-step's operands
+// come from memory that other XCDs have just written, 1.5 - 2 us away, and the larger tiles' two steps of prefetch cover
+// a quarter of that (a 256-deep product took 31 us with 128 x 128 tiles).  Here four waves of 32 x 32 work on k-steps of
+// 32, the fp32 operands of the four steps ahead are in registers (16 values per thread and step), C is fetched before
+// the first step, and two LDS stages leave room for three workgroups on a CU.
+//
+// A thread holds eight consecutive k of one row of A and of one column of B, i.e. one 16-byte chunk of its row in every
+// plane.  A row of a plane is 32 bf16 = four chunks, the chunk index XOR-ed with bits 2..3 of the row: the sixteen
+// consecutive rows that a 16-byte read is served at a time then fall into distinct banks.
+constexpr int SK = 32, S_RING = 4;
+constexpr int S_PLANE = 64 * SK * 2, S_STAGE = 6 * S_PLANE;  // bytes
+
+__device__ __forceinline__ int small_off(int row, int chunk) { return row * 64 + ((chunk ^ ((row >> 2) & 3)) << 4); }
+
+struct SmallSlab {
+  float a[8], b[8];
+};
+
+template <bool TRANS_B>
+__global__ __launch_bounds__(256, 2) void gemm_x3_small_kernel(GemmF32 g, int tiles_x, int tiles_y) {
+  __shared__ __attribute__((aligned(16))) unsigned char smem[2 * S_STAGE];
+  // the tile order of gemm_x3_kernel (rows of tiles dealt to the XCDs, longest contractions first)
+  const bool by_columns = g.b_lower_tri && !g.a_lower_tri && !g.c_lower;
+  const int major = by_columns ? tiles_x : tiles_y, minor = by_columns ? tiles_y : tiles_x;
+  const int id = blockIdx.x;
+  const int x = (id + (int)blockIdx.z * (major & 7)) & 7, j = id >> 3;
+  const int i = j / minor, t = j - i * minor;
+  const int rrow = 8 * i + ((i & 1) ? 7 - x : x);
+  if (rrow >= major) return;
+  const int ty = by_columns ? t : ((g.a_lower_tri || g.c_lower) ? tiles_y - 1 - rrow : rrow);
+  const int tx = by_columns ? rrow : t;
+  const int m0 = ty * 64, n0 = tx * 64;
+  if (g.c_lower && n0 > m0) return;
+  const int b1 = (int)blockIdx.z % g.batch, b2 = (int)blockIdx.z / g.batch;
+  const float* A = g.A + (int64_t)b1 * g.stride_a + (int64_t)b2 * g.stride2_a;
+  const float* B = g.B + (int64_t)b1 * g.stride_b + (int64_t)b2 * g.stride2_b;
+  float* Cm = g.C + (int64_t)b1 * g.stride_c + (int64_t)b2 * g.stride2_c;
+  const int k_begin = g.b_lower_tri ? n0 : 0;  // n0 is a multiple of SK
+  int k_end = (g.kc_last > 0 && b1 == g.batch - 1) ? g.kc_last : g.Kc;
+  if (g.a_lower_tri && m0 + 64 < k_end) k_end = m0 + 64;
+  const int nsteps = (k_end - k_begin) / SK;
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int ar = tid >> 2, ac = tid & 3;                       // A (and B when transposed): row, chunk of eight k
+  const int bc = TRANS_B ? ar : lane, bk = TRANS_B ? ac : wave;  // B: column, chunk; untransposed a wave reads 64 columns
+  const float* const ap = A + (int64_t)(m0 + ar) * g.lda + ac * 8;
+  const float* const bp = TRANS_B ? B + (int64_t)(n0 + bc) * g.ldb + bk * 8 : B + (int64_t)(bk * 8) * g.ldb + n0 + bc;
+  auto load = [&](SmallSlab& s, int k) {
+    const float4 a0 = *(const float4*)(ap + k), a1 = *(const float4*)(ap + k + 4);
+    s.a[0] = a0.x; s.a[1] = a0.y; s.a[2] = a0.z; s.a[3] = a0.w; s.a[4] = a1.x; s.a[5] = a1.y; s.a[6] = a1.z; s.a[7] = a1.w;
+    if (TRANS_B) {
+      const float4 v0 = *(const float4*)(bp + k), v1 = *(const float4*)(bp + k + 4);
+      s.b[0] = v0.x; s.b[1] = v0.y; s.b[2] = v0.z; s.b[3] = v0.w; s.b[4] = v1.x; s.b[5] = v1.y; s.b[6] = v1.z; s.b[7] = v1.w;
+    } else {
+      const float* const src = bp + (int64_t)k * g.ldb;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s.b[e] = src[(int64_t)e * g.ldb];
+    }
+  };
+  auto put = [&](const float (&v)[8], unsigned char* dst) {
+    uint32_t p[3][4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) split3(v[2 * e], v[2 * e + 1], p[0][e], p[1][e], p[2][e]);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) *(uint4*)(dst + q * S_PLANE) = make_uint4(p[q][0], p[q][1], p[q][2], p[q][3]);
+  };
+  auto store = [&](const SmallSlab& s, unsigned char* stage) {
+    put(s.a, stage + small_off(ar, ac));
+    put(s.b, stage + 3 * S_PLANE + small_off(bc, bk));
+  };
+
+  // C through one descriptor per wave, fetched now: its latency is covered by the contraction
+  const int wm_u = __builtin_amdgcn_readfirstlane(wm), wn_u = __builtin_amdgcn_readfirstlane(wn);
+  float* const c0 = Cm + (int64_t)(m0 + wm_u * 32) * g.ldc + n0 + wn_u * 32;
+  const int lane_bytes = ((lane >> 5) * 4 * (int)g.ldc + (lane & 31)) * 4;
+  const int row_bytes = (int)g.ldc * 4;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(c0, 0, 0x7fffffff, 0x00020000);
+
+  f32x16_t acc;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+  SmallSlab ring[S_RING];
+  float cv[16];
+  const int r = lane & 31, ch = lane >> 5;
+  const int k_last = k_end - SK;
+  auto clampk = [&](int k) { return k < k_last ? k : k_last; };
+  if (nsteps > 0) {
+#pragma unroll
+    for (int n = 0; n < S_RING; ++n) load(ring[n], clampk(k_begin + n * SK));
+  }
+  if (g.beta != 0.f) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      cv[v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rsrc, lane_bytes, ((v / 4) * 8 + (v & 3)) * row_bytes, 0));
+  }
+  if (nsteps > 0) {
+    store(ring[0], smem);
+    load(ring[0], clampk(k_begin + S_RING * SK));
+    __syncthreads();
+    constexpr int PA[6] = {2, 1, 0, 1, 0, 0};
+    constexpr int PB[6] = {0, 1, 2, 0, 1, 0};
+    // step ks (n = ks % S_RING): multiply from stage ks % 2 while slab ks + 1 goes to the other stage and its registers
+    // take step ks + 1 + S_RING.  Fetches past the end re-read the final slab; what they store is never multiplied.
+    auto step = [&](auto tag, int ks) {
+      constexpr int n = decltype(tag)::value, m = (n + 1) % S_RING;
+      const unsigned char* cur = smem + (n & 1) * S_STAGE;
+#pragma unroll
+      for (int kk = 0; kk < SK / 16; ++kk) {
+        uint4 af[3], bf[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          af[q] = *(const uint4*)(cur + q * S_PLANE + small_off(wm * 32 + r, 2 * kk + ch));
+          bf[q] = *(const uint4*)(cur + (3 + q) * S_PLANE + small_off(wn * 32 + r, 2 * kk + ch));
+        }
+#pragma unroll
+        for (int pr = 0; pr < 6; ++pr) acc = mfma_bf16(af[PA[pr]], bf[PB[pr]], acc);
+      }
+      store(ring[m], smem + ((n + 1) & 1) * S_STAGE);
+      load(ring[m], clampk(k_begin + (ks + 1 + S_RING) * SK));
+      __syncthreads();
+    };
+    for (int ks = 0; ks < nsteps; ks += S_RING) {
+      step(std::integral_constant<int, 0>{}, ks);
+      if (ks + 1 >= nsteps) break;
+      step(std::integral_constant<int, 1>{}, ks + 1);
+      if (ks + 2 >= nsteps) break;
+      step(std::integral_constant<int, 2>{}, ks + 2);
+      if (ks + 3 >= nsteps) break;
+      step(std::integral_constant<int, 3>{}, ks + 3);
+    }
+  }
+  const bool diag = g.c_lower && n0 == m0;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    float res = g.alpha * acc[v];
+    if (g.beta != 0.f) res += g.beta * cv[v];
+    if (diag && wn * 32 + (lane & 31) > wm * 32 + (v / 4) * 8 + (lane >> 5) * 4 + (v & 3)) continue;
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, res), rsrc, lane_bytes,
+                                          ((v / 4) * 8 + (v & 3)) * row_bytes, 0);
+  }
+}
+static_assert(S_RING == 4, "the loop above is written out for four slabs");
+
+template <bool TRANS_B>
+int launch_x3_small(const GemmF32& g, hipStream_t st) {
+  const int tiles_x = g.N / 64, tiles_y = g.M / 64;
+  const int nb2 = g.batch2 > 1 ? g.batch2 : 1;
+  const bool by_columns = g.b_lower_tri && !g.a_lower_tri && !g.c_lower;  // as in the kernel's tile order
+  const int major = by_columns ? tiles_x : tiles_y, minor = by_columns ? tiles_y : tiles_x;
+  const unsigned grid_x = 8u * (unsigned)((major + 7) / 8) * (unsigned)minor;
+  hipLaunchKernelGGL((gemm_x3_small_kernel<TRANS_B>), dim3(grid_x, 1, (unsigned)(g.batch * nb2)), dim3(256), 0, st, g, tiles_x,
+                     tiles_y);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? 0 : 1000 + (int)e;
+}
+
 int g_x3_mode = 1;  // 0 = never, 1 = when the shape fits and is big enough
 
 }  // namespace
@@ -342,15 +500,30 @@ int llmc_gemm_x3(const GemmF32& g, hipStream_t st) {
   // strip's origin): wider rows than this go to the fp32 kernel's 64-bit path
   if (g.ldc >= (1 << 22)) return -1;
   // Whether a product is split depends on its own shape only, never on how many independent problems
-  // (batch2) share the launch, so that a grouped call gives the bits of its single calls.  Both tile shapes
+  // (batch2) share the launch, so that a grouped call gives the bits of its single calls.  All tile shapes
   // add the partial products of an element in the same order, so the choice between them is free.
-  if (g.M % 128 || g.N % 128 || (int64_t)(g.M / 128) * (g.N / 128) * g.batch < 16) return -1;
+  // (from contractions of 256 on: the fp32 kernel's 64-wide tiles take 7 us at 128, 11 against 10 us at 256)
+  const bool fit64 = g.M % 64 == 0 && g.N % 64 == 0 && g.Kc >= 256 && g.Kc % SK == 0 && g.kc_last % SK == 0;
+  const bool fit128 = g.M % 128 == 0 && g.N % 128 == 0;
+  if (!fit64 && !(fit128 && (int64_t)(g.M / 128) * (g.N / 128) * g.batch >= 16)) return -1;
+  // The tile: what each shape's workgroups take, in units of 7.4 us for a contraction of 512 (measured with 1 .. 8 passes
+  // of the chip).  256 x 256: one per CU, 13 a pass.  128 x 128: two per CU, 7 a pass, 5 when each has a CU to itself.
+  // 64 x 64: 3 a pass of two per CU, 2 with a CU each; the steps at the diagonal of a triangular operand waste least
+  // there (0.6 of the time per tile).  Beyond one pass the workgroups follow each other without waiting, half a pass is the tail.
   const int64_t nbatch = (int64_t)g.batch * nb2;
-  // 256-wide tiles when they alone fill the chip (one workgroup per CU), 128-wide ones otherwise
   const bool fit256 = g.M % 256 == 0 && g.N % 256 == 0;
-  int64_t t256 = fit256 ? (int64_t)(g.M / 256) * (g.N / 256) * nbatch : 0;
-  if (g.c_lower && fit256) t256 = t256 / 2 + (g.M / 256) * nbatch / 2;
-  if (fit256 && t256 >= 192)
+  auto cost = [&](int edge, int per_cu, float pass, float alone) {
+    const int64_t rows = g.M / edge, cols = g.N / edge;
+    const int64_t tiles = (g.c_lower ? rows * cols / 2 + rows / 2 : rows * cols) * nbatch;
+    const float full = 256.f * per_cu;
+    return tiles <= 256 ? alone : (tiles <= full ? pass : pass * (tiles / full + 0.5f));
+  };
+  constexpr float NEVER = 1e30f;
+  const float c256 = fit256 ? cost(256, 1, 13.f, 13.f) : NEVER;
+  const float c128 = fit128 ? cost(128, 2, 7.f, 5.f) : NEVER;
+  const float c64 = fit64 ? cost(64, 2, 3.f, 2.f) * (g.a_lower_tri || g.b_lower_tri ? 0.6f : 1.f) : NEVER;
+  if (c256 <= c128 && c256 <= c64)
     return g.trans_b ? launch_x3<64, 128, 4, 2, true>(g, st) : launch_x3<64, 128, 4, 2, false>(g, st);
+  if (c64 < c128) return g.trans_b ? launch_x3_small<true>(g, st) : launch_x3_small<false>(g, st);
   return g.trans_b ? launch_x3<64, 64, 2, 2, true>(g, st) : launch_x3<64, 64, 2, 2, false>(g, st);
 }

@@ -63,3 +63,31 @@ def test_sgemm_rejects_bad_arguments():
     assert lib.llmc_sgemm(0, 8, a.data_ptr(), 8, a.data_ptr(), 8, 8, 8, 8, 1.0, 0.0, 0, 0, st) == -1
     assert lib.llmc_sgemm(a.data_ptr(), 8, a.data_ptr(), 8, a.data_ptr(), 4, 8, 8, 8, 1.0, 0.0, 0, 0, st) == -5
     assert lib.llmc_sgemm(a.data_ptr(), 8, a.data_ptr(), 8, a.data_ptr(), 8, 8, 8, 8, 1.0, 0.0, 0, 64, st) == -13
+
+
+@pytest.mark.parametrize("M,N,Kc,trans_b,flags,alpha,beta", [
+    (64, 64, 256, False, 0, 1.0, 0.0),      # one tile, as few k-steps as the split product takes
+    (64, 192, 288, True, 0, -1.0, 1.0),     # a contraction that is no multiple of the four steps in flight
+    (192, 320, 352, False, 0, -1.0, 1.0),
+    (448, 448, 256, True, 1, -1.0, 1.0),    # lower triangle only, diagonal tiles
+    (320, 256, 256, False, 4, 1.0, 0.0),    # contractions from 256 down to 64: two steps
+    (256, 320, 256, False, 2, -1.0, 0.0),
+])
+def test_sgemm_small_tiles(M, N, Kc, trans_b, flags, alpha, beta):
+    """Products of a few 64 x 64 tiles: within the fp32 matrix instruction's error, nothing outside C written."""
+    from llmcompressor_amd import ops
+
+    A, B, Bp, C0 = _operands(M, N, Kc, trans_b, flags, seed=M + N + Kc + flags)
+    ref = alpha * (A.double() @ Bp.double()) + beta * C0.double()
+    bound = A.double().abs() @ Bp.double().abs() + C0.double().abs()
+    wide = torch.full((M + 2, N + 8), 7.0, device="cuda")
+    C = wide[1:M + 1, 4:N + 4]
+    C.copy_(C0)
+    ops.sgemm_(C, A, B, alpha=alpha, beta=beta, trans_b=trans_b, flags=flags)
+    err = ((C.double() - ref).abs() / bound)
+    if flags & 1:
+        assert torch.equal(torch.triu(C, 1), torch.triu(C0, 1))
+        err = torch.tril(err)
+    assert err.max().item() < 8 * 2 ** -24, err.max().item() * 2 ** 24
+    C.fill_(7.0)
+    assert bool((wide == 7.0).all())
