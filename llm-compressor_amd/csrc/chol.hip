@@ -164,137 +164,156 @@ __global__ __launch_bounds__(1024) void hinv_copyin_rows_kernel(const float* __r
 // b > 0 then solves its own 64 rows of block column m against it, after bringing them up to date with the
 // region's earlier steps, and takes the new columns' contribution off its own diagonal block -- so that block
 // is complete when its turn comes.  The rows below the region are not on the spine: they are solved against
-// the whole region afterwards, one launch (chol_region_rows_kernel), 64 rows per workgroup, the block row kept
-// in LDS from one block column to the next.
+// the whole region afterwards, one launch (chol_region_rows_kernel), the solved block columns kept in LDS from one to
+// the next.
 //
 // The inverses of the diagonal blocks' factors go to a side array Xs (block c0 / 64 at Xs + (c0 / 64) * 4096, dense
 // 64 x 64) and not over the diagonal block itself: within one launch every workgroup reads that block, whenever it
 // happens to start, so nothing may overwrite it before the launch has ended.  chol_scatter_diag_kernel moves them
 // into the diagonal blocks once the factorisation is complete (where the inversion expects them).
+//
+// Sixteen waves: eight run the factorisation, whose chain keeps one of them busy at a time; meanwhile the other eight bring
+// the workgroup's rows up to date with the region's earlier steps, operands straight from memory.  11.7, 14, 15 and
+// 9 us for the four steps (13, 14.5, 18 and 10 us one after the other).
+constexpr int STEP_NT = 1024;
 struct RegionStepLds {
   cholblk::FactorScratch fs;
   float Abuf[NB][cholblk::LDD];
-  float Bbuf[NB][cholblk::LDD];
 };
 
-__global__ __launch_bounds__(cholblk::NT) void chol_region_step_kernel(float* __restrict__ A, int Kp, int r0, int m,
-                                                                       int K, HinvScalars* sc, float* __restrict__ Xs,
-                                                                       int64_t xs_stride) {
+__global__ __launch_bounds__(STEP_NT) void chol_region_step_kernel(float* __restrict__ A, int Kp, int r0, int m, int K,
+                                                                   HinvScalars* sc, float* __restrict__ Xs,
+                                                                   int64_t xs_stride) {
   using namespace cholblk;
   A += (int64_t)blockIdx.y * Kp * Kp;  // grouped call: blockIdx.y = problem
   Xs += (int64_t)blockIdx.y * xs_stride;
   sc += blockIdx.y;
   extern __shared__ __attribute__((aligned(16))) unsigned char region_smem[];
   RegionStepLds& L = *(RegionStepLds*)region_smem;
-  const int tid = threadIdx.x, w = tid >> 6, r = tid & 63;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), r = tid & 63;
   const int b = blockIdx.x;                // 0: owner of the diagonal block; b > 0: row block m + b of the region
   const int c0 = r0 + NB * m;              // the step's block column
   const int64_t rows = c0 + (int64_t)NB * b;
-  // the diagonal block's loads are issued first: their latency hides behind the products below
-  const float* dsrc = A + (int64_t)(c0 + r) * Kp + c0 + 8 * w;
-  const float4 d0 = *(const float4*)dsrc, d1 = *(const float4*)(dsrc + 4);
-  Acc64 acc, dg;
-  if (b > 0) {
-    // own rows of block column m, brought up to date with the region's earlier steps:
-    // acc = A[rows, c0..] - sum_{i<m} A[rows, cols_i] A[c0 rows, cols_i]^T
-    acc_load(acc, A + rows * Kp + c0, Kp, w, r);
-    acc_load(dg, A + rows * Kp + rows, Kp, w, r);  // this row block's own diagonal block, needed at the very end
-    for (int i = 0; i < m; ++i) {
-      BlockFetch fa, fb;
-      fa.fetch(A + rows * Kp + r0 + NB * i, Kp, tid);
-      fb.fetch(A + (int64_t)c0 * Kp + r0 + NB * i, Kp, tid);
-      if (i > 0) __syncthreads();  // the previous product has read the buffers
-      fa.put(L.Abuf, tid);
-      fb.put(L.Bbuf, tid);
-      __syncthreads();
-      mm64_nt<true>(acc, L.Abuf, L.Bbuf, w, r);
-    }
-  }
-  L.fs.AT[8 * w + 0][r] = d0.x; L.fs.AT[8 * w + 1][r] = d0.y; L.fs.AT[8 * w + 2][r] = d0.z; L.fs.AT[8 * w + 3][r] = d0.w;
-  L.fs.AT[8 * w + 4][r] = d1.x; L.fs.AT[8 * w + 5][r] = d1.y; L.fs.AT[8 * w + 6][r] = d1.z; L.fs.AT[8 * w + 7][r] = d1.w;
-  __syncthreads();
-  const int bad = factor_invert_64(L.fs);
-  if (b == 0) {
-    // first failing pivot, 1-based index in the ORIGINAL (un-reversed) ordering
-    if (tid == 0 && bad < NB && c0 + bad < K) atomicCAS(&sc->info, 0, K - (c0 + bad));
+  // this wave's tile (w / 4, w % 4) of the row block's own diagonal block, needed at the very end
+  v4f dg = {0.f, 0.f, 0.f, 0.f};
+  float* const dgp = A + rows * Kp + rows;
+  if (w < NT / 64) {
+    const float* dsrc = A + (int64_t)(c0 + r) * Kp + c0 + 8 * w;
+    const float4 d0 = *(const float4*)dsrc, d1 = *(const float4*)(dsrc + 4);
+    if (b > 0) dg = tile_load(dgp, Kp, w, r);
+    factor_block_put(L.fs, d0, d1, w, r);
+    const int bad = factor_invert_64(L.fs);
+    if (b == 0) {
+      // first failing pivot, 1-based index in the ORIGINAL (un-reversed) ordering
+      if (tid == 0 && bad < NB && c0 + bad < K) atomicCAS(&sc->info, 0, K - (c0 + bad));
 #pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      const int idx = tid + NT * n, row = idx >> 4, c4 = (idx & 15) * 4;
-      *(float4*)(Xs + (int64_t)(c0 / NB) * NB * NB + row * NB + c4) = *(const float4*)&L.fs.X[row][c4];
+      for (int n = 0; n < 2; ++n) {
+        const int idx = tid + NT * n, row = idx >> 4, c4 = (idx & 15) * 4;
+        *(float4*)(Xs + (int64_t)(c0 / NB) * NB * NB + row * NB + c4) = *(const float4*)&L.fs.X[row][c4];
+      }
     }
-    return;
+  } else {
+    if (b > 0) {
+      // rows of block column m, tiles 2 (w - 8) and 2 (w - 8) + 1: A[rows, c0..] - sum_{i<m} A[rows, cols_i] A[c0 rows, cols_i]^T
+      dg = tile_load(dgp, Kp, w, r);
+      // product i (i < m <= 2 here) runs while slab i is factored, its operands in flight since the slab before (all
+      // of them at the start: 17 instead of 15 us for m = 2)
+      const int t0 = 2 * (w - NT / 64);
+      const float* const xp = A + (rows + 16 * (t0 >> 2)) * Kp + r0;
+      const float* const yp = A + (int64_t)(c0 + 16 * (t0 & 3)) * Kp + r0;
+      v4f acc0 = tile_load(A + rows * Kp + c0, Kp, t0, r), acc1 = tile_load(A + rows * Kp + c0, Kp, t0 + 1, r);
+      Operand64 x, y0, y1;
+      auto fetch = [&](int i) {
+        x = operand_load(xp + NB * i, Kp, r);
+        y0 = operand_load(yp + NB * i, Kp, r);
+        y1 = operand_load(yp + 16 * (int64_t)Kp + NB * i, Kp, r);
+      };
+      if (m > 0) fetch(0);
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        if (i < m) {
+          acc0 = tile_mm<true>(acc0, x, y0);
+          acc1 = tile_mm<true>(acc1, x, y1);
+          if (i + 1 < m) fetch(i + 1);
+        } else if (i == m) {
+          tile_store(acc0, &L.Abuf[0][0], LDD, t0, r);
+          tile_store(acc1, &L.Abuf[0][0], LDD, t0 + 1, r);
+        }
+        __syncthreads();
+        __syncthreads();
+      }
+      for (int n = 7; n < FACTOR_BARRIERS; ++n) __syncthreads();
+    } else {
+      for (int n = 0; n < FACTOR_BARRIERS; ++n) __syncthreads();
+    }
   }
-  // solve: R = acc * inv(L_mm)^T  (the barriers inside the factorisation separate this from the last product)
-  acc_store(acc, &L.Abuf[0][0], LDD, w, r);
-  __syncthreads();
-  Acc64 sol = {};
-  mm64_nt<false>(sol, L.Abuf, L.fs.X, w, r);
-  acc_store(sol, A + rows * Kp + c0, Kp, w, r);
+  if (b == 0) return;
+  // solve, one tile per wave: R = Abuf * inv(L_mm)^T
+  v4f sol = {0.f, 0.f, 0.f, 0.f};
+  sol = tile_mm<false>(sol, operand_load(&L.Abuf[16 * (w >> 2)][0], LDD, r), operand_load(&L.fs.X[16 * (w & 3)][0], LDD, r));
   __syncthreads();  // every wave has read Abuf
-  acc_store(sol, &L.Abuf[0][0], LDD, w, r);
-  // the new columns' contribution to this row block's own diagonal block: D_b -= R R^T
+  tile_store(sol, &L.Abuf[0][0], LDD, w, r);
+  tile_store(sol, A + rows * Kp + c0, Kp, w, r);
   __syncthreads();
-  mm64_nt<true>(dg, L.Abuf, L.Abuf, w, r);
-  acc_store(dg, A + rows * Kp + rows, Kp, w, r);
+  // the new columns' contribution to this row block's own diagonal block: D_b -= R R^T
+  dg = tile_mm<true>(dg, operand_load(&L.Abuf[16 * (w >> 2)][0], LDD, r), operand_load(&L.Abuf[16 * (w & 3)][0], LDD, r));
+  tile_store(dg, dgp, Kp, w, r);
 }
 
+// Rows below the region against its nb block columns, 16 RT rows per workgroup, one 16 x 16 tile per wave (RT x 4 waves,
+// wave w: rows 16 (w / 4), columns 16 (w % 4) of each block column).  What bounds it is the chain of ten 64-deep products
+// per tile, 16 dependent matrix instructions each: the factor's operands come straight from memory, the next block's
+// while the current product runs, so that the waves meet only where a solved block column passes through LDS.  Few rows
+// per workgroup while that leaves them a CU each: 10 us for a 256-wide region, 22 us with 64 rows and the factor staged
+// in LDS.  Every RT applies the same operations to an element in the same order.
+template <int RT>
 struct RegionRowsLds {
-  float R[4][NB][cholblk::LDD];  // the workgroup's solved blocks of the region's block columns
-  float Abuf[NB][cholblk::LDD];
-  float Bbuf[NB][cholblk::LDD];
+  float R[4][16 * RT][cholblk::LDD];  // the solved blocks of the region's block columns
+  float S[16 * RT][cholblk::LDD];
 };
 
-// rows row_start + 64 * blockIdx.x .. of the nb block columns of the region at r0, whose diagonal region is done
-__global__ __launch_bounds__(cholblk::NT) void chol_region_rows_kernel(float* __restrict__ A, int Kp, int r0, int nb,
-                                                                       int row_start, const float* __restrict__ Xs,
-                                                                       int64_t xs_stride) {
+template <int RT>
+__global__ __launch_bounds__(256 * RT) void chol_region_rows_kernel(float* __restrict__ A, int Kp, int r0, int nb,
+                                                                    int row_start, const float* __restrict__ Xs,
+                                                                    int64_t xs_stride) {
   using namespace cholblk;
   A += (int64_t)blockIdx.y * Kp * Kp;
   Xs += (int64_t)blockIdx.y * xs_stride;
   extern __shared__ __attribute__((aligned(16))) unsigned char rows_smem[];
-  RegionRowsLds& L = *(RegionRowsLds*)rows_smem;
-  const int tid = threadIdx.x, w = tid >> 6, r = tid & 63;
-  const int64_t rows = row_start + (int64_t)NB * blockIdx.x;
-  // schedule: for block column j the factor blocks (j, 0) .. (j, j-1) at A[r0 + 64 j rows, r0 + 64 i columns], then
-  // the inverse of the diagonal block's factor from the side array.  One block ahead is in flight while the current
-  // product runs.
-  const float* xs0 = Xs + (int64_t)(r0 / NB) * NB * NB;
-  BlockFetch next;
-  next.fetch(xs0, NB, tid);
-  Acc64 own[4];  // the workgroup's rows of the region's block columns: all loads in flight from the start
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    if (j < nb) acc_load(own[j], A + rows * Kp + r0 + NB * j, Kp, w, r);
-  bool first = true;
+  RegionRowsLds<RT>& L = *(RegionRowsLds<RT>*)rows_smem;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = threadIdx.x & 63;
+  const int ti = w >> 2, tj = w & 3;
+  float* const own = A + (row_start + (int64_t)blockIdx.x * 16 * RT) * Kp + r0;
+  const float* const xs = Xs + (int64_t)(r0 / NB) * NB * NB + 16 * tj * NB;
+  const float* const fac = A + (int64_t)(r0 + 16 * tj) * Kp + r0;
+  // operand of product i of block column j: the factor block (j, i), or the inverse of the diagonal block's factor
+  auto factor_operand = [&](int j, int i) {
+    return i < j ? operand_load(fac + (int64_t)NB * j * Kp + NB * i, Kp, r) : operand_load(xs + (int64_t)j * NB * NB, NB, r);
+  };
+  Operand64 next = factor_operand(0, 0);
+  v4f acc = tile_load(own, Kp, w, r);
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     if (j >= nb) break;
-    Acc64 acc = own[j];
-    for (int i = 0; i <= j; ++i) {
-      if (!first) __syncthreads();  // the previous product has read Bbuf (and Abuf)
-      first = false;
-      next.put(L.Bbuf, tid);
-      {  // the block after this one
-        int nj = j, ni = i + 1;
-        if (ni > nj) { nj = j + 1; ni = 0; }
-        if (nj < nb) {
-          if (ni == nj)
-            next.fetch(xs0 + (int64_t)nj * NB * NB, NB, tid);
-          else
-            next.fetch(A + (int64_t)(r0 + NB * nj) * Kp + r0 + NB * ni, Kp, tid);
-        }
-      }
-      if (i == j) acc_store(acc, &L.Abuf[0][0], LDD, w, r);
-      __syncthreads();
-      if (i < j) {
-        mm64_nt<true>(acc, L.R[i], L.Bbuf, w, r);
-      } else {
-        Acc64 sol = {};
-        mm64_nt<false>(sol, L.Abuf, L.Bbuf, w, r);
-        acc_store(sol, A + rows * Kp + r0 + NB * j, Kp, w, r);
-        acc_store(sol, &L.R[j][0][0], LDD, w, r);  // read by later products, after the barriers in between
-      }
+    v4f ahead = acc;
+    if (j + 1 < nb) ahead = tile_load(own + NB * (j + 1), Kp, w, r);
+#pragma unroll
+    for (int i = 0; i < j; ++i) {
+      const Operand64 y = next;
+      next = factor_operand(j, i + 1);
+      acc = tile_mm<true>(acc, operand_load(&L.R[i][16 * ti][0], LDD, r), y);
     }
+    const Operand64 y = next;
+    if (j + 1 < nb) next = factor_operand(j + 1, 0);
+    tile_store(acc, &L.S[0][0], LDD, w, r);
+    __syncthreads();
+    v4f sol = {0.f, 0.f, 0.f, 0.f};
+    sol = tile_mm<false>(sol, operand_load(&L.S[16 * ti][0], LDD, r), y);
+    tile_store(sol, own + NB * j, Kp, w, r);
+    tile_store(sol, &L.R[j][0][0], LDD, w, r);
+    __syncthreads();
+    acc = ahead;
   }
 }
 
@@ -380,7 +399,7 @@ inline int64_t hinv_temp_floats(int64_t Kp) { return Kp * Kp / 4 > NB * Kp ? Kp 
 // region's update as one product.
 inline int chol_factor(float* A, int Kp, int K, HinvScalars* sc, float* Xs, int64_t xs_stride, int n, hipStream_t st) {
   static const int cfg_step = set_dynamic_lds(chol_region_step_kernel, sizeof(RegionStepLds));
-  static const int cfg_rows = set_dynamic_lds(chol_region_rows_kernel, sizeof(RegionRowsLds));
+  static const int cfg_rows = set_dynamic_lds(chol_region_rows_kernel<4>, sizeof(RegionRowsLds<4>));
   if (cfg_step) return cfg_step;
   if (cfg_rows) return cfg_rows;
   const int64_t mat = (int64_t)Kp * Kp;
@@ -403,16 +422,21 @@ inline int chol_factor(float* A, int Kp, int K, HinvScalars* sc, float* Xs, int6
         if (rc) return rc;
       }
       for (int m = 0; m < nb; ++m) {
-        hipLaunchKernelGGL(chol_region_step_kernel, dim3(nb - m, n), dim3(cholblk::NT), sizeof(RegionStepLds), st, A, Kp,
+        hipLaunchKernelGGL(chol_region_step_kernel, dim3(nb - m, n), dim3(STEP_NT), sizeof(RegionStepLds), st, A, Kp,
                            r0, m, K, sc, Xs, xs_stride);
         LLMC_LAUNCH_STATUS();
       }
-      const int below = (Kp - (r0 + rw)) / NB;
-      if (below > 0) {
-        hipLaunchKernelGGL(chol_region_rows_kernel, dim3(below, n), dim3(cholblk::NT), sizeof(RegionRowsLds), st, A, Kp,
-                           r0, nb, r0 + rw, (const float*)Xs, xs_stride);
+      const int below = (Kp - (r0 + rw)) / 16;  // tile rows below the region
+#define LLMC_ROWS(RT)                                                                                              \
+  hipLaunchKernelGGL((chol_region_rows_kernel<RT>), dim3(below / RT, n), dim3(256 * RT), sizeof(RegionRowsLds<RT>), \
+                     st, A, Kp, r0, nb, r0 + rw, (const float*)Xs, xs_stride)
+      if (below > 0) {  // a multiple of four; two workgroups per CU at most before they take more rows each
+        if ((int64_t)below * n <= 512) LLMC_ROWS(1);
+        else if ((int64_t)below * n <= 1024) LLMC_ROWS(2);
+        else LLMC_ROWS(4);
         LLMC_LAUNCH_STATUS();
       }
+#undef LLMC_ROWS
     }
     const int M2 = Kp - (k0 + pw);
     if (M2 > 0) {

@@ -2,25 +2,26 @@
 //
 // factor_invert_64: Cholesky factor L of one 64 x 64 block and X = L^-1, left in LDS.
 //
-// The block lives in LDS column-major; a column slab of 16 is factored by one wave with a row of the block in
-// each lane (lane r = row r, the slab's 16 entries of that row in 16 registers), so a pivot row's entries reach
-// every row as scalars (v_readlane) and nothing crosses waves inside a slab.  A lone wave issues one vector
-// instruction every eight cycles on this part, so the slab loop is trimmed to what the chain needs:
-//
-//   * the columns stay unscaled (the L D L^T form): the rank-1 update of column c by pivot column j is
-//     a[c] -= a[j] * (a_c[j] / d_j); the serial chain from one pivot to the next is readlane -> reciprocal ->
-//     multiply -> readlane -> fma, and no square root sits on it;
+// The block lives in LDS; a column slab of 16 is factored by one wave.  What bounds it is that wave's issue: 64 pivots,
+// one after the other, a vector instruction every 5.5 cycles and a dependent one every 9.  So the slab loop holds what
+// the chain needs and nothing else:
+//   * every row of 16 lanes keeps its own copy of the slab's diagonal rows (`b`, lane i = row i, 16 columns in
+//     registers), so that a pivot's multipliers are operands of the updates themselves (v_fmac_f32_dpp with
+//     row_newbcast: lane c of the own row of lanes); with v_readlane into scalars each took an instruction of its own
+//     and a wait;
+//   * a second set of registers (`a`) takes the same column operations: 48 lanes hold the rows below the diagonal block,
+//     the first 16 lanes hold rows of the identity, which end up as the transposed inverse of the unit-lower factor --
+//     no separate inversion;
+//   * the columns stay unscaled (the L D L^T form): the update of column c by pivot column j is
+//     x[c] -= x[j] * (b_c[j] / d_j), and no square root sits on the chain;
 //   * a pivot that is not positive and finite is only recorded (one ballot per slab): what follows it is
-//     discarded by the caller, so no fix-up sits on the chain either;
-//   * what the other phases need goes to LDS once per slab: V (the unscaled columns), T (V D^-1, the unit-lower
-//     factor) and 1/sqrt(d) per row.
-//
-// Between two slabs all eight waves apply the rank-16 update to the columns still to come
-// (A[r][c] -= sum_t V[r][t] T[c][t], T read as LDS broadcasts), and while wave k+1 factors its slab, waves 4-7
-// invert slab k: the elimination on an identity with the unit-lower factor needs no row scaling and, run over all
-// 64 rows, leaves X_kk = L_kk^-1 in the rows of the diagonal block and W_k = -L[below, k] X_kk in the rows below.
-// The off-diagonal blocks of X follow by doubling, X21 = X22 (-L21 X11) at widths 16 and 32, as 16 x 16 tiles on
-// v_mfma_f32_16x16x4_f32.
+//     discarded by the caller, so no fix-up sits on the chain either.
+// Between two slabs the next slab's columns are updated on v_mfma_f32_16x16x4_f32 (one 16 x 16 tile per wave); the
+// columns after it, and everything of the inverse that can be formed by then, follow in the other waves while the next
+// slab is factored.  With X_kk = L_kk^-1 and W_k = -L[below, k] X_kk, the parts of X below the diagonal are
+//   X_10 = X_11 W_0[1],  Z_0 = W_0[2..3] - L[2..3, 1] X_10,  X_2c = X_22 Z_c[2],  X_3c = X_33 (Z_c[3] + W_2[3] Z_c[2])
+// with Z_1 = W_1[2..3] for column c = 1, and X_32 = X_33 W_2[3]: one product with X_33 is left after the last slab.
+// About 6 us in all (with scalar multipliers, a vector-unit update and the inverse after each slab: 7.8 us).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -36,288 +37,263 @@ constexpr int LDP = 20;  // LDS row stride of a 16-wide slab
 
 struct FactorScratch {
   float X[NB][LDD];      // the result: inverse of the factor, zeros above the diagonal
-  float AT[NB][LDD];     // the block, column-major: AT[c][r] = A[r][c]; the doubling reuses it for -L21 X11
-  float V[4][NB][LDP];   // V[k][r][t]: unscaled factored columns of slab k (L = V D^-1/2)
-  float T[4][NB][LDP];   // T[k][r][t] = V[k][r][t] / d: the unit-lower factor
+  float AT[NB][LDD];     // the block, column-major: AT[c][r] = A[r][c], columns from 16 on
+  float P[NB][LDP];      // the current slab's columns, row-major
+  float V[3][NB][LDP];   // V[k][r][t]: unscaled factored columns of slab k below its diagonal block (L = V D^-1/2)
+  float T[3][NB][LDP];   // T[k][r][t] = V[k][r][t] / d: the unit-lower factor
+  float Y[4][16][LDP];   // Y[k]: inverse of slab k's 16 x 16 unit-lower factor, row-major
   float W[3][NB][LDP];   // W[k][r][c] = -(L[r, slab k] X_kk)[c] for the rows r below slab k's diagonal block
+  float Z[2][16][LDP];   // Z_0[2], Z_0[3]
+  float Q[2][16][LDP];   // Z_c[3] + W_2[3] Z_c[2], c = 0, 1
   float rs[NB];          // 1 / L[r][r]
   int bad;               // smallest column whose pivot was not positive and finite, NB if none
   int pad[3];
 };
 
-__device__ __forceinline__ float lane_value(float v, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+// v in lane LI of every row of 16 lanes, for the whole row
+template <int LI>
+__device__ __forceinline__ float row_lane(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x150 + LI, 0xf, 0xf, true));
+}
+// x[c] -= x_j * (lane c's t), c = J + 1 .. 15, in ascending order.  Written out in assembly because the compiler does
+// not fold a broadcast with two uses into its multiply-adds.  A vector register may be read across lanes two
+// wait states after it was written: hence the wait before the first (t) and, where the caller reads x[J + 1] across
+// lanes (PIVOT), behind it.
+template <int J, bool PIVOT, int C = J + 1>
+__device__ __forceinline__ void eliminate(float (&x)[16], float xj, float t) {
+  if constexpr (C < 16) {
+    if constexpr (C == J + 1 && PIVOT)
+      asm volatile("s_nop 1\n\tv_fmac_f32_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf\n\ts_nop 1"
+                   : "+v"(x[C]) : "v"(t), "v"(xj), "n"(C));
+    else if constexpr (C == J + 1)
+      asm volatile("s_nop 1\n\tv_fmac_f32_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                   : "+v"(x[C]) : "v"(t), "v"(xj), "n"(C));
+    else
+      asm volatile("v_fmac_f32_dpp %0, -%1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf"
+                   : "+v"(x[C]) : "v"(t), "v"(xj), "n"(C));
+    eliminate<J, PIVOT, C + 1>(x, xj, t);
+  }
 }
 
-// Slab K, in one wave, lane r = row r.
-template <int K>
-__device__ __forceinline__ void factor_slab(int r, FactorScratch& s) {
-  float a[16], t[16], myd = 1.f;
-#pragma unroll
-  for (int c = 0; c < 16; ++c) a[c] = s.AT[16 * K + c][r];
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int jr = 16 * K + j;
-    const float d = lane_value(a[j], jr);
-    t[j] = a[j] * __builtin_amdgcn_rcpf(d);
-    // the multipliers are read into distinct scalar registers first and applied afterwards: a scalar register
-    // written by a readlane cannot feed the very next vector instruction, and one register reused for every
-    // pair serialises them
-    float m[16];
-#pragma unroll
-    for (int c = j + 1; c < 16; ++c) m[c] = lane_value(t[j], 16 * K + c);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int c = j + 1; c < 16; ++c) a[c] = fmaf(-a[j], m[c], a[c]);
-    myd = r == jr ? a[j] : myd;
-    __builtin_amdgcn_sched_barrier(0);
+template <int J>
+__device__ __forceinline__ void pivots(float (&b)[16], float (&a)[16], float (&rd)[16], float& myd, int i) {
+  if constexpr (J < 16) {
+    rd[J] = __builtin_amdgcn_rcpf(row_lane<J>(b[J]));
+    myd = i == J ? b[J] : myd;
+    const float t = b[J] * rd[J];
+    eliminate<J, true>(b, b[J], t);
+    eliminate<J, false>(a, a[J], t);
+    pivots<J + 1>(b, a, rd, myd, i);
   }
+}
+
+// Slab K, in one wave.
+template <int K>
+__device__ __forceinline__ void factor_slab(int lane, FactorScratch& s) {
+  const int i = lane & 15, g = lane >> 4;
+  const int row = 16 * (K + g) + i;         // g = 0: row of the diagonal block (and identity row i); g > 0: a row below
+  const bool below = g > 0 && K + g < 4;
+  float b[16], a[16], rd[16], myd = 1.f;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    *(float4*)&s.V[K][r][4 * q] = make_float4(a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]);
-    *(float4*)&s.T[K][r][4 * q] = make_float4(t[4 * q], t[4 * q + 1], t[4 * q + 2], t[4 * q + 3]);
+    const float4 x = *(const float4*)&s.P[16 * K + i][4 * q];
+    b[4 * q] = x.x; b[4 * q + 1] = x.y; b[4 * q + 2] = x.z; b[4 * q + 3] = x.w;
+    float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (below) y = *(const float4*)&s.P[row][4 * q];
+    a[4 * q] = y.x; a[4 * q + 1] = y.y; a[4 * q + 2] = y.z; a[4 * q + 3] = y.w;
+  }
+  if (g == 0) {
+#pragma unroll
+    for (int c = 0; c < 16; ++c) a[c] = c == i ? 1.f : 0.f;
+  }
+  pivots<0>(b, a, rd, myd, i);
+  if (K < 3 && below) {
+    constexpr int KK = K < 3 ? K : 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      *(float4*)&s.V[KK][row][4 * q] = make_float4(a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]);
+      *(float4*)&s.T[KK][row][4 * q] = make_float4(a[4 * q] * rd[4 * q], a[4 * q + 1] * rd[4 * q + 1],
+                                                   a[4 * q + 2] * rd[4 * q + 2], a[4 * q + 3] * rd[4 * q + 3]);
+    }
+  }
+  if (g == 0) {
+#pragma unroll
+    for (int c = 0; c < 16; ++c) s.Y[K][c][i] = a[c];
   }
   // per row of the diagonal block: 1/sqrt(d) (hardware estimate plus one Newton step) and the pivot check.  A
   // pivot that is zero, negative, infinite or NaN gives an estimate that is infinite, zero or NaN, and the
   // Newton step turns each of those into NaN.
-  const bool diag = r >= 16 * K && r < 16 * K + 16;
   float rs = __builtin_amdgcn_rsqf(myd);
   rs = rs * (1.5f - 0.5f * myd * rs * rs);
-  if (diag) s.rs[r] = rs;
-  const unsigned long long failed = __ballot(diag && !(rs > 0.f && rs < 3.0e38f && myd <= 3.0e38f));
-  if (failed != 0ull && r == 0 && s.bad == NB) s.bad = __builtin_ctzll(failed);  // slabs run in ascending order
+  if (g == 0) s.rs[row] = rs;
+  const unsigned long long failed = __ballot(g == 0 && !(rs > 0.f && rs < 3.0e38f && myd <= 3.0e38f));
+  if (failed != 0ull && lane == 0 && s.bad == NB) s.bad = 16 * K + __builtin_ctzll(failed);  // slabs run in ascending order
 }
 
-// Rank-16 update by slab k of the columns still to come, shared by the eight waves: wave v takes NC / 8 columns.
-template <int K>
-__device__ __forceinline__ void update_trailing(int r, int v, FactorScratch& s) {
-  constexpr int NC = (48 - 16 * K) / 8;  // 6, 4, 2
-  float p[16];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const float4 x = *(const float4*)&s.V[K][r][4 * q];
-    p[4 * q] = x.x; p[4 * q + 1] = x.y; p[4 * q + 2] = x.z; p[4 * q + 3] = x.w;
-  }
-  const int c0 = 16 * (K + 1) + v * NC;
-  float acc[NC];
-#pragma unroll
-  for (int i = 0; i < NC; ++i) acc[i] = s.AT[c0 + i][r];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    float4 tv[NC];
-#pragma unroll
-    for (int i = 0; i < NC; ++i) tv[i] = *(const float4*)&s.T[K][c0 + i][4 * q];  // one address per wave: broadcast
-#pragma unroll
-    for (int i = 0; i < NC; ++i) acc[i] = fmaf(-p[4 * q], tv[i].x, acc[i]);
-#pragma unroll
-    for (int i = 0; i < NC; ++i) acc[i] = fmaf(-p[4 * q + 1], tv[i].y, acc[i]);
-#pragma unroll
-    for (int i = 0; i < NC; ++i) acc[i] = fmaf(-p[4 * q + 2], tv[i].z, acc[i]);
-#pragma unroll
-    for (int i = 0; i < NC; ++i) acc[i] = fmaf(-p[4 * q + 3], tv[i].w, acc[i]);
-  }
-#pragma unroll
-  for (int i = 0; i < NC; ++i) s.AT[c0 + i][r] = acc[i];
-}
-
-// Elimination on an identity with the unit-lower form of slab K, one of four helper waves (h = 0..3): the wave
-// owns the columns h, h+4, h+8, h+12 of the slab's 16.  Rows of the diagonal block end up holding X_kk (after the
-// row scaling by 1/L[r][r]), rows below it W_k.
-template <int K>
-__device__ __forceinline__ void invert_slab(int r, int h, FactorScratch& s) {
-  float tl[16];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const float4 x = *(const float4*)&s.T[K][r][4 * q];
-    tl[4 * q] = x.x; tl[4 * q + 1] = x.y; tl[4 * q + 2] = x.z; tl[4 * q + 3] = x.w;
-  }
-  float y[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) y[i] = (r == 16 * K + h + 4 * i) ? 1.f : 0.f;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int jr = 16 * K + j;
-    const float vm = r > jr ? tl[j] : 0.f;  // column j of the unit-lower factor, below its diagonal
-    float m[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) m[i] = lane_value(y[i], jr);  // row jr of the columns h + 4i: 1 on its own diagonal
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) y[i] = fmaf(-vm, m[i], y[i]);
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  if (r >= 16 * K && r < 16 * K + 16) {
-    const float rs = s.rs[r];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s.X[r][16 * K + h + 4 * i] = y[i] * rs;
-  } else if (K < 3 && r >= 16 * K + 16) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) s.W[K < 3 ? K : 0][r][h + 4 * i] = y[i];
-  }
-}
-
-// one 16 x 16 tile on the matrix cores: acc += A(16 x 4n) * B(4n x 16), A[i][k] at A + i * lda + k scaled by
-// ascale[k] when given and negated when NEG, B[k][c] at B + k * ldb + c, all in LDS.  Result layout: lane l holds
-// column l % 16, rows 4 * (l / 16) + v.
-template <int N4, bool NEG>
-__device__ __forceinline__ v4f tile16(v4f acc, const float* A, int lda, const float* B, int ldb, int lane,
-                                      const float* ascale = nullptr) {
+// acc - A B^T over 16 inner indices, A[i][k] at A + i * LDP + k, B[c][k] at B + c * LDP + k
+__device__ __forceinline__ v4f tile16_nt(v4f acc, const float* A, const float* B, int lane) {
   const int i = lane & 15, g = lane >> 4;
-#pragma unroll
-  for (int kk = 0; kk < N4; ++kk) {
-    float av = A[i * lda + 4 * kk + g];
-    if (ascale) av *= ascale[4 * kk + g];
-    const float bv = B[(4 * kk + g) * ldb + i];
-    if (NEG) av = -av;
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc, 0, 0, 0);
-  }
+  const float4 av = *(const float4*)(A + i * LDP + 4 * g), bv = *(const float4*)(B + i * LDP + 4 * g);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(-av.x, bv.x, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(-av.y, bv.y, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(-av.z, bv.z, acc, 0, 0, 0);
+  acc = __builtin_amdgcn_mfma_f32_16x16x4f32(-av.w, bv.w, acc, 0, 0, 0);
   return acc;
 }
+// tile (ti, tj) of the block, less slab K's contribution: into P (the next slab's columns) or back into AT
+template <int K>
+__device__ __forceinline__ void update_tile(FactorScratch& s, int ti, int tj, bool to_panel, int lane) {
+  const int c = lane & 15, g = lane >> 4;
+  float* const at = &s.AT[16 * tj + c][16 * ti + 4 * g];
+  const float4 x = *(const float4*)at;
+  v4f acc = {x.x, x.y, x.z, x.w};
+  acc = tile16_nt(acc, &s.V[K][16 * ti][0], &s.T[K][16 * tj][0], lane);
+  if (to_panel) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) s.P[16 * ti + 4 * g + v][c] = acc[v];
+  } else {
+    *(float4*)at = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  }
+}
+// 16 x 16 tile A B (+ C) into `out` (row stride ldo); A's columns scaled by ascale, its rows by rscale, negated with NEG
+template <bool NEG>
+__device__ __forceinline__ void product_tile(const float* A, int lda, const float* B, int ldb, const float* C, int ldc,
+                                             float* out, int ldo, int lane, const float* ascale = nullptr,
+                                             const float* rscale = nullptr) {
+  const int c = lane & 15, g = lane >> 4;
+  v4f acc = {0.f, 0.f, 0.f, 0.f};
+  if (C) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[v] = C[(4 * g + v) * ldc + c];
+  }
+  const float rsc = rscale ? rscale[c] : 1.f;
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) {
+    float av = A[c * lda + 4 * kk + g];
+    if (ascale) av *= ascale[4 * kk + g];
+    if (rscale) av *= rsc;
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(NEG ? -av : av, B[(4 * kk + g) * ldb + c], acc, 0, 0, 0);
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) out[(4 * g + v) * ldo + c] = acc[v];
+}
+// X_kk = Y_k with its rows scaled by 1/L[r][r]
+__device__ __forceinline__ void diagonal_tile(FactorScratch& s, int k, int lane) {
+  const int r = lane >> 2, q = lane & 3;
+  const float4 y = *(const float4*)&s.Y[k][r][4 * q];
+  const float f = s.rs[16 * k + r];
+  *(float4*)&s.X[16 * k + r][16 * k + 4 * q] = make_float4(y.x * f, y.y * f, y.z * f, y.w * f);
+}
 
-// s.AT holds the 64 x 64 block to factor, column-major (its lower triangle incl. the diagonal is used; the caller
-// passes a barrier after writing it)  ->  s.X = inverse of its lower Cholesky factor, exact zeros above the
-// diagonal.  Every thread of the 512 calls it.  Returns, in every thread, the smallest column whose pivot was not
+// the caller's share: row r of the block, columns 8 w .. 8 w + 7, as the 512 threads (w = tid / 64, r = tid % 64) hold it
+__device__ __forceinline__ void factor_block_put(FactorScratch& s, float4 d0, float4 d1, int w, int r) {
+  if (w < 2) {
+    *(float4*)&s.P[r][8 * w] = d0;
+    *(float4*)&s.P[r][8 * w + 4] = d1;
+    return;
+  }
+  s.AT[8 * w + 0][r] = d0.x; s.AT[8 * w + 1][r] = d0.y; s.AT[8 * w + 2][r] = d0.z; s.AT[8 * w + 3][r] = d0.w;
+  s.AT[8 * w + 4][r] = d1.x; s.AT[8 * w + 5][r] = d1.y; s.AT[8 * w + 6][r] = d1.z; s.AT[8 * w + 7][r] = d1.w;
+}
+
+// factor_block_put() has been called by every thread of the 512 (its lower triangle incl. the diagonal is used); no
+// barrier is needed in between  ->  s.X = inverse of the block's lower Cholesky factor, exact zeros above the
+// diagonal.  Every one of the 512 threads calls it.  Returns, in every thread, the smallest column whose pivot was not
 // positive and finite (NB if none; the numbers computed after such a pivot are meaningless).  Ends with a
-// barrier: s.X is readable by all on return.
+// barrier: s.X is readable by all on return.  FACTOR_BARRIERS barriers in all.
+constexpr int FACTOR_BARRIERS = 9;
 __device__ __forceinline__ int factor_invert_64(FactorScratch& s) {
-  const int tid = threadIdx.x, w = tid >> 6, r = tid & 63;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), r = tid & 63;
   if (tid == 0) s.bad = NB;
-  for (int i = tid; i < NB * LDD / 4; i += NT) ((float4*)&s.X[0][0])[i] = make_float4(0.f, 0.f, 0.f, 0.f);
   __syncthreads();
 
-  if (w == 0) factor_slab<0>(r, s);
-  __syncthreads();
-  update_trailing<0>(r, w, s);
-  __syncthreads();
-  if (w == 1) factor_slab<1>(r, s);
-  if (w >= 4) invert_slab<0>(r, w - 4, s);
-  __syncthreads();
-  update_trailing<1>(r, w, s);
-  __syncthreads();
-  if (w == 2) factor_slab<2>(r, s);
-  if (w >= 4) invert_slab<1>(r, w - 4, s);
-  __syncthreads();
-  update_trailing<2>(r, w, s);
-  __syncthreads();
-  if (w == 3) factor_slab<3>(r, s);
-  if (w >= 4) invert_slab<2>(r, w - 4, s);
-  __syncthreads();
-  if (w >= 4) invert_slab<3>(r, w - 4, s);
-  __syncthreads();
-
-  float (*Z)[LDD] = s.AT;  // the block itself is no longer needed: rows 0..31 take -L21 X11 of the 32-wide step
-  // ---- doubling, width 16: X[16.., 0..16) = X_11 W_0[16..32) (wave 0), X[48.., 32..48) = X_33 W_2[48..64) (wave 1)
-  if (w < 2) {
-    const int lo = 2 * w, hi = 2 * w + 1;
-    v4f acc = {0.f, 0.f, 0.f, 0.f};
-    acc = tile16<4, false>(acc, &s.X[16 * hi][16 * hi], LDD, &s.W[lo][16 * hi][0], LDP, r);
-    const int c = r & 15, g = r >> 4;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) s.X[16 * hi + 4 * g + v][16 * lo + c] = acc[v];
+  if (w == 0) {
+    factor_slab<0>(r, s);
+  } else {
+    for (int i = tid - 64; i < NB * 16; i += NT - 64) {  // the tiles above the diagonal
+      const int row = i >> 4, c4 = (i & 15) * 4;
+      if ((c4 >> 4) > (row >> 4)) *(float4*)&s.X[row][c4] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
   }
   __syncthreads();
-  // ---- width 32, first half: Z = -L21 X11 for rows 32..63: columns 16..31 are W_1 as it stands (waves 2, 3 copy
-  // it), columns 0..15 are W_0 - L[32.., 16..32) X_10 (waves 0, 1: one 16-row tile each; L = V scaled by 1/sqrt(d)
-  // of its column)
-  if (w < 2) {
-    const int c = r & 15, g = r >> 4;
-    v4f acc;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) acc[v] = s.W[0][32 + 16 * w + 4 * g + v][c];
-    acc = tile16<4, true>(acc, &s.V[1][32 + 16 * w][0], LDP, &s.X[16][0], LDD, r, &s.rs[16]);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) Z[16 * w + 4 * g + v][c] = acc[v];
-  } else if (w < 4) {
-    const int row = (w - 2) * 16 + (r >> 2), q = r & 3;
-    *(float4*)&Z[row][16 + 4 * q] = *(const float4*)&s.W[1][32 + row][4 * q];
-  }
+  if (w < 3) update_tile<0>(s, 1 + w, 1, true, r);
+  if (w == 3) diagonal_tile(s, 0, r);
   __syncthreads();
-  // ---- width 32, second half: X[32.., 0..32) = X22 Z, one 16 x 16 tile per wave 0..3 (X22 is lower triangular: the
-  // upper tile row stops at 16)
-  if (w < 4) {
-    const int ti = w >> 1, tj = w & 1;
-    const int c = r & 15, g = r >> 4;
-    v4f acc = {0.f, 0.f, 0.f, 0.f};
-    acc = tile16<4, false>(acc, &s.X[32 + 16 * ti][32], LDD, &Z[0][16 * tj], LDD, r);
-    if (ti == 1) acc = tile16<4, false>(acc, &s.X[48][48], LDD, &Z[16][16 * tj], LDD, r);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) s.X[32 + 16 * ti + 4 * g + v][16 * tj + c] = acc[v];
-  }
+  if (w == 0) factor_slab<1>(r, s);
+  if (w == 1) update_tile<0>(s, 2, 2, false, r);
+  if (w == 2) update_tile<0>(s, 3, 2, false, r);
+  if (w == 3) update_tile<0>(s, 3, 3, false, r);
+  if (w >= 4 && w < 7)
+    product_tile<true>(&s.T[0][16 * (w - 3)][0], LDP, &s.Y[0][0][0], LDP, nullptr, 0, &s.W[0][16 * (w - 3)][0], LDP, r);
+  __syncthreads();
+  if (w < 2) update_tile<1>(s, 2 + w, 2, true, r);
+  if (w == 2) diagonal_tile(s, 1, r);
+  __syncthreads();
+  if (w == 0) factor_slab<2>(r, s);
+  if (w == 1) update_tile<1>(s, 3, 3, false, r);
+  if (w == 2 || w == 3) product_tile<true>(&s.T[1][16 * w][0], LDP, &s.Y[1][0][0], LDP, nullptr, 0, &s.W[1][16 * w][0], LDP, r);
+  if (w == 4) product_tile<false>(&s.X[16][16], LDD, &s.W[0][16][0], LDP, nullptr, 0, &s.X[16][0], LDD, r);
+  __syncthreads();
+  if (w == 0) update_tile<2>(s, 3, 3, true, r);
+  if (w == 1) diagonal_tile(s, 2, r);
+  if (w == 2 || w == 3)
+    product_tile<true>(&s.V[1][16 * w][0], LDP, &s.X[16][0], LDD, &s.W[0][16 * w][0], LDP, &s.Z[w - 2][0][0], LDP, r, &s.rs[16]);
+  if (w == 4) product_tile<true>(&s.T[2][48][0], LDP, &s.Y[2][0][0], LDP, nullptr, 0, &s.W[2][48][0], LDP, r);
+  __syncthreads();
+  if (w == 0) factor_slab<3>(r, s);
+  if (w == 1) product_tile<false>(&s.X[32][32], LDD, &s.Z[0][0][0], LDP, nullptr, 0, &s.X[32][0], LDD, r);
+  if (w == 2) product_tile<false>(&s.X[32][32], LDD, &s.W[1][32][0], LDP, nullptr, 0, &s.X[32][16], LDD, r);
+  if (w == 3) product_tile<false>(&s.W[2][48][0], LDP, &s.Z[0][0][0], LDP, &s.Z[1][0][0], LDP, &s.Q[0][0][0], LDP, r);
+  if (w == 4) product_tile<false>(&s.W[2][48][0], LDP, &s.W[1][32][0], LDP, &s.W[1][48][0], LDP, &s.Q[1][0][0], LDP, r);
+  __syncthreads();
+  // X_33 as its unscaled form and the row scale: its own tile is written at the same time
+  if (w < 2) product_tile<false>(&s.Y[3][0][0], LDP, &s.Q[w][0][0], LDP, nullptr, 0, &s.X[48][16 * w], LDD, r, nullptr, &s.rs[48]);
+  if (w == 2) product_tile<false>(&s.Y[3][0][0], LDP, &s.W[2][48][0], LDP, nullptr, 0, &s.X[48][32], LDD, r, nullptr, &s.rs[48]);
+  if (w == 3) diagonal_tile(s, 3, r);
   __syncthreads();
   return s.bad;
 }
 
 }  // namespace cholblk
 
-// ---- 64 x 64 products on the matrix cores, for the kernels that keep a block row of the factorisation in one
-// workgroup.  A 64 x 64 result is 16 tiles of 16 x 16; wave w of the eight owns the tiles (w / 2, 2 * (w % 2) + e),
-// e = 0, 1.  Tile layout of v_mfma_f32_16x16x4_f32: lane l holds column l % 16, rows 4 * (l / 16) + v.
+// ---- 64-deep products on the matrix cores, one 16 x 16 tile per wave.  Tile layout of v_mfma_f32_16x16x4_f32: lane l
+// holds column l % 16, rows 4 * (l / 16) + v.  Tile t of a 64 x 64 block: rows 16 (t / 4), columns 16 (t % 4).
 namespace cholblk {
 
-struct Acc64 {
-  v4f t[2];
+// 16 rows of 64 values as the matrix instruction takes them: the k index a lane group feeds into an instruction is free
+// as long as both operands agree, so lane group g = lane / 16 takes k = 16 g .. 16 g + 15 of row lane % 16 and reads
+// its 16 values as four 16-byte loads.
+struct Operand64 {
+  float4 v[4];
 };
-
-// acc (+/-)= A * B^T with A and B row-major 64 x 64 blocks in LDS (row stride LDD).  The k index a lane group
-// feeds into a matrix instruction is free as long as both operands agree, so lane group g takes k = 16 g .. 16 g + 15
-// and reads its 16 values as four 16-byte loads.
+__device__ __forceinline__ Operand64 operand_load(const float* p, int64_t ld, int lane) {
+  const float* src = p + (int64_t)(lane & 15) * ld + 16 * (lane >> 4);
+  Operand64 o;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) o.v[q] = *(const float4*)(src + 4 * q);
+  return o;
+}
+// acc +/- X Y^T
 template <bool NEG>
-__device__ __forceinline__ void mm64_nt(Acc64& acc, const float (*A)[LDD], const float (*B)[LDD], int w, int lane) {
-  const int i = lane & 15, g = lane >> 4, ti = w >> 1;
-  float a[16];
+__device__ __forceinline__ v4f tile_mm(v4f acc, const Operand64& x, const Operand64& y) {
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const float4 x = *(const float4*)&A[16 * ti + i][16 * g + 4 * q];
-    a[4 * q] = NEG ? -x.x : x.x; a[4 * q + 1] = NEG ? -x.y : x.y; a[4 * q + 2] = NEG ? -x.z : x.z; a[4 * q + 3] = NEG ? -x.w : x.w;
+    const float4 a = x.v[q], b = y.v[q];
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(NEG ? -a.x : a.x, b.x, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(NEG ? -a.y : a.y, b.y, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(NEG ? -a.z : a.z, b.z, acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(NEG ? -a.w : a.w, b.w, acc, 0, 0, 0);
   }
-#pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    const int tj = 2 * (w & 1) + e;
-    float b[16];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const float4 x = *(const float4*)&B[16 * tj + i][16 * g + 4 * q];
-      b[4 * q] = x.x; b[4 * q + 1] = x.y; b[4 * q + 2] = x.z; b[4 * q + 3] = x.w;
-    }
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) acc.t[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[kk], b[kk], acc.t[e], 0, 0, 0);
-  }
+  return acc;
 }
-
-// the wave's two tiles of a 64 x 64 block at `p` (row stride ld, global or LDS)
-__device__ __forceinline__ void acc_load(Acc64& acc, const float* p, int64_t ld, int w, int lane) {
-  const int i = lane & 15, g = lane >> 4, ti = w >> 1;
-#pragma unroll
-  for (int e = 0; e < 2; ++e)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) acc.t[e][v] = p[(int64_t)(16 * ti + 4 * g + v) * ld + 16 * (2 * (w & 1) + e) + i];
+__device__ __forceinline__ v4f tile_load(const float* p, int64_t ld, int t, int lane) {
+  const float* src = p + (int64_t)(16 * (t >> 2) + 4 * (lane >> 4)) * ld + 16 * (t & 3) + (lane & 15);
+  return v4f{src[0], src[ld], src[2 * ld], src[3 * ld]};
 }
-__device__ __forceinline__ void acc_store(const Acc64& acc, float* p, int64_t ld, int w, int lane) {
-  const int i = lane & 15, g = lane >> 4, ti = w >> 1;
+__device__ __forceinline__ void tile_store(v4f acc, float* p, int64_t ld, int t, int lane) {
+  float* dst = p + (int64_t)(16 * (t >> 2) + 4 * (lane >> 4)) * ld + 16 * (t & 3) + (lane & 15);
 #pragma unroll
-  for (int e = 0; e < 2; ++e)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) p[(int64_t)(16 * ti + 4 * g + v) * ld + 16 * (2 * (w & 1) + e) + i] = acc.t[e][v];
+  for (int v = 0; v < 4; ++v) dst[v * ld] = acc[v];
 }
-
-// a 64 x 64 block of a row-major global matrix through registers into a row-major LDS block: fetch() issues the
-// loads (two 16-byte loads per thread), put() stores them, so that a product can run in between
-struct BlockFetch {
-  float4 v[2];
-  __device__ __forceinline__ void fetch(const float* src, int64_t ld, int tid) {
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      const int idx = tid + NT * n;
-      v[n] = *(const float4*)(src + (int64_t)(idx >> 4) * ld + (idx & 15) * 4);
-    }
-  }
-  __device__ __forceinline__ void put(float (*dst)[LDD], int tid) const {
-#pragma unroll
-    for (int n = 0; n < 2; ++n) {
-      const int idx = tid + NT * n;
-      *(float4*)&dst[idx >> 4][(idx & 15) * 4] = v[n];
-    }
-  }
-};
 
 }  // namespace cholblk

@@ -798,3 +798,25 @@ def test_gptq_column_loop_at_tile_edges(R, K, blocksize, case):
     same = (got == expected.to(W.dtype)).float().mean().item()
     assert same > 0.985, same
     assert abs(loss.item() - loss_e.item()) <= 0.01 * loss_e.item() + 1e-9
+
+
+@pytest.mark.parametrize("K,n", [(320, 3), (1088, 12), (1088, 24)])
+def test_hinv_grouped_rows_per_workgroup(K, n):
+    """The rows below a region are solved 16, 32 or 64 to a workgroup, by how many there are in all; with 1088 columns
+    the grouped calls take 32 and 64 where the single ones take 16.  Same bits."""
+    from llmcompressor_amd import ops
+
+    torch.manual_seed(K + n)
+    Hs = []
+    for _ in range(n):
+        x = torch.randn(2 * K, K, device="cuda") * torch.exp(torch.randn(K, device="cuda"))
+        Hs.append((x.t() @ x).contiguous())
+    U, dead, info = ops.gptq_hinv_grouped([h.clone() for h in Hs], None, [2.0] * n, 0.01)
+    assert int(info.abs().sum()) == 0
+    for b in (0, n - 1):
+        Ub, _, _ = ops.gptq_hinv_(Hs[b].clone(), None, divisor=2.0)
+        assert torch.equal(U[b], Ub)
+        Hd = Hs[b].double() / 2
+        Hd.diagonal().add_(0.01 * Hd.diagonal().mean())
+        err = (Ub.double().t() @ Ub.double() @ Hd - torch.eye(K, device="cuda", dtype=torch.float64)).abs().max()
+        assert err < 1e-3, err
