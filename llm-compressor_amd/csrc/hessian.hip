@@ -149,42 +149,61 @@ __device__ __forceinline__ void tile_epilogue(float* __restrict__ H, int64_t ldh
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave >> 1, wn = wave & 1;
   const bool diag = i0 == j0;
-  if (FAST_EPI && i0 + BT <= K && j0 + BT <= K) {
-    // interior tile: no bounds checks, so the 16-byte loads of a whole row of MFMA tiles are
-    // issued back to back before the first use
+  // Interior tiles need no bounds checks, so the 16-byte loads of a whole row of MFMA tiles are issued back to back
+  // before the first use.  A tile that reaches past K does the same with clamped addresses and stores what lies inside:
+  // with K a multiple of 4 a quad is inside or outside as a whole.  (Element by element, each load waiting for the
+  // one before, an edge tile took 70 us, ten times an interior one, and 300 x 2000 spent 60 of 89 us there.)
+  // NB: MFMA tiles whose loads are in flight together (fewer at an edge: registers).
+  auto fast_rows = [&](auto edge_tag) {
+    constexpr bool EDGE = decltype(edge_tag)::value;
+    constexpr int NB = EDGE ? 1 : MI;
 #pragma unroll
     for (int a = 0; a < MI; ++a) {
       if (a_only >= 0 && a != a_only) continue;
-      float4 old[MI][4];
+      const int rbase = i0 + wm * (BT / 2) + a * 32 + (lane >> 5) * 4;
 #pragma unroll
-      for (int b = 0; b < MI; ++b) {
-        const int col = j0 + wn * (BT / 2) + b * 32 + (lane & 31);
-        const int rbase = i0 + wm * (BT / 2) + a * 32 + (lane >> 5) * 4;
+      for (int b0 = 0; b0 < MI; b0 += NB) {
+        float4 old[NB][4];
 #pragma unroll
-        for (int vq = 0; vq < 4; ++vq) old[b][vq] = *(const float4*)(H + (int64_t)col * ldh + rbase + vq * 8);
-      }
+        for (int b = 0; b < NB; ++b) {
+          const int col = j0 + wn * (BT / 2) + (b0 + b) * 32 + (lane & 31);
 #pragma unroll
-      for (int b = 0; b < MI; ++b) {
-        const int col = j0 + wn * (BT / 2) + b * 32 + (lane & 31);
-        const int rbase = i0 + wm * (BT / 2) + a * 32 + (lane >> 5) * 4;
-#pragma unroll
-        for (int vq = 0; vq < 4; ++vq) {
-          const int r0 = rbase + vq * 8;
-          float4 o;
-          o.x = old[b][vq].x + alpha * acc[a][b][vq * 4 + 0];
-          o.y = old[b][vq].y + alpha * acc[a][b][vq * 4 + 1];
-          o.z = old[b][vq].z + alpha * acc[a][b][vq * 4 + 2];
-          o.w = old[b][vq].w + alpha * acc[a][b][vq * 4 + 3];
-          *(float4*)(H + (int64_t)col * ldh + r0) = o;
-          if (!diag) {
-            H[(int64_t)(r0 + 0) * ldh + col] = o.x;
-            H[(int64_t)(r0 + 1) * ldh + col] = o.y;
-            H[(int64_t)(r0 + 2) * ldh + col] = o.z;
-            H[(int64_t)(r0 + 3) * ldh + col] = o.w;
+          for (int vq = 0; vq < 4; ++vq) {
+            const int c = EDGE ? min(col, K - 1) : col, r = EDGE ? min(rbase + vq * 8, K - 4) : rbase + vq * 8;
+            old[b][vq] = *(const float4*)(H + (int64_t)c * ldh + r);
           }
         }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+          const int col = j0 + wn * (BT / 2) + (b0 + b) * 32 + (lane & 31);
+#pragma unroll
+          for (int vq = 0; vq < 4; ++vq) {
+            const int r0 = rbase + vq * 8;
+            float4 o;
+            o.x = old[b][vq].x + alpha * acc[a][b0 + b][vq * 4 + 0];
+            o.y = old[b][vq].y + alpha * acc[a][b0 + b][vq * 4 + 1];
+            o.z = old[b][vq].z + alpha * acc[a][b0 + b][vq * 4 + 2];
+            o.w = old[b][vq].w + alpha * acc[a][b0 + b][vq * 4 + 3];
+            if (EDGE && (col >= K || r0 >= K)) continue;
+            *(float4*)(H + (int64_t)col * ldh + r0) = o;
+            if (!diag) {
+              H[(int64_t)(r0 + 0) * ldh + col] = o.x;
+              H[(int64_t)(r0 + 1) * ldh + col] = o.y;
+              H[(int64_t)(r0 + 2) * ldh + col] = o.z;
+              H[(int64_t)(r0 + 3) * ldh + col] = o.w;
+            }
+          }
+        }
+        if (EDGE) __builtin_amdgcn_sched_barrier(0);
       }
     }
+  };
+  if (FAST_EPI && i0 + BT <= K && j0 + BT <= K) {
+    fast_rows(std::false_type{});
+    return;
+  }
+  if (FAST_EPI && (K & 3) == 0) {
+    fast_rows(std::true_type{});
     return;
   }
 #pragma unroll
@@ -617,16 +636,17 @@ struct Choice {
 // Phases for BT-wide tiles.  Whole rounds of NUM_WG tiles first.  When `split`, the R tiles left
 // over are cut along the tokens so that they fill a round too: R <= 128 -> one phase of
 // floor(256/R) chunks per tile; R > 128 -> 128 tiles in two chunks, then the rest as before.  A
-// chunk keeps at least 4 slabs.  time_us is a rough model (measured microseconds per slab and per
-// epilogue of one tile, partial tiles through the workspace at 3 TB/s) used only to pick between
-// candidates.
+// chunk keeps at least 4 slabs.  time_us is a rough model used only to pick between candidates, fitted to 26 sizes from
+// 2 x 10568 to 16384 x 2048: 256-wide tiles take 1.15 us per slab with half the chip's CUs at work and 1.9 with all,
+// and 33 us for the epilogue of a round, 45 for every further one; 128-wide tiles, two to a CU, take 0.62 us per
+// slab and 8 us while they are few and grow with their number from there; partial tiles pass through the workspace
+// at 3 TB/s.
 Choice make_choice(int bt, int64_t T, int64_t K, bool split) {
   Choice c;
   c.bt = bt;
   const int nb = (int)((K + bt - 1) / bt);
   const int nt = nb * (nb + 1) / 2;
   const int nslab = (int)((T + BK - 1) / BK);
-  const double slab_us = bt == 256 ? 1.75 : 0.7, epi_us = bt == 256 ? 35.0 : 10.0, chunk_epi_us = 5.0;
   Plan& plan = c.plan;
   plan.nphase = 0;
   int wg = 0, tile0 = 0, ws_tile = 0;
@@ -641,8 +661,15 @@ Choice make_choice(int bt, int64_t T, int64_t K, bool split) {
     wg += ((items + 7) / 8) * 8;
     tile0 += ntiles;
     if (sp > 1) ws_tile += items;
-    const int rounds = (items + NUM_WG - 1) / NUM_WG;
-    c.time_us += rounds * (((nslab + sp - 1) / sp) * slab_us + (sp > 1 ? chunk_epi_us : epi_us));
+    const int rounds = (items + NUM_WG - 1) / NUM_WG, slabs = (nslab + sp - 1) / sp;
+    if (bt == 256) {
+      const double fill = (double)items / (rounds * NUM_WG);
+      c.time_us += rounds * slabs * (1.15 + (fill > 0.5 ? 1.5 * (fill - 0.5) : 0.0));
+      c.time_us += sp > 1 ? 5.0 * rounds : 33.0 + 45.0 * (rounds - 1);
+    } else {
+      const double busy = 0.0042 * items;
+      c.time_us += slabs * (busy > 0.62 ? busy : 0.62) + (sp > 1 ? 5.0 + 0.01 * items : 8.0 + 0.07 * items);
+    }
   };
   int slimit = nslab / 4;
   if (slimit > 16) slimit = 16;

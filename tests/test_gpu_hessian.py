@@ -257,3 +257,24 @@ def test_hessian_fp32_activations(T, K):
     Hn = H0.cuda()
     ops.hessian_accumulate_(Hn, x.cuda().contiguous(), assume_symmetric=False)
     assert _rel(Hn.cpu(), H0.double() + 2 * x.double().t() @ x.double()) < TOL
+
+
+@pytest.mark.parametrize("K", [4, 132, 260, 388, 1020, 1028, 1030])
+@pytest.mark.parametrize("T", [3, 300])
+def test_hessian_tiles_that_reach_past_the_last_column(T, K):
+    """Edge tiles with whole quads (K a multiple of 4) and without; memory around H stays as it was."""
+    from llmcompressor_amd import ops
+
+    torch.manual_seed(K + T)
+    x = torch.randn(T, K, device="cuda").bfloat16()
+    s = torch.randn(K, K, device="cuda")
+    wide = torch.full((K + 2, K + 8), 7.0, device="cuda")
+    H = wide[1:K + 1, 4:K + 4]
+    H.copy_(s + s.t())
+    ref = H.double() + 2 * x.double().t() @ x.double()
+    ops.hessian_accumulate_(H, x)
+    assert torch.equal(H, H.t())
+    bound = H.double().abs() + 2 * x.double().abs().t() @ x.double().abs()
+    assert ((H.double() - ref).abs() / bound).max().item() < 1e-5
+    H.fill_(7.0)
+    assert bool((wide == 7.0).all())
