@@ -1,14 +1,12 @@
 // GPTQ quantize_weight: blocked column loop with error feedback.
 //
 // Rows of W are independent given the inverse-Hessian factor U, so a workgroup owns a set of rows and never
-// synchronises with another one inside a block of columns.  The block's 128x128 slice of U sits in LDS, a
-// row's columns of the block in registers.  Per column: quantise, form err = (w - q)/U[i][i] and subtract
-// err * U[i][c] from the columns behind it (U is zero below the diagonal, so no masking is needed).
-//   * quantiser (gptq_block_kernel): 4 lanes per row, 32 columns per lane as 8 runs of 4 neighbouring
-//     columns; a run is quantised start to finish inside its lane (layout described at the Q* constants).
-//   * SparseGPT (sgpt_block_kernel): 16 lanes per row, 8 columns per lane; the column's value and prune flag
-//     are broadcast inside the team and every lane forms the error.
-// After the block, W[:, i2:] -= Err * U[i1:i2, i2:] runs as a matrix-core GEMM (llmc_gemm_f32).
+// synchronises with another one inside a group of columns.  Per column: quantise, form err = (w - q)/U[i][i] and
+// subtract err * U[i][c] from the columns behind it (U is zero below the diagonal, so no masking is needed).
+//   * quantiser: one launch per group of up to 512 columns (gptq_group.h has the layout).
+//   * SparseGPT (sgpt_block_kernel): one launch per block, 16 lanes per row, 8 columns per lane; the block's slice of
+//     U sits in LDS, the column's value and prune flag are broadcast inside the team and every lane forms the error.
+// After the group, W[:, gend:] -= Err * U[g0:gend, gend:] runs as a matrix-core GEMM (llmc_gemm_f32).
 #include <vector>
 
 #include "gemm_f32.h"
