@@ -46,9 +46,20 @@ void require_gpu(const Tensor& t) {
               " tensor (there is no CPU fallback)");
 }
 
+// The dispatcher picks these implementations when any argument is on the GPU, so every tensor is checked by itself:
+// first the one that names the call's device, then the others against it, before a pointer is taken.
+void require_beside(const Tensor& first, const Tensor& t) {
+  require_gpu(t);
+  TORCH_CHECK(t.device() == first.device(), "expected every tensor on ", first.device(), ", got one on ", t.device());
+}
+void require_beside(const Tensor& first, const optional<Tensor>& t) {
+  if (t.has_value()) require_beside(first, *t);
+}
+
 const void* ptr(const optional<Tensor>& t) { return t.has_value() ? t->const_data_ptr() : nullptr; }
 
 void require_rows(const Tensor& x) {
+  require_gpu(x);
   TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1, "expected a 2-D tensor with unit column stride");
 }
 
@@ -57,10 +68,10 @@ Tensor scratch(const Tensor& like, int64_t bytes) {
   return at::empty({bytes}, like.options().dtype(at::kByte));
 }
 
-// the kernels read the global scale as one fp32 value
-optional<Tensor> global32(const optional<Tensor>& gs) {
+// the kernels read the global scale as one fp32 value beside the call's first tensor
+optional<Tensor> global32(const Tensor& first, const optional<Tensor>& gs) {
   if (!gs.has_value()) return gs;
-  require_gpu(*gs);
+  require_beside(first, gs);
   return gs->to(at::kFloat).contiguous();
 }
 
@@ -68,7 +79,8 @@ optional<Tensor> global32(const optional<Tensor>& gs) {
 
 void hessian_launch(Tensor& H, const Tensor& X, double alpha, bool symmetric, bool use_workspace, float* count,
                     float add) {
-  require_gpu(X);
+  require_gpu(H);
+  require_beside(H, X);
   TORCH_CHECK(H.scalar_type() == at::kFloat && H.dim() == 2 && H.size(0) == H.size(1) && H.stride(1) == 1,
               "hessian_accum_: H must be a square fp32 matrix with unit column stride");
   TORCH_CHECK(X.dim() >= 1 && X.size(-1) == H.size(0), "hessian_accum_: X must be [..., ", H.size(0), "]");
@@ -90,8 +102,11 @@ void hessian_accum_(Tensor& H, const Tensor& X, double alpha, bool symmetric, bo
 
 void hessian_accum_counted_(Tensor& H, const Tensor& X, Tensor& count, double samples, double alpha, bool symmetric,
                             bool use_workspace) {
-  TORCH_CHECK(count.device() == H.device() && count.scalar_type() == at::kFloat && count.numel() == 1,
-              "hessian_accum_counted_: the sample count must be one fp32 value on H's device");
+  require_gpu(H);
+  require_beside(H, X);
+  require_beside(H, count);
+  TORCH_CHECK(count.scalar_type() == at::kFloat && count.numel() == 1,
+              "hessian_accum_counted_: the sample count must be one fp32 value");
   hessian_launch(H, X, alpha, symmetric, use_workspace, count.data_ptr<float>(), (float)samples);
 }
 
@@ -129,6 +144,7 @@ Pair minmax_observe_blocks(const Tensor& W, int64_t bh, int64_t bw) {
 }
 
 Pair minmax_observe_strided(const Tensor& x, int64_t n0, int64_t n1, int64_t group, int64_t s0, int64_t s1) {
+  require_gpu(x);
   const int dt = dtype_code(x);
   Guard guard(x.device());
   Tensor mn = at::empty({n1}, x.options()), mx = at::empty({n1}, x.options());
@@ -185,6 +201,7 @@ Pair mse_observe_blocks(const Tensor& W, int64_t bh, int64_t bw, int64_t fmt, in
 Pair mse_observe_strided(const Tensor& x, int64_t n0, int64_t n1, int64_t group, int64_t s0, int64_t s1, int64_t fmt,
                          int64_t bits, bool symmetric, int64_t mode, double maxshrink, int64_t patience, double grid,
                          double norm, double expand) {
+  require_gpu(x);
   const int dt = dtype_code(x), steps = search_steps(maxshrink, grid);
   Guard guard(x.device());
   Tensor mn = at::empty({n1}, x.options()), mx = at::empty({n1}, x.options());
@@ -199,9 +216,14 @@ Pair mse_observe_strided(const Tensor& x, int64_t n0, int64_t n1, int64_t group,
 
 // ---- scales
 
+void require_stats(const Tensor& first, at::TensorList mins, at::TensorList maxs) {
+  require_gpu(first);
+  for (const Tensor& t : mins) require_beside(first, t);
+  for (const Tensor& t : maxs) require_beside(first, t);
+}
+
 void global_scale_into(at::TensorList mins, at::TensorList maxs, const Tensor& out) {
   const Tensor& mn0 = mins[0];
-  require_gpu(mn0);
   Guard guard(mn0.device());
   void* st = stream_of(mn0);
   const int64_t nws = llmc_global_scale_workspace_bytes();
@@ -216,22 +238,25 @@ void global_scale_into(at::TensorList mins, at::TensorList maxs, const Tensor& o
 }
 
 Tensor global_scale(at::TensorList mins, at::TensorList maxs) {
+  require_stats(mins[0], mins, maxs);
   Tensor out = at::empty({1}, mins[0].options().dtype(at::kFloat));
   global_scale_into(mins, maxs, out);
   return out;
 }
 
 void global_scale_into_(at::TensorList mins, at::TensorList maxs, Tensor& out) {
-  TORCH_CHECK(out.scalar_type() == at::kFloat && out.numel() == 1 && out.device() == mins[0].device(),
-              "global_scale_into_: the output must be one fp32 value on the statistics' device");
+  require_stats(out, mins, maxs);
+  TORCH_CHECK(out.scalar_type() == at::kFloat && out.numel() == 1,
+              "global_scale_into_: the output must be one fp32 value");
   global_scale_into(mins, maxs, out);
 }
 
 std::tuple<Tensor, Tensor, optional<Tensor>> qparams(const Tensor& min_vals, const Tensor& max_vals, int64_t fmt,
                                                      int64_t bits, bool symmetric, int64_t mode,
                                                      const optional<Tensor>& global_scale, bool want_codes) {
-  require_gpu(max_vals);
-  const optional<Tensor> gs = global32(global_scale);
+  require_gpu(min_vals);
+  require_beside(min_vals, max_vals);
+  const optional<Tensor> gs = global32(min_vals, global_scale);
   const Tensor mn = min_vals.contiguous(), mx = max_vals.contiguous();
   const int dt = dtype_code(mn);
   Guard guard(mn.device());
@@ -251,16 +276,19 @@ std::tuple<Tensor, Tensor, optional<Tensor>> qparams(const Tensor& min_vals, con
 // or one byte per group where the parameter holds the stored codes; `zp` has one byte per group
 void qparams_into_(const Tensor& min_vals, const Tensor& max_vals, Tensor& scale, const optional<Tensor>& zp,
                    int64_t fmt, int64_t bits, bool symmetric, int64_t mode, const optional<Tensor>& global_scale) {
-  const optional<Tensor> gs = global32(global_scale);
+  require_gpu(min_vals);
+  require_beside(min_vals, max_vals);
+  require_beside(min_vals, scale);
+  require_beside(min_vals, zp);
+  const optional<Tensor> gs = global32(min_vals, global_scale);
   const Tensor mn = min_vals.contiguous(), mx = max_vals.contiguous();
   const int dt = dtype_code(mn);
   const bool coded = scale.element_size() == 1;
   const int sdt = mode == LLMC_SCALE_NVFP4 ? LLMC_F32 : dt;
-  TORCH_CHECK(scale.device() == mn.device() && scale.is_contiguous() && scale.numel() == mn.numel() &&
+  TORCH_CHECK(scale.is_contiguous() && scale.numel() == mn.numel() &&
                   (coded ? mode != LLMC_SCALE_PLAIN : dtype_code(scale) == sdt),
               "qparams_into_: the scale does not fit the statistics");
-  TORCH_CHECK(!zp.has_value() || (zp->device() == mn.device() && zp->is_contiguous() && zp->element_size() == 1 &&
-                                  zp->numel() == mn.numel()),
+  TORCH_CHECK(!zp.has_value() || (zp->is_contiguous() && zp->element_size() == 1 && zp->numel() == mn.numel()),
               "qparams_into_: the zero point does not fit the statistics");
   Guard guard(mn.device());
   check(llmc_calculate_qparams(mn.const_data_ptr(), mx.const_data_ptr(), mn.numel(), dt, (int)fmt, (int)bits,
@@ -278,13 +306,21 @@ int scale_code(const Tensor& scale) {
   return dtype_code(scale);
 }
 
+void require_quantize(const Tensor& x, const Tensor& scale, const optional<Tensor>& zero_point,
+                      const optional<Tensor>& g_idx, const optional<Tensor>& global_scale) {
+  require_rows(x);
+  require_beside(x, scale);
+  require_beside(x, zero_point);
+  require_beside(x, g_idx);
+  require_beside(x, global_scale);
+}
+
 Tensor quantize_launch(const Tensor& x, const Tensor& scale_, const optional<Tensor>& zero_point, int64_t fmt,
                        int64_t bits, int64_t row_div, int64_t srow, int64_t col_div, int64_t out_mode,
                        const optional<Tensor>& g_idx_, const optional<Tensor>& global_scale,
                        optional<at::ScalarType> out_dtype, int64_t* shape_out) {
-  require_gpu(scale_);
-  require_rows(x);
-  const optional<Tensor> gs = global32(global_scale);
+  require_quantize(x, scale_, zero_point, g_idx_, global_scale);
+  const optional<Tensor> gs = global32(x, global_scale);
   const int64_t R = x.size(0), K = x.size(1);
   const Tensor scale = scale_.contiguous();
   optional<Tensor> zp, g_idx;
@@ -333,6 +369,7 @@ Tensor quant_pack(const Tensor& x, const Tensor& scale, const optional<Tensor>& 
 Pair quant_pack_shaped(const Tensor& x, const Tensor& scale, const optional<Tensor>& zp, int64_t fmt, int64_t bits,
                        int64_t row_div, int64_t srow, int64_t col_div, int64_t out_mode,
                        const optional<Tensor>& g_idx, const optional<Tensor>& global_scale) {
+  require_quantize(x, scale, zp, g_idx, global_scale);
   Tensor shape = at::empty({2}, x.options().dtype(at::kLong));
   Tensor out = quantize_launch(x, scale, zp, fmt, bits, row_div, srow, col_div, out_mode, g_idx, global_scale,
                                c10::nullopt, shape.data_ptr<int64_t>());
@@ -354,6 +391,7 @@ Pair fp8_dynamic_per_token(const Tensor& X, int64_t fmt, int64_t bits, int64_t o
 
 // fake-quantised activations of any shape whose last dimension holds the columns: each row's, or each group's, own scale
 Tensor dynamic_token_quantize(const Tensor& x, int64_t fmt, int64_t bits) {
+  require_gpu(x);
   const Tensor X = x.contiguous();
   Guard guard(X.device());
   const int64_t K = X.size(-1), N = X.numel() / K;
@@ -366,7 +404,8 @@ Tensor dynamic_token_quantize(const Tensor& x, int64_t fmt, int64_t bits) {
 
 Tensor dynamic_group_quantize(const Tensor& x, int64_t group, int64_t fmt, int64_t bits, int64_t mode,
                               const optional<Tensor>& global_scale) {
-  const optional<Tensor> gs = global32(global_scale);
+  require_gpu(x);
+  const optional<Tensor> gs = global32(x, global_scale);
   const Tensor X = x.contiguous();
   Guard guard(X.device());
   const int64_t K = X.size(-1), N = X.numel() / K;
