@@ -216,10 +216,22 @@ Pair mse_observe_strided(const Tensor& x, int64_t n0, int64_t n1, int64_t group,
 
 // ---- scales
 
-void require_stats(const Tensor& first, at::TensorList mins, at::TensorList maxs) {
-  require_gpu(first);
-  for (const Tensor& t : mins) require_beside(first, t);
-  for (const Tensor& t : maxs) require_beside(first, t);
+// the kernels walk a minimum and its maximum by one index and read both in one dtype
+void require_pair(const Tensor& mn, const Tensor& mx) {
+  TORCH_CHECK_VALUE(mn.numel() == mx.numel() && mn.scalar_type() == mx.scalar_type(),
+                    "minima and maxima must agree in size and dtype, got ", mn.sizes(), " ", mn.scalar_type(), " and ",
+                    mx.sizes(), " ", mx.scalar_type());
+}
+
+void require_stats(at::TensorList mins, at::TensorList maxs) {
+  TORCH_CHECK_VALUE(!mins.empty() && mins.size() == maxs.size(), "expected one array of maxima per array of minima and "
+                    "at least one of each, got ", mins.size(), " of minima and ", maxs.size(), " of maxima");
+  require_gpu(mins[0]);
+  for (size_t i = 0; i < mins.size(); ++i) {
+    require_beside(mins[0], mins[i]);
+    require_beside(mins[0], maxs[i]);
+    require_pair(mins[i], maxs[i]);
+  }
 }
 
 void global_scale_into(at::TensorList mins, at::TensorList maxs, const Tensor& out) {
@@ -238,14 +250,15 @@ void global_scale_into(at::TensorList mins, at::TensorList maxs, const Tensor& o
 }
 
 Tensor global_scale(at::TensorList mins, at::TensorList maxs) {
-  require_stats(mins[0], mins, maxs);
+  require_stats(mins, maxs);
   Tensor out = at::empty({1}, mins[0].options().dtype(at::kFloat));
   global_scale_into(mins, maxs, out);
   return out;
 }
 
 void global_scale_into_(at::TensorList mins, at::TensorList maxs, Tensor& out) {
-  require_stats(out, mins, maxs);
+  require_stats(mins, maxs);
+  require_beside(mins[0], out);
   TORCH_CHECK(out.scalar_type() == at::kFloat && out.numel() == 1,
               "global_scale_into_: the output must be one fp32 value");
   global_scale_into(mins, maxs, out);
@@ -256,6 +269,7 @@ std::tuple<Tensor, Tensor, optional<Tensor>> qparams(const Tensor& min_vals, con
                                                      const optional<Tensor>& global_scale, bool want_codes) {
   require_gpu(min_vals);
   require_beside(min_vals, max_vals);
+  require_pair(min_vals, max_vals);
   const optional<Tensor> gs = global32(min_vals, global_scale);
   const Tensor mn = min_vals.contiguous(), mx = max_vals.contiguous();
   const int dt = dtype_code(mn);
@@ -278,6 +292,7 @@ void qparams_into_(const Tensor& min_vals, const Tensor& max_vals, Tensor& scale
                    int64_t fmt, int64_t bits, bool symmetric, int64_t mode, const optional<Tensor>& global_scale) {
   require_gpu(min_vals);
   require_beside(min_vals, max_vals);
+  require_pair(min_vals, max_vals);
   require_beside(min_vals, scale);
   require_beside(min_vals, zp);
   const optional<Tensor> gs = global32(min_vals, global_scale);

@@ -67,3 +67,25 @@ def test_a_tensor_of_another_gpu_in_any_place_is_refused(name, position):
     args = [_fake("cuda:1" if i == position else "cuda:0", *s, dtype=d) for i, (s, d) in enumerate(tensors)]
     with pytest.raises(RuntimeError, match="expected every tensor on cuda:"):
         _call(name, *build(*args))
+
+
+def _stats(*sizes, dtype=torch.float32):
+    return [_fake("cuda:0", n, dtype=dtype) for n in sizes]
+
+
+@pytest.mark.parametrize("mins,maxs", [((4,), ()), ((4, 4), (4,)), ((4,), (4, 4)), ((), ())])
+def test_global_scale_refuses_lists_that_do_not_pair_up(mins, maxs):
+    out = _fake("cuda:0", 1, dtype=torch.float32)
+    with pytest.raises(ValueError, match="one array of maxima per array of minima"):
+        _call("global_scale_into_", _stats(*mins), _stats(*maxs), out)
+    with pytest.raises(ValueError, match="one array of maxima per array of minima"):
+        _call("global_scale", _stats(*mins), _stats(*maxs))
+
+
+@pytest.mark.parametrize("mn,mx", [((8, torch.float32), (4, torch.float32)), ((4, torch.float32), (4, torch.bfloat16))])
+def test_minima_and_maxima_of_another_size_or_dtype_are_refused(mn, mx):
+    a, b = (_fake("cuda:0", n, dtype=d) for n, d in (mn, mx))
+    for call in (lambda: _call("global_scale", [b, a], [b, b]), lambda: _call("qparams", a, b, 0, 4, True),
+                 lambda: _call("qparams_into_", a, b, a, None, 0, 4, True)):
+        with pytest.raises(ValueError, match="must agree in size and dtype"):
+            call()
