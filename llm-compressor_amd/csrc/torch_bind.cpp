@@ -11,6 +11,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
+#include <cmath>
 #include <tuple>
 
 #include "llmc_amd.h"
@@ -157,6 +158,7 @@ Pair minmax_observe_strided(const Tensor& x, int64_t n0, int64_t n1, int64_t gro
 // ---- MSE observers
 
 int search_steps(double maxshrink, double grid) {
+  TORCH_CHECK_VALUE(std::isfinite(maxshrink * grid), "MSE observer: maxshrink * grid is not finite");
   const int64_t steps = (int64_t)(maxshrink * grid);
   TORCH_CHECK_VALUE(steps <= 256, "MSE observer: int(maxshrink*grid)=", steps,
                     " search steps exceed the supported 256");
@@ -404,9 +406,14 @@ Pair fp8_dynamic_per_token(const Tensor& X, int64_t fmt, int64_t bits, int64_t o
   return {out, scale};
 }
 
+void require_columns(const Tensor& x) {
+  require_gpu(x);
+  TORCH_CHECK_VALUE(x.dim() > 0 && x.size(-1) > 0, "expected a value with columns, got ", x.sizes());
+}
+
 // fake-quantised activations of any shape whose last dimension holds the columns: each row's, or each group's, own scale
 Tensor dynamic_token_quantize(const Tensor& x, int64_t fmt, int64_t bits) {
-  require_gpu(x);
+  require_columns(x);
   const Tensor X = x.contiguous();
   Guard guard(X.device());
   const int64_t K = X.size(-1), N = X.numel() / K;
@@ -419,7 +426,7 @@ Tensor dynamic_token_quantize(const Tensor& x, int64_t fmt, int64_t bits) {
 
 Tensor dynamic_group_quantize(const Tensor& x, int64_t group, int64_t fmt, int64_t bits, int64_t mode,
                               const optional<Tensor>& global_scale) {
-  require_gpu(x);
+  require_columns(x);
   const optional<Tensor> gs = global32(x, global_scale);
   const Tensor X = x.contiguous();
   Guard guard(X.device());

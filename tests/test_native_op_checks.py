@@ -89,3 +89,18 @@ def test_minima_and_maxima_of_another_size_or_dtype_are_refused(mn, mx):
                  lambda: _call("qparams_into_", a, b, a, None, 0, 4, True)):
         with pytest.raises(ValueError, match="must agree in size and dtype"):
             call()
+
+
+@pytest.mark.parametrize("shape", [(0,), (3, 0), (0, 0), ()])
+def test_a_value_without_columns_is_refused(shape):
+    x = _fake("cuda:0", *shape)
+    for call in (lambda: _call("dynamic_token_quantize", x, 1, 8), lambda: _call("dynamic_group_quantize", x, 16, 1, 8)):
+        with pytest.raises(ValueError, match="a value with columns"):
+            call()
+
+
+@pytest.mark.parametrize("maxshrink,grid", [(float("nan"), 100.0), (0.2, float("inf")), (1e300, 1e300)])
+def test_a_search_range_that_is_not_finite_is_refused(maxshrink, grid):
+    w = _fake("cuda:0", 4, 32)
+    with pytest.raises(ValueError, match="not finite"):
+        _call("mse_observe", w, 16, 0, 4, True, 0, maxshrink, 5, grid)
