@@ -86,14 +86,16 @@ void hessian_launch(Tensor& H, const Tensor& X, double alpha, bool symmetric, bo
               "hessian_accum_: H must be a square fp32 matrix with unit column stride");
   TORCH_CHECK(X.dim() >= 1 && X.size(-1) == H.size(0), "hessian_accum_: X must be [..., ", H.size(0), "]");
   const int dt = dtype_code(X);
-  const bool rows = X.dim() == 2 && X.stride(1) == 1;
+  // rows that lie at least K apart are read where they are; an expanded value's overlap
+  const bool rows = X.dim() == 2 && X.stride(1) == 1 && X.stride(0) >= X.size(1);
   const Tensor x = rows ? X : X.reshape({-1, X.size(-1)}).contiguous();
+  const int64_t ldx = rows ? x.stride(0) : x.size(1);  // (the stride of a single contiguous row can be anything)
   Guard guard(H.device());
   const int64_t nws = use_workspace && dt != LLMC_F32 ? llmc_hessian_workspace_bytes(x.size(0), x.size(1)) : 0;
   const Tensor ws = nws ? scratch(H, nws) : Tensor();
-  check(llmc_hessian_accumulate_counted(H.data_ptr<float>(), H.stride(0), x.const_data_ptr(), x.stride(0), x.size(0),
-                                        x.size(1), dt, (float)alpha, symmetric ? LLMC_HESSIAN_ASSUME_SYMMETRIC : 0,
-                                        count, add, nws ? ws.data_ptr() : nullptr, nws, stream_of(H)),
+  check(llmc_hessian_accumulate_counted(H.data_ptr<float>(), H.stride(0), x.const_data_ptr(), ldx, x.size(0), x.size(1),
+                                        dt, (float)alpha, symmetric ? LLMC_HESSIAN_ASSUME_SYMMETRIC : 0, count, add,
+                                        nws ? ws.data_ptr() : nullptr, nws, stream_of(H)),
         "llmc_hessian_accumulate");
 }
 

@@ -278,3 +278,20 @@ def test_hessian_tiles_that_reach_past_the_last_column(T, K):
     assert ((H.double() - ref).abs() / bound).max().item() < 1e-5
     H.fill_(7.0)
     assert bool((wide == 7.0).all())
+
+
+@pytest.mark.parametrize("shape", [(64, 256), (1, 256), (2, 32, 256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_hessian_hook_takes_values_whose_rows_overlap(shape, dtype):
+    """An expanded value repeats its memory: its rows lie less than a row apart, and the hook copies it first."""
+    from llmcompressor_amd.modifiers.gptq.gptq_quantize import accumulate_hessian
+
+    K = shape[-1]
+    linear = torch.nn.Linear(K, 1, bias=False, device="cuda")
+    row = torch.randn(K, device="cuda").to(dtype)
+    for x in (row.expand(shape), torch.randn(K + 64, device="cuda").to(dtype).as_strided(shape, (1,) * len(shape))):
+        got, want = torch.zeros(K, K, device="cuda"), torch.zeros(K, K, device="cuda")
+        n0, n1 = torch.zeros((), device="cuda"), torch.zeros((), device="cuda")
+        got, n0 = accumulate_hessian(x, linear, got, n0)
+        want, n1 = accumulate_hessian(x.clone(memory_format=torch.contiguous_format), linear, want, n1)
+        assert torch.equal(got, want) and n0.item() == n1.item() > 0
