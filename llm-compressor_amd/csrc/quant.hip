@@ -493,6 +493,9 @@ int log2_exact(int64_t v) {  // log2 of a power of two, -1 otherwise
   return n;
 }
 
+// units are numbered in 32 bits, with room for the last workgroup's lanes past the end
+bool units_fit(int64_t R, int64_t per_row) { return R <= ((1LL << 32) - 256) / per_row; }
+
 void walk_rows(RowsWalk& w, int64_t R, int64_t K, int e) {
   w.per_row = (uint32_t)(K / e);
   w.units = (uint32_t)(R * w.per_row);
@@ -504,7 +507,7 @@ void walk_rows(RowsWalk& w, int64_t R, int64_t K, int e) {
 bool try_launch_rows(const QuantParams& p, hipStream_t st) {
   if (p.x_dt == LLMC_F32 || p.g_idx || p.K % 8 || p.ldx % 8 || ((uintptr_t)p.x & 15)) return false;
   const int e = p.K % 16 ? 8 : 16;
-  if (p.K > (1LL << 30) || p.R > (1LL << 32) / (p.K / e) - 256) return false;
+  if (p.K > (1LL << 30) || !units_fit(p.R, p.K / e)) return false;
   const int sm = p.gscale ? SM_GLOBAL
                  : p.scale_dt == LLMC_E8M0 ? SM_E8M0
                  : p.scale_dt == LLMC_F32 || p.scale_dt == LLMC_E4M3 ? SM_F32 : SM_SAME;
@@ -895,7 +898,7 @@ extern "C" int llmc_dynamic_group_quantize(const void* x, int32_t x_dtype, int64
                                            const float* global_scale, void* out, int64_t ldo, void* stream) {
   LLMC_CHECK_ARG(x && N > 0 && K > 0 && (((uintptr_t)x) & 15) == 0, 1);
   LLMC_CHECK_ARG(x_dtype == LLMC_BF16 || (x_dtype == LLMC_F16 && scale_mode != LLMC_SCALE_MXFP4), 2);
-  LLMC_CHECK_ARG(K <= (1LL << 30) && N <= (1LL << 32) / ((K + 15) / 16) - 256, 4);
+  LLMC_CHECK_ARG(K <= (1LL << 30) && units_fit(N, (K + 15) / 16), 4);
   LLMC_CHECK_ARG(ldx >= K && ldx % 8 == 0, 5);
   const int lg = log2_exact(group);
   LLMC_CHECK_ARG(lg >= 4 && lg <= 10 && K % group == 0, 6);

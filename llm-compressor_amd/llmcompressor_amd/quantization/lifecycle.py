@@ -215,9 +215,12 @@ def _run_quantize(x, scale, zero_point, args: QuantizationArgs, out_mode, g_idx=
 
 def _fused_group_mode(x2: torch.Tensor, args: QuantizationArgs, global_scale) -> Optional[int]:
     """The scale mode of llmc_dynamic_group_quantize when it takes these arguments, else None: symmetric groups of a
-    power of two between 16 and 1024 columns of 16-bit values, integers of 4 or 8 bits."""
+    power of two between 16 and 1024 columns of 16-bit values, integers of 4 or 8 bits, runs of 16 columns numbered
+    in 32 bits and a row of at most 2^30."""
     g = args.group_size
     if not args.symmetric or g < 16 or g > 1024 or g & (g - 1) or x2.data_ptr() % 16:
+        return None
+    if x2.shape[1] > 1 << 30 or x2.numel() // 16 > (1 << 32) - 256:
         return None
     if args.type == QuantizationType.INT and args.num_bits not in (4, 8):
         return None

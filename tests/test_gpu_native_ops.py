@@ -159,3 +159,14 @@ def test_mse_search_over_blocks_equals_its_rows_form(rows, cols, bh, bw):
     if bh * bw % 8 == 0 and (bh * bw // 8) & (bh * bw // 8 - 1) == 0 and bh * bw <= 512:
         return  # such groups take the other kernel, whose sums run in another order
     assert torch.equal(mn.reshape(-1), emn.reshape(-1)) and torch.equal(mx.reshape(-1), emx.reshape(-1))
+
+
+def test_dynamic_groups_of_one_very_wide_row():
+    """2^28 columns in one row are 2^24 runs of 16: far below the 2^32 that the kernel numbers."""
+    from llmcompressor_amd import ops
+
+    llmc = _llmc()
+    x = torch.randn(1, 1 << 28, device="cuda", dtype=torch.bfloat16)
+    got = llmc.dynamic_group_quantize(x, 32, ops.FMT_FP8, 8)
+    want = llmc.dynamic_group_quantize(x.view(1 << 14, -1), 32, ops.FMT_FP8, 8)
+    assert torch.equal(got.view_as(want), want)
