@@ -110,12 +110,18 @@ def _run(weight, scale, zp, args: QuantizationArgs, mode, g_idx=None, global_sca
 
 
 def _tensor_of(module: torch.nn.Module, name: str) -> Optional[torch.Tensor]:
-    """``module.<name>`` without the failing attribute lookups (a microsecond each) for the names it does not have."""
+    """``module.<name>`` or None, without the failing attribute lookup (a microsecond) where the name can only be in the
+    module's own dicts: a class with its own ``__getattr__`` (a wrapper that forwards to the module it holds), or with
+    the name itself (a property), is asked the ordinary way."""
+    cls = type(module)
+    if (cls.__getattr__ is not torch.nn.Module.__getattr__ or cls.__getattribute__ is not object.__getattribute__
+            or hasattr(cls, name)):
+        return getattr(module, name, None)
     d = module.__dict__
-    for where in (d["_parameters"], d["_buffers"], d):
+    for where in (d, d["_parameters"], d["_buffers"], d["_modules"]):
         if name in where:
             return where[name]
-    return getattr(module, name, None) if hasattr(type(module), name) else None
+    return None
 
 
 def compress_module(module: torch.nn.Module, fmt: Optional[str] = None) -> Dict[str, torch.Tensor]:
