@@ -206,7 +206,7 @@ class Observer(torch.nn.Module):
                      global_scale: Optional[torch.Tensor]) -> bool:
         """``get_qparams`` written straight into a module's parameters (device tensors; the scale parameter may hold
         stored codes), without the temporaries and copies in between.  False, with nothing done, where the
-        parameters' shapes or dtypes ask for the conversions of the general path."""
+        parameters' shapes, dtypes or devices ask for the conversions and copies of the general path."""
         if type(self).get_qparams is not Observer.get_qparams or type(self).get_global_scale is not Observer.get_global_scale:
             return False
         args, mn, mx = self.args, self.min_vals, self.max_vals
@@ -218,14 +218,15 @@ class Observer(torch.nn.Module):
             fits = scale.dtype in (torch.float8_e4m3fn, torch.float32)
         else:
             fits = scale.dtype == torch.uint8 and mn.dtype == torch.bfloat16
-        if not (fits and scale.is_cuda and scale.shape == mn.shape and scale.is_contiguous()):
+        if not (fits and scale.is_cuda and scale.device == mn.device and scale.shape == mn.shape and scale.is_contiguous()):
             return False
         if zero_point is not None and not (
                 zero_point.device == scale.device and zero_point.shape == mn.shape and zero_point.is_contiguous()
                 and (zero_point.dtype == torch.int8 or (args.symmetric and zero_point.element_size() == 1))):
             return False
         if grouped:
-            if global_scale is None or global_scale.dtype != torch.float32 or global_scale.shape != (1,):
+            if (global_scale is None or global_scale.device != mn.device or global_scale.dtype != torch.float32
+                    or global_scale.shape != (1,)):
                 return False
             stats = self.fusion_handler.get_fused_statistics()
             llmc.global_scale_into_([s["min_vals"] for s in stats], [s["max_vals"] for s in stats], global_scale)
