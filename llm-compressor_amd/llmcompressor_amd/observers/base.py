@@ -162,8 +162,11 @@ class Observer(torch.nn.Module):
 
     def update_statistics(self, min_vals: torch.Tensor, max_vals: torch.Tensor) -> None:
         """Fold a fresh (min, max) into the running statistics (memoryless: replace)."""
-        own = self.__dict__  # plain tensors: nothing for Module.__setattr__ to register
-        own["min_vals"], own["max_vals"] = min_vals, max_vals
+        if self._buffers or self._parameters:  # a subclass may have registered them
+            self.min_vals, self.max_vals = min_vals, max_vals
+        else:  # plain tensors: nothing for Module.__setattr__ to register
+            own = self.__dict__
+            own["min_vals"], own["max_vals"] = min_vals, max_vals
 
     def update_statistics_from_observed(self, observed: torch.Tensor) -> None:
         """Reference entry point: ``observed`` is already flattened to (num_observations, *qparam_shape, group)."""

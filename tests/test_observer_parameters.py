@@ -35,3 +35,19 @@ def test_parameters_of_another_device_are_left_to_the_general_path(monkeypatch, 
     assert done is (not where)
     assert calls == ([] if where else ["global_scale", "qparams"] if grouped else ["qparams"])
     assert observer.has_statistics is bool(where)
+
+
+def test_statistics_that_a_subclass_registers_are_written_where_it_keeps_them():
+    class Buffered(Observer):
+        def __init__(self, **kw):
+            super().__init__(**kw)
+            self.register_buffer("min_vals", torch.zeros(2))
+            self.register_buffer("max_vals", torch.zeros(2))
+
+    args = preset_name_to_scheme("W8A16", ["Linear"]).weights
+    observer = Buffered(base_name="weight", args=args)
+    observer.update_statistics(torch.tensor([-1.0, -2.0]), torch.tensor([3.0, 4.0]))
+    assert observer.state_dict()["min_vals"].tolist() == [-1.0, -2.0]
+    assert observer.state_dict()["max_vals"].tolist() == [3.0, 4.0]
+    observer.delete_statistics()
+    assert not observer.has_statistics
