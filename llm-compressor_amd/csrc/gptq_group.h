@@ -12,8 +12,8 @@
 //     inside a turn; after the last turn of a run every lane holds its columns' values and errors;
 //   * a turn's four errors reach the team as DPP operands (an immediate lane number, hence the unrolled turns), without
 //     a pass through LDS;
-//   * a division is two operations (two_step_div below); a wave that meets a divisor or a value outside the range
-//     where that holds repeats its block with plain divisions.
+//   * a division is three operations (quotient() below); a wave that meets a divisor or a value outside the range
+//     where that gives the IEEE quotient repeats its block with plain divisions.
 // Before block b is quantised, the group's earlier errors are taken off its columns on the matrix cores,
 // W[:, b] - E U[:, b], as 16 x 16 tiles accumulated by v_mfma_f32_16x16x4_f32 in fp32.
 //
@@ -89,19 +89,25 @@ constexpr int q_smem(int team, bool has_zp) {
 #ifdef LLMC_GPTQ_GROUP_KERNELS
 namespace {
 
-// x / s in two operations from yh = 1/s rounded (hardware estimate and one Newton step) and yl = (1/s - yh) rounded:
-// RN(x * yh + RN(x * yl)).  The sum before the last rounding is within 2^-46 (relative) of x / s, so the result is the
-// IEEE quotient except where x / s lies within 2^-22 of an ulp of a midpoint between two floats, where it is the
-// other neighbour: an error of at most 0.5000003 ulp against 0.5.  Holds while s is in [2^-100, 2^100] and x is finite;
-// outside, the reciprocal is NaN (or the result is not finite) and the caller falls back to plain divisions.  The
-// addend +0 of the low product turns a -0 quotient into +0, as adding a zero point of zero does.
-__device__ __forceinline__ void two_step_reciprocal(const float s, float& yh, float& yl) {
-  const float a = fabsf(s), y0 = __builtin_amdgcn_rcpf(s), y = fmaf(fmaf(-s, y0, 1.0f), y0, y0);
-  const bool ok = a >= 0x1p-100f && a <= 0x1p100f;
-  yl = fmaf(-s, y, 1.0f) * y;
-  yh = ok ? y : __builtin_nanf("");
+// The IEEE quotient x / s in three operations, from y = 1/s (hardware estimate, within an ulp, and one Newton step):
+// q = RN(x y) is within 1.5 ulp of x / s, its residual x - q s is exact, and RN(q + residual * y) errs by no more than
+// 1.5 * 2^-24 ulp (3 * 2^-24 where y is an ulp off) before its own rounding.  A quotient of two 24-bit numbers keeps
+// 2^-25 ulp and multiples of that from every midpoint, so only numerators within a few such steps of one can go wrong;
+// all 360 million of those up to 16 steps were tried, and every numerator of the 32 divisors whose y need not be the
+// rounded reciprocal.  Two pairs fail, with the significands 0xfffffd and 0xffffff as divisors; those are refused.
+// Refused divisors (also outside [2^-46, 2^46], where a quotient that matters could under- or overflow on the way) have
+// a NaN reciprocal, and the caller falls back to plain divisions.  A numerator below 2^-100 has a subnormal residual, so
+// its quotient can be an ulp off: as a value's it rounds to zero on every grid either way, and as an error's it is
+// 2^-54 at most.  The residual's +0 turns a -0 quotient into +0, as adding a zero point of zero does.
+__device__ __forceinline__ float quotient_reciprocal(const float s) {
+  const float y0 = __builtin_amdgcn_rcpf(s), y = fmaf(fmaf(-s, y0, 1.0f), y0, y0);
+  const bool ok = s >= 0x1p-46f && s <= 0x1p46f && (__float_as_uint(s) & 0x7ffffdu) != 0x7ffffdu;
+  return ok ? y : __builtin_nanf("");
 }
-__device__ __forceinline__ float two_step_div(float x, float yh, float yl) { return fmaf(x, yh, fmaf(x, yl, 0.0f)); }
+__device__ __forceinline__ float quotient(float x, float s, float y) {
+  const float q = x * y;
+  return fmaf(fmaf(-q, s, x), y, q);
+}
 
 template <int SD>
 __device__ __forceinline__ float round_sd(float x) {
@@ -121,9 +127,9 @@ __device__ __forceinline__ float grid_value(float v, float qmin, float qmax) {
 
 // a lane's run: 4 columns of one row, and everything about those columns that its evaluation needs
 struct QRun {
-  float w[QG], s[QG], yh[QG], yl[QG], z[QG];  // values, scales, their reciprocals, zero points
-  float dh[QG], dl[QG];                       // minus reciprocals of U's diagonal; with EXACT dh holds the diagonal
-  float u01, u02, u03, u12, u13, u23;         // the 4 x 4 diagonal block of U above its diagonal
+  float w[QG], s[QG], y[QG], z[QG];    // values, scales, their reciprocals, zero points
+  float dn[QG], dy[QG];                // minus U's diagonal and its reciprocals
+  float u01, u02, u03, u12, u13, u23;  // the 4 x 4 diagonal block of U above its diagonal
 };
 struct QResult {
   float q[QG], e[QG];  // dequantised values and negated scaled errors
@@ -141,13 +147,13 @@ template <int FMT, int SD, bool HAS_ZP, bool EXACT>
 __device__ __forceinline__ void gptq_run(const QRun& r, QResult& o, float qmin, float qmax) {
   float w1 = r.w[1], w2 = r.w[2], w3 = r.w[3];
   auto column = [&](float wv, int m) {
-    float v = EXACT ? wv / r.s[m] + 0.0f : two_step_div(wv, r.yh[m], r.yl[m]);
+    float v = EXACT ? wv / r.s[m] + 0.0f : quotient(wv, r.s[m], r.y[m]);
     if (HAS_ZP) v = v + r.z[m];
     float dq = grid_value<FMT, EXACT>(v, qmin, qmax);
     if (HAS_ZP) dq = round_sd<SD>(dq - r.z[m]);
     o.q[m] = round_sd<SD>(dq * r.s[m]);
     const float x = __fsub_rn(wv, o.q[m]);
-    o.e[m] = EXACT ? -(x / r.dh[m]) : two_step_div(x, r.dh[m], r.dl[m]);
+    o.e[m] = EXACT ? x / r.dn[m] : quotient(x, r.dn[m], r.dy[m]);
     return o.e[m];
   };
   const float e0 = column(r.w[0], 0);
@@ -305,8 +311,8 @@ struct USlice {
   }
 };
 
-// column constants of a block, for thread i < 128 (column i): Ds[comp][quad] float4 with comp 0 = -1/d high parts, 1 = low
-// parts, 2 = u01 u02 u03 u12, 3 = u13 u23
+// column constants of a block, for thread i < 128 (column i): Ds[comp][quad] float4 with comp 0 = -d, 1 = -1/d,
+// 2 = u01 u02 u03 u12, 3 = u13 u23
 struct DColumn {
   float u[QG];  // U[i][4 (i/4) .. + 3]; only entries from the diagonal on are used
   __device__ __forceinline__ void fetch(const float* __restrict__ base, int64_t ldu, int count, int i) {
@@ -322,13 +328,11 @@ struct DColumn {
     float v[QG];
 #pragma unroll
     for (int k = 0; k < QG; ++k) v[k] = i < count && (i & ~3) + k < count ? u[k] : 0.f;
-    const float d = m == 0 ? v[0] : (m == 1 ? v[1] : (m == 2 ? v[2] : v[3]));
-    float dh, dl;
-    two_step_reciprocal(i < count ? d : 1.f, dh, dl);
+    const float di = m == 0 ? v[0] : (m == 1 ? v[1] : (m == 2 ? v[2] : v[3])), d = i < count ? di : 1.f;
     float* q = Ds + quad * 4;
     constexpr int COMP = GB / QG * 4;
-    q[m] = -dh;
-    q[COMP + m] = -dl;
+    q[m] = -d;
+    q[COMP + m] = -quotient_reciprocal(d);
     if (m == 0) {
       q[2 * COMP + 0] = v[1];
       q[2 * COMP + 1] = v[2];
@@ -345,8 +349,8 @@ __device__ __forceinline__ void load_d(QRun& r, const float* __restrict__ Ds, in
   constexpr int COMP = GB / QG * 4;
   const float4 a = *(const float4*)(Ds + quad * 4), b = *(const float4*)(Ds + COMP + quad * 4);
   const float4 c = *(const float4*)(Ds + 2 * COMP + quad * 4), d = *(const float4*)(Ds + 3 * COMP + quad * 4);
-  r.dh[0] = a.x; r.dh[1] = a.y; r.dh[2] = a.z; r.dh[3] = a.w;
-  r.dl[0] = b.x; r.dl[1] = b.y; r.dl[2] = b.z; r.dl[3] = b.w;
+  r.dn[0] = a.x; r.dn[1] = a.y; r.dn[2] = a.z; r.dn[3] = a.w;
+  r.dy[0] = b.x; r.dy[1] = b.y; r.dy[2] = b.z; r.dy[3] = b.w;
   r.u01 = c.x; r.u02 = c.y; r.u03 = c.z; r.u12 = c.w; r.u13 = d.x; r.u23 = d.y;
 }
 
@@ -625,12 +629,8 @@ __global__ __launch_bounds__(Q_THREADS) void gptq_group_kernel(GptqGroupParams p
         r.w[m] = w[J][m];
         r.s[m] = s[J][m];
         r.z[m] = z[J][m];
-        two_step_reciprocal(r.s[m], r.yh[m], r.yl[m]);
-        bad = bad | (r.yh[m] != r.yh[m]);
-        if (EXACT) {
-          const int c = J * SPAN + tl * QG + m;
-          r.dh[m] = c < count ? p.U[(int64_t)(i1 + c) * p.ldu + i1 + c] : 1.f;
-        }
+        r.y[m] = quotient_reciprocal(r.s[m]);
+        bad = bad | (r.y[m] != r.y[m]);
       }
       if constexpr (UNROLL && !EXACT) {
         float ep[QG];
@@ -652,7 +652,7 @@ __global__ __launch_bounds__(Q_THREADS) void gptq_group_kernel(GptqGroupParams p
     float total = 0.f;
 #pragma unroll
     for (int J = 0; J < NRUN; ++J) total += run_loss(o[J]);
-    if (__any(bad || !(total < 0x1p100f))) {
+    if (__any(bad || !(total < 0x1p60f))) {  // every quotient stayed below 2^128 then, or its NaN is in the total
       load_w();
       all_runs(std::true_type{});
     }

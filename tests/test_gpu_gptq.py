@@ -3,6 +3,7 @@
 Tolerances (north star): GPTQ codes agree on >= 99.9 % of the weights and the layer
 reconstruction error ||(W - Q) X|| is within 1 % of the oracle's.
 """
+import numpy as np
 import pytest
 import torch
 
@@ -820,3 +821,83 @@ def test_hinv_grouped_rows_per_workgroup(K, n):
         Hd.diagonal().add_(0.01 * Hd.diagonal().mean())
         err = (Ub.double().t() @ Ub.double() @ Hd - torch.eye(K, device="cuda", dtype=torch.float64)).abs().max()
         assert err < 1e-3, err
+
+
+def _hard_errors(rng, divisors, per_divisor):
+    """Pairs of 24-bit significands (x, d) whose quotient lies as close to a midpoint between two floats as any does:
+    |2^k x - M d| is 1 to 8 for an odd M.  -> d [divisors], x [per_divisor, divisors], float32 in [0.5, 1)."""
+    ds, xs = [], []
+    while len(ds) < divisors:
+        d, row = int(rng.integers(1 << 23, 1 << 24)) | 1, []
+        for k in (24, 25):
+            inverse = pow(1 << k, -1, d)
+            for c in range(1, 9):
+                for sign in (1, -1):
+                    x = sign * c * inverse % d
+                    x += d * -(-max(0, (1 << 23) - x) // d)  # the first of its residue class from 2^23 on
+                    M = ((1 << k) * x - sign * c) // d
+                    if 1 << 23 <= x < 1 << 24 and 1 << 24 < M < 1 << 25 and M % 2:
+                        row.append(x)
+        if len(row) >= per_divisor:
+            ds.append(d)
+            xs.append(row[:per_divisor])
+    scale = np.float32(2.0 ** -24)
+    return np.array(ds, np.float32) * scale, np.array(xs, np.float32).T * scale
+
+
+@pytest.mark.parametrize("R", [16, 4128])
+@pytest.mark.parametrize("case", ["int8_f32", "int4_bf16", "fp8_bf16", "fp4_f32_global"])
+def test_gptq_errors_are_ieee_quotients(R, case):
+    """err = (w - q) / d at quotients 2^-25 to 2^-22 ulp from a midpoint.  A column quantised to zero passes its error to
+    a column that holds the IEEE quotient and counts its last place: nothing may be left there."""
+    from llmcompressor_amd import ops
+
+    K, half = 512, 64
+    d, x = _hard_errors(np.random.default_rng(7), K // 2, 8)
+    sources = np.arange(K).reshape(-1, 2 * half)[:, :half].reshape(-1)
+    targets = sources + half
+    rows = np.resize(np.arange(8), R)
+    W, scale = np.zeros((R, K), np.float32), np.full((R, K), 64.0, np.float32)  # 64: every source rounds to zero
+    want = x / d
+    W[:, sources] = x[rows]
+    W[:, targets] = want[rows]
+    scale[:, targets] = np.exp2(np.floor(np.log2(want[rows])) - 23)
+    U = np.zeros((K, K), np.float32)
+    U[sources, sources], U[targets, targets], U[sources, targets] = d, 1.0, 1.0
+    fmt, bits = {"int8": (ops.FMT_INT, 8), "int4": (ops.FMT_INT, 4), "fp8": (ops.FMT_FP8, 8),
+                 "fp4": (ops.FMT_FP4, 4)}[case.split("_")[0]]
+    sd = torch.bfloat16 if "bf16" in case else torch.float32
+    if case.startswith("fp8"):
+        scale[:, sources] = 65536.0  # e4m3 has values down to 2^-9
+    gs = torch.ones(1, device="cuda") if "global" in case else None
+    columns = torch.arange(K, dtype=torch.int32, device="cuda")
+    got, _ = ops.gptq_quantize(torch.from_numpy(W).cuda(), torch.from_numpy(U).cuda(), torch.from_numpy(scale).cuda().to(sd),
+                               None, fmt, bits, 1, K, g_idx=columns, global_scale=gs)
+    assert torch.count_nonzero(got) == 0, torch.count_nonzero(got).item()
+
+
+@pytest.mark.parametrize("R", [16, 4128])
+def test_gptq_values_are_rounded_from_ieee_quotients(R):
+    """x / s next to a midpoint between n + 1/2 and its float neighbour: the IEEE quotient decides whether the value
+    rounds to n or n + 1."""
+    from llmcompressor_amd import ops
+
+    rng, K = np.random.default_rng(11), 512
+    x, s = np.zeros(K, np.float32), np.ones(K, np.float32)
+    for i in range(K):
+        while True:
+            n = float(rng.integers(1, 126)) + 0.5
+            e = int(np.floor(np.log2(n)))
+            M = 2 * int(n * 2.0 ** (23 - e)) + int(rng.choice([-1, 1]))  # a midpoint beside n + 1/2, in units of 2^(e - 24)
+            c = int(rng.choice([-3, -2, -1, 1, 2, 3]))
+            S = (-c * pow(M, -1, 1 << 24)) % (1 << 24)
+            X = (M * S + c) >> 24
+            if S >= 1 << 23 and 1 << 23 <= X < 1 << 24 and (M * S + c) % (1 << 24) == 0:
+                break
+        x[i], s[i] = np.float32(X) * np.float32(2.0 ** (e - 24)), np.float32(S) * np.float32(2.0 ** -24)
+    want = np.rint(x / s) * s
+    columns = torch.arange(K, dtype=torch.int32, device="cuda")
+    W = torch.from_numpy(x).cuda().expand(R, K).contiguous()
+    got, _ = ops.gptq_quantize(W, torch.eye(K, device="cuda"), torch.from_numpy(s).cuda(), None, ops.FMT_INT, 8, 1, 0,
+                               g_idx=columns)
+    assert torch.equal(got, torch.from_numpy(want).cuda().expand(R, K))
