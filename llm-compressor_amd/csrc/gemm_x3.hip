@@ -334,6 +334,13 @@ int launch_x3(const GemmF32& g, hipStream_t st) {
 // A thread holds eight consecutive k of one row of A and of one column of B, i.e. one 16-byte chunk of its row in every
 // plane.  A row of a plane is 32 bf16 = four chunks, the chunk index XOR-ed with bits 2..3 of the row: the sixteen
 // consecutive rows that a 16-byte read is served at a time then fall into distinct banks.
+//
+// TWO_SUMS: the leading products a0 b0 and the five small ones have an accumulator each, added at the end.  In one
+// accumulator every matrix instruction rounds the whole sum, six times per 16 k; in two it is rounded once.  Error against
+// fp64 as a share of the fp32 instruction's, one sum -> two: ordinary operands 0.80 - 0.87 -> 0.32, one product per sum
+// 1.30 -> 1.02, a triangular operand whose diagonal outweighs all before it 1.5 -> 1.7 (the fp32 instruction rounds such a
+// sum once, 2.5e-8).  The factor U of 512, 768, 1024 columns, whose inverse these products form: 4.7, 5.0, 5.2e-7 ->
+// 4.5, 4.6, 5.1e-7 (by the fp32 instruction 4.8, 5.2, 5.2e-7).  The time is the same.
 constexpr int SK = 32, S_RING = 4;
 constexpr int S_PLANE = 64 * SK * 2, S_STAGE = 6 * S_PLANE;  // bytes
 
@@ -343,7 +350,7 @@ struct SmallSlab {
   float a[8], b[8];
 };
 
-template <bool TRANS_B>
+template <bool TRANS_B, bool TWO_SUMS>
 __global__ __launch_bounds__(256, 2) void gemm_x3_small_kernel(GemmF32 g, int tiles_x, int tiles_y) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[2 * S_STAGE];
   // the tile order of gemm_x3_kernel (rows of tiles dealt to the XCDs, longest contractions first)
@@ -404,9 +411,9 @@ __global__ __launch_bounds__(256, 2) void gemm_x3_small_kernel(GemmF32 g, int ti
   const int row_bytes = (int)g.ldc * 4;
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(c0, 0, 0x7fffffff, 0x00020000);
 
-  f32x16_t acc;
+  f32x16_t acc, low;  // low: the products behind a0 b0 (TWO_SUMS)
 #pragma unroll
-  for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+  for (int v = 0; v < 16; ++v) acc[v] = low[v] = 0.f;
   SmallSlab ring[S_RING];
   float cv[16];
   const int r = lane & 31, ch = lane >> 5;
@@ -441,7 +448,12 @@ __global__ __launch_bounds__(256, 2) void gemm_x3_small_kernel(GemmF32 g, int ti
           bf[q] = *(const uint4*)(cur + (3 + q) * S_PLANE + small_off(wn * 32 + r, 2 * kk + ch));
         }
 #pragma unroll
-        for (int pr = 0; pr < 6; ++pr) acc = mfma_bf16(af[PA[pr]], bf[PB[pr]], acc);
+        for (int pr = 0; pr < 6; ++pr) {
+          if (TWO_SUMS && pr < 5)
+            low = mfma_bf16(af[PA[pr]], bf[PB[pr]], low);
+          else
+            acc = mfma_bf16(af[PA[pr]], bf[PB[pr]], acc);
+        }
       }
       store(ring[m], smem + ((n + 1) & 1) * S_STAGE);
       load(ring[m], clampk(k_begin + (ks + 1 + S_RING) * SK));
@@ -460,7 +472,7 @@ __global__ __launch_bounds__(256, 2) void gemm_x3_small_kernel(GemmF32 g, int ti
   const bool diag = g.c_lower && n0 == m0;
 #pragma unroll
   for (int v = 0; v < 16; ++v) {
-    float res = g.alpha * acc[v];
+    float res = g.alpha * (TWO_SUMS ? acc[v] + low[v] : acc[v]);
     if (g.beta != 0.f) res += g.beta * cv[v];
     if (diag && wn * 32 + (lane & 31) > wm * 32 + (v / 4) * 8 + (lane >> 5) * 4 + (v & 3)) continue;
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, res), rsrc, lane_bytes,
@@ -469,14 +481,14 @@ __global__ __launch_bounds__(256, 2) void gemm_x3_small_kernel(GemmF32 g, int ti
 }
 static_assert(S_RING == 4, "the loop above is written out for four slabs");
 
-template <bool TRANS_B>
+template <bool TRANS_B, bool TWO_SUMS>
 int launch_x3_small(const GemmF32& g, hipStream_t st) {
   const int tiles_x = g.N / 64, tiles_y = g.M / 64;
   const int nb2 = g.batch2 > 1 ? g.batch2 : 1;
   const bool by_columns = g.b_lower_tri && !g.a_lower_tri && !g.c_lower;  // as in the kernel's tile order
   const int major = by_columns ? tiles_x : tiles_y, minor = by_columns ? tiles_y : tiles_x;
   const unsigned grid_x = 8u * (unsigned)((major + 7) / 8) * (unsigned)minor;
-  hipLaunchKernelGGL((gemm_x3_small_kernel<TRANS_B>), dim3(grid_x, 1, (unsigned)(g.batch * nb2)), dim3(256), 0, st, g, tiles_x,
+  hipLaunchKernelGGL((gemm_x3_small_kernel<TRANS_B, TWO_SUMS>), dim3(grid_x, 1, (unsigned)(g.batch * nb2)), dim3(256), 0, st, g, tiles_x,
                      tiles_y);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? 0 : 1000 + (int)e;
@@ -500,12 +512,16 @@ int llmc_gemm_x3(const GemmF32& g, hipStream_t st) {
   // strip's origin): wider rows than this go to the fp32 kernel's 64-bit path
   if (g.ldc >= (1 << 22)) return -1;
   // Whether a product is split depends on its own shape only, never on how many independent problems
-  // (batch2) share the launch, so that a grouped call gives the bits of its single calls.  All tile shapes
-  // add the partial products of an element in the same order, so the choice between them is free.
-  // (from contractions of 256 on: the fp32 kernel's 64-wide tiles take 7 us at 128, 11 against 10 us at 256)
+  // (batch2) share the launch, so that a grouped call gives the bits of its single calls.  From sixteen 128-wide tiles
+  // on, all tile shapes add the partial products of an element in the same order, so the choice between them is free.
+  // Products of fewer tiles, the lower levels of the triangular inverse and narrow panels, have 64-wide ones with two
+  // sums (from contractions of 256 on: the fp32 kernel's 64-wide tiles take 7 us at 128, 11 against 10 us at 256).
   const bool fit64 = g.M % 64 == 0 && g.N % 64 == 0 && g.Kc >= 256 && g.Kc % SK == 0 && g.kc_last % SK == 0;
   const bool fit128 = g.M % 128 == 0 && g.N % 128 == 0;
-  if (!fit64 && !(fit128 && (int64_t)(g.M / 128) * (g.N / 128) * g.batch >= 16)) return -1;
+  if (!(fit128 && (int64_t)(g.M / 128) * (g.N / 128) * g.batch >= 16)) {
+    if (!fit64) return -1;
+    return g.trans_b ? launch_x3_small<true, true>(g, st) : launch_x3_small<false, true>(g, st);
+  }
   // The tile: what each shape's workgroups take, in units of 7.4 us for a contraction of 512 (measured with 1 .. 8 passes
   // of the chip).  256 x 256: one per CU, 13 a pass.  128 x 128: two per CU, 7 a pass, 5 when each has a CU to itself.
   // 64 x 64: 3 a pass of two per CU, 2 with a CU each; the steps at the diagonal of a triangular operand waste least
@@ -520,10 +536,10 @@ int llmc_gemm_x3(const GemmF32& g, hipStream_t st) {
   };
   constexpr float NEVER = 1e30f;
   const float c256 = fit256 ? cost(256, 1, 13.f, 13.f) : NEVER;
-  const float c128 = fit128 ? cost(128, 2, 7.f, 5.f) : NEVER;
+  const float c128 = cost(128, 2, 7.f, 5.f);
   const float c64 = fit64 ? cost(64, 2, 3.f, 2.f) * (g.a_lower_tri || g.b_lower_tri ? 0.6f : 1.f) : NEVER;
   if (c256 <= c128 && c256 <= c64)
     return g.trans_b ? launch_x3<64, 128, 4, 2, true>(g, st) : launch_x3<64, 128, 4, 2, false>(g, st);
-  if (c64 < c128) return g.trans_b ? launch_x3_small<true>(g, st) : launch_x3_small<false>(g, st);
+  if (c64 < c128) return g.trans_b ? launch_x3_small<true, false>(g, st) : launch_x3_small<false, false>(g, st);
   return g.trans_b ? launch_x3<64, 64, 2, 2, true>(g, st) : launch_x3<64, 64, 2, 2, false>(g, st);
 }
