@@ -747,18 +747,16 @@ def test_factor_forms_agree_over_shapes_and_formats(R, K, fmt_name, bits, group,
             assert q.round().min() >= grid.min() and q.round().max() <= grid.max()
 
 
-def _column_loop(W, U, scale_cols, zp_cols, grid, sd):
-    """The column loop written out in fp32: scales and zero points per element, ``grid`` rounds a quotient."""
-    W = W.float().clone()
-    loss = torch.zeros((), device=W.device)
+def _loop_in_fp64(W, U, Q, scale_cols, zp_cols):
+    """The column loop in fp64 along the decisions Q: the value that each column holds when its turn comes, and half the
+    sum of its squared errors."""
+    W, U, Q = W.double().clone(), U.double(), Q.double()
+    loss = torch.zeros((), device=W.device, dtype=torch.float64)
     for i in range(W.shape[1]):
-        s, z = scale_cols[:, i], zp_cols[:, i]
-        q = ((grid(W[:, i] / s + z) - z).to(sd).float() * s).to(sd).float()
-        err = (W[:, i] - q) / U[i, i]
+        err = (W[:, i] - Q[:, i]) / U[i, i]
         loss += (err * err).sum() / 2
-        W[:, i] = q
         W[:, i + 1:] -= err[:, None] * U[i, i + 1:]
-    return W, loss
+    return W / scale_cols.double() + zp_cols.double(), loss
 
 
 @pytest.mark.parametrize("R,K,blocksize", [(1, 1, 128), (15, 129, 128), (16, 256, 128), (17, 516, 128), (33, 700, 37),
@@ -766,11 +764,17 @@ def _column_loop(W, U, scale_cols, zp_cols, grid, sd):
 @pytest.mark.parametrize("case", ["int4_bf16", "int4_zp_f16", "int8_f32", "fp8_bf16", "fp4_f32_global", "fp4_f16"])
 def test_gptq_column_loop_at_tile_edges(R, K, blocksize, case):
     """Partial blocks and groups, block widths that leave every access unaligned, a last workgroup of one row, and
-    weights on both sides of the line between 16 and 8 lanes per row, for formats with unrolled turns and with loops."""
+    weights on both sides of the line between 16 and 8 lanes per row, for formats with unrolled turns and with loops.
+
+    The loop is followed in fp64 along the kernel's own decisions, so that one value next to a rounding boundary does
+    not take the rest of its row with it: every decision has to be the nearest point of the grid, but for the error that
+    fp32 can have gathered by then.  A column is updated K times at most, each update rounding a sum no larger than the
+    column ever gets, and brings in its error's own rounding (of w - q and of the division) times U / d; twice 2^-24
+    each, as the matrix instruction may truncate."""
     from llmcompressor_amd import ops
 
     torch.manual_seed(R + K)
-    W = (torch.randn(R, K, device="cuda") * 0.02).bfloat16()
+    W = (torch.randn(R, K, device="cuda") * 0.02).bfloat16().float()  # in fp32 the decisions come back unrounded
     U = torch.triu(torch.randn(K, K, device="cuda") * 0.05, 1) + torch.diag(torch.rand(K, device="cuda") + 0.5)
     U_in = U + torch.tril(torch.full((K, K), float("nan"), device="cuda"), -1)  # what is below must not be read
     sd = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[case.split("_")[-1].replace("global", "f32")]
@@ -781,9 +785,9 @@ def test_gptq_column_loop_at_tile_edges(R, K, blocksize, case):
     if "int" in case:
         fmt, bits, grid = ops.FMT_INT, 8 if "int8" in case else 4, lambda v: torch.round(v.clamp(-qmax - 1, qmax))
     elif "fp8" in case:
-        fmt, bits, grid = ops.FMT_FP8, 8, lambda v: v.clamp(-qmax, qmax).to(torch.float8_e4m3fn).float()
+        fmt, bits, grid = ops.FMT_FP8, 8, lambda v: v.clamp(-qmax, qmax).to(torch.float8_e4m3fn).to(v.dtype)
     else:
-        points = torch.tensor([0, .5, 1, 1.5, 2, 3, 4, 6.], device="cuda")
+        points = torch.tensor([0, .5, 1, 1.5, 2, 3, 4, 6.], device="cuda", dtype=torch.float64)
 
         def grid(v):
             a = v.abs().clamp(max=6.0)
@@ -792,13 +796,20 @@ def test_gptq_column_loop_at_tile_edges(R, K, blocksize, case):
             return torch.copysign(r, v)
         fmt, bits = ops.FMT_FP4, 4
     s = scale.float() / gs if gs is not None else scale.float()
-    expected, loss_e = _column_loop(W, U, s.expand(R, K), (zp.float() if zp is not None else torch.zeros_like(s)).expand(R, K),
-                                    grid, torch.float32 if gs is not None else sd)
+    z = zp.double() if zp is not None else torch.zeros_like(s, dtype=torch.float64)
     got, loss = ops.gptq_quantize(W, U_in, scale, zp, fmt, bits, 1, 1, global_scale=gs, blocksize=blocksize)
-    # another order of the sums moves a value across a rounding boundary now and then, and what follows with it
-    same = (got == expected.to(W.dtype)).float().mean().item()
-    assert same > 0.985, same
-    assert abs(loss.item() - loss_e.item()) <= 0.01 * loss_e.item() + 1e-9
+    v, loss_e = _loop_in_fp64(W, U, got, s.expand(R, K), z.expand(R, K))
+    chosen = grid(got.double() / s.double() + z)  # the grid's points are far apart beside the rounding of got
+    sd_step = 2.0 ** {torch.bfloat16: -9, torch.float16: -12, torch.float32: -25}[torch.float32 if gs is not None else sd]
+    assert bool(((got.double() - (chosen - z) * s.double()).abs() <= 2 * sd_step * got.double().abs() + 1e-12).all())
+    spread = (U.double().abs() / U.double().diagonal()[:, None]).triu(1).sum(0).max()
+    largest = (v - z).abs().amax() + 1
+    bound = 2 * 2.0 ** -24 * largest * (K + 2 * spread)
+    excess = (v - chosen).abs() - (v - grid(v)).abs()
+    assert bool((excess <= 2 * bound).all()), (excess.max().item(), bound.item())
+    # the loss: every error off by the bound at most, and K / 8 fp32 additions per lane
+    slack = 2 * bound * s.double().max() / U.double().diagonal().min() * (2 * loss_e * R * K) ** 0.5 + K / 8 * 2.0 ** -24 * loss_e
+    assert abs(loss.double() - loss_e) <= slack + 1e-12, (loss.item(), loss_e.item(), slack.item())
 
 
 @pytest.mark.parametrize("K,n", [(320, 3), (1088, 12), (1088, 24)])
