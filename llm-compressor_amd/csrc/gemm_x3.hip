@@ -338,9 +338,7 @@ int launch_x3(const GemmF32& g, hipStream_t st) {
 // TWO_SUMS: the leading products a0 b0 and the five small ones have an accumulator each, added at the end.  In one
 // accumulator every matrix instruction rounds the whole sum, six times per 16 k; in two it is rounded once.  Error against
 // fp64 as a share of the fp32 instruction's, one sum -> two: ordinary operands 0.80 - 0.87 -> 0.32, one product per sum
-// 1.30 -> 1.02, a triangular operand whose diagonal outweighs all before it 1.5 -> 1.7 (the fp32 instruction rounds such a
-// sum once, 2.5e-8).  The factor U of 512, 768, 1024 columns, whose inverse these products form: 4.7, 5.0, 5.2e-7 ->
-// 4.5, 4.6, 5.1e-7 (by the fp32 instruction 4.8, 5.2, 5.2e-7).  The time is the same.
+// 1.30 -> 1.02.  The time is the same.
 constexpr int SK = 32, S_RING = 4;
 constexpr int S_PLANE = 64 * SK * 2, S_STAGE = 6 * S_PLANE;  // bytes
 
@@ -514,12 +512,14 @@ int llmc_gemm_x3(const GemmF32& g, hipStream_t st) {
   // Whether a product is split depends on its own shape only, never on how many independent problems
   // (batch2) share the launch, so that a grouped call gives the bits of its single calls.  From sixteen 128-wide tiles
   // on, all tile shapes add the partial products of an element in the same order, so the choice between them is free.
-  // Products of fewer tiles, the lower levels of the triangular inverse and narrow panels, have 64-wide ones with two
-  // sums (from contractions of 256 on: the fp32 kernel's 64-wide tiles take 7 us at 128, 11 against 10 us at 256).
+  // Products of fewer tiles, the far updates of weights of few rows, have 64-wide ones with two sums, from contractions
+  // of 512 on.  The fp32 instruction keeps the shorter ones, which are the lower levels of the triangular inverse: it takes
+  // 11 us against 10 at 256, and where a triangle's diagonal outweighs all before it, it rounds the sum once (2.5e-8,
+  // against 3.8e-8 split with one sum and 4.5e-8 with two).
   const bool fit64 = g.M % 64 == 0 && g.N % 64 == 0 && g.Kc >= 256 && g.Kc % SK == 0 && g.kc_last % SK == 0;
   const bool fit128 = g.M % 128 == 0 && g.N % 128 == 0;
   if (!(fit128 && (int64_t)(g.M / 128) * (g.N / 128) * g.batch >= 16)) {
-    if (!fit64) return -1;
+    if (!fit64 || g.Kc < 512) return -1;
     return g.trans_b ? launch_x3_small<true, true>(g, st) : launch_x3_small<false, true>(g, st);
   }
   // The tile: what each shape's workgroups take, in units of 7.4 us for a contraction of 512 (measured with 1 .. 8 passes

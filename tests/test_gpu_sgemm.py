@@ -54,7 +54,7 @@ def test_sgemm_matches_fp64(M, N, Kc, trans_b, flags, alpha, beta):
     assert errs["auto"] <= 1.5 * errs["fp32"] + 1e-8
 
 
-@pytest.mark.parametrize("M,N,Kc", [(64, 64, 256), (192, 64, 320), (256, 256, 512), (128, 1024, 512), (4160, 512, 512)])
+@pytest.mark.parametrize("M,N,Kc", [(64, 64, 512), (192, 64, 544), (256, 256, 1024), (128, 1024, 512), (4160, 512, 512)])
 @pytest.mark.parametrize("trans_b", [False, True])
 def test_sgemm_below_sixteen_large_tiles_is_closer_than_the_fp32_instruction(M, N, Kc, trans_b):
     """These products round their whole sum once per 16 k where the fp32 instruction rounds it 16 times: a quarter of
@@ -84,12 +84,19 @@ def test_sgemm_rejects_bad_arguments():
 
 
 @pytest.mark.parametrize("M,N,Kc,trans_b,flags,alpha,beta", [
-    (64, 64, 256, False, 0, 1.0, 0.0),      # one tile, as few k-steps as the split product takes
-    (64, 192, 288, True, 0, -1.0, 1.0),     # a contraction that is no multiple of the four steps in flight
+    (64, 64, 256, False, 0, 1.0, 0.0),      # one tile of the fp32 instruction
+    (64, 192, 288, True, 0, -1.0, 1.0),
     (192, 320, 352, False, 0, -1.0, 1.0),
     (448, 448, 256, True, 1, -1.0, 1.0),    # lower triangle only, diagonal tiles
-    (320, 256, 256, False, 4, 1.0, 0.0),    # contractions from 256 down to 64: two steps
+    (320, 256, 256, False, 4, 1.0, 0.0),
     (256, 320, 256, False, 2, -1.0, 0.0),
+    (64, 64, 512, False, 0, 1.0, 0.0),      # split: one tile, as few k-steps as it takes with two sums
+    (64, 192, 544, True, 0, -1.0, 1.0),     # a contraction that is no multiple of the four steps in flight
+    (192, 320, 608, False, 0, -1.0, 1.0),
+    (448, 448, 512, True, 1, -1.0, 1.0),    # lower triangle only, diagonal tiles
+    (320, 512, 512, False, 4, 1.0, 0.0),    # contractions from 512 down to 64: two steps
+    (512, 320, 512, False, 2, -1.0, 0.0),
+    (640, 640, 256, True, 1, -1.0, 1.0),    # from sixteen 128-wide tiles on: one sum
 ])
 def test_sgemm_small_tiles(M, N, Kc, trans_b, flags, alpha, beta):
     """Products of a few 64 x 64 tiles: within the fp32 matrix instruction's error, nothing outside C written."""
