@@ -109,19 +109,23 @@ def _run(weight, scale, zp, args: QuantizationArgs, mode, g_idx=None, global_sca
     return op(weight.contiguous(), scale, zpa, fmt, bits, row_div, srow, col_div, mode, g_idx, global_scale)
 
 
-def _tensor_of(module: torch.nn.Module, name: str) -> Optional[torch.Tensor]:
-    """``module.<name>`` or None, without the failing attribute lookup (a microsecond) where the name can only be in the
-    module's own dicts: a class with its own ``__getattr__`` (a wrapper that forwards to the module it holds), or with
-    the name itself (a property), is asked the ordinary way."""
+def _tensors_of(module: torch.nn.Module):
+    """The function ``name -> module.<name> or None``, without the failing attribute lookup (a microsecond) where the name
+    can only be in the module's own dicts.  A class with its own ``__getattr__`` (a wrapper that forwards to the module it
+    holds), or with the name itself (a property), is asked the ordinary way."""
     cls = type(module)
-    if (cls.__getattr__ is not torch.nn.Module.__getattr__ or cls.__getattribute__ is not object.__getattribute__
-            or hasattr(cls, name)):
-        return getattr(module, name, None)
+    if cls.__getattr__ is not torch.nn.Module.__getattr__ or cls.__getattribute__ is not object.__getattribute__:
+        return lambda name: getattr(module, name, None)
     d = module.__dict__
-    for where in (d, d["_parameters"], d["_buffers"], d["_modules"]):
-        if name in where:
-            return where[name]
-    return None
+    own = (d["_parameters"], d["_buffers"], d, d["_modules"])
+
+    def lookup(name):
+        for where in own:
+            if name in where:
+                return where[name]
+        return getattr(module, name, None) if hasattr(cls, name) else None
+
+    return lookup
 
 
 def compress_module(module: torch.nn.Module, fmt: Optional[str] = None) -> Dict[str, torch.Tensor]:
@@ -129,13 +133,14 @@ def compress_module(module: torch.nn.Module, fmt: Optional[str] = None) -> Dict[
     scheme: QuantizationScheme = module.quantization_scheme
     args = scheme.weights
     fmt = fmt or infer_format(scheme)
+    tensor = _tensors_of(module)
     weight = module.weight.data
     scale = module.weight_scale.data
-    zp = _tensor_of(module, "weight_zero_point")
+    zp = tensor("weight_zero_point")
     zp = None if zp is None else zp.data
-    gs = _tensor_of(module, "weight_global_scale")
+    gs = tensor("weight_global_scale")
     gs = None if gs is None else gs.data.to(torch.float32)
-    g_idx = _tensor_of(module, "weight_g_idx")
+    g_idx = tensor("weight_g_idx")
     g_idx = None if g_idx is None else g_idx.data
     out: Dict[str, torch.Tensor] = {}
     if fmt == CompressionFormat.pack_quantized:
@@ -171,7 +176,7 @@ def compress_module(module: torch.nn.Module, fmt: Optional[str] = None) -> Dict[
     else:
         raise ValueError(f"unsupported compression format {fmt}")
     for name in ("input_scale", "input_zero_point", "input_global_scale", "output_scale", "output_zero_point"):
-        t = _tensor_of(module, name)
+        t = tensor(name)
         if t is None:
             continue
         if name.endswith("zero_point"):  # zero points of symmetric arguments are all zero and are not stored
@@ -179,7 +184,7 @@ def compress_module(module: torch.nn.Module, fmt: Optional[str] = None) -> Dict[
             if act is None or act.symmetric:
                 continue
         out[name] = t.data
-    bias = _tensor_of(module, "bias")
+    bias = tensor("bias")
     if bias is not None:
         out["bias"] = bias.data
     return out

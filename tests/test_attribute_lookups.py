@@ -4,7 +4,7 @@ import types
 import pytest
 import torch
 
-from llmcompressor_amd.compressors import _tensor_of
+from llmcompressor_amd.compressors import _tensors_of
 from llmcompressor_amd.modifiers.quantization.calibration import observe, update_qparams
 
 
@@ -73,10 +73,10 @@ def test_tensors_of_a_module_are_found_as_attributes():
     linear.register_buffer("weight_g_idx", torch.arange(4))
     linear.input_scale = torch.ones(1)  # neither parameter nor buffer
     for module in (linear, Forwarding(linear)):
-        assert _tensor_of(module, "bias") is linear.bias
-        assert _tensor_of(module, "weight_g_idx") is linear.weight_g_idx
-        assert _tensor_of(module, "input_scale") is linear.input_scale
-        assert _tensor_of(module, "weight_zero_point") is None
-    assert _tensor_of(torch.nn.Linear(4, 4, bias=False), "bias") is None
+        assert _tensors_of(module)("bias") is linear.bias
+        assert _tensors_of(module)("weight_g_idx") is linear.weight_g_idx
+        assert _tensors_of(module)("input_scale") is linear.input_scale
+        assert _tensors_of(module)("weight_zero_point") is None
+    assert _tensors_of(torch.nn.Linear(4, 4, bias=False))("bias") is None
     own = WithProperty(4, 4)
-    assert _tensor_of(own, "weight_zero_point") is own.bias
+    assert _tensors_of(own)("weight_zero_point") is own.bias
