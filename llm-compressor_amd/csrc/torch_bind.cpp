@@ -117,15 +117,20 @@ void hessian_accum_counted_(Tensor& H, const Tensor& X, Tensor& count, double sa
 
 using Pair = std::tuple<Tensor, Tensor>;
 
-Pair minmax_observe(const Tensor& W, int64_t group) {
+// `workspace`: scratch memory that the caller keeps; without it the call takes its own
+Pair minmax_observe(const Tensor& W, int64_t group, const optional<Tensor>& workspace) {
   require_rows(W);
+  require_beside(W, workspace);
   const int dt = dtype_code(W);
   TORCH_CHECK_VALUE(group > 0 && W.size(1) % group == 0, "llmc_minmax_groups: argument 6 rejected");
   Guard guard(W.device());
   const int64_t R = W.size(0), K = W.size(1);
   Tensor mn = at::empty({R, K / group}, W.options()), mx = at::empty({R, K / group}, W.options());
-  const int64_t nws = llmc_minmax_workspace_bytes();
-  const Tensor ws = scratch(W, nws);
+  TORCH_CHECK_VALUE(!workspace.has_value() || (workspace->scalar_type() == at::kByte && workspace->is_contiguous() &&
+                                               ((uintptr_t)workspace->data_ptr() & 15) == 0),
+                    "minmax_observe: the workspace must be contiguous bytes, 16-byte aligned");
+  const Tensor ws = workspace.has_value() ? *workspace : scratch(W, llmc_minmax_workspace_bytes());
+  const int64_t nws = ws.numel();
   check(llmc_minmax_groups(W.const_data_ptr(), dt, R, K, W.stride(0), group, mn.data_ptr(), mx.data_ptr(),
                            ws.data_ptr(), nws, stream_of(W)),
         "llmc_minmax_groups");

@@ -29,11 +29,11 @@ def _require_gpu(*ts: torch.Tensor) -> None:
 _llmc = None
 
 
-def _native_ops():
+def _native():
     """The registered operators (torch_ops.py imports this module, so they are looked up at the first call)."""
     global _llmc
-    from .torch_ops import llmc as _llmc
-
+    if _llmc is None:
+        from .torch_ops import llmc as _llmc
     return _llmc
 
 
@@ -46,7 +46,7 @@ def hessian_accumulate_(H: torch.Tensor, x: torch.Tensor, alpha: float = 2.0, as
     fixed order, so results stay reproducible); without it every output tile is one workgroup.  `count` (fp32, one
     value on H's device) is raised by `samples` in the same launch."""
     _require_gpu(H, x)
-    llmc = _llmc or _native_ops()
+    llmc = _native()
     if count is not None:
         llmc.hessian_accum_counted_(H, x, count, samples, alpha, assume_symmetric, use_workspace)
     else:
@@ -150,7 +150,6 @@ def hessian_accumulate_grouped_(Hs, xs, alpha: float = 2.0, assume_symmetric: bo
 FMT_INT, FMT_FP8, FMT_FP4 = 0, 1, 2
 SCALE_PLAIN, SCALE_NVFP4, SCALE_MXFP4 = 0, 1, 2
 OUT_FAKEQUANT, OUT_CODES, OUT_PACKED = 0, 1, 2
-_TD = {BF16: torch.bfloat16, F16: torch.float16, F32: torch.float32}
 
 class _WorkspaceStore(dict):
     """The scratch buffers of one host thread, keyed by (device, stream)."""
@@ -204,45 +203,24 @@ def _dt(t: torch.Tensor) -> int:
         raise TypeError(f"unsupported dtype {t.dtype}; expected bf16/f16/f32") from None
 
 
+# The short operators below are implemented natively behind torch.ops.llmc (csrc/torch_bind.cpp), which the package
+# calls directly; these are their names among the other tensor-level entry points.
+
 def minmax_groups(w: torch.Tensor, group: int):
     """min/max of each run of `group` consecutive columns of w [R,K] -> two [R, K/group] tensors."""
     _require_gpu(w)
-    assert w.ndim == 2 and w.stride(1) == 1
-    R, K = w.shape
-    mn = torch.empty((R, K // group), dtype=w.dtype, device=w.device)
-    mx = torch.empty_like(mn)
-    ws = _workspace(w.device, 1 << 16)
-    with torch.cuda.device(w.device):
-        rc = _lib.lib().llmc_minmax_groups(w.data_ptr(), _dt(w), R, K, w.stride(0), group, mn.data_ptr(),
-                                           mx.data_ptr(), ws.data_ptr(), ws.numel(), _stream(w))
-    _lib.check(rc, "llmc_minmax_groups")
-    return mn, mx
+    return _native().minmax_observe(w, group, _workspace(w.device, 1 << 16))
 
 
 def minmax_blocks(w: torch.Tensor, bh: int, bw: int):
     _require_gpu(w)
-    assert w.ndim == 2 and w.stride(1) == 1
-    R, K = w.shape
-    shape = ((R + bh - 1) // bh, (K + bw - 1) // bw)
-    mn = torch.empty(shape, dtype=w.dtype, device=w.device)
-    mx = torch.empty_like(mn)
-    with torch.cuda.device(w.device):
-        rc = _lib.lib().llmc_minmax_blocks(w.data_ptr(), _dt(w), R, K, w.stride(0), bh, bw, mn.data_ptr(),
-                                           mx.data_ptr(), _stream(w))
-    _lib.check(rc, "llmc_minmax_blocks")
-    return mn, mx
+    return _native().minmax_observe_blocks(w, bh, bw)
 
 
 def minmax_strided(x: torch.Tensor, n0: int, n1: int, group: int, s0: int, s1: int):
     """x viewed as (n0, n1, group) with element strides (s0, s1, 1): reduce dims (0,-1) -> [n1]."""
     _require_gpu(x)
-    mn = torch.empty((n1,), dtype=x.dtype, device=x.device)
-    mx = torch.empty_like(mn)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().llmc_minmax_strided(x.data_ptr(), _dt(x), n0, n1, group, s0, s1, mn.data_ptr(),
-                                            mx.data_ptr(), _stream(x))
-    _lib.check(rc, "llmc_minmax_strided")
-    return mn, mx
+    return _native().minmax_observe_strided(x, n0, n1, group, s0, s1)
 
 
 def _gs32(global_scale):
@@ -254,98 +232,30 @@ def _gs32(global_scale):
 
 def global_scale_from_stats(stats):
     """NVFP4 global scale from the (min, max) arrays of every observer of a fused group -> fp32 [1]."""
-    mn0 = stats[0][0]
-    _require_gpu(mn0)
-    absmax = torch.zeros(1, dtype=torch.float32, device=mn0.device)
-    out = torch.empty(1, dtype=torch.float32, device=mn0.device)
-    with torch.cuda.device(mn0.device):
-        for mn, mx in stats:
-            mn, mx = mn.contiguous(), mx.contiguous()
-            rc = _lib.lib().llmc_absmax_accumulate(mn.data_ptr(), mx.data_ptr(), mn.numel(), _dt(mn),
-                                                   absmax.data_ptr(), _stream(mn0))
-            _lib.check(rc, "llmc_absmax_accumulate")
-        rc = _lib.lib().llmc_generate_gparam(absmax.data_ptr(), _dt(mn0), out.data_ptr(), _stream(mn0))
-    _lib.check(rc, "llmc_generate_gparam")
-    return out
+    mins, maxs = [mn for mn, _ in stats], [mx for _, mx in stats]
+    _require_gpu(*mins, *maxs)
+    return _native().global_scale(mins, maxs)
 
 
 def calculate_qparams(mn, mx, fmt: int, bits: int, symmetric: bool, scale_mode: int = SCALE_PLAIN,
                       global_scale=None, want_codes: bool = False):
     """(min,max) -> (scale, zero_point int8, scale_code uint8|None); shapes follow `mn`."""
-    global_scale = _gs32(global_scale)
-    _require_gpu(mn, mx)
-    mn, mx = mn.contiguous(), mx.contiguous()
-    sdt = torch.float32 if scale_mode == SCALE_NVFP4 else mn.dtype
-    scale = torch.empty(mn.shape, dtype=sdt, device=mn.device)
-    zp = torch.zeros(mn.shape, dtype=torch.int8, device=mn.device)
-    codes = torch.empty(mn.shape, dtype=torch.uint8, device=mn.device) if want_codes else None
-    with torch.cuda.device(mn.device):
-        rc = _lib.lib().llmc_calculate_qparams(
-            mn.data_ptr(), mx.data_ptr(), mn.numel(), _dt(mn), fmt, bits, 1 if symmetric else 0, scale_mode,
-            _ptr(global_scale), scale.data_ptr(), _DT[sdt], 0 if symmetric else zp.data_ptr(), _ptr(codes),
-            _stream(mn))
-    _lib.check(rc, "llmc_calculate_qparams")
-    return scale, zp, codes
+    _require_gpu(mn, mx, global_scale)
+    return _native().qparams(mn, mx, fmt, bits, bool(symmetric), scale_mode, global_scale, want_codes)
 
 
 def quantize(x, scale, zero_point, fmt: int, bits: int, row_div: int, scale_row_stride: int, col_div: int,
              out_mode: int = OUT_FAKEQUANT, g_idx=None, global_scale=None, out_dtype=None):
     """Element-wise quantise of x [R,K]; see llmc_quantize in include/llmc_amd.h for the scale indexing."""
-    global_scale = _gs32(global_scale)
-    _require_gpu(x, scale)
-    assert x.ndim == 2 and x.stride(1) == 1
-    R, K = x.shape
-    scale = scale.contiguous()
-    if zero_point is not None:
-        zero_point = zero_point.contiguous()
-        assert zero_point.dtype == torch.int8
-    if g_idx is not None:
-        g_idx = g_idx.to(torch.int32).contiguous()
-    if out_mode == OUT_FAKEQUANT:
-        out_dtype = out_dtype or x.dtype
-        out = torch.empty((R, K), dtype=out_dtype, device=x.device)
-        odt, ldo = _DT[out_dtype], K
-    elif out_mode == OUT_CODES:
-        tdt = torch.int8 if fmt == FMT_INT else (torch.float8_e4m3fn if fmt == FMT_FP8 else torch.uint8)
-        out = torch.empty((R, K), dtype=tdt, device=x.device)
-        odt, ldo = 0, K
-    else:
-        if fmt == FMT_INT:
-            pf = 32 // bits
-            ldo = (K + pf - 1) // pf
-            out = torch.empty((R, ldo), dtype=torch.int32, device=x.device)
-        elif fmt == FMT_FP4:
-            ldo = (K + 1) // 2
-            out = torch.empty((R, ldo), dtype=torch.uint8, device=x.device)
-        else:
-            ldo = K
-            out = torch.empty((R, K), dtype=torch.float8_e4m3fn, device=x.device)
-        odt = 0
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().llmc_quantize(
-            x.data_ptr(), _dt(x), R, K, x.stride(0), scale.data_ptr(), _dt(scale), _ptr(zero_point),
-            _ptr(g_idx), _ptr(global_scale), fmt, bits, row_div, scale_row_stride, col_div, out_mode,
-            out.data_ptr(), odt, ldo, _stream(x))
-    _lib.check(rc, "llmc_quantize")
-    return out
+    _require_gpu(x, scale, zero_point, g_idx, global_scale)
+    return _native().quant_pack(x, scale, zero_point, fmt, bits, row_div, scale_row_stride, col_div, out_mode, g_idx,
+                                global_scale, out_dtype)
 
 
 def dynamic_per_token_quantize(x, fmt: int = FMT_FP8, bits: int = 8, out_mode: int = OUT_FAKEQUANT):
     """x [N,K] bf16/f16 -> (fake-quantised x | code bytes, per-row scale [N,1])."""
     _require_gpu(x)
-    assert x.ndim == 2 and x.stride(1) == 1
-    N, K = x.shape
-    scale = torch.empty((N, 1), dtype=x.dtype, device=x.device)
-    if out_mode == OUT_FAKEQUANT:
-        out = torch.empty((N, K), dtype=x.dtype, device=x.device)
-    else:
-        out = torch.empty((N, K), dtype=torch.float8_e4m3fn if fmt == FMT_FP8 else torch.int8, device=x.device)
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().llmc_dynamic_per_token_quantize(x.data_ptr(), _dt(x), N, K, x.stride(0), fmt, bits,
-                                                        out_mode, out.data_ptr(), K, scale.data_ptr(),
-                                                        _stream(x))
-    _lib.check(rc, "llmc_dynamic_per_token_quantize")
-    return out, scale
+    return _native().fp8_dynamic_per_token(x, fmt, bits, out_mode)
 
 
 FACTOR_INVERSE, FACTOR_GROUPS, FACTOR_GROUP_WIDTH = 0, 1, 512
@@ -520,30 +430,12 @@ def sparsegpt_sparsify(weight, U, sparsity: float, prune_n: int = 0, prune_m: in
     return out, loss
 
 
-def _mse_common(maxshrink, grid, patience, norm, expand):
-    steps = int(maxshrink * grid)
-    if steps > 256:
-        raise ValueError(f"MSE observer: int(maxshrink*grid)={steps} search steps exceed the supported 256")
-    return steps, float(grid), int(patience), float(norm), float(expand)
-
-
 def mse_observe_groups(w, group: int, fmt: int, bits: int, symmetric: bool, scale_mode: int = SCALE_PLAIN,
                        maxshrink=0.20, patience=5, grid=100.0, norm=2.4, expand=1.0):
     """MSE grid search per run of `group` columns of w [R,K] -> (min, max) [R, K/group]."""
     _require_gpu(w)
-    assert w.ndim == 2 and w.stride(1) == 1
-    R, K = w.shape
-    steps, grid, patience, norm, expand = _mse_common(maxshrink, grid, patience, norm, expand)
-    n = R * (K // group)
-    mn = torch.empty((R, K // group), dtype=w.dtype, device=w.device)
-    mx = torch.empty_like(mn)
-    ws = _workspace(w.device, _lib.lib().llmc_mse_workspace_bytes(n))
-    with torch.cuda.device(w.device):
-        rc = _lib.lib().llmc_mse_observe_groups(
-            w.data_ptr(), _dt(w), R, K, w.stride(0), group, fmt, bits, 1 if symmetric else 0, scale_mode, steps,
-            grid, patience, norm, expand, mn.data_ptr(), mx.data_ptr(), ws.data_ptr(), ws.numel(), _stream(w))
-    _lib.check(rc, "llmc_mse_observe_groups")
-    return mn, mx
+    return _native().mse_observe(w, group, fmt, bits, bool(symmetric), scale_mode, maxshrink, patience, grid, norm,
+                                 expand)
 
 
 def sumsq_accumulate_(total: torch.Tensor, x: torch.Tensor):
@@ -609,34 +501,15 @@ def imatrix_observe_groups(w, group: int, fmt: int, bits: int, symmetric: bool, 
 def mse_observe_strided(x, n0: int, n1: int, group: int, s0: int, s1: int, fmt: int, bits: int, symmetric: bool,
                         scale_mode: int = SCALE_PLAIN, maxshrink=0.20, patience=5, grid=100.0, norm=2.4, expand=1.0):
     _require_gpu(x)
-    steps, grid, patience, norm, expand = _mse_common(maxshrink, grid, patience, norm, expand)
-    mn = torch.empty((n1,), dtype=x.dtype, device=x.device)
-    mx = torch.empty_like(mn)
-    ws = _workspace(x.device, _lib.lib().llmc_mse_workspace_bytes(n1))
-    with torch.cuda.device(x.device):
-        rc = _lib.lib().llmc_mse_observe_strided(
-            x.data_ptr(), _dt(x), n0, n1, group, s0, s1, fmt, bits, 1 if symmetric else 0, scale_mode, steps, grid,
-            patience, norm, expand, mn.data_ptr(), mx.data_ptr(), ws.data_ptr(), ws.numel(), _stream(x))
-    _lib.check(rc, "llmc_mse_observe_strided")
-    return mn, mx
+    return _native().mse_observe_strided(x, n0, n1, group, s0, s1, fmt, bits, bool(symmetric), scale_mode, maxshrink,
+                                         patience, grid, norm, expand)
 
 
 def mse_observe_blocks(w, bh: int, bw: int, fmt: int, bits: int, symmetric: bool, scale_mode: int = SCALE_PLAIN,
                        maxshrink=0.20, patience=5, grid=100.0, norm=2.4, expand=1.0):
     _require_gpu(w)
-    assert w.ndim == 2 and w.stride(1) == 1
-    R, K = w.shape
-    steps, grid, patience, norm, expand = _mse_common(maxshrink, grid, patience, norm, expand)
-    shape = ((R + bh - 1) // bh, (K + bw - 1) // bw)
-    mn = torch.empty(shape, dtype=w.dtype, device=w.device)
-    mx = torch.empty_like(mn)
-    ws = _workspace(w.device, _lib.lib().llmc_mse_workspace_bytes(shape[0] * shape[1]))
-    with torch.cuda.device(w.device):
-        rc = _lib.lib().llmc_mse_observe_blocks(
-            w.data_ptr(), _dt(w), R, K, w.stride(0), bh, bw, fmt, bits, 1 if symmetric else 0, scale_mode, steps,
-            grid, patience, norm, expand, mn.data_ptr(), mx.data_ptr(), ws.data_ptr(), ws.numel(), _stream(w))
-    _lib.check(rc, "llmc_mse_observe_blocks")
-    return mn, mx
+    return _native().mse_observe_blocks(w, bh, bw, fmt, bits, bool(symmetric), scale_mode, maxshrink, patience, grid,
+                                        norm, expand)
 
 
 def _imatrix_steps(maxshrink, grid):

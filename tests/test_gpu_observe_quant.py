@@ -361,3 +361,19 @@ def test_global_scale_matches_oracle_for_many_absmax_values(dtype):
         if got != want:
             bad.append((v.item(), got, want))
     assert not bad, bad[:5]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_global_scale_in_two_steps_equals_the_one_call(dtype):
+    """llmc_absmax_accumulate over every array and llmc_generate_gparam, for callers of the C ABI that keep the cell."""
+    from llmcompressor_amd import _lib, ops
+
+    torch.manual_seed(5)
+    arrays = [torch.randn(n, device="cuda").to(dtype) for n in (1, 2055, 70000)]
+    stats = [(-t.abs(), t.abs() * 0.5) for t in arrays]
+    lib, st = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    cell, out = torch.zeros(1, device="cuda"), torch.empty(1, device="cuda")
+    for mn, mx in stats:
+        assert lib.llmc_absmax_accumulate(mn.data_ptr(), mx.data_ptr(), mn.numel(), ops._DT[dtype], cell.data_ptr(), st) == 0
+    assert lib.llmc_generate_gparam(cell.data_ptr(), ops._DT[dtype], out.data_ptr(), st) == 0
+    assert torch.equal(out, ops.global_scale_from_stats(stats))
