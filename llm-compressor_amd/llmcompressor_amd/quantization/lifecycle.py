@@ -225,6 +225,8 @@ def _fused_group_mode(x2: torch.Tensor, args: QuantizationArgs, global_scale) ->
     if args.type == QuantizationType.INT and args.num_bits not in (4, 8):
         return None
     mode = scale_mode(args, global_scale is not None)
+    if global_scale is not None and mode != ops.SCALE_NVFP4:  # the general path divides by it whatever the mode
+        return None
     if x2.dtype != torch.bfloat16 and (x2.dtype != torch.float16 or mode == ops.SCALE_MXFP4):
         return None
     return mode
