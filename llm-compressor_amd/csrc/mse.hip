@@ -131,8 +131,8 @@ __global__ __launch_bounds__(256) void mse_team_kernel(MseParams p, int64_t ngro
     mn = fminf(mn, __shfl_xor(mn, o, 64));
     mx = fmaxf(mx, __shfl_xor(mx, o, 64));
   }
-  mn = round_rt(mn * p.expand, p.dt);
-  mx = round_rt(mx * p.expand, p.dt);
+  mn = round_rt(product<LLMC_F16>(mn, p.expand), p.dt);
+  mx = round_rt(product<LLMC_F16>(mx, p.expand), p.dt);
   float best = p.dt == LLMC_BF16 ? 3.3895313892515355e38f : p.dt == LLMC_F16 ? 65504.0f : 3.4028234663852886e38f;
   if (p.err32) best = 3.4028234663852886e38f;
   float wt[8];
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void mse_team_kernel(MseParams p, int64_t ngro
   for (int wd = 0; wd < MASK_WORDS; ++wd) mask[wd] = 0ull;
   for (int i = 0; i < p.steps; ++i) {
     const float pi = step_factor(i, p.grid);
-    const float smin = round_rt(mn * pi, p.dt), smax = round_rt(mx * pi, p.dt);
+    const float smin = round_rt(product<LLMC_F16>(mn, pi), p.dt), smax = round_rt(product<LLMC_F16>(mx, pi), p.dt);
     float s, zp;
     int e;
     qparams_from_minmax(smin, smax, p.dt, f, p.symmetric != 0, p.scale_mode, 1.f, &s, &zp, &e);
@@ -353,7 +353,7 @@ struct StepScale {
   }
   __device__ __forceinline__ void at(float factor, float* s, float* zp) const {
     if (RULE == RULE_SYM) {
-      const float a = round16_finite<DT>(amax * factor);
+      const float a = round16_finite<DT>(product<DT>(amax, factor));
       float q;
       if (corrected) {  // rhalf is correctly rounded, so one residual step gives the correctly rounded quotient
         q = a * rhalf;
@@ -377,7 +377,7 @@ struct StepScale {
       }
     }
     int e;
-    qparams_from_minmax(round_to<DT>(mn * factor), round_to<DT>(mx * factor), DT, f, RULE != RULE_ASYM,
+    qparams_from_minmax(round_to<DT>(product<DT>(mn, factor)), round_to<DT>(product<DT>(mx, factor)), DT, f, RULE != RULE_ASYM,
                         RULE == RULE_SYM_MX ? LLMC_SCALE_MXFP4 : LLMC_SCALE_PLAIN, 1.f, s, zp, &e);
   }
 };
@@ -444,8 +444,8 @@ __global__ __launch_bounds__(TAB ? TEAM_BLOCK : 256) void mse_team_fast_kernel(M
       mn = fminf(mn, __shfl_xor(mn, o, 64));
       mx = fmaxf(mx, __shfl_xor(mx, o, 64));
     }
-    mn = round_to<DT>(mn * p.expand);
-    mx = round_to<DT>(mx * p.expand);
+    mn = round_to<DT>(product<DT>(mn, p.expand));
+    mx = round_to<DT>(product<DT>(mx, p.expand));
     const bool values_plain = range.plain();
     float best = largest_finite<DT>();
     uint64_t mask[MW];
@@ -668,8 +668,8 @@ __global__ __launch_bounds__(ROW_THREADS* UNITS, 4) void mse_rows_fast_kernel(Ms
     __syncthreads();  // (also the table, the first time)
     mn = fminf(fminf(shm[unit][0], shm[unit][1]), fminf(shm[unit][2], shm[unit][3]));
     mx = fmaxf(fmaxf(shm[unit][4], shm[unit][5]), fmaxf(shm[unit][6], shm[unit][7]));
-    mn = round_to<DT>(mn * p.expand);
-    mx = round_to<DT>(mx * p.expand);
+    mn = round_to<DT>(product<DT>(mn, p.expand));
+    mx = round_to<DT>(product<DT>(mx, p.expand));
     const bool values_plain = range.plain();
     const StepScale<DT, FMT, RULE> scales(mn, mx, f);
     float s_prev = -1.f;
@@ -810,8 +810,8 @@ __global__ __launch_bounds__(256) void mse_generic_kernel(MseParams p, GenericLa
   __syncthreads();
   mn = fminf(fminf(shm[0], shm[1]), fminf(shm[2], shm[3]));
   mx = fmaxf(fmaxf(shm[4], shm[5]), fmaxf(shm[6], shm[7]));
-  mn = round_rt(mn * p.expand, p.dt);
-  mx = round_rt(mx * p.expand, p.dt);
+  mn = round_rt(product<LLMC_F16>(mn, p.expand), p.dt);
+  mx = round_rt(product<LLMC_F16>(mx, p.expand), p.dt);
   float best = p.dt == LLMC_BF16 ? 3.3895313892515355e38f : p.dt == LLMC_F16 ? 65504.0f : 3.4028234663852886e38f;
   if (p.err32) best = 3.4028234663852886e38f;
   uint64_t mask[MASK_WORDS];
@@ -819,7 +819,7 @@ __global__ __launch_bounds__(256) void mse_generic_kernel(MseParams p, GenericLa
   for (int wd = 0; wd < MASK_WORDS; ++wd) mask[wd] = 0ull;
   for (int i = 0; i < p.steps; ++i) {
     const float pi = step_factor(i, p.grid);
-    const float smin = round_rt(mn * pi, p.dt), smax = round_rt(mx * pi, p.dt);
+    const float smin = round_rt(product<LLMC_F16>(mn, pi), p.dt), smax = round_rt(product<LLMC_F16>(mx, pi), p.dt);
     float s, zp;
     int e_;
     qparams_from_minmax(smin, smax, p.dt, f, p.symmetric != 0, p.scale_mode, 1.f, &s, &zp, &e_);
@@ -884,8 +884,8 @@ __global__ __launch_bounds__(256) void mse_select_kernel(const uint64_t* __restr
   const float mn = load_rt(min0, i, dt), mx = load_rt(max0, i, dt);
   // no recorded improvement (e.g. non-finite errors): the reference keeps the un-shrunk range
   const float pb = best < 0 ? 1.0f : step_factor(best, grid);
-  store_rt(min_out, i, best < 0 ? mn : round_rt(mn * pb, dt), dt);
-  store_rt(max_out, i, best < 0 ? mx : round_rt(mx * pb, dt), dt);
+  store_rt(min_out, i, best < 0 ? mn : round_rt(product<LLMC_F16>(mn, pb), dt), dt);
+  store_rt(max_out, i, best < 0 ? mx : round_rt(product<LLMC_F16>(mx, pb), dt), dt);
 }
 
 inline int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }

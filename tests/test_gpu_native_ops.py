@@ -170,3 +170,32 @@ def test_dynamic_groups_of_one_very_wide_row():
     got = llmc.dynamic_group_quantize(x, 32, ops.FMT_FP8, 8)
     want = llmc.dynamic_group_quantize(x.view(1 << 14, -1), 32, ops.FMT_FP8, 8)
     assert torch.equal(got.view_as(want), want)
+
+
+@pytest.mark.parametrize("form", ["lanes", "rows", "blocks"])
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_mse_search_over_f16_rounds_the_shrunk_range_twice(form, symmetric):
+    """The range times the shrink factor is an fp32 value before it is an f16 one.  Every f16 magnitude between 8 and 16
+    where rounding the exact product to f16 at once gives another value, with one other value in its group (a sum of two
+    does not depend on its order): 28 of the 4000 symmetric searches end elsewhere when rounded once."""
+    from oracle import observers as O
+
+    args = F.QArgs(num_bits=4, strategy="group", group_size=8, symmetric=symmetric)
+    a = (torch.arange(1024) * 2.0 ** -7 + 8).half()
+    factors = torch.tensor([1.0 - i / 100.0 for i in range(20)]).float()
+    twice = (a.float()[:, None] * factors).half()
+    step = torch.where(a[:, None].double() * factors.double() < 8, 2.0 ** -8, 2.0 ** -7)
+    once = torch.round(a[:, None].double() * factors.double() / step) * step
+    a = a[(twice.double() != once).any(1)]
+    w = torch.zeros(4000, 8, dtype=torch.float16)
+    w[:, 3] = -a[torch.arange(4000) % len(a)]
+    w[:, 6] = ((torch.rand(4000, generator=torch.Generator().manual_seed(0)) * 2 - 1) * w[:, 3].float()).half()
+    want = O.grid_search_mse(O.flatten_for_calibration(w, "weight", args), args)
+    if form == "rows":  # two bytes off a 16-byte boundary
+        x = torch.cat([w.view(-1)[:1], w.view(-1)]).cuda()[1:].view(4000, 8)
+    else:
+        x = w.cuda()
+    got = (_llmc().mse_observe_blocks(x, 1, 8, 0, 4, symmetric) if form == "blocks"
+           else _llmc().mse_observe(x, 8, 0, 4, symmetric))
+    for g, e in zip(got, want):
+        assert torch.equal(g.cpu().reshape(-1), e.reshape(-1)), (g.cpu().reshape(-1) != e.reshape(-1)).sum()
