@@ -524,20 +524,27 @@ int llmc_gemm_x3(const GemmF32& g, hipStream_t st) {
   }
   // The tile: what each shape's workgroups take, in units of 7.4 us for a contraction of 512 (measured with 1 .. 8 passes
   // of the chip).  256 x 256: one per CU, 13 a pass.  128 x 128: two per CU, 7 a pass, 5 when each has a CU to itself.
-  // 64 x 64: 3 a pass of two per CU, 2 with a CU each; the steps at the diagonal of a triangular operand waste least
-  // there (0.6 of the time per tile).  Beyond one pass the workgroups follow each other without waiting, half a pass is the tail.
+  // 64 x 64: 3 a pass of two per CU, 2 with a CU each.  Beyond one pass the workgroups follow each other without waiting,
+  // half a pass is the tail.  With a triangular operand a tile's contraction is half as long on average, and the longest
+  // one bounds the call while the passes are few: lines through 14 products of 512 to 8192 columns, 0.2 to 24 passes
+  // (as 0.6 of the rectangular time, 6144 x 8192 x 8192 took 64 x 64 tiles and 3.14 ms; 256 x 256 take 2.11).
   const int64_t nbatch = (int64_t)g.batch * nb2;
   const bool fit256 = g.M % 256 == 0 && g.N % 256 == 0;
-  auto cost = [&](int edge, int per_cu, float pass, float alone) {
+  const bool tri = g.a_lower_tri || g.b_lower_tri;
+  struct Line {
+    float base, slope, least;
+  };
+  auto cost = [&](int edge, int per_cu, float pass, float alone, Line triangle) {
     const int64_t rows = g.M / edge, cols = g.N / edge;
     const int64_t tiles = (g.c_lower ? rows * cols / 2 + rows / 2 : rows * cols) * nbatch;
     const float full = 256.f * per_cu;
+    if (tri) return fmaxf(triangle.base + triangle.slope * (tiles / full), triangle.least);
     return tiles <= 256 ? alone : (tiles <= full ? pass : pass * (tiles / full + 0.5f));
   };
   constexpr float NEVER = 1e30f;
-  const float c256 = fit256 ? cost(256, 1, 13.f, 13.f) : NEVER;
-  const float c128 = cost(128, 2, 7.f, 5.f);
-  const float c64 = fit64 ? cost(64, 2, 3.f, 2.f) * (g.a_lower_tri || g.b_lower_tri ? 0.6f : 1.f) : NEVER;
+  const float c256 = fit256 ? cost(256, 1, 13.f, 13.f, {4.0f, 4.6f, 8.8f}) : NEVER;
+  const float c128 = cost(128, 2, 7.f, 5.f, {1.4f, 3.0f, 4.0f});
+  const float c64 = fit64 ? cost(64, 2, 3.f, 2.f, {0.4f, 1.1f, 1.8f}) : NEVER;
   if (c256 <= c128 && c256 <= c64)
     return g.trans_b ? launch_x3<64, 128, 4, 2, true>(g, st) : launch_x3<64, 128, 4, 2, false>(g, st);
   if (c64 < c128) return g.trans_b ? launch_x3_small<true, false>(g, st) : launch_x3_small<false, false>(g, st);
