@@ -636,11 +636,14 @@ struct Choice {
 // Phases for BT-wide tiles.  Whole rounds of NUM_WG tiles first.  When `split`, the R tiles left
 // over are cut along the tokens so that they fill a round too: R <= 128 -> one phase of
 // floor(256/R) chunks per tile; R > 128 -> 128 tiles in two chunks, then the rest as before.  A
-// chunk keeps at least 4 slabs.  time_us is a rough model used only to pick between candidates, fitted to 26 sizes from
-// 2 x 10568 to 16384 x 2048: 256-wide tiles take 1.15 us per slab with half the chip's CUs at work and 1.9 with all,
-// and 33 us for the epilogue of a round, 45 for every further one; 128-wide tiles, two to a CU, take 0.62 us per
-// slab and 8 us while they are few and grow with their number from there; partial tiles pass through the workspace
-// at 3 TB/s.
+// chunk keeps at least 4 slabs.  time_us is a rough model used only to pick between candidates, fitted to the four
+// candidates' times at 456 sizes (16 to 32768 tokens, 256 to 14336 columns; rms error 11 %): the pick is 0.5 % slower than
+// the best of the four on average and 16 % at most.  256-wide tiles take 1.18 us per slab with up to half the chip's CUs at
+// work and 1.72 with all; the epilogue of a round takes 25 to 38 us, 54 more for every further one, 12 where partial
+// tiles are written.  128-wide tiles, two to a CU, take 0.55 us per slab while there is at most one to a CU or so and 1.18
+// with two; their epilogues grow with their number, faster from 1200 tiles on, where H leaves the last-level cache.
+// Partial tiles pass through the workspace at 5.8 TB/s.  (A fit to 26 sizes before this one charged 128-wide tiles in
+// token chunks twice their time: 16384 x 768 took 48 us, 29 now; 4096 x 1536 46 and 29.)
 Choice make_choice(int bt, int64_t T, int64_t K, bool split) {
   Choice c;
   c.bt = bt;
@@ -663,12 +666,15 @@ Choice make_choice(int bt, int64_t T, int64_t K, bool split) {
     if (sp > 1) ws_tile += items;
     const int rounds = (items + NUM_WG - 1) / NUM_WG, slabs = (nslab + sp - 1) / sp;
     if (bt == 256) {
-      const double fill = (double)items / (rounds * NUM_WG);
-      c.time_us += rounds * slabs * (1.15 + (fill > 0.5 ? 1.5 * (fill - 0.5) : 0.0));
-      c.time_us += sp > 1 ? 5.0 * rounds : 33.0 + 45.0 * (rounds - 1);
+      auto slab_us = [](double fill) { return 1.18 + (fill > 0.5 ? 1.08 * (fill - 0.5) : 0.0); };
+      const int full = items / NUM_WG, rest = items % NUM_WG;
+      c.time_us += slabs * (full * slab_us(1.0) + (rest ? slab_us((double)rest / NUM_WG) : 0.0));
+      c.time_us += sp > 1 ? 12.0 * rounds : 25.0 + 54.0 * (rounds - 1) + 13.0 * (full ? 1.0 : (double)rest / NUM_WG);
     } else {
-      const double busy = 0.0042 * items;
-      c.time_us += slabs * (busy > 0.62 ? busy : 0.62) + (sp > 1 ? 5.0 + 0.01 * items : 8.0 + 0.07 * items);
+      auto slab_us = [](int n) { return 0.55 + (n > 196 ? 0.002 * (n - 196) : 0.0); };
+      const int full = items / (2 * NUM_WG), rest = items % (2 * NUM_WG);
+      c.time_us += slabs * (full * slab_us(2 * NUM_WG) + (rest ? slab_us(rest) : 0.0));
+      c.time_us += (sp > 1 ? 1.3 + 0.008 * items : 6.7 + 0.04 * items) + (items > 1200 ? 0.118 * (items - 1200) : 0.0);
     }
   };
   int slimit = nslab / 4;
@@ -694,7 +700,7 @@ Choice make_choice(int bt, int64_t T, int64_t K, bool split) {
   }
   c.nsplit_tiles = nt - (c.first_split_phase < plan.nphase ? plan.ph[c.first_split_phase].tile0 : nt);
   c.ws_bytes = (int64_t)ws_tile * bt * bt * 4;
-  c.time_us += c.ws_bytes * 2 / 3e6 + (ws_tile ? 15.0 : 0.0);  // partial tiles written and read back, reduce kernel
+  c.time_us += c.ws_bytes * 2 / 5.8e6 + (ws_tile ? 9.0 : 0.0);  // partial tiles written and read back, reduce kernel
   c.grid = wg;
   return c;
 }
