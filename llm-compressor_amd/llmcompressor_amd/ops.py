@@ -117,7 +117,7 @@ def hessian_accumulate_grouped_(Hs, xs, alpha: float = 2.0, assume_symmetric: bo
     x_ref = next((x for x in xs if x.shape[0] > 0), None)
     if x_ref is None:
         return Hs
-    _require_gpu(H0, x_ref)
+    _require_gpu(H0, *(x for x in xs if x.shape[0] > 0))
     if x_ref.dtype not in (torch.bfloat16, torch.float16):
         raise TypeError(f"hessian_accumulate_grouped_: unsupported activation dtype {x_ref.dtype}")
     n = len(Hs)
@@ -274,7 +274,7 @@ def gptq_hinv_(H: torch.Tensor, perm=None, divisor: float = 1.0, percdamp: float
     outside them.
 
     Returns (U (= H), dead uint8 [K], info int32 [1] on device)."""
-    _require_gpu(H)
+    _require_gpu(H, perm)
     assert H.dtype == torch.float32 and H.ndim == 2 and H.shape[0] == H.shape[1] and H.stride(1) == 1
     K = H.shape[0]
     dead = torch.empty(K, dtype=torch.uint8, device=H.device)
@@ -298,7 +298,7 @@ def gptq_hinv_grouped(Hs, perms=None, divisors=None, percdamp: float = 0.01, for
 
     n = len(Hs)
     H0 = Hs[0]
-    _require_gpu(H0)
+    _require_gpu(H0, perms)
     K = H0.shape[0]
     for H in Hs:
         assert H.dtype == torch.float32 and H.shape == (K, K) and H.stride(1) == 1 and H.stride(0) == H0.stride(0)
@@ -328,8 +328,8 @@ def gptq_quantize(weight, U, scale, zero_point, fmt: int, bits: int, row_div: in
                   form: int = FACTOR_INVERSE):
     """The GPTQ column loop on a factor of the given form (see gptq_hinv_).  Returns (quantised-dequantised weight
     in weight.dtype, loss fp32 [1])."""
+    _require_gpu(weight, U, scale, zero_point, global_scale, g_idx, perm, dead)
     global_scale = _gs32(global_scale)
-    _require_gpu(weight, U, scale)
     assert weight.ndim == 2 and weight.stride(1) == 1 and U.stride(1) == 1
     R, K = weight.shape
     scale = scale.contiguous()
@@ -364,7 +364,7 @@ def gptq_quantize_grouped(weights, U, scales, zero_points, fmt: int, bits: int, 
 
     n = len(weights)
     w0 = weights[0]
-    _require_gpu(w0, U)
+    _require_gpu(*weights, U, *scales, *(zero_points or ()), *(global_scales or ()), *(g_idxs or ()), perms, dead)
     R, K = w0.shape
     keep = []
 
@@ -406,7 +406,7 @@ def sparsegpt_sparsify(weight, U, sparsity: float, prune_n: int = 0, prune_m: in
                        blocksize: int = 128, preserve_sparsity_mask: bool = False, form: int = FACTOR_INVERSE):
     """The SparseGPT column loop on the factor U of gptq_hinv_ (of the given form).  Returns (pruned weight in
     weight.dtype, loss fp32 [1])."""
-    _require_gpu(weight, U)
+    _require_gpu(weight, U, dead)
     assert weight.ndim == 2 and weight.stride(1) == 1 and U.stride(1) == 1
     R, K = weight.shape
     if prune_n:

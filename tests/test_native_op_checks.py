@@ -104,3 +104,24 @@ def test_a_search_range_that_is_not_finite_is_refused(maxshrink, grid):
     w = _fake("cuda:0", 4, 32)
     with pytest.raises(ValueError, match="not finite"):
         _call("mse_observe", w, 16, 0, 4, True, 0, maxshrink, 5, grid)
+
+
+def _gptq_args(host):
+    f32, bf = torch.float32, torch.bfloat16
+    made = {"weight": ((4, 32), bf), "U": ((32, 32), f32), "scale": ((4, 1), bf), "zero_point": ((4, 1), torch.int8),
+            "g_idx": ((32,), torch.int32), "perm": ((32,), torch.int32), "dead": ((32,), torch.uint8), "global_scale": ((1,), f32)}
+    return {k: _host(*s, dtype=d) if k == host else _fake("cuda:0", *s, dtype=d) for k, (s, d) in made.items()}
+
+
+@pytest.mark.parametrize("host", list(_gptq_args("")))
+def test_the_column_loop_refuses_a_host_tensor_in_any_place(host):
+    from llmcompressor_amd import ops
+
+    a = _gptq_args(host)
+    with pytest.raises(RuntimeError, match="device tensors only; got a cpu tensor"):
+        ops.gptq_quantize(a["weight"], a["U"], a["scale"], a["zero_point"], 0, 4, 1, 1, g_idx=a["g_idx"], perm=a["perm"],
+                          dead=a["dead"], global_scale=a["global_scale"])
+    with pytest.raises(RuntimeError, match="device tensors only; got a cpu tensor"):
+        ops.gptq_quantize_grouped([a["weight"]], a["U"][None], [a["scale"]], [a["zero_point"]], 0, 4, 1, 1,
+                                  g_idxs=[a["g_idx"]], perms=a["perm"][None], dead=a["dead"][None],
+                                  global_scales=[a["global_scale"]])
