@@ -855,7 +855,7 @@ inline GptqWork gptq_work(char* p, int64_t n, int64_t R, int64_t K) {
 // product per block).
 //
 // Rows per workgroup: 16 while that is at most one workgroup per CU (4096 rows in all), 32 beyond: a pass of the chip
-// over the group takes 45 us with 16 rows each and 63 us with 32 (see gptq_group.h).  Both give the same bits.
+// over the group takes 48 us with 16 rows each and 65-70 us with 32 (see gptq_group.h).  Both give the same bits.
 constexpr int64_t Q_FEW_ROWS = 16 * 256;
 static int gptq_column_loop(GptqGroupParams p, bool has_zp, int n, int64_t R, int64_t K, int bs,
                             const GptqWork& w, int form, hipStream_t st) {
