@@ -24,6 +24,7 @@ count over the shorter time.  Prints ONE JSON line.
 from __future__ import annotations
 
 import argparse
+import gc
 import json
 import os
 import sys
@@ -546,6 +547,7 @@ def probe_oneshot_moe(batches=16, tokens=2048, layers=2, vocab=32000):
             peak = torch.cuda.max_memory_allocated() / 2 ** 30
             del model
             active_session().reset()  # the session still refers to the model it compressed
+            gc.collect()  # a model is a cycle: left to itself it may count in the next row's peak
             torch.cuda.empty_cache()
             if best is None or dt < best[0]:
                 best = (dt, peak)
