@@ -110,6 +110,63 @@ def test_column_loop_on_two_term_products(R, K, spread):
     assert torch.allclose(errs[0], errs[1], rtol=0.02)
 
 
+def _exact_loop(W, H, scale, percdamp):
+    """int4 codes of 128-column groups by the column loop in 64 bits, from the 64-bit factor of H."""
+    K = H.shape[0]
+    Hd = H.double().cpu() + percdamp * H.diagonal().double().mean().cpu() * torch.eye(K, dtype=torch.float64)
+    V = torch.linalg.cholesky(Hd.flip(0, 1)).flip(0, 1)
+    U = torch.linalg.solve_triangular(V, torch.eye(K, dtype=torch.float64), upper=True).cuda()
+    W, codes = W.double().clone(), torch.empty(W.shape, device=W.device)
+    for j in range(K):
+        s = scale[:, j // 128].double()
+        codes[:, j] = torch.round(W[:, j] / s).clamp(-8, 7)
+        W[:, j + 1:] -= ((W[:, j] - codes[:, j] * s) / U[j, j])[:, None] * U[j, j + 1:]
+    return codes
+
+
+def _two_sets(K, T, seed, other):
+    """Activations of which the channels `other` never fire together with the rest."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn(T, K, device="cuda", generator=g)
+    x *= torch.logspace(-0.5, 0.5, K, device="cuda")[torch.randperm(K, device="cuda", generator=g)]
+    x[:T // 4, ~other] = 0
+    x[T // 4:, other] = 0
+    return x
+
+
+def _loop_agreement(x, percdamp, form, seed):
+    """Share of the int4 codes of a column loop on x^T x that are those of 64 bits."""
+    from llmcompressor_amd import ops
+
+    K, R = x.shape[1], 256
+    H = (x.double().T @ x.double()).float()
+    H = (H + H.T) / 2
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    w = torch.randn(R, K, device="cuda", generator=g) * 0.02
+    scale = w.view(R, K // 128, 128).abs().amax(-1) / 7.5
+    U, info = _chain(H, form, percdamp)
+    assert info == 0
+    q, _ = ops.gptq_quantize(w, U, scale, None, ops.FMT_INT, 4, 1, K // 128, form=form,
+                             g_idx=torch.arange(K, dtype=torch.int32, device="cuda") // 128)
+    codes = torch.round(q / scale.repeat_interleave(128, 1))
+    return (codes == _exact_loop(w, H, scale, percdamp)).float().mean().item()
+
+
+@pytest.mark.parametrize("channels", [1, 8])
+@pytest.mark.parametrize("exponent", [0, -15, -20, -40])
+def test_rows_of_the_factor_without_later_columns(channels, exponent):
+    """Channels of the first group that fire only by themselves: their rows of the factor are zero beyond the diagonal
+    block, and what the loop keeps of their weights must not push the other columns out of the products' range, however
+    small the Hessian is."""
+    from llmcompressor_amd import ops
+
+    K = 1536
+    other = torch.zeros(K, dtype=torch.bool, device="cuda")
+    other[torch.arange(channels, device="cuda") * 37] = True
+    x = _two_sets(K, 3 * K, 5 + channels, other) * 2.0 ** exponent
+    assert _loop_agreement(x, 0.01, ops.FACTOR_GROUPS, seed=2) >= 0.999
+
+
 @pytest.mark.parametrize("K", [1, 3, 64, 65, 1023, 1025, 16384])
 def test_diagonal_order_at_the_edges_of_its_workgroups(K):
     from llmcompressor_amd import ops
