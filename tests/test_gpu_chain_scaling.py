@@ -43,6 +43,36 @@ def test_factor_against_64_bits(K):
     assert err.max().item() < K ** 0.5 * 2 ** -24 * 30, err.max().item()
 
 
+def _common_directions(K):
+    """Channels that all read the same 64 directions, most of the quiet ones' energy: the first updates of the factorisation
+    take nearly all of the matrix away, and the rounding of their sums is what is left."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn(2 * K, K, device="cuda", generator=g)
+    x *= torch.logspace(-1, 1, K, device="cuda")[torch.randperm(K, device="cuda", generator=g)]
+    x += torch.randn(2 * K, 64, device="cuda", generator=g) @ (torch.randn(64, K, device="cuda", generator=g) * 0.3)
+    x = x[:, x.square().sum(0).argsort(descending=True)].contiguous()
+    H = torch.zeros(K, K, dtype=torch.float64, device="cuda")
+    for part in x.split(2048):
+        H += part.double().T @ part.double()
+    return (H / (2 * K)).float()
+
+
+# Bounds: what three-term products give in the same panels of 256 columns (512 from 8192 on).  Measured 6.2e-6, 7.2e-6 and
+# 1.47e-5; 8.3e-6, 9.9e-6 and 1.95e-5 with panels twice as wide, whose sums are rounded twice as often.
+@pytest.mark.parametrize("K,bound", [(3072, 7.28e-6), (4096, 8.47e-6), (8192, 1.62e-5)])
+def test_sums_of_an_update_are_short(K, bound):
+    H = _common_directions(K)
+    V, info = _chain(H, form=1)
+    assert info == 0
+    Hd = H.double().cpu()
+    Hd += 0.01 * Hd.diagonal().mean() * torch.eye(K, dtype=torch.float64)
+    want = torch.linalg.cholesky(Hd.flip(0, 1)).flip(0, 1).cuda()
+    block = torch.arange(K, device="cuda").flip(0) // 512  # inside these blocks V holds the inverse
+    far = block[:, None] != block[None, :]
+    err = ((V.double() - want)[far].norm() / want[far].norm()).item()
+    assert err < bound, err
+
+
 @pytest.mark.parametrize("K,form", [(320, 0), (1000, 0), (1152, 1), (2304, 0)])
 @pytest.mark.parametrize("shift", [-60, 24])
 def test_powers_of_two_pass_through(K, form, shift):
