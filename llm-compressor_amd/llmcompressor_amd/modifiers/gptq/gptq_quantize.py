@@ -253,9 +253,11 @@ def finish_weight_group(ctx, blocksize: int = 128):
     n, order, mods, keys = ctx["n"], ctx["order"], ctx["mods"], ctx["keys"]
     perms, all_perms, U, dead, info = ctx["perms"], ctx["all_perms"], ctx["U"], ctx["dead"], ctx["info"]
     form = ctx["form"]
-    if ops.gptq_quantize_form(U.shape[-1], blocksize) != ops.gptq_quantize_form(U.shape[-1], ctx["blocksize"]):
+    if ops.gptq_factor_form(U.shape[-1], blocksize) != ops.gptq_factor_form(U.shape[-1], ctx["blocksize"]):
         raise ValueError(f"finish_weight_group: block size {blocksize} does not fit the factors, which were prepared "
                          f"for block size {ctx['blocksize']}")
+    if form == ops.FACTOR_GROUPS:  # its loop runs in blocks of 128; the block size only regroups fp32 sums
+        blocksize = max(blocksize, 128)
     prep = []
     base_g_idx = {}
     for j, m in enumerate(mods):

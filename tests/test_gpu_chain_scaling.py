@@ -207,3 +207,39 @@ def test_diagonal_order_at_the_edges_of_its_workgroups(K):
     got = ops.diag_argsort_desc(Hs)
     for row, H in zip(got, Hs):
         assert torch.equal(row, torch.argsort(H.diagonal(), descending=True, stable=True))
+
+
+def _linears(K, rows, count, seed=0):
+    """(modules, their Hessians): W4A16 in groups of 128 columns, static activation order."""
+    from llmcompressor_amd.modifiers.quantization.calibration import initialize_observer
+    from llmcompressor_amd.quantization import initialize_module_for_quantization, preset_name_to_scheme
+
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    mods = []
+    for i in range(count):
+        m = torch.nn.Linear(K, rows, bias=False, dtype=torch.bfloat16, device="cuda")
+        m.weight.data = (torch.randn(rows, K, device="cuda", generator=g) * 0.02).bfloat16()
+        initialize_module_for_quantization(m, preset_name_to_scheme("W4A16", ["Linear"]))
+        initialize_observer(m, "weight")
+        mods.append(m)
+    return mods, [_hessian(K, 2 * K, seed + 10 + i) for i in range(count)]
+
+
+@torch.no_grad()
+@pytest.mark.parametrize("K", [1024, 1536])
+def test_weight_group_finished_in_another_block_size(K):
+    """The halves of ``quantize_weight_group`` take block sizes of their own: the block size only regroups fp32 sums, whatever
+    form of the factor the first half has asked for (below 8192 columns, where that depends on it)."""
+    from llmcompressor_amd.modifiers.gptq.gptq_quantize import (begin_weight_group, finish_weight_group,
+                                                                quantize_weight_group)
+    from llmcompressor_amd.modifiers.quantization.calibration import observe
+
+    mods, Hs = _linears(K, 256, 3)
+    divisors = [1.0] * len(mods)
+    observe(mods, "weight")
+    want = quantize_weight_group(mods, Hs, divisors)
+    for first, second in ((128, 64), (64, 128)):
+        observe(mods, "weight")
+        got = finish_weight_group(begin_weight_group(mods, Hs, divisors, blocksize=first), second)
+        agree = torch.stack([(a[1]["weight"] == b[1]["weight"]).float().mean() for a, b in zip(got, want)])
+        assert agree.min().item() >= 0.999, (first, second, agree)

@@ -606,6 +606,23 @@ def test_gptq_job_planning():
     assert mod._plan_jobs(list(mods)) == mods
 
 
+@pytest.mark.parametrize("K,refused", [(512, False), (1536, False), (4096, False), (8192, True), (1600, False)])
+def test_gptq_block_size_of_a_group_in_two_halves(K, refused):
+    """``finish_weight_group`` refuses a block size only where the first half's asked for a factor that the loop of the other
+    cannot read and has always been refused: from 8192 columns on."""
+    from llmcompressor_amd import ops
+    from llmcompressor_amd.modifiers.gptq.gptq_quantize import finish_weight_group
+
+    for first, second in ((128, 64), (64, 128), (128, 256), (32, 96)):
+        ctx = dict(n=0, order=[], mods=[], keys=[], perms=None, all_perms=None, U=torch.empty(0, K, K), dead=None, info=None,
+                   form=ops.gptq_quantize_form(K, first), blocksize=first)
+        if refused and (first < 128) != (second < 128):
+            with pytest.raises(ValueError, match="does not fit the factors"):
+                finish_weight_group(ctx, second)
+        else:
+            assert finish_weight_group(ctx, second) == []
+
+
 def test_observed_kv_cache_stand_in():
     """The stand-in for ``past_key_values`` shows keys and values to the module's observers and defers to the
     real cache when there is one."""
