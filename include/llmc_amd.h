@@ -295,7 +295,8 @@ int llmc_dynamic_per_token_quantize(const void* x, int32_t x_dtype, int64_t N, i
  * third of its arithmetic.  The blocks are aligned to the last column: [K-512, K), [K-1024, K-512), ..., and a
  * first block of the K % 512 columns that are left.  llmc_gptq_quantize takes either form and gives the same
  * result up to fp32 rounding, and so does llmc_sparsegpt_sparsify (its block size must then be 128).
- * llmc_gptq_quantize_form(K, blocksize) is the form the library prefers for a quantize_weight call,
+ * llmc_gptq_quantize_form_rows(R, K, blocksize) is the form the library prefers for a quantize_weight call on R rows,
+ * llmc_gptq_quantize_form(K, blocksize) the same for a weight of few rows (at most K),
  * llmc_gptq_factor_form(K, blocksize) the one for any column loop (sparsify_weight's).
  */
 enum {
@@ -305,6 +306,7 @@ enum {
 };
 int32_t llmc_gptq_factor_form(int64_t K, int32_t blocksize);
 int32_t llmc_gptq_quantize_form(int64_t K, int32_t blocksize);
+int32_t llmc_gptq_quantize_form_rows(int64_t R, int64_t K, int32_t blocksize);
 int64_t llmc_gptq_hinv_workspace_bytes(int64_t K);
 int llmc_gptq_hinv(float* H, int64_t ldh, int64_t K, const int32_t* perm, float divisor,
                    float percdamp, int32_t form, uint8_t* dead_out, void* workspace,
@@ -328,6 +330,12 @@ int llmc_gptq_hinv_grouped(const float* const* H, int64_t ldh, int32_t n, int64_
                            const int32_t* const* perm, const float* divisors, float percdamp,
                            int32_t form, uint8_t* dead_out, float* U_out, int64_t ldu, void* workspace,
                            int64_t workspace_bytes, int32_t* info_out, void* stream);
+/* The same where the loops of some problems want the other form: the first n_inverse problems get
+ * LLMC_FACTOR_INVERSE whatever `form` says. */
+int llmc_gptq_hinv_grouped_forms(const float* const* H, int64_t ldh, int32_t n, int64_t K,
+                                 const int32_t* const* perm, const float* divisors, float percdamp,
+                                 int32_t form, uint8_t* dead_out, float* U_out, int64_t ldu, void* workspace,
+                                 int64_t workspace_bytes, int32_t* info_out, int32_t n_inverse, void* stream);
 
 /* ---- a8/a9: GPTQ block column loop ---------------------------------------------
  * Replaces the loop of quantize_weight (gptq_quantize.py:88-92,144-146,167-250):

@@ -129,7 +129,7 @@ def quantize_weight_tensors(weight: torch.Tensor, observer, quant_args: Quantiza
     # dead columns, damping, Cholesky -> inverse -> upper factor; identity on failure
     # (where the width allows it the chain stops at the Cholesky factor of H outside 512-column diagonal blocks
     # and the column loop works from that: same result up to fp32 rounding, a third less arithmetic in the chain)
-    form = ops.gptq_quantize_form(num_columns, blocksize)
+    form = ops.gptq_quantize_form(num_columns, blocksize, num_rows)
     dead, info = llmc.gptq_prepare_hinv_(H, perm, float(hessian_divisor), float(percdamp), form)
     U = H  # overwritten in place by the factor
 
@@ -209,19 +209,21 @@ def begin_weight_group(modules, hessians, hessian_divisors, percdamp: float = 0.
     enqueue the chains of several sets, observe the weights while they run, and finish afterwards."""
     n = len(modules)
     keys = [group_key(m, m.quantization_scheme.weights, H) for m, H in zip(modules, hessians)]
-    # members of one column-loop set next to each other, so that their factors are one slice of the batch
-    order = sorted(range(n), key=lambda i: (keys.index(keys[i]), i))
+    # the form of the factor that each member's loop is given by itself (those of the full inverse in front), and members of one
+    # column-loop set next to each other, so that their factors are one slice of the batch
+    forms = [ops.gptq_quantize_form(m.weight.shape[1], blocksize, m.weight.shape[0]) for m in modules]
+    order = sorted(range(n), key=lambda i: (forms[i] != ops.FACTOR_INVERSE, keys.index(keys[i]), i))
     mods = [modules[i] for i in order]
     Hs = [hessians[i] for i in order]
     divs = [hessian_divisors[i] for i in order]
-    keys = [keys[i] for i in order]
+    keys, forms = [keys[i] for i in order], [forms[i] for i in order]
     # Members that were given the very same Hessian tensor (Linears fed one input: q/k/v, gate/up) with the same
-    # divisor and the same ordering rule have the same column order and the same factor: the chain runs once per
-    # distinct Hessian and the members take copies of its results.
+    # divisor, the same ordering rule and the same form have the same column order and the same factor: the chain runs once
+    # per distinct Hessian and the members take copies of its results.
     ordered = [bool(m.quantization_scheme.weights.actorder) for m in mods]
     first_of, source = {}, []
-    for i, (H, d, o) in enumerate(zip(Hs, divs, ordered)):
-        source.append(first_of.setdefault((id(H), float(d), o), i))
+    for i, (H, d, o, f) in enumerate(zip(Hs, divs, ordered, forms)):
+        source.append(first_of.setdefault((id(H), float(d), o, f), i))
     distinct = sorted(set(source))
     shared = len(distinct) < n
     uH, udiv, uord = [Hs[i] for i in distinct], [divs[i] for i in distinct], [ordered[i] for i in distinct]
@@ -233,8 +235,9 @@ def begin_weight_group(modules, hessians, hessian_divisors, percdamp: float = 0.
     else:
         single = [_diag_order([H])[0] if o else None for o, H in zip(uord, uH)]
         perms = torch.stack(single) if single[0] is not None else None
-    form = ops.gptq_quantize_form(uH[0].shape[0], blocksize)
-    U, dead, info = llmc.gptq_prepare_hinv_grouped(uH, perms, [float(d) for d in udiv], float(percdamp), form)
+    inverses = sum(forms[i] == ops.FACTOR_INVERSE for i in distinct)
+    U, dead, info = llmc.gptq_prepare_hinv_grouped(uH, perms, [float(d) for d in udiv], float(percdamp), form=forms[-1],
+                                                   n_inverse=inverses)
     if shared:
         slot = {i: j for j, i in enumerate(distinct)}
         # through pinned memory, so that the host does not wait for the chain it has just enqueued
@@ -244,7 +247,7 @@ def begin_weight_group(modules, hessians, hessian_divisors, percdamp: float = 0.
             perms = perms[take]
             all_perms = perms if all_perms is not None else None
     return dict(n=n, order=order, mods=mods, keys=keys, perms=perms, all_perms=all_perms, U=U, dead=dead, info=info,
-                form=form, blocksize=blocksize)
+                forms=forms, blocksize=blocksize)
 
 
 def finish_weight_group(ctx, blocksize: int = 128):
@@ -252,12 +255,9 @@ def finish_weight_group(ctx, blocksize: int = 128):
     column loops on the factors of ``begin_weight_group``, and the results in the caller's order."""
     n, order, mods, keys = ctx["n"], ctx["order"], ctx["mods"], ctx["keys"]
     perms, all_perms, U, dead, info = ctx["perms"], ctx["all_perms"], ctx["U"], ctx["dead"], ctx["info"]
-    form = ctx["form"]
     if ops.gptq_factor_form(U.shape[-1], blocksize) != ops.gptq_factor_form(U.shape[-1], ctx["blocksize"]):
         raise ValueError(f"finish_weight_group: block size {blocksize} does not fit the factors, which were prepared "
                          f"for block size {ctx['blocksize']}")
-    if form == ops.FACTOR_GROUPS:  # its loop runs in blocks of 128; the block size only regroups fp32 sums
-        blocksize = max(blocksize, 128)
     prep = []
     base_g_idx = {}
     for j, m in enumerate(mods):
@@ -294,11 +294,14 @@ def finish_weight_group(ctx, blocksize: int = 128):
         part = prep[at:end]
         first = part[0]
         fmt, bits = kernel_format(first["args"])
+        form, bs = ctx["forms"][at], blocksize
+        if form == ops.FACTOR_GROUPS:  # its loop runs in blocks of 128; the block size only regroups fp32 sums
+            bs = max(bs, 128)
         if end - at == 1:
             outs[at], losses[at] = llmc.gptq_quantize(
                 first["W"], U[at], first["kscale"], first["zp"], fmt, bits, first["row_div"], first["srow"],
                 g_idx=first["g_idx"], perm=first["perm"], dead=dead[at], global_scale=first["qp"]["global_scale"],
-                blocksize=blocksize, form=form)
+                blocksize=bs, form=form)
         else:
             has_gs = first["qp"]["global_scale"] is not None
             o, l = llmc.gptq_quantize_grouped(
@@ -306,7 +309,7 @@ def finish_weight_group(ctx, blocksize: int = 128):
                 None if first["zp"] is None else [p["zp"] for p in part], fmt, bits, first["row_div"], first["srow"],
                 g_idxs=None if first["g_idx"] is None else [p["g_idx"] for p in part],
                 perms=None if perms is None else perms[at:end], dead=dead[at:end],
-                global_scales=[p["qp"]["global_scale"] for p in part] if has_gs else None, blocksize=blocksize,
+                global_scales=[p["qp"]["global_scale"] for p in part] if has_gs else None, blocksize=bs,
                 form=form)
             for b in range(end - at):
                 outs[at + b], losses[at + b] = o[b], l[b]

@@ -268,9 +268,10 @@ def gptq_factor_form(K: int, blocksize: int = 128) -> int:
     return int(_lib.lib().llmc_gptq_factor_form(int(K), int(blocksize)))
 
 
-def gptq_quantize_form(K: int, blocksize: int = 128) -> int:
-    """gptq_factor_form for a quantize_weight call, whose loop is faster on FACTOR_GROUPS: from 1536 columns on."""
-    return int(_lib.lib().llmc_gptq_quantize_form(int(K), int(blocksize)))
+def gptq_quantize_form(K: int, blocksize: int = 128, rows: int = 0) -> int:
+    """gptq_factor_form for a quantize_weight call on a weight of ``rows`` rows, whose loop is faster on FACTOR_GROUPS: from
+    1536 columns on for weights of at most K rows, from 4096 on for all."""
+    return int(_lib.lib().llmc_gptq_quantize_form_rows(int(rows), int(K), int(blocksize)))
 
 
 def gptq_hinv_(H: torch.Tensor, perm=None, divisor: float = 1.0, percdamp: float = 0.01, form: int = FACTOR_INVERSE):
@@ -296,9 +297,11 @@ def gptq_hinv_(H: torch.Tensor, perm=None, divisor: float = 1.0, percdamp: float
     return H, dead, info
 
 
-def gptq_hinv_grouped(Hs, perms=None, divisors=None, percdamp: float = 0.01, form: int = FACTOR_INVERSE):
+def gptq_hinv_grouped(Hs, perms=None, divisors=None, percdamp: float = 0.01, form: int = FACTOR_INVERSE,
+                      n_inverse: int = 0):
     """gptq_hinv_ for n Hessians of one width in lock-step.  Hs: list of fp32 [K,K] (left untouched); perms:
-    int32 [n,K] tensor or None; divisors: list of floats.  Returns (U [n,K,K] fp32, dead [n,K] uint8, info [n])."""
+    int32 [n,K] tensor or None; divisors: list of floats; the first n_inverse get FACTOR_INVERSE whatever ``form`` says.
+    Returns (U [n,K,K] fp32, dead [n,K] uint8, info [n])."""
     import ctypes
 
     n = len(Hs)
@@ -321,9 +324,9 @@ def gptq_hinv_grouped(Hs, perms=None, divisors=None, percdamp: float = 0.01, for
     nbytes = _lib.lib().llmc_gptq_hinv_grouped_workspace_bytes(n, K)
     ws = _workspace(H0.device, nbytes)
     with torch.cuda.device(H0.device):
-        rc = _lib.lib().llmc_gptq_hinv_grouped(hp, H0.stride(0), n, K, pp, dv, float(percdamp), int(form),
-                                              dead.data_ptr(), U.data_ptr(), K, ws.data_ptr(), ws.numel(),
-                                              info.data_ptr(), _stream(H0))
+        rc = _lib.lib().llmc_gptq_hinv_grouped_forms(hp, H0.stride(0), n, K, pp, dv, float(percdamp), int(form),
+                                                    dead.data_ptr(), U.data_ptr(), K, ws.data_ptr(), ws.numel(),
+                                                    info.data_ptr(), int(n_inverse), _stream(H0))
     _lib.check(rc, "llmc_gptq_hinv_grouped")
     return U, dead, info
 

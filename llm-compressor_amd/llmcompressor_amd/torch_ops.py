@@ -72,8 +72,9 @@ def _gptq_prepare_hinv_(H, perm=None, divisor=1.0, percdamp=0.01, form=0):
     return dead, info
 
 
-def _gptq_prepare_hinv_grouped(Hs, perms=None, divisors=None, percdamp=0.01, form=0):
-    return _impl.gptq_hinv_grouped(list(Hs), perms, None if divisors is None else list(divisors), percdamp, form=form)
+def _gptq_prepare_hinv_grouped(Hs, perms=None, divisors=None, percdamp=0.01, form=0, n_inverse=0):
+    return _impl.gptq_hinv_grouped(list(Hs), perms, None if divisors is None else list(divisors), percdamp, form=form,
+                                   n_inverse=n_inverse)
 
 
 def _gptq_quantize(W, Hinv, scale, zero_point, fmt, num_bits, row_div, scale_row_stride, g_idx=None, perm=None,
@@ -100,7 +101,7 @@ def _sparsegpt_sparsify(W, Hinv, sparsity, prune_n=0, prune_m=0, dead=None, bloc
 _register("gptq_prepare_hinv_(Tensor(a!) H, Tensor? perm=None, float divisor=1.0, float percdamp=0.01, int form=0) "
           "-> (Tensor dead, Tensor info)", _gptq_prepare_hinv_)
 _register("gptq_prepare_hinv_grouped(Tensor[] Hs, Tensor? perms=None, float[]? divisors=None, float percdamp=0.01, "
-          "int form=0) "
+          "int form=0, int n_inverse=0) "
           "-> (Tensor U, Tensor dead, Tensor info)", _gptq_prepare_hinv_grouped)
 _register("gptq_quantize(Tensor W, Tensor Hinv, Tensor scale, Tensor? zero_point, int fmt, int num_bits, int row_div, "
           "int scale_row_stride, Tensor? g_idx=None, Tensor? perm=None, Tensor? dead=None, Tensor? global_scale=None, "

@@ -615,7 +615,7 @@ def test_gptq_block_size_of_a_group_in_two_halves(K, refused):
 
     for first, second in ((128, 64), (64, 128), (128, 256), (32, 96)):
         ctx = dict(n=0, order=[], mods=[], keys=[], perms=None, all_perms=None, U=torch.empty(0, K, K), dead=None, info=None,
-                   form=ops.gptq_quantize_form(K, first), blocksize=first)
+                   forms=[], blocksize=first)
         if refused and (first < 128) != (second < 128):
             with pytest.raises(ValueError, match="does not fit the factors"):
                 finish_weight_group(ctx, second)
