@@ -34,7 +34,7 @@ from ..quantization.calibration import observe, update_qparams
 from ..quantization.quantization import QuantizationMixin
 from ..utils.concurrent import SIDE_STREAMS, run_on_streams
 from ..utils.hessian_staging import HessianStagingMixin
-from .gptq_quantize import (accumulate_hessian, begin_weight_group, finish_weight_group, make_empty_hessian,
+from .gptq_quantize import (GROUP_MAX_BYTES, accumulate_hessian, begin_weight_group, finish_weight_group, make_empty_hessian,
                             quantize_weight, quantize_weight_group,
                             width_key)
 
@@ -78,7 +78,8 @@ class GPTQModifier(Modifier, QuantizationMixin, HessianStagingMixin):
     :param group_min_modules: when at least this many Linears of one ``compress_module_list`` call have the same
         number of input features (the experts of an MoE layer; q/k/v/o/gate/up of a decoder layer), their
         Cholesky chains run in lock-step in grouped kernels, and so do the column loops of those among them
-        that share shape and scheme (0 = never); ``group_max_bytes`` bounds the work buffers of one such job
+        that share shape and scheme (0 = never); ``group_max_bytes`` bounds the work buffers of one such job (sets
+        are split for the chains, and their column loops run over fewer problems at a time)
     :param compress_concurrency: how many modules of one ``compress_module_list`` call are quantised at the
         same time, each on its own HIP stream (1 = one after the other, the reference's behaviour)
 
@@ -97,7 +98,7 @@ class GPTQModifier(Modifier, QuantizationMixin, HessianStagingMixin):
     share_identical_inputs: bool = True
     compress_concurrency: int = 4
     group_min_modules: int = 3
-    group_max_bytes: int = 8 << 30
+    group_max_bytes: int = GROUP_MAX_BYTES
     stage_by_reference: bool = True
     stage_max_bytes: int = 16 << 30
 
@@ -350,7 +351,7 @@ class GPTQModifier(Modifier, QuantizationMixin, HessianStagingMixin):
             if len(members) < max(2, self.group_min_modules):
                 continue
             K = members[0].weight.shape[1]
-            # factors + work matrices: about 10 K^2 bytes per problem
+            # factors + the chain's work matrices: about 10 K^2 bytes per problem (finish_weight_group bounds the loops')
             per_call = max(1, min(len(members), int(self.group_max_bytes // (10 * K * K))))
             for i in range(0, len(members), per_call):
                 part = members[i:i + per_call]
@@ -386,7 +387,7 @@ class GPTQModifier(Modifier, QuantizationMixin, HessianStagingMixin):
     def _end_set(self, begun):
         part, names, ctx = begun
         with torch.no_grad():
-            results = finish_weight_group(ctx, self.block_size)
+            results = finish_weight_group(ctx, self.block_size, self.group_max_bytes)
         return part, names, results
 
     def _finish_sets(self, launched, consumed_on=None):

@@ -193,14 +193,29 @@ def width_key(module: torch.nn.Module, quant_args: QuantizationArgs, hessian: to
     return (module.weight.shape[1], module.weight.device, hessian.stride(0), bool(quant_args.actorder))
 
 
-def quantize_weight_group(modules, hessians, hessian_divisors, blocksize: int = 128, percdamp: float = 0.01):
+GROUP_MAX_BYTES = 8 << 30
+
+
+def loop_slices(count: int, rows: int, columns: int, form: int, budget: int) -> list[tuple[int, int]]:
+    """[begin, end) of the problems that share a lock-step column loop, equal runs whose work buffers stay within ``budget``
+    bytes (one problem at least).  A run of them has the bits of single calls, so the cut changes no result."""
+    one = ops.gptq_quantize_grouped_workspace_bytes(1, rows, columns, form)  # each further problem takes no more
+    most = max(1, min(count, budget // one))
+    runs = -(-count // most)
+    ends = [count * (i + 1) // runs for i in range(runs)]
+    return list(zip([0] + ends, ends))
+
+
+def quantize_weight_group(modules, hessians, hessian_divisors, blocksize: int = 128, percdamp: float = 0.01,
+                          max_bytes: int = GROUP_MAX_BYTES):
     """``quantize_weight`` for several Linears of one width at once (the experts of an MoE layer, or the
     projections of a decoder layer that read the hidden state): one lock-step Cholesky chain for all of them,
     and one lock-step column loop per set of equal shape and scheme, instead of a chain of small kernels per
-    module.  Same results as calling ``quantize_weight`` on each.  Returns a list of
+    module.  Same results as calling ``quantize_weight`` on each.  ``max_bytes`` bounds the factors and the column loops'
+    work buffers (those of one problem are never split).  Returns a list of
     (loss tensor, q_param_dict, info tensor) in the order of ``modules``."""
     return finish_weight_group(begin_weight_group(modules, hessians, hessian_divisors, percdamp, blocksize),
-                               blocksize)
+                               blocksize, max_bytes)
 
 
 def begin_weight_group(modules, hessians, hessian_divisors, percdamp: float = 0.01, blocksize: int = 128):
@@ -250,7 +265,7 @@ def begin_weight_group(modules, hessians, hessian_divisors, percdamp: float = 0.
                 forms=forms, blocksize=blocksize)
 
 
-def finish_weight_group(ctx, blocksize: int = 128):
+def finish_weight_group(ctx, blocksize: int = 128, max_bytes: int = GROUP_MAX_BYTES):
     """Second half of ``quantize_weight_group``: quantisation parameters from the weight observers, the lock-step
     column loops on the factors of ``begin_weight_group``, and the results in the caller's order."""
     n, order, mods, keys = ctx["n"], ctx["order"], ctx["mods"], ctx["keys"]
@@ -286,11 +301,15 @@ def finish_weight_group(ctx, blocksize: int = 128):
                          kscale=effective_scale(qp["scale"], quant_args, W.dtype)))
 
     outs, losses = [None] * n, [None] * n
-    at = 0
+    budget = max_bytes - U.numel() * U.element_size()
+    runs, at = [], 0
     while at < n:
         end = at + 1
         while end < n and keys[end] == keys[at]:
             end += 1
+        runs += [(at + b, at + e) for b, e in loop_slices(end - at, *mods[at].weight.shape, ctx["forms"][at], budget)]
+        at = end
+    for at, end in runs:
         part = prep[at:end]
         first = part[0]
         fmt, bits = kernel_format(first["args"])
@@ -313,7 +332,6 @@ def finish_weight_group(ctx, blocksize: int = 128):
                 form=form)
             for b in range(end - at):
                 outs[at + b], losses[at + b] = o[b], l[b]
-        at = end
 
     results = [None] * n
     for j, (m, p) in enumerate(zip(mods, prep)):

@@ -362,6 +362,10 @@ def gptq_quantize(weight, U, scale, zero_point, fmt: int, bits: int, row_div: in
     return out, loss
 
 
+def gptq_quantize_grouped_workspace_bytes(n: int, rows: int, columns: int, form: int = FACTOR_INVERSE) -> int:
+    return int(_lib.lib().llmc_gptq_quantize_grouped_workspace_bytes(int(n), int(rows), int(columns), int(form)))
+
+
 def gptq_quantize_grouped(weights, U, scales, zero_points, fmt: int, bits: int, row_div: int, scale_row_stride: int,
                           g_idxs=None, perms=None, dead=None, global_scales=None, blocksize: int = 128,
                           form: int = FACTOR_INVERSE):
@@ -395,8 +399,7 @@ def gptq_quantize_grouped(weights, U, scales, zero_points, fmt: int, bits: int, 
         perms = perms.to(torch.int32).contiguous()
     outs = [torch.empty((R, K), dtype=w0.dtype, device=w0.device) for _ in range(n)]
     loss = torch.empty(n, dtype=torch.float32, device=w0.device)
-    nbytes = _lib.lib().llmc_gptq_quantize_grouped_workspace_bytes(n, R, K, int(form))
-    ws = _workspace(w0.device, nbytes)
+    ws = _workspace(w0.device, gptq_quantize_grouped_workspace_bytes(n, R, K, form))
     wp = (ctypes.c_void_p * n)(*[w.data_ptr() for w in weights])
     op = (ctypes.c_void_p * n)(*[o.data_ptr() for o in outs])
     sp, zp = ptrs(scales), ptrs(zero_points)

@@ -623,6 +623,23 @@ def test_gptq_block_size_of_a_group_in_two_halves(K, refused):
             assert finish_weight_group(ctx, second) == []
 
 
+@pytest.mark.parametrize("count,rows,K", [(100, 8192, 2048), (128, 768, 2048), (384, 768, 768), (7, 28672, 4096), (1, 128256, 8192)])
+def test_gptq_loops_of_a_group_stay_within_their_memory(count, rows, K):
+    """Every problem in one run of a lock-step loop, no run's work buffers above the bound (8 GiB with the factors, which the
+    loop of 100 weights of 8192 x 2048 exceeded with 20), no more runs than that takes."""
+    from llmcompressor_amd import ops
+    from llmcompressor_amd.modifiers.gptq.gptq_quantize import GROUP_MAX_BYTES, loop_slices
+
+    for form in (ops.FACTOR_INVERSE, ops.FACTOR_GROUPS):
+        bytes_of = lambda n: ops.gptq_quantize_grouped_workspace_bytes(n, rows, K, form)  # noqa: E731
+        for budget in (GROUP_MAX_BYTES - 4 * K * K * count, 3 * bytes_of(1), 0):
+            runs = loop_slices(count, rows, K, form, budget)
+            assert [b for b, _ in runs] == [0] + [e for _, e in runs[:-1]] and runs[-1][1] == count
+            most = max(e - b for b, e in runs)
+            assert most == 1 or bytes_of(most) <= budget
+            assert len(runs) == 1 or bytes_of(-(-count // (len(runs) - 1))) > budget
+
+
 def test_observed_kv_cache_stand_in():
     """The stand-in for ``past_key_values`` shows keys and values to the module's observers and defers to the
     real cache when there is one."""
