@@ -53,6 +53,7 @@ int llmc_gemm_x3(const GemmF32& g, hipStream_t st);
 void llmc_gemm_x3_set_mode(int mode);
 
 // The product of operands whose range is known, split into two f16 terms (gemm_x2.hip): |A| and |B| (scaled, where scales
-// are given) at most 2^15, at least one element of a row that matters near 2^13.  Takes what llmc_gemm_x2_fits.
+// are given) at most 2^15, at least one element of a row that matters near 2^13.  A B^T without scales, A B with them; takes
+// what llmc_gemm_x2_fits.
 bool llmc_gemm_x2_fits(const GemmF32& g);
 int llmc_gemm_x2(const GemmF32& g, hipStream_t st);
