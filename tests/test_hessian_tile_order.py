@@ -1,6 +1,22 @@
-"""The Hessian kernel numbers the tiles of the upper triangle whole super-tiles first (`tile_coords` in csrc/hessian.hip): a
-restatement of that order, which has to reach every tile once, and to keep the 32 tiles that one L2 serves together."""
+"""The Hessian kernel numbers the tiles of the upper triangle whole super-tiles first (`tile_coords` in
+csrc/hessian_tiles.h, compiled for the host here): a restatement of that order, which the function has to follow, has to reach
+every tile once, and to keep the 32 tiles that one L2 serves together."""
+import ctypes
+import os
+import subprocess
+
 import pytest
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "llm-compressor_amd", "csrc")
+WRAPPER = """
+#define __host__
+#define __device__
+#define __forceinline__ inline
+#include "hessian_tiles.h"
+extern "C" void tiles(int n, int nb, int SH, int SW, int* ij) {
+  for (int c = 0; c < n; ++c) tile_coords(c, nb, SH, SW, ij[2 * c], ij[2 * c + 1]);
+}
+"""
 
 
 def _tiles(nb, SH, SW):
@@ -40,3 +56,20 @@ def test_groups_of_32_share_their_panels(nb):
     groups = [tiles[x * per + g:x * per + g + 32] for x in range(8) for g in range(0, per, 32)]
     panels = [len({p for t in group for p in t}) for group in groups]
     assert sum(panels) / len(panels) <= 12.5
+
+
+@pytest.fixture(scope="module")
+def compiled(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("tiles") / "tiles.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", f"-I{CSRC}", "-x", "c++", "-", "-o", lib],
+                   input=WRAPPER.encode(), check=True)
+    return ctypes.CDLL(lib).tiles
+
+
+@pytest.mark.parametrize("SH,SW", [(4, 8), (8, 8)])
+def test_the_kernel_takes_the_tiles_in_this_order(compiled, SH, SW):
+    for nb in range(1, 90):
+        want = list(_tiles(nb, SH, SW))
+        got = ((ctypes.c_int * 2) * (len(want) + 1))()
+        compiled(len(want) + 1, nb, SH, SW, ctypes.byref(got))
+        assert [tuple(t) for t in got] == want + [(-1, -1)]
