@@ -314,8 +314,8 @@ def _zipf_routing(T, n, gen):
 
 
 @pytest.mark.parametrize("scheme", ["w4a16", "nvfp4"])
-@pytest.mark.parametrize("R,K", [(768, 2048), (2048, 768)])
-def test_moe_layer_grouped_gptq_against_the_oracle(R, K, scheme):
+@pytest.mark.parametrize("R,K,form", [(768, 2048, 0), (2048, 768, 0), (768, 2048, 1)])  # 1: what quantize_weight_group takes there
+def test_moe_layer_grouped_gptq_against_the_oracle(R, K, form, scheme):
     """128 expert Linears of one shape in one lock-step call (Hessians from the grouped launch over the Zipf-routed
     tokens, activation ordering by each expert's diagonal); three experts (thousands of tokens, about K/2 tokens, a
     handful) are then run through the oracle's accumulate_hessian / quantize_weight on the same tokens: Hessian <= 1e-5,
@@ -355,10 +355,11 @@ def test_moe_layer_grouped_gptq_against_the_oracle(R, K, scheme):
         scales.append(s)
         gidx.append(base[perms[b].long()])
     fmt = ops.FMT_INT if scheme == "w4a16" else ops.FMT_FP4
-    U, dead, info = ops.gptq_hinv_grouped([H.clone() for H in Hs], perms, [1.0] * n, 0.01)
+    assert form in (ops.FACTOR_INVERSE, ops.gptq_quantize_form(K, 128, R))
+    U, dead, info = ops.gptq_hinv_grouped([H.clone() for H in Hs], perms, [1.0] * n, 0.01, form=form)
     assert int(info.abs().sum()) == 0
     outs, loss = ops.gptq_quantize_grouped(Ws, U, scales, None, fmt, 4, 1, K // group, g_idxs=gidx, perms=perms,
-                                           dead=dead, global_scales=gss if gss else None)
+                                           dead=dead, global_scales=gss if gss else None, form=form)
     torch.cuda.synchronize()
     assert torch.count_nonzero(outs[17]) == 0 and torch.count_nonzero(outs[127]) == 0
     if scheme == "w4a16":

@@ -1,5 +1,5 @@
-"""GPU: the Cholesky chain works on D H D, D a diagonal of powers of two, and takes its trailing updates as two-term f16
-products, whose operands that scaling keeps in range (gptq_quantize.py:144-164 is the chain's definition)."""
+"""GPU: the Cholesky chain works on D H D, D a diagonal of powers of two, and from 3072 columns on takes its updates as
+two-term f16 products, whose operands that scaling keeps in range (gptq_quantize.py:144-164 is the chain's definition)."""
 import pytest
 import torch
 
@@ -21,12 +21,13 @@ def _chain(H, form=0, percdamp=0.01):
     return U, int(info.item())
 
 
-# trailing matrices of one tile and less, of odd numbers of 64-wide tiles, of whole 128- and 256-wide ones, with regions
-# cut short by the width; 8320: 512-wide panels, the last one of a single block column
-@pytest.mark.parametrize("K", [320, 384, 576, 832, 1280, 2304, 4160, 8320])
+# trailing matrices of one tile and less, of odd numbers of 64-wide tiles, of whole 128-wide ones, with regions cut short by the
+# width.  Two-term products from 3072 on: 3136 and 4160 on 64-wide tiles only, the others on 128-wide ones
+# too; 512-wide panels from 8320 on, whose second regions take a product of their own, the last one of 128 columns there
+@pytest.mark.parametrize("K", [320, 384, 576, 832, 1280, 2304, 3072, 3136, 4160, 8320, 11008])
 def test_factor_against_64_bits(K):
     H = _hessian(K, 2 * K, seed=K)
-    form = 1 if K == 8320 else 0  # there the factor itself outside the 512-wide diagonal blocks: no long inverse
+    form = 1 if K >= 8320 else 0  # there the factor itself outside the 512-wide diagonal blocks: no long inverse
     U, info = _chain(H, form)
     assert info == 0
     Hd = H.double().cpu()
@@ -73,7 +74,7 @@ def test_sums_of_an_update_are_short(K, bound):
     assert err < bound, err
 
 
-@pytest.mark.parametrize("K,form", [(320, 0), (1000, 0), (1152, 1), (2304, 0)])
+@pytest.mark.parametrize("K,form", [(320, 0), (1000, 0), (1152, 1), (2304, 0), (3072, 0), (3136, 0), (4224, 1)])
 @pytest.mark.parametrize("shift", [-60, 24])
 def test_powers_of_two_pass_through(K, form, shift):
     """Without damping, scaling row and column c of H by 2^e[c] scales column c of the inverse factor by 2^-e[c] and row c
@@ -92,15 +93,18 @@ def test_powers_of_two_pass_through(K, form, shift):
     assert torch.equal(Us, want)
 
 
-@pytest.mark.parametrize("K", [320, 1280])
+# (row, column): eliminated from the last column on, so the pivot of the lower index fails.  The last ones go through all of
+# the chain's products, as infinities in the two-term ones (1e18 against diagonal entries near 1), before their pivot comes
+@pytest.mark.parametrize("K,at", [(320, (5, 40)), (1280, (5, 40)), (3072, (5, 40)), (3072, (5, 3000)), (3136, (1500, 3100)),
+                                  (4224, (64, 4200))])
 @pytest.mark.parametrize("big", [1e4, 1e18])
-def test_indefinite_matrix_is_found_at_its_pivot(K, big):
+def test_indefinite_matrix_is_found_at_its_pivot(K, at, big):
     """An off-diagonal entry far above what a positive matrix allows leaves the range of the products, in the row whose
     pivot fails for it; nothing before that pivot may notice."""
     H = _hessian(K, 2 * K, seed=K + 2, spread=0.3)
-    H[5, 40] = H[40, 5] = big  # eliminated from the last column on: pivot 5 fails
+    H[at[0], at[1]] = H[at[1], at[0]] = big
     U, info = _chain(H)
-    assert info == 6
+    assert info == at[0] + 1
     assert torch.equal(U, torch.eye(K, device="cuda"))
 
 
@@ -228,6 +232,23 @@ def test_rows_of_the_factor_without_later_columns(channels, exponent):
     other[torch.arange(channels, device="cuda") * 37] = True
     x = _two_sets(K, 3 * K, 5 + channels, other) * 2.0 ** exponent
     assert _loop_agreement(x, 0.01, ops.FACTOR_GROUPS, seed=2) >= 0.999
+
+
+@pytest.mark.parametrize("percdamp", [0.01, 1e-6])
+@pytest.mark.parametrize("louder", [4, 8, 14])
+def test_loud_channels_that_fire_apart(louder, percdamp):
+    """Half of the channels 2^louder times as loud as the others, which never fire together with them: the row scales follow
+    the loud ones, and the sums of the others, which they add nothing to, keep their codes.  (An element 2^-14 below a row's
+    largest loses bits below 2^-38 of that, and the damping keeps what a column is divided by above percdamp^(1/2) of the
+    loudest channels' norm: 2^-38 K^(1/2) / percdamp^(1/2) of a quantisation step at most.)"""
+    from llmcompressor_amd import ops
+
+    K = 1536
+    other = torch.rand(K, generator=torch.Generator().manual_seed(louder)).cuda() < 0.5
+    x = _two_sets(K, 3 * K, louder, other)
+    x[:, other] *= 2.0 ** louder
+    groups, inverse = (_loop_agreement(x, percdamp, form, seed=3) for form in (ops.FACTOR_GROUPS, ops.FACTOR_INVERSE))
+    assert groups >= 0.999 and groups >= inverse - 0.0005, (groups, inverse)
 
 
 @pytest.mark.parametrize("K", [1, 3, 64, 65, 1023, 1025, 16384])

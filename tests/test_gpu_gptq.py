@@ -243,8 +243,9 @@ def test_gptq_zero_hessian_zeroes_weight_and_failure_is_rtn():
     assert torch.equal(wq.cpu(), rtn)
 
 
+@pytest.mark.parametrize("own_form", [False, True])  # the inverse factor; the form that quantize_weight asks for
 @pytest.mark.parametrize("R,K,T", [(1024, 4096, 8192), (512, 14336, 32768)])
-def test_gptq_full_size_properties(R, K, T):
+def test_gptq_full_size_properties(R, K, T, own_form):
     """Llama-3-8B widths (the oracle would take minutes here): size-independent properties.
     Every output value lies on its group's int4 grid; GPTQ's layer reconstruction error beats
     round-to-nearest's; rescaling H leaves the codes unchanged; a narrower block width regroups the
@@ -265,10 +266,12 @@ def test_gptq_full_size_properties(R, K, T):
     g_idx = (torch.arange(K, dtype=torch.int32, device="cuda") // g)[perm]
 
     def run(Hin, blocksize=128, divisor=float(T)):
-        U, dead, info = ops.gptq_hinv_(Hin.clone(), perm, divisor=divisor)
+        form = ops.gptq_quantize_form(K, blocksize, R) if own_form else ops.FACTOR_INVERSE
+        assert form == (ops.FACTOR_GROUPS if own_form and blocksize == 128 else ops.FACTOR_INVERSE)
+        U, dead, info = ops.gptq_hinv_(Hin.clone(), perm, divisor=divisor, form=form)
         assert int(info.item()) == 0
         wq, loss = ops.gptq_quantize(w, U, scale, None, ops.FMT_INT, 4, 1, K // g, g_idx=g_idx, perm=perm, dead=dead,
-                                     blocksize=blocksize)
+                                     blocksize=blocksize, form=form)
         return wq, loss, U
 
     wq, loss, U = run(H)
@@ -290,6 +293,8 @@ def test_gptq_full_size_properties(R, K, T):
     # block width only regroups fp32 sums
     wq_b, _, _ = run(H, blocksize=64)
     assert (wq_b == wq).float().mean().item() >= CODE_AGREEMENT
+    if own_form:
+        return
     # U^T U = (P^T H P / n + damp I)^-1 on sampled columns
     Hp = (H[perm][:, perm] / T).double()
     damp = 0.01 * torch.diag(Hp).mean()
