@@ -172,6 +172,25 @@ def test_dynamic_groups_of_one_very_wide_row():
     assert torch.equal(got.view_as(want), want)
 
 
+# 64 MiB is where the last rows come first: just below, just above with 0 to 7 blocks left over, a row of eight-column lanes
+@pytest.mark.parametrize("rows,cols", [(8192, 4096), (8193, 4096), (8200, 4112), (9001, 4112), (8448, 4096), (16385, 2056)])
+def test_large_inputs_from_the_end(rows, cols):
+    """Every row of an input that is walked from its end has the values that it has in an input walked in order."""
+    from llmcompressor_amd import ops
+
+    llmc = _llmc()
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    x = torch.randn(rows, cols, device="cuda", dtype=torch.bfloat16, generator=g)
+    scale = torch.rand(rows, 1, device="cuda", generator=g).bfloat16() + 0.25
+    parts = [slice(i, i + 4000) for i in range(0, rows, 4000)]
+    for mode in (ops.OUT_FAKEQUANT, ops.OUT_CODES, ops.OUT_PACKED):
+        quantised = [llmc.quant_pack(x[p], scale[p], None, ops.FMT_INT, 4, 1, 1, cols, mode, None, None) for p in [slice(None)] + parts]
+        assert torch.equal(quantised[0], torch.cat(quantised[1:]))
+    if cols % 16 == 0:
+        dynamic = [llmc.dynamic_group_quantize(x[p], 16, ops.FMT_FP8, 8) for p in [slice(None)] + parts]
+        assert torch.equal(dynamic[0], torch.cat(dynamic[1:]))
+
+
 @pytest.mark.parametrize("form", ["lanes", "rows", "blocks"])
 @pytest.mark.parametrize("symmetric", [True, False])
 def test_mse_search_over_f16_rounds_the_shrunk_range_twice(form, symmetric):
