@@ -226,8 +226,13 @@ struct GroupArgs {
   float* H[GROUP_MAX];
   const uint16_t* X[GROUP_MAX];
   int T[GROUP_MAX];
+  int spread;    // of each of the first `spread` problems every XCD takes an eighth of the tiles, before
   int first[9];  // XCD x takes tiles [first[x], first[x + 1]) of all the problems' tiles laid end to end
 };
+// first tile of the eighth (with next = 1, of the one behind it) of problem p's tiles that XCD x takes
+__host__ __device__ __forceinline__ int spread_first(int x, int p, int ntiles, int next = 0) {
+  return (((x + p) & 7) + next) * ntiles / 8;
+}
 struct NoGroup {
   static constexpr bool grouped = false;
   static constexpr bool segmented = false;
@@ -254,10 +259,20 @@ __global__ __launch_bounds__(256) void hessian_syrk_kernel(float* __restrict__ H
                                                             unsigned* __restrict__ pace) {
   int group_tile = 0;
   if constexpr (GRP::grouped) {
-    const int flat = grp.first[blockIdx.x & 7] + (int)(blockIdx.x >> 3);
-    if (flat >= grp.first[(blockIdx.x & 7) + 1]) return;
-    const int p = flat / plan.ph[0].ntiles;
-    group_tile = flat - p * plan.ph[0].ntiles;
+    const int x = blockIdx.x & 7, ntiles = plan.ph[0].ntiles;
+    int at = (int)(blockIdx.x >> 3), p = 0;
+    for (; p < grp.spread; ++p) {
+      const int lo = spread_first(x, p, ntiles), n = spread_first(x, p, ntiles, 1) - lo;
+      group_tile = lo + at;
+      if (at < n) break;
+      at -= n;
+    }
+    if (p == grp.spread) {
+      at += grp.first[x];
+      if (at >= grp.first[x + 1]) return;
+      p = at / ntiles;
+      group_tile = at - p * ntiles;
+    }
     Tfull = grp.T[p];
     H = grp.H[p];
     Xfull = grp.X[p];
@@ -906,46 +921,62 @@ extern "C" int llmc_hessian_accumulate_segments(float* H, int64_t ldh, const voi
   return launch_choice(x_dtype, c, H, ldh, nullptr, ldx, T, K, alpha, flags, ws, pace, st, &segs, {});
 }
 
-// Divides the tiles of n problems (tokens in grp.T, all positive) among the 8 XCDs, one contiguous run each with an eighth
-// of the slabs, and returns the longest run's number of tiles.  An XCD's 32 workgroups then work on one problem or two, whose
-// panels they share in their L2.  (Dealt to all eight XCDs problem by problem, every XCD reads every problem, the last one has
-// fewer tiles than the others, and problems of six tiles leave two XCDs without work: 32 problems of 6144 x 2048 976 -> 941 us,
-// 128 of 4096 x 768 560 -> 457, with 1 to 4000 tokens 420 -> 282, of width 2048 1852 -> 1745; 4 x 6000 x 2048 142 -> 141.)
-// Problems of unequal token counts are first put in an order in which every run starts with its longest.
-int deal_to_xcds(GroupArgs& grp, int n, int ntiles) {
+// Divides the tiles of n problems (tokens in grp.T, all positive) among the 8 XCDs, an eighth of the work each, and returns the
+// largest number of tiles that one of them gets.  A tile's work is its slabs and its epilogue, which takes as long as EPILOGUE
+// slabs (by slabs alone the run of the shortest problems was by far the longest where tokens are few).
+//   Problems of at most 64 tiles are laid end to end and cut into one contiguous run per XCD, whose 32 workgroups then work on
+// one problem or two and share its panels in their L2; problem by problem every XCD reads every problem and, with tiles that are
+// no multiple of eight, one of them has fewer than the others.  Those of them whose tiles are long go to all XCDs
+// all the same, longest first: a run of them would take whole passes of its XCD's CUs, three where two and a half are its share.
+//   Wider problems all go to all XCDs: an eighth of one is already a run of neighbouring tiles, and with all XCDs on one
+// problem the longest come first everywhere and the shortest fill the last pass.
+// In us, problem by problem / now, tokens shared out evenly, at random and as 1 / rank^1.1: 128 problems of 2048 columns, 32768
+// tokens, 925 / 839, 931 / 830, 943 / 842; 32 with 24576 311 / 299, 329 / 305, 361 / 296; 60 of 1408 columns, 24000 tokens, 328 / 299,
+// 331 / 298, 364 / 308; 16 of 4096 columns, 30000 tokens, 799 / 788, 762 / 756, 781 / 778; 8 of 14336, 32768 tokens, 8144 / 7342,
+// 8366 / 7505, 8319 / 7476; 128 of 768, 32768 tokens, 274 / 270, 280 / 278, 325 / 289.
+constexpr int64_t EPILOGUE = 20;
+constexpr int RUN_MAX_TILES = 64;
+int deal_to_xcds(GroupArgs& grp, int n, int ntiles, int tiles_at_once) {
   bool equal = true;
   for (int i = 1; i < n; ++i) equal = equal && grp.T[i] == grp.T[0];
-  if (!equal) {
-    int by_tokens[GROUP_MAX];
-    for (int i = 0; i < n; ++i) by_tokens[i] = i;
-    std::stable_sort(by_tokens, by_tokens + n, [&](int a, int b) { return grp.T[a] > grp.T[b]; });
-    const GroupArgs given = grp;
-    int at = 0;
-    for (int x = 0; x < 8; ++x)
-      for (int r = 0; r * 8 < n; ++r) {
-        const int j = r * 8 + ((r & 1) ? 7 - x : x);  // back and forth: the eight lists come out about equally long
-        if (j >= n) continue;
-        grp.H[at] = given.H[by_tokens[j]];
-        grp.X[at] = given.X[by_tokens[j]];
-        grp.T[at++] = given.T[by_tokens[j]];
-      }
-  }
-  auto slabs = [&](int i) { return ((int64_t)grp.T[i] + BK - 1) / BK; };
+  auto work = [&](int i) { return ((int64_t)grp.T[i] + BK - 1) / BK + EPILOGUE; };  // of a tile of problem i
   int64_t total = 0;
-  for (int i = 0; i < n; ++i) total += slabs(i) * ntiles;
-  int64_t before = 0;  // slabs of the problems before i
-  int x = 1, most = 0;
-  grp.first[0] = 0;
-  for (int i = 0; i < n; ++i) {
-    const int64_t end = before + slabs(i) * ntiles;
-    // run x starts at the tile nearest to its share's beginning
-    for (; x < 8 && total * x <= end * 8; ++x)
-      grp.first[x] = i * ntiles + (int)((total * x - before * 8 + slabs(i) * 4) / (slabs(i) * 8));
-    before = end;
+  for (int i = 0; i < n; ++i) total += work(i) * ntiles;
+  grp.spread = 0;
+  if (!equal || ntiles > RUN_MAX_TILES) {
+    int order[GROUP_MAX];  // the spread ones by their length, the others as given
+    for (int i = 0; i < n; ++i) order[i] = i;
+    std::stable_sort(order, order + n, [&](int a, int b) { return grp.T[a] > grp.T[b]; });
+    // long: an XCD gets through fewer than four passes of such tiles
+    while (grp.spread < n && (ntiles > RUN_MAX_TILES || work(order[grp.spread]) * 4 * 8 * tiles_at_once > total)) ++grp.spread;
+    std::sort(order + grp.spread, order + n);
+    const GroupArgs given = grp;
+    for (int i = 0; i < n; ++i) {
+      grp.H[i] = given.H[order[i]];
+      grp.X[i] = given.X[order[i]];
+      grp.T[i] = given.T[order[i]];
+    }
   }
-  grp.first[8] = n * ntiles;
-  for (x = 0; x < 8; ++x) most = std::max(most, grp.first[x + 1] - grp.first[x]);
-  return most;
+  // run x ends where XCDs 0 .. x have their eighths: what they hold of the spread problems, then the runs
+  int tiles[8];
+  int64_t held = 0, before = 0;  // before: work of the problems laid end to end in front of problem i
+  int i = grp.spread;
+  grp.first[0] = i * ntiles;
+  for (int x = 0; x < 8; ++x) {
+    tiles[x] = 0;
+    for (int p = 0; p < grp.spread; ++p) {
+      const int c = spread_first(x, p, ntiles, 1) - spread_first(x, p, ntiles);
+      tiles[x] += c;
+      held += c * work(p);
+    }
+    const int64_t end = total * (x + 1) / 8 - held;
+    while (i < n && before + work(i) * ntiles <= end) before += work(i++) * ntiles;
+    int cut = n * ntiles;
+    if (x < 7 && i < n) cut = i * ntiles + (end > before ? (int)((end - before + work(i) / 2) / work(i)) : 0);  // the nearest tile
+    grp.first[x + 1] = std::max(cut, grp.first[x]);
+    tiles[x] += grp.first[x + 1] - grp.first[x];
+  }
+  return *std::max_element(tiles, tiles + 8);
 }
 
 template <int BT, int DT>
@@ -959,7 +990,7 @@ int launch_grouped(GroupArgs& grp, int n, int64_t ldh, int64_t ldx, int64_t K, f
     hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
     if (e != hipSuccess) return 1000 + (int)e;
   }
-  const int most = deal_to_xcds(grp, n, c.plan.ph[0].ntiles);
+  const int most = deal_to_xcds(grp, n, c.plan.ph[0].ntiles, BT == 256 ? 32 : 64);
   hipLaunchKernelGGL(kern, dim3(8 * most), dim3(256), smem, st, (float*)nullptr, ldh, (const uint16_t*)nullptr, ldx, 0,
                      (int)K, alpha, sym, nb, c.plan, (float*)nullptr, grp, (unsigned*)nullptr);
   LLMC_LAUNCH_STATUS();

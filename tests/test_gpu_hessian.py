@@ -297,10 +297,14 @@ def test_hessian_hook_takes_values_whose_rows_overlap(shape, dtype):
         assert torch.equal(got, want) and n0.item() == n1.item() > 0
 
 
-@pytest.mark.parametrize("K", [136, 256, 768, 1032])
-@pytest.mark.parametrize("tokens", [[70], [64, 0, 65], [130] * 8, [1, 2, 300, 0, 64, 128, 63, 129, 700], [5] * 131, list(range(0, 129))])
+# the last three: some problems long enough to be spread over the XCDs among others in runs; 1536 columns: 21 tiles a problem;
+# 3072: 78, which are all spread
+@pytest.mark.parametrize("K,tokens", [(K, t) for K in (136, 256, 768, 1032) for t in (
+    [70], [64, 0, 65], [130] * 8, [1, 2, 300, 0, 64, 128, 63, 129, 700], [5] * 131, list(range(0, 129)))] + [
+    (K, t) for K in (136, 256, 768, 1032, 1536) for t in ([9, 5000] + [3] * 70, [3000, 0, 40, 2500, 1] + [64] * 40, [6000] + [1] * 128)] + [
+    (3072, [130, 7, 0, 400]), (3072, [64] * 3)])
 def test_grouped_tiles_are_taken_once_each(K, tokens):
-    """The tiles of all problems of a grouped call are laid end to end and cut into one run per XCD.  Small integers: every sum
+    """The tiles of all problems of a grouped call are divided among the XCDs, in runs or spread over all of them.  Small integers: every sum
     is exact in fp32, so a tile left out or taken twice shows, whatever the order of the sums."""
     from llmcompressor_amd import ops
 
