@@ -263,6 +263,19 @@ def test_diagonal_order_at_the_edges_of_its_workgroups(K):
         assert torch.equal(row, torch.argsort(H.diagonal(), descending=True, stable=True))
 
 
+# either side of 72000 entries, from where on they are sorted and not counted; more problems than one launch takes
+@pytest.mark.parametrize("n,K", [(71, 1000), (72, 1000), (70, 1024), (71, 1024), (128, 2048), (256, 513), (300, 100), (600, 352)])
+def test_diagonal_order_of_many_problems(n, K):
+    from llmcompressor_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(n)
+    diagonals = torch.randint(-50, 51, (n, K), device="cuda", generator=g).float()
+    space = torch.zeros(n, K, K, device="cuda")
+    space.diagonal(dim1=1, dim2=2).copy_(diagonals)
+    got = ops.diag_argsort_desc(list(space))
+    assert torch.equal(got, torch.argsort(diagonals, dim=1, descending=True, stable=True))
+
+
 def _linears(K, rows, count, seed=0):
     """(modules, their Hessians): W4A16 in groups of 128 columns, static activation order."""
     from llmcompressor_amd.modifiers.quantization.calibration import initialize_observer
