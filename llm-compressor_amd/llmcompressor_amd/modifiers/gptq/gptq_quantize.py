@@ -226,7 +226,10 @@ def begin_weight_group(modules, hessians, hessian_divisors, percdamp: float = 0.
     keys = [group_key(m, m.quantization_scheme.weights, H) for m, H in zip(modules, hessians)]
     # the form of the factor that each member's loop is given by itself (those of the full inverse in front), and members of one
     # column-loop set next to each other, so that their factors are one slice of the batch
-    forms = [ops.gptq_quantize_form(m.weight.shape[1], blocksize, m.weight.shape[0]) for m in modules]
+    columns = hessians[0].shape[0]
+    rows = [k[0][0] if k is not None else m.weight.shape[0] for k, m in zip(keys, modules)]
+    form_of = {r: ops.gptq_quantize_form(columns, blocksize, r) for r in set(rows)}
+    forms = [form_of[r] for r in rows]
     order = sorted(range(n), key=lambda i: (forms[i] != ops.FACTOR_INVERSE, keys.index(keys[i]), i))
     mods = [modules[i] for i in order]
     Hs = [hessians[i] for i in order]
