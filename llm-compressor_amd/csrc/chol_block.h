@@ -34,20 +34,27 @@ constexpr int NB = 64;
 constexpr int NT = 512;  // threads per workgroup
 constexpr int LDD = 68;  // LDS row stride (floats) of a 64-wide block: 16-byte aligned rows, staggered banks
 constexpr int LDP = 20;  // LDS row stride of a 16-wide slab
+constexpr int LDA = 52;  // ... of a column of the 48 x 48 block behind the first slab
+constexpr int LOW_ROWS = 48 + 32 + 16;
 
+// 63 KB: with what a region's workgroup keeps beside it (chol_region.h), two workgroups fit a CU.
 struct FactorScratch {
-  float X[NB][LDD];      // the result: inverse of the factor, zeros above the diagonal
-  float AT[NB][LDD];     // the block, column-major: AT[c][r] = A[r][c], columns from 16 on
-  float P[NB][LDP];      // the current slab's columns, row-major
-  float V[3][NB][LDP];   // V[k][r][t]: unscaled factored columns of slab k below its diagonal block (L = V D^-1/2)
-  float T[3][NB][LDP];   // T[k][r][t] = V[k][r][t] / d: the unit-lower factor
-  float Y[4][16][LDP];   // Y[k]: inverse of slab k's 16 x 16 unit-lower factor, row-major
-  float W[3][NB][LDP];   // W[k][r][c] = -(L[r, slab k] X_kk)[c] for the rows r below slab k's diagonal block
-  float Z[2][16][LDP];   // Z_0[2], Z_0[3]
-  float Q[2][16][LDP];   // Z_c[3] + W_2[3] Z_c[2], c = 0, 1
-  float rs[NB];          // 1 / L[r][r]
-  int bad;               // smallest column whose pivot was not positive and finite, NB if none
+  float X[NB][LDD];          // the result: inverse of the factor, zeros above the diagonal
+  float AT[NB - 16][LDA];    // the block, column-major: at(c, r) = A[r][c], columns and rows from 16 on
+  float P[NB][LDP];          // the current slab's columns, row-major
+  float V[LOW_ROWS][LDP];    // low(V, k, r)[t]: unscaled factored columns of slab k below its diagonal block (L = V D^-1/2)
+  float T[LOW_ROWS][LDP];    // low(T, k, r)[t] = V / d: the unit-lower factor
+  float W[LOW_ROWS][LDP];    // low(W, k, r)[c] = -(L[r, slab k] X_kk)[c]
+  float Y[4][16][LDP];       // Y[k]: inverse of slab k's 16 x 16 unit-lower factor, row-major
+  float Z[2][16][LDP];       // Z_0[2], Z_0[3]
+  float rs[NB];              // 1 / L[r][r]
+  int bad;                   // smallest column whose pivot was not positive and finite, NB if none
   int pad[3];
+  __device__ float* at(int c, int r) { return &AT[c - 16][r - 16]; }
+  // row r of slab k: only the rows below the slab's diagonal block are kept, 48 + 32 + 16 of them
+  __device__ static float* low(float (*m)[LDP], int k, int r) { return m[r - 16 + (k == 0 ? 0 : k == 1 ? 32 : 48)]; }
+  // Q_c = Z_c[3] + W_2[3] Z_c[2], c = 0, 1: in rows of P that the last slab does not use
+  __device__ float* q(int c) { return P[16 * c]; }
 };
 
 // v in lane LI of every row of 16 lanes, for the whole row
@@ -111,8 +118,8 @@ __device__ __forceinline__ void factor_slab(int lane, FactorScratch& s) {
     constexpr int KK = K < 3 ? K : 0;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      *(float4*)&s.V[KK][row][4 * q] = make_float4(a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]);
-      *(float4*)&s.T[KK][row][4 * q] = make_float4(a[4 * q] * rd[4 * q], a[4 * q + 1] * rd[4 * q + 1],
+      *(float4*)(s.low(s.V, KK, row) + 4 * q) = make_float4(a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]);
+      *(float4*)(s.low(s.T, KK, row) + 4 * q) = make_float4(a[4 * q] * rd[4 * q], a[4 * q + 1] * rd[4 * q + 1],
                                                    a[4 * q + 2] * rd[4 * q + 2], a[4 * q + 3] * rd[4 * q + 3]);
     }
   }
@@ -144,10 +151,10 @@ __device__ __forceinline__ v4f tile16_nt(v4f acc, const float* A, const float* B
 template <int K>
 __device__ __forceinline__ void update_tile(FactorScratch& s, int ti, int tj, bool to_panel, int lane) {
   const int c = lane & 15, g = lane >> 4;
-  float* const at = &s.AT[16 * tj + c][16 * ti + 4 * g];
+  float* const at = s.at(16 * tj + c, 16 * ti + 4 * g);
   const float4 x = *(const float4*)at;
   v4f acc = {x.x, x.y, x.z, x.w};
-  acc = tile16_nt(acc, &s.V[K][16 * ti][0], &s.T[K][16 * tj][0], lane);
+  acc = tile16_nt(acc, s.low(s.V, K, 16 * ti), s.low(s.T, K, 16 * tj), lane);
   if (to_panel) {
 #pragma unroll
     for (int v = 0; v < 4; ++v) s.P[16 * ti + 4 * g + v][c] = acc[v];
@@ -192,18 +199,21 @@ __device__ __forceinline__ void factor_block_put(FactorScratch& s, float4 d0, fl
     *(float4*)&s.P[r][8 * w + 4] = d1;
     return;
   }
-  s.AT[8 * w + 0][r] = d0.x; s.AT[8 * w + 1][r] = d0.y; s.AT[8 * w + 2][r] = d0.z; s.AT[8 * w + 3][r] = d0.w;
-  s.AT[8 * w + 4][r] = d1.x; s.AT[8 * w + 5][r] = d1.y; s.AT[8 * w + 6][r] = d1.z; s.AT[8 * w + 7][r] = d1.w;
+  if (r < 16) return;  // above the diagonal
+  float* const at = s.at(8 * w, r);
+  at[0 * LDA] = d0.x; at[1 * LDA] = d0.y; at[2 * LDA] = d0.z; at[3 * LDA] = d0.w;
+  at[4 * LDA] = d1.x; at[5 * LDA] = d1.y; at[6 * LDA] = d1.z; at[7 * LDA] = d1.w;
 }
 
 // factor_block_put() has been called by every thread of the 512 (its lower triangle incl. the diagonal is used); no
 // barrier is needed in between  ->  s.X = inverse of the block's lower Cholesky factor, exact zeros above the
 // diagonal.  Every one of the 512 threads calls it.  Returns, in every thread, the smallest column whose pivot was not
 // positive and finite (NB if none; the numbers computed after such a pivot are meaningless).  Ends with a
-// barrier: s.X is readable by all on return.  FACTOR_BARRIERS barriers in all.
-constexpr int FACTOR_BARRIERS = 9;
-__device__ __forceinline__ int factor_invert_64(FactorScratch& s) {
-  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), r = tid & 63;
+// barrier: s.X is readable by all on return.  Waves 4 to 7 call beside() once while each of the four slabs is factored (1.5
+// us each, in which they have at most one tile to form).
+template <typename Beside>
+__device__ __forceinline__ int factor_invert_64(FactorScratch& s, int tid, Beside beside) {
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), r = tid & 63;
   if (tid == 0) s.bad = NB;
   __syncthreads();
 
@@ -215,6 +225,7 @@ __device__ __forceinline__ int factor_invert_64(FactorScratch& s) {
       if ((c4 >> 4) > (row >> 4)) *(float4*)&s.X[row][c4] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
   }
+  if (w >= 4) beside();
   __syncthreads();
   if (w < 3) update_tile<0>(s, 1 + w, 1, true, r);
   if (w == 3) diagonal_tile(s, 0, r);
@@ -224,31 +235,34 @@ __device__ __forceinline__ int factor_invert_64(FactorScratch& s) {
   if (w == 2) update_tile<0>(s, 3, 2, false, r);
   if (w == 3) update_tile<0>(s, 3, 3, false, r);
   if (w >= 4 && w < 7)
-    product_tile<true>(&s.T[0][16 * (w - 3)][0], LDP, &s.Y[0][0][0], LDP, nullptr, 0, &s.W[0][16 * (w - 3)][0], LDP, r);
+    product_tile<true>(s.low(s.T, 0, 16 * (w - 3)), LDP, &s.Y[0][0][0], LDP, nullptr, 0, s.low(s.W, 0, 16 * (w - 3)), LDP, r);
+  if (w >= 4) beside();
   __syncthreads();
   if (w < 2) update_tile<1>(s, 2 + w, 2, true, r);
   if (w == 2) diagonal_tile(s, 1, r);
   __syncthreads();
   if (w == 0) factor_slab<2>(r, s);
   if (w == 1) update_tile<1>(s, 3, 3, false, r);
-  if (w == 2 || w == 3) product_tile<true>(&s.T[1][16 * w][0], LDP, &s.Y[1][0][0], LDP, nullptr, 0, &s.W[1][16 * w][0], LDP, r);
-  if (w == 4) product_tile<false>(&s.X[16][16], LDD, &s.W[0][16][0], LDP, nullptr, 0, &s.X[16][0], LDD, r);
+  if (w == 2 || w == 3) product_tile<true>(s.low(s.T, 1, 16 * w), LDP, &s.Y[1][0][0], LDP, nullptr, 0, s.low(s.W, 1, 16 * w), LDP, r);
+  if (w == 4) product_tile<false>(&s.X[16][16], LDD, s.low(s.W, 0, 16), LDP, nullptr, 0, &s.X[16][0], LDD, r);
+  if (w >= 4) beside();
   __syncthreads();
   if (w == 0) update_tile<2>(s, 3, 3, true, r);
   if (w == 1) diagonal_tile(s, 2, r);
   if (w == 2 || w == 3)
-    product_tile<true>(&s.V[1][16 * w][0], LDP, &s.X[16][0], LDD, &s.W[0][16 * w][0], LDP, &s.Z[w - 2][0][0], LDP, r, &s.rs[16]);
-  if (w == 4) product_tile<true>(&s.T[2][48][0], LDP, &s.Y[2][0][0], LDP, nullptr, 0, &s.W[2][48][0], LDP, r);
+    product_tile<true>(s.low(s.V, 1, 16 * w), LDP, &s.X[16][0], LDD, s.low(s.W, 0, 16 * w), LDP, &s.Z[w - 2][0][0], LDP, r, &s.rs[16]);
+  if (w == 4) product_tile<true>(s.low(s.T, 2, 48), LDP, &s.Y[2][0][0], LDP, nullptr, 0, s.low(s.W, 2, 48), LDP, r);
   __syncthreads();
   if (w == 0) factor_slab<3>(r, s);
   if (w == 1) product_tile<false>(&s.X[32][32], LDD, &s.Z[0][0][0], LDP, nullptr, 0, &s.X[32][0], LDD, r);
-  if (w == 2) product_tile<false>(&s.X[32][32], LDD, &s.W[1][32][0], LDP, nullptr, 0, &s.X[32][16], LDD, r);
-  if (w == 3) product_tile<false>(&s.W[2][48][0], LDP, &s.Z[0][0][0], LDP, &s.Z[1][0][0], LDP, &s.Q[0][0][0], LDP, r);
-  if (w == 4) product_tile<false>(&s.W[2][48][0], LDP, &s.W[1][32][0], LDP, &s.W[1][48][0], LDP, &s.Q[1][0][0], LDP, r);
+  if (w == 2) product_tile<false>(&s.X[32][32], LDD, s.low(s.W, 1, 32), LDP, nullptr, 0, &s.X[32][16], LDD, r);
+  if (w == 3) product_tile<false>(s.low(s.W, 2, 48), LDP, &s.Z[0][0][0], LDP, &s.Z[1][0][0], LDP, s.q(0), LDP, r);
+  if (w == 4) product_tile<false>(s.low(s.W, 2, 48), LDP, s.low(s.W, 1, 32), LDP, s.low(s.W, 1, 48), LDP, s.q(1), LDP, r);
+  if (w >= 4) beside();
   __syncthreads();
   // X_33 as its unscaled form and the row scale: its own tile is written at the same time
-  if (w < 2) product_tile<false>(&s.Y[3][0][0], LDP, &s.Q[w][0][0], LDP, nullptr, 0, &s.X[48][16 * w], LDD, r, nullptr, &s.rs[48]);
-  if (w == 2) product_tile<false>(&s.Y[3][0][0], LDP, &s.W[2][48][0], LDP, nullptr, 0, &s.X[48][32], LDD, r, nullptr, &s.rs[48]);
+  if (w < 2) product_tile<false>(&s.Y[3][0][0], LDP, s.q(w), LDP, nullptr, 0, &s.X[48][16 * w], LDD, r, nullptr, &s.rs[48]);
+  if (w == 2) product_tile<false>(&s.Y[3][0][0], LDP, s.low(s.W, 2, 48), LDP, nullptr, 0, &s.X[48][32], LDD, r, nullptr, &s.rs[48]);
   if (w == 3) diagonal_tile(s, 3, r);
   __syncthreads();
   return s.bad;

@@ -1,0 +1,408 @@
+// A 256-wide region of the blocked Cholesky factorisation in one launch (chol.hip).
+//
+// The serial spine of the factorisation is one 64 x 64 diagonal block after the other.  Inside a region of up to four such
+// blocks everything that hangs on them runs in this launch, one workgroup per task, and what crosses workgroups is handed
+// over through memory:
+//   spine            factors and inverts diagonal block m (inverse X_m), solves row block m + 1 against it
+//                    (R = A[m+1, m] X_m^T), takes R R^T off diagonal block m + 1, and goes on with that one
+//   row block b > 1  of the region: its columns m < b - 1 as the X_m arrive, with the updates that they make to its later
+//                    columns and to its diagonal block; then hands A[b, b-1] and the diagonal block to the spine
+//   rows below       32 rows to a workgroup, two independent sets of 16: each block column solved as its X arrives
+// One launch per step, with every workgroup factoring the block for itself, and one more for the rows below took 49.8 and
+// 10.2 us for a region of a 4096-wide matrix, 4.5 us of each launch being the launch; 45 us now.  What bounds the region is
+// the spine: the 64 x 64 factor-and-invert (one wave's instruction issue, chol_block.h) and two products per step, 8.6 us.
+// Whole chains: 4096 columns 1323 -> 1114 us, 14336 9.0 -> 8.1 ms, 128 of 2048 8.16 -> 7.95 ms.
+//
+// 512 threads and at most 80 KB of LDS to a workgroup: two fit a CU, and one fits beside a workgroup of the 128-wide
+// products.  With 1024 threads and 131 KB a launch needed CUs of its own, and beside another stream's products every third
+// launch waited for one to run out (280 us).
+//
+// Handing over.  The L2s of the eight XCDs do not see each other's writes within a launch.  A producer stores with sc1
+// (through its L2, to where every XCD reads), waits for its stores and counts up a word in memory; a consumer polls that
+// word and then loads.  Its loads may use the caches: nothing that is handed over lies in a line that was touched earlier
+// in the launch by anyone but its producer (side buffers of their own; the caches start the launch without them).  One
+// hand-over of 16 KB, store to loaded, takes 1.3 us; with agent-scope fences, which write back and invalidate whole caches,
+// 3.5, and 17 with 240 workgroups listening.
+//
+// Progress.  A workgroup takes its task by a ticket when it starts to run, so whoever waits, waits for tasks that already
+// run or come next: the core tasks (spine, row blocks) of all problems come first, a problem's next to each other, then the
+// rows below.  A launch holds at most two workgroups whose partners have not started, whatever else occupies the chip.  A
+// wait that has not ended after 20 s (it cannot, short of a fault) gives up: info becomes -1, every task of the problem
+// leaves, and the result is the identity as for any failed factorisation.
+#pragma once
+#include "chol_block.h"
+
+namespace cholregion {
+using namespace cholblk;
+
+struct HinvScalars {
+  float damp;
+  int info;
+};
+
+constexpr int REGION_NT = NT;
+constexpr int ROWS = 32;  // of a task below the region
+constexpr int MAX_BLOCKS = 4;
+constexpr int BLOCK = NB * NB;
+// words of a problem that count hand-overs, each in a line of its own; they grow over the whole factorisation
+constexpr int SYNC_LINE = 32;
+constexpr int SYNC_X = 0;                                // + m: X_m, 16 per region
+constexpr int SYNC_ROW = SYNC_X + MAX_BLOCKS - 1;        // + j (1..3): solved blocks (j, i), i < j, 16 each
+constexpr int SYNC_NEXT = SYNC_ROW + MAX_BLOCKS - 2;     // + b (2, 3): A[b, b-1] and diagonal block b, 16 per region
+constexpr int SYNC_TICKET = SYNC_NEXT + MAX_BLOCKS;      // of problem 0: tickets of all launches
+constexpr int SYNC_WORDS = (SYNC_TICKET + 1) * SYNC_LINE;
+// floats of a problem that hold what is handed over besides X: solved blocks (j, i), then A[b, b-1] and diagonal block b
+constexpr int SIDE_NEXT = 6 * BLOCK;
+constexpr int SIDE_FLOATS = SIDE_NEXT + 4 * BLOCK;
+
+struct RegionArgs {
+  float* A;            // work matrices, one every Kp^2 floats
+  float* Xs;           // inverses of the diagonal blocks' factors (block c / 64 at (c / 64) * 4096), one set every xs_stride floats
+  float* side;         // SIDE_FLOATS per problem, side_stride apart
+  uint32_t* sync;      // SYNC_WORDS per problem, zero before the first region
+  HinvScalars* sc;
+  int64_t xs_stride, side_stride;
+  int Kp, K, r0, nb;   // region: block columns r0 .. r0 + 64 nb
+  int n, tiles;        // problems; sets of ROWS rows below the region
+  uint32_t ticket0;    // tickets of the launches before
+  uint32_t region;     // regions before this one, all of MAX_BLOCKS blocks
+};
+
+struct CoreLds {
+  FactorScratch fs;
+  float S[NB][LDD];  // rows to be solved, then solved
+};
+struct RowsLds {
+  float R[MAX_BLOCKS - 1][ROWS][LDD];  // the solved block columns
+  float S[ROWS][LDD];
+};
+struct RegionLds {
+  union {
+    CoreLds core;
+    RowsLds rows;
+  };
+  int word, gave_up;
+};
+static_assert(sizeof(RegionLds) <= 80 * 1024, "two workgroups to a CU");
+
+// tasks of a problem that come first: the spine and the row blocks from 2 on
+__host__ __device__ inline int core_tasks(int nb) { return nb > 2 ? nb - 1 : 1; }
+// block (j, i), i < j, of the side buffer
+__device__ __forceinline__ int solved_block(int j, int i) { return (j * (j - 1) / 2 + i) * BLOCK; }
+__device__ __forceinline__ int next_block(int b) { return SIDE_NEXT + (b - 2) * 2 * BLOCK; }
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+constexpr int SC1 = 16;  // through the L2
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t block_rsrc(float* block) {
+  return __builtin_amdgcn_make_buffer_rsrc(block, 0, BLOCK * 4, 0x00027000);
+}
+__device__ __forceinline__ void store4_through(__amdgpu_buffer_rsrc_t rs, int at, float4 v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(v4i, v), rs, at * 4, 0, SC1);
+}
+// tile t of a dense 64 x 64 block
+__device__ __forceinline__ void tile_store_through(v4f acc, __amdgpu_buffer_rsrc_t rs, int t, int lane) {
+  const int at = (16 * (t >> 2) + 4 * (lane >> 4)) * NB + 16 * (t & 3) + (lane & 15);
+#pragma unroll
+  for (int v = 0; v < 4; ++v)
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(acc[v]), rs, (at + v * NB) * 4, 0, SC1);
+}
+// this wave's stores have arrived; count `add` on `word`
+__device__ __forceinline__ void publish(uint32_t* word, uint32_t add, int lane) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (lane == 0) __hip_atomic_fetch_add(word, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool reached(const uint32_t* word, uint32_t target) {
+  const bool there = (int)(__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target) >= 0;
+  asm volatile("" ::: "memory");  // what is loaded next is loaded after the word
+  return there;
+}
+// false: gave up
+__device__ __forceinline__ bool poll(const uint32_t* word, uint32_t target) {
+  if (reached(word, target)) return true;
+  const uint64_t start = __builtin_readsteadycounter();  // 100 MHz
+  do {
+    __builtin_amdgcn_s_sleep(2);
+    if (reached(word, target)) return true;
+  } while (__builtin_readsteadycounter() - start < 2000000000ull);
+  return false;
+}
+// for the whole workgroup; a barrier on either side
+__device__ __forceinline__ bool wait_for(RegionLds& L, const uint32_t* word, uint32_t target, HinvScalars* sc) {
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const bool ok = poll(word, target);
+    if (!ok) atomicExch(&sc->info, -1);
+    L.gave_up = !ok;
+  }
+  __syncthreads();
+  return !L.gave_up;
+}
+
+// a problem's pointers
+struct Region {
+  float* A;
+  float* Xs;  // of the region's first block
+  float* side;
+  uint32_t* sync;
+  HinvScalars* sc;
+  int Kp, K, r0, nb;
+  uint32_t done;  // hand-overs of one kind in the regions before
+  __device__ uint32_t* word(int which) const { return sync + which * SYNC_LINE; }
+  // count of SYNC_ROW + j once `blocks` blocks of this region have arrived
+  __device__ uint32_t row_target(int j, int blocks) const { return (done * j + blocks) * 16u; }
+  __device__ uint32_t target() const { return (done + 1) * 16u; }
+};
+
+__device__ __forceinline__ void spine(const Region& g, RegionLds& lds, int thread) {
+  CoreLds& L = lds.core;
+  const int w = __builtin_amdgcn_readfirstlane(thread >> 6);
+  const int64_t ld = g.Kp;
+  {
+    const int r = thread & 63;
+    const float* src = g.A + (int64_t)(g.r0 + r) * ld + g.r0 + 8 * w;
+    factor_block_put(L.fs, *(const float4*)src, *(const float4*)(src + 4), w, r);
+  }
+  for (int m = 0; m < g.nb; ++m) {
+    const int c0 = g.r0 + NB * m;
+    const bool more = m + 1 < g.nb;
+    int tid = thread;
+    asm("" : "+v"(tid));  // the many addresses that follow from it are formed where they are used, not kept (and spilled)
+    const int r = tid & 63;
+    // What waves 4 to 7 do beside the factorisation: the row block solved last goes out, the next one (A[m+1, m] into S,
+    // the tiles on and below the diagonal of block m + 1 into registers, three or two per wave) comes in.
+    const int t = (tid - NT / 2) & (NT / 2 - 1), row = t >> 4, c4 = (t & 15) * 4, q = w & 3;
+    auto tile_row = [](int i) { return i < 1 ? 0 : i < 3 ? 1 : i < 6 ? 2 : 3; };
+    auto tile_col = [&](int i) { return i - tile_row(i) * (tile_row(i) + 1) / 2; };
+    float4 in0, in1, in2, in3;  // (an array ends up in scratch memory)
+    v4f dg[3];
+    enum { WANTED, COMING, THERE };
+    int state = more ? WANTED : THERE, turn = 0;
+    uint32_t* const ready = g.word(SYNC_NEXT + m + 1);
+    auto fetch = [&]() {
+      const float* const src = m == 0 ? g.A + (int64_t)(c0 + NB) * ld + c0 : g.side + next_block(m + 1);
+      const float* const dsrc = m == 0 ? src + NB : src + BLOCK;
+      const int64_t sld = m == 0 ? ld : NB;
+      const float* const at = src + row * sld + c4;
+      in0 = *(const float4*)at;
+      in1 = *(const float4*)(at + 16 * sld);
+      in2 = *(const float4*)(at + 32 * sld);
+      in3 = *(const float4*)(at + 48 * sld);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int d = min(q + 4 * i, 9);
+        dg[i] = tile_load(dsrc, sld, tile_row(d) * 4 + tile_col(d), r);
+      }
+      state = COMING;
+    };
+    auto put = [&]() {
+      *(float4*)&L.S[row][c4] = in0;
+      *(float4*)&L.S[row + 16][c4] = in1;
+      *(float4*)&L.S[row + 32][c4] = in2;
+      *(float4*)&L.S[row + 48][c4] = in3;
+      state = THERE;
+    };
+    if (w >= 4 && m == 0 && more) fetch();
+    const int bad = factor_invert_64(L.fs, tid, [&]() {
+      if (turn == 0 && m > 0) {
+        const __amdgpu_buffer_rsrc_t out = block_rsrc(g.side + solved_block(m, m - 1));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float4 v = *(const float4*)&L.S[row + 16 * i][c4];
+          store4_through(out, (row + 16 * i) * NB + c4, v);
+          *(float4*)(g.A + (int64_t)(c0 + row + 16 * i) * ld + c0 - NB + c4) = v;
+        }
+        publish(g.word(SYNC_ROW + m), 4, r);
+      }
+      if (state == COMING)
+        put();
+      else if (state == WANTED && reached(ready, g.target()))
+        fetch();
+      ++turn;
+    });
+    // first failing pivot, 1-based index in the ORIGINAL (un-reversed) ordering
+    if (tid == 0 && bad < NB && c0 + bad < g.K) atomicCAS(&g.sc->info, 0, g.K - (c0 + bad));
+    {
+      const __amdgpu_buffer_rsrc_t xs = block_rsrc(g.Xs + m * BLOCK);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int idx = tid + NT * i, xr = idx >> 4, xc = (idx & 15) * 4;
+        store4_through(xs, xr * NB + xc, *(const float4*)&L.fs.X[xr][xc]);
+      }
+    }
+    if (!more) {
+      publish(g.word(SYNC_X + m), 2, r);
+      return;
+    }
+    if (w >= 4) {
+      if (state == WANTED) {
+        if (!poll(ready, g.target()) && r == 0) {
+          atomicExch(&g.sc->info, -1);
+          lds.gave_up = 1;
+        }
+        fetch();
+      }
+      if (state == COMING) put();
+    }
+    __syncthreads();
+    if (lds.gave_up) return;
+    // R = S X_m^T, two tiles per wave
+    v4f sol0 = {0.f, 0.f, 0.f, 0.f}, sol1 = sol0;
+    const int st = (w >> 1) * 4 + (w & 1) * 2;
+    {
+      const Operand64 x = operand_load(&L.S[16 * (w >> 1)][0], LDD, r);
+      sol0 = tile_mm<false>(sol0, x, operand_load(&L.fs.X[32 * (w & 1)][0], LDD, r));
+      sol1 = tile_mm<false>(sol1, x, operand_load(&L.fs.X[32 * (w & 1) + 16][0], LDD, r));
+    }
+    __syncthreads();  // every wave has read S
+    tile_store(sol0, &L.S[0][0], LDD, st, r);
+    tile_store(sol1, &L.S[0][0], LDD, st + 1, r);
+    publish(g.word(SYNC_X + m), 2, r);
+    __syncthreads();
+    // the next block less R R^T, straight to where the factorisation takes it
+    if (w >= 4) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const int d = q + 4 * i;
+        if (d > 9) continue;
+        const int ti = tile_row(d), tj = tile_col(d);
+        const v4f v = tile_mm<true>(dg[i], operand_load(&L.S[16 * ti][0], LDD, r), operand_load(&L.S[16 * tj][0], LDD, r));
+        const int c = r & 15, k = 16 * ti + 4 * (r >> 4);
+        if (tj == 0) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) L.fs.P[k + e][c] = v[e];
+        } else {
+          *(float4*)L.fs.at(16 * tj + c, k) = make_float4(v[0], v[1], v[2], v[3]);
+        }
+      }
+    }
+  }
+}
+
+// row block b >= 2 of the region, wave w: tiles (w / 2, 2 (w % 2)) and the one beside it of every block
+__device__ __forceinline__ void row_block(const Region& g, RegionLds& lds, int b, int tid) {
+  CoreLds& L = lds.core;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), r = tid & 63;
+  const int tr = 16 * (w >> 1), tc = 32 * (w & 1), t0 = (w >> 1) * 4 + (w & 1) * 2;
+  const int64_t ld = g.Kp;
+  float* const own = g.A + (int64_t)(g.r0 + NB * b) * ld + g.r0;
+  v4f acc[MAX_BLOCKS - 1][2], dg[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+#pragma unroll
+    for (int c = 0; c < MAX_BLOCKS - 1; ++c) {
+      if (c < b) acc[c][i] = tile_load(own + NB * c, ld, t0 + i, r);
+    }
+    dg[i] = tile_load(own + NB * b, ld, t0 + i, r);
+  }
+#pragma unroll
+  for (int m = 0; m < MAX_BLOCKS - 2; ++m) {
+    if (m + 1 >= b) break;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) tile_store(acc[m][i], &L.S[0][0], LDD, t0 + i, r);
+    if (!wait_for(lds, g.word(SYNC_X + m), g.target(), g.sc)) return;
+    v4f sol[2];
+    {
+      const Operand64 x = operand_load(&L.S[tr][0], LDD, r);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        sol[i] = tile_mm<false>(v4f{0.f, 0.f, 0.f, 0.f}, x, operand_load(g.Xs + m * BLOCK + (tc + 16 * i) * NB, NB, r));
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) tile_store(sol[i], &L.S[0][0], LDD, t0 + i, r);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int idx = tid + NT * i, row = idx >> 4, c4 = (idx & 15) * 4;
+      const float4 out = *(const float4*)&L.S[row][c4];
+      store4_through(block_rsrc(g.side + solved_block(b, m)), row * NB + c4, out);
+      *(float4*)(own + row * ld + NB * m + c4) = out;
+    }
+    const Operand64 x = operand_load(&L.S[tr][0], LDD, r);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) dg[i] = tile_mm<true>(dg[i], x, operand_load(&L.S[tc + 16 * i][0], LDD, r));
+    publish(g.word(SYNC_ROW + b), 2, r);
+#pragma unroll
+    for (int c = m + 1; c < MAX_BLOCKS - 1; ++c) {
+      if (c >= b) break;
+      if (!wait_for(lds, g.word(SYNC_ROW + c), g.row_target(c, m + 1), g.sc)) return;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        acc[c][i] = tile_mm<true>(acc[c][i], x, operand_load(g.side + solved_block(c, m) + (tc + 16 * i) * NB, NB, r));
+    }
+    // (S is written again only after the waits' barriers: every wave has its operands by then)
+    if (m + 2 == b) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        tile_store_through(acc[m + 1][i], block_rsrc(g.side + next_block(b)), t0 + i, r);
+        tile_store_through(dg[i], block_rsrc(g.side + next_block(b) + BLOCK), t0 + i, r);
+      }
+      publish(g.word(SYNC_NEXT + b), 2, r);
+    }
+  }
+}
+
+// rows 32 tile .. 32 tile + 31 below the region, wave w: rows 16 (w / 4), columns 16 (w % 4) of each block column
+__device__ __forceinline__ void rows_below(const Region& g, RegionLds& lds, int tile, int tid) {
+  RowsLds& L = lds.rows;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6), r = tid & 63, s = 16 * (w >> 2), tc = w & 3;
+  const int64_t ld = g.Kp;
+  float* const own = g.A + (int64_t)(g.r0 + NB * g.nb + ROWS * tile + s) * ld + g.r0;
+  v4f acc = tile_load(own, ld, tc, r);
+#pragma unroll
+  for (int j = 0; j < MAX_BLOCKS; ++j) {
+    if (j >= g.nb) break;
+    v4f ahead = acc;
+    if (j + 1 < g.nb) ahead = tile_load(own + NB * (j + 1), ld, tc, r);
+    if (j > 0) {
+      // the solved blocks arrive before the inverse of the diagonal block does
+      if (!wait_for(lds, g.word(SYNC_ROW + j), g.row_target(j, j), g.sc)) return;
+#pragma unroll
+      for (int i = 0; i < j; ++i)
+        acc = tile_mm<true>(acc, operand_load(&L.R[i][s][0], LDD, r),
+                            operand_load(g.side + solved_block(j, i) + 16 * tc * NB, NB, r));
+    }
+    tile_store(acc, &L.S[s][0], LDD, tc, r);
+    if (!wait_for(lds, g.word(SYNC_X + j), g.target(), g.sc)) return;
+    v4f sol = {0.f, 0.f, 0.f, 0.f};
+    sol = tile_mm<false>(sol, operand_load(&L.S[s][0], LDD, r), operand_load(g.Xs + j * BLOCK + 16 * tc * NB, NB, r));
+    tile_store(sol, own + NB * j, ld, tc, r);
+    if (j + 1 < MAX_BLOCKS) tile_store(sol, &L.R[j < MAX_BLOCKS - 1 ? j : 0][s][0], LDD, tc, r);
+    acc = ahead;
+  }
+}
+
+__global__ __launch_bounds__(REGION_NT) void chol_region_kernel(RegionArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char region_smem[];
+  RegionLds& lds = *(RegionLds*)region_smem;
+  const int tid = threadIdx.x;
+  const int cores = core_tasks(a.nb), all = a.n * cores;
+  auto problem_of = [&](int task) { return task < all ? task / cores : (task - all) / a.tiles; };
+  if (tid == 0) {
+    const int task = (int)(atomicAdd(a.sync + SYNC_TICKET * SYNC_LINE, 1u) - a.ticket0);
+    lds.word = task;
+    lds.gave_up = a.sc[problem_of(task)].info < 0;  // in an earlier region
+  }
+  __syncthreads();
+  if (lds.gave_up) return;
+  const int task = __builtin_amdgcn_readfirstlane(lds.word), problem = problem_of(task);
+  Region g;
+  g.A = a.A + (int64_t)problem * a.Kp * a.Kp;
+  g.Xs = a.Xs + problem * a.xs_stride + (int64_t)(a.r0 / NB) * BLOCK;
+  g.side = a.side + problem * a.side_stride;
+  g.sync = a.sync + (int64_t)problem * SYNC_WORDS;
+  g.sc = a.sc + problem;
+  g.Kp = a.Kp; g.K = a.K; g.r0 = a.r0; g.nb = a.nb;
+  g.done = a.region;
+  if (task < all) {
+    const int role = task - problem * cores;
+    if (role == 0)
+      spine(g, lds, tid);
+    else
+      row_block(g, lds, role + 1, tid);
+  } else {
+    rows_below(g, lds, task - all - problem * a.tiles, tid);
+  }
+}
+
+}  // namespace cholregion
