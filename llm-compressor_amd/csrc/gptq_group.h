@@ -15,7 +15,11 @@
 //   * a division is three operations (quotient() below); a wave that meets a divisor or a value outside the range
 //     where that gives the IEEE quotient repeats its block with plain divisions.
 // Before block b is quantised, the group's earlier errors are taken off its columns on the matrix cores,
-// W[:, b] - E U[:, b], as 16 x 16 tiles accumulated by v_mfma_f32_16x16x4_f32 in fp32.
+// W[:, b] - E U[:, b], as 16 x 16 tiles accumulated by v_mfma_f32_16x16x4_f32 in fp32.  In the left-looking form the same
+// products bring in what the group owes to all earlier columns, P U[group, group]: E starts out as P in LDS, a block's own
+// columns of it are multiplied ahead of the block before, and its errors are added to them.  As a pass over the pieces of P,
+// a 512-wide product and a pass that formed D this took three launches more per group: with them 4096 x 4096 2441 -> 2202
+// us (a whole call), 4096 x 14336 19.7 -> 19.1 ms, 32 of 768 x 2048 5341 -> 5000 us.
 //
 // A workgroup is four waves that run the chain, one per SIMD, and four that prepare the next block meanwhile: its slice
 // of U, its scales and the part of its tiles that does not wait for the current block.
@@ -58,12 +62,23 @@ struct GptqGroupParams {
   int64_t row_div, srow;
   int fmt, bits;
   int sd;           // dtype the dequantised value is formed in
-  float* E;         // scaled errors of the group, negated, row stride Q_LDE
+  float* E;         // scaled errors of the group, negated, row stride Q_LDE; NULL with P or D
   float* loss_rows; // [R], written by the first group and added to by the others
   // grouped call: problem blockIdx.y takes scale / zp / gscale / g_idx from items and its Wf, U, E and
   // loss rows at these strides (in elements)
   const GptqItem* items;
   int64_t u_stride, w_stride, e_stride;
+  // the left-looking form (gptq.hip), blocks of 128 columns: `pieces` matrices [.., Q_LDE] whose sum P times U[group, group]
+  // the group's 512 columns take from the columns before them (0: nothing), and D (NULL: nobody reads it), the group's
+  // columns of W minus the quantised ones over k_scale, [.., ldw] like Wf, with the rows' largest values so far and the
+  // scales that follow from them
+  const float* P;
+  int pieces;
+  int64_t piece_stride, p_stride;
+  float* D;
+  const float* k_scale;  // [K] per problem
+  float *row_max, *row_scale;
+  int64_t ks_stride, rows_stride;
 };
 
 typedef void (*GptqGroupKernel)(GptqGroupParams);
@@ -79,11 +94,21 @@ constexpr int Q_UHALF = GB / 2;
 constexpr int Q_U = Q_UHALF * GB + Q_UHALF * Q_UHALF;  // LDS slice of U: rows 0..63 whole, rows 64..127 from column 64 on
 constexpr int Q_D = GB / QG * 16;               // LDS column constants: four float4 per quad of columns
 constexpr int Q_LDS_W = GB + 4;                 // LDS row stride of a block's values
-constexpr int Q_LDS_E = (GROUP - 1) * GB + 4;   // LDS row stride of the group's errors
+constexpr int Q_LDS_E = GROUP * GB + 4;         // LDS row stride of the group's errors (and P)
 constexpr int Q_THREADS = 512;
 constexpr int q_rows(int team) { return 256 / team; }
 constexpr int q_smem(int team, bool has_zp) {
-  return (Q_U + Q_D + q_rows(team) * ((has_zp ? 3 : 2) * Q_LDS_W + Q_LDS_E)) * 4;
+  return (Q_U + Q_D + q_rows(team) * (2 * Q_LDS_W + Q_LDS_E)) * 4 + (has_zp ? q_rows(team) * Q_LDS_W : 0);
+}
+
+// the power of two that brings m >= 0 into [2^13, 2^14), the largest one for m = 0; 1 where m is not finite
+constexpr int SCALE_MAX_EXP = 100;
+__device__ __forceinline__ float scale_to_2_13(float m) {
+  if (!(m <= 3.4028234e38f)) return 1.f;
+  int e = 14 - SCALE_MAX_EXP;
+  if (m > 0.f) (void)frexpf(m, &e);  // m in [2^(e-1), 2^e)
+  e = 14 - e;
+  return ldexpf(1.f, e < -SCALE_MAX_EXP ? -SCALE_MAX_EXP : (e > SCALE_MAX_EXP ? SCALE_MAX_EXP : e));
 }
 
 #ifdef LLMC_GPTQ_GROUP_KERNELS
@@ -176,6 +201,9 @@ __device__ __forceinline__ float team_value(float v) {
   const int lo = __builtin_amdgcn_mov_dpp(x, 0x150 + LI, 0xf, 0xf, true);
   return __int_as_float(TEAM == 16 ? lo : __builtin_amdgcn_update_dpp(lo, x, 0x158 + (LI & 7), 0xf, 0xc, false));
 }
+
+// of a normal power of two up to 2^126: its exponent negated
+__device__ __forceinline__ float reciprocal_of_power_of_2(float s) { return __uint_as_float(0x7f000000u - __float_as_uint(s)); }
 
 __device__ __forceinline__ void add_row(float (&w)[QG], float e, const float4& u) {
   w[0] = fmaf(e, u.x, w[0]);
@@ -398,21 +426,20 @@ struct BChunk {
     }
   }
 };
+// The sums start from zero and the chain adds them to W, in one rounding: they are the size of a quantisation step, the
+// weights several of them, and every instruction rounds a sum.
 template <int NR>
 struct Tiles {
   f32x4_t acc[NR][2];
-  __device__ __forceinline__ void load(const float* __restrict__ W, int64_t ldw, int col0, int col1, int q) {
+  __device__ __forceinline__ void clear() {
 #pragma unroll
     for (int t = 0; t < NR; ++t)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        acc[t][0][i] = load_at<float>(W, (t * 16 + i) * ldw, (uint32_t)(4 * q) * (uint32_t)ldw + (uint32_t)col0);
-        acc[t][1][i] = load_at<float>(W, (t * 16 + i) * ldw, (uint32_t)(4 * q) * (uint32_t)ldw + (uint32_t)col1);
-      }
+      for (int i = 0; i < 4; ++i) acc[t][0][i] = acc[t][1][i] = 0.f;
   }
   // E: the workgroup's rows at the chunk's first column
   __device__ __forceinline__ void multiply(const BChunk& b, const float* __restrict__ E, int lde, bool vec, int len, int c,
-                                           int q) {
+                                           int q, bool second_only = false) {
 #pragma unroll
     for (int t = 0; t < NR; ++t) {
       const float* src = E + (t * 16 + c) * lde + KL * q;
@@ -433,7 +460,7 @@ struct Tiles {
       }
 #pragma unroll
       for (int j = 0; j < KL; ++j) {
-        acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b.b0[j], acc[t][0], 0, 0, 0);
+        if (!second_only) acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b.b0[j], acc[t][0], 0, 0, 0);
         acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b.b1[j], acc[t][1], 0, 0, 0);
       }
     }
@@ -470,19 +497,50 @@ __global__ __launch_bounds__(Q_THREADS) void gptq_group_kernel(GptqGroupParams p
   extern __shared__ __attribute__((aligned(16))) float qsmem[];
   float* const Us = qsmem;                       // slice of U of this block
   float* const Ds = Us + Q_U;                    // its column constants
-  float* const Es = Ds + Q_D;                    // the group's errors
+  float* const Es = Ds + Q_D;                    // P, then P plus the errors of the finished blocks
   float* const Ws = Es + ROWS * Q_LDS_E;         // the block's values after the group's earlier errors
   float* const Ss = Ws + ROWS * Q_LDS_W;         // scales
-  float* const Zs = Ss + ROWS * Q_LDS_W;         // zero points (HAS_ZP only)
+  int8_t* const Zs = (int8_t*)(Ss + ROWS * Q_LDS_W);  // zero points (HAS_ZP only)
   if (p.items) {
     const GptqItem it = p.items[blockIdx.y];
     p.scale = it.scale; p.zp = it.zp; p.gscale = it.gscale; p.g_idx = it.g_idx;
     p.Wf += (int64_t)blockIdx.y * p.w_stride;
     p.U += (int64_t)blockIdx.y * p.u_stride;
-    p.E += (int64_t)blockIdx.y * p.e_stride;
+    if (p.E) p.E += (int64_t)blockIdx.y * p.e_stride;
     p.loss_rows += (int64_t)blockIdx.y * p.R;
+    p.P += (int64_t)blockIdx.y * p.p_stride;
+    if (p.D) p.D += (int64_t)blockIdx.y * p.w_stride;
+    p.k_scale += (int64_t)blockIdx.y * p.ks_stride;
+    p.row_max += (int64_t)blockIdx.y * p.rows_stride;
+    p.row_scale += (int64_t)blockIdx.y * p.rows_stride;
   }
   const int row0 = blockIdx.x * ROWS;
+  const bool has_p = p.pieces > 0;
+  // P, its pieces added in their order, by all threads: `half` of the workgroup's float4s to a role
+  auto load_p = [&](int half) {
+    constexpr int N = ROWS * GROUP * GB / 4 / Q_THREADS;  // per thread
+    const int tid = opaque(threadIdx.x & 255);
+    const float* src = p.P + (int64_t)row0 * Q_LDE + (int64_t)half * (N * 256 * 4);
+    float4 v[N];
+#pragma unroll
+    for (int n = 0; n < N; ++n) v[n] = *(const float4*)(src + (tid + n * 256) * 4);
+#pragma unroll 1
+    for (int k = 1; k < p.pieces; ++k) {
+      src += p.piece_stride;
+      float4 x[N];
+#pragma unroll
+      for (int n = 0; n < N; ++n) x[n] = *(const float4*)(src + (tid + n * 256) * 4);
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        v[n].x += x[n].x; v[n].y += x[n].y; v[n].z += x[n].z; v[n].w += x[n].w;
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) {
+      const int f = half * (N * 256) + tid + n * 256;
+      *(float4*)&Es[(f >> 7) * Q_LDS_E + (f & 127) * 4] = v[n];
+    }
+  };
   const bool vec_u = (p.ldu & 3) == 0 && (p.bs & 3) == 0 && ((uintptr_t)p.U & 15) == 0;
 
   // Barriers, in the order in which both roles pass them: "ready" (a block's slice, scales and values are in LDS), "read"
@@ -529,27 +587,40 @@ __global__ __launch_bounds__(Q_THREADS) void gptq_group_kernel(GptqGroupParams p
           }
           const int o = team * Q_LDS_W + J * SPAN + tl * QG;
           *(float4*)&Ss[o] = make_float4(s[4 * J], s[4 * J + 1], s[4 * J + 2], s[4 * J + 3]);
-          if (HAS_ZP) *(float4*)&Zs[o] = make_float4(z[4 * J], z[4 * J + 1], z[4 * J + 2], z[4 * J + 3]);
+          if (HAS_ZP) *(char4*)&Zs[o] = make_char4((int8_t)z[4 * J], (int8_t)z[4 * J + 1], (int8_t)z[4 * J + 2], (int8_t)z[4 * J + 3]);
         }
       }
       phase_end();
-      if (kc > 0) {
+      if (has_p && kc == 0) {
+        load_p(1);
+        __syncthreads();  // P
+      }
+      if (kc > 0 || has_p) {
         const int c = lane & 15, q = lane >> 4;
         const int ct0 = wave * 16 + c, ct1 = ct0 + Q_UHALF;
         const int col0 = ct0 < count ? ct0 : count - 1, col1 = ct1 < count ? ct1 : count - 1;
         const float* const Uc = p.U + (int64_t)p.g0 * p.ldu + i2;
         Tiles<NR> tiles;
-        tiles.load(p.Wf + (int64_t)row0 * p.ldw + i2, p.ldw, col0, col1, q);
+        tiles.clear();
+        if (has_p) {  // the block's own columns of P; U's rows from 64 on are zero in the columns before them
+          BChunk b;
+          b.fetch(base, p.ldu, KS, col0, col1, q);
+          tiles.multiply(b, Es + kc, Q_LDS_E, true, KS, c, q);
+          b.fetch(base + (int64_t)KS * p.ldu, p.ldu, KS, col0, col1, q);
+          tiles.multiply(b, Es + kc + KS, Q_LDS_E, true, KS, c, q, true);
+        }
         tiles.accumulate(Uc, p.ldu, Es, Q_LDS_E, last, p.bs, col0, col1, c, q);
         phase_end();
-        // rows of U for the errors of the block before, in flight until they are there
-        const int len0 = p.bs < KS ? p.bs : KS, len1 = p.bs - len0;
-        BChunk b0, b1;
-        b0.fetch(Uc + (int64_t)last * p.ldu, p.ldu, len0, col0, col1, q);
-        if (len1 > 0) b1.fetch(Uc + (int64_t)(last + KS) * p.ldu, p.ldu, len1, col0, col1, q);
-        __syncthreads();  // errors
-        tiles.multiply(b0, Es + last, Q_LDS_E, (last & 3) == 0 && len0 == KS, len0, c, q);
-        if (len1 > 0) tiles.multiply(b1, Es + last + KS, Q_LDS_E, (last & 3) == 0 && len1 == KS, len1, c, q);
+        if (kc > 0) {
+          // rows of U for the errors of the block before, in flight until they are there
+          const int len0 = p.bs < KS ? p.bs : KS, len1 = p.bs - len0;
+          BChunk b0, b1;
+          b0.fetch(Uc + (int64_t)last * p.ldu, p.ldu, len0, col0, col1, q);
+          if (len1 > 0) b1.fetch(Uc + (int64_t)(last + KS) * p.ldu, p.ldu, len1, col0, col1, q);
+          __syncthreads();  // errors
+          tiles.multiply(b0, Es + last, Q_LDS_E, (last & 3) == 0 && len0 == KS, len0, c, q);
+          if (len1 > 0) tiles.multiply(b1, Es + last + KS, Q_LDS_E, (last & 3) == 0 && len1 == KS, len1, c, q);
+        }
 #pragma unroll
         for (int t = 0; t < NR; ++t)
 #pragma unroll
@@ -570,7 +641,11 @@ __global__ __launch_bounds__(Q_THREADS) void gptq_group_kernel(GptqGroupParams p
   // ---- the chain
   const QFormat f = make_qformat(FMT, p.bits);   // the format is a compile-time constant here
   const bool vec_w = (p.bs & 3) == 0;
-  float loss = 0.f;
+  float loss = 0.f, dmax = 0.f;
+  if (has_p) {
+    load_p(0);
+    __syncthreads();  // P
+  }
 #pragma unroll 1
   for (int i1 = p.g0; i1 < p.gend; i1 += p.bs) {
     const int count = p.gend - i1 < p.bs ? p.gend - i1 : p.bs;
@@ -580,32 +655,40 @@ __global__ __launch_bounds__(Q_THREADS) void gptq_group_kernel(GptqGroupParams p
     const bool live = row < p.R;
     float* const wrow = p.Wf + (int64_t)row * p.ldw;
     float* const erow = p.E + (int64_t)row * Q_LDE;
-    __syncthreads();  // ready
     float w[NRUN][QG], s[NRUN][QG], z[NRUN][QG];
-    auto load_w = [&]() {
+    auto load_w = [&]() {  // as they are in memory
 #pragma unroll
       for (int J = 0; J < NRUN; ++J) {
         const int c = J * SPAN + tl * QG;
         float4 v;
-        if (kc > 0)
-          v = *(const float4*)&Ws[team * Q_LDS_W + c];
-        else if (vec_w)
+        if (vec_w)
           v = *(const float4*)&wrow[i1 + (c < count ? c : 0)];
         else
           v = make_float4(wrow[i1 + (c < count ? c : 0)], wrow[i1 + (c + 1 < count ? c + 1 : 0)],
                           wrow[i1 + (c + 2 < count ? c + 2 : 0)], wrow[i1 + (c + 3 < count ? c + 3 : 0)]);
-        w[J][0] = live && c + 0 < count ? v.x : 0.f;
-        w[J][1] = live && c + 1 < count ? v.y : 0.f;
-        w[J][2] = live && c + 2 < count ? v.z : 0.f;
-        w[J][3] = live && c + 3 < count ? v.w : 0.f;
+        w[J][0] = v.x; w[J][1] = v.y; w[J][2] = v.z; w[J][3] = v.w;
+      }
+    };
+    auto add_sums = [&]() {
+#pragma unroll
+      for (int J = 0; J < NRUN; ++J) {
+        const int c = J * SPAN + tl * QG;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (kc > 0 || has_p) v = *(const float4*)&Ws[team * Q_LDS_W + c];
+        w[J][0] = live && c + 0 < count ? w[J][0] + v.x : 0.f;
+        w[J][1] = live && c + 1 < count ? w[J][1] + v.y : 0.f;
+        w[J][2] = live && c + 2 < count ? w[J][2] + v.z : 0.f;
+        w[J][3] = live && c + 3 < count ? w[J][3] + v.w : 0.f;
       }
     };
     load_w();
+    __syncthreads();  // ready
+    add_sums();
 #pragma unroll
     for (int J = 0; J < NRUN; ++J) {
       const int o = team * Q_LDS_W + J * SPAN + tl * QG;
       const float4 a = *(const float4*)&Ss[o];
-      const float4 b = HAS_ZP ? *(const float4*)&Zs[o] : make_float4(0.f, 0.f, 0.f, 0.f);
+      const char4 b = HAS_ZP ? *(const char4*)&Zs[o] : make_char4(0, 0, 0, 0);
       s[J][0] = a.x; s[J][1] = a.y; s[J][2] = a.z; s[J][3] = a.w;
       z[J][0] = b.x; z[J][1] = b.y; z[J][2] = b.z; z[J][3] = b.w;
     }
@@ -654,6 +737,7 @@ __global__ __launch_bounds__(Q_THREADS) void gptq_group_kernel(GptqGroupParams p
     for (int J = 0; J < NRUN; ++J) total += run_loss(o[J]);
     if (__any(bad || !(total < 0x1p60f))) {  // every quotient stayed below 2^128 then, or its NaN is in the total
       load_w();
+      add_sums();
       all_runs(std::true_type{});
     }
     __builtin_amdgcn_s_setprio(0);
@@ -662,7 +746,13 @@ __global__ __launch_bounds__(Q_THREADS) void gptq_group_kernel(GptqGroupParams p
       for (int J = 0; J < NRUN; ++J) {
         const int c = J * SPAN + tl * QG;
         if (vec_w && c + QG <= count) {
-          *(float4*)&Es[team * Q_LDS_E + kc + c] = make_float4(o[J].e[0], o[J].e[1], o[J].e[2], o[J].e[3]);
+          float4* const at = (float4*)&Es[team * Q_LDS_E + kc + c];
+          float4 v = make_float4(o[J].e[0], o[J].e[1], o[J].e[2], o[J].e[3]);
+          if (has_p) {
+            const float4 x = *at;
+            v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w;
+          }
+          *at = v;
         } else {
 #pragma unroll
           for (int m = 0; m < QG; ++m)
@@ -687,15 +777,23 @@ __global__ __launch_bounds__(Q_THREADS) void gptq_group_kernel(GptqGroupParams p
 #pragma unroll
       for (int J = 0; J < NRUN; ++J) {
         const int c = J * SPAN + tl * QG;
+        if (p.D) {  // (in whole blocks) the weights as they came are still in Wf
+          const float4 w0 = *(const float4*)&wrow[i1 + c], ks = *(const float4*)&p.k_scale[i1 + c];
+          float4 d = make_float4(w0.x - o[J].q[0], w0.y - o[J].q[1], w0.z - o[J].q[2], w0.w - o[J].q[3]);
+          d.x *= reciprocal_of_power_of_2(ks.x); d.y *= reciprocal_of_power_of_2(ks.y);
+          d.z *= reciprocal_of_power_of_2(ks.z); d.w *= reciprocal_of_power_of_2(ks.w);
+          dmax = fmaxf(dmax, fmaxf(fmaxf(fabsf(d.x), fabsf(d.y)), fmaxf(fabsf(d.z), fabsf(d.w))));
+          *(float4*)&p.D[(int64_t)row * p.ldw + i1 + c] = d;
+        }
         if (vec_w && c + QG <= count) {
           *(float4*)&wrow[i1 + c] = make_float4(o[J].q[0], o[J].q[1], o[J].q[2], o[J].q[3]);
-          *(float4*)&erow[kc + c] = make_float4(o[J].e[0], o[J].e[1], o[J].e[2], o[J].e[3]);
+          if (p.E) *(float4*)&erow[kc + c] = make_float4(o[J].e[0], o[J].e[1], o[J].e[2], o[J].e[3]);
         } else {
 #pragma unroll
           for (int m = 0; m < QG; ++m)
             if (c + m < count) {
               wrow[i1 + c + m] = o[J].q[m];
-              erow[kc + c + m] = o[J].e[m];
+              if (p.E) erow[kc + c + m] = o[J].e[m];
             }
         }
       }
@@ -706,6 +804,15 @@ __global__ __launch_bounds__(Q_THREADS) void gptq_group_kernel(GptqGroupParams p
   loss += __shfl_xor(loss, 4, 8);
   const int row = row0 + (int)threadIdx.x / TEAM;
   if (row < p.R && threadIdx.x % TEAM == 0) p.loss_rows[row] = (p.g0 == 0 ? 0.f : p.loss_rows[row]) + loss * 0.5f;
+  if (p.D) {
+#pragma unroll
+    for (int k = 1; k < TEAM; k *= 2) dmax = fmaxf(dmax, __shfl_xor(dmax, k, TEAM));
+    if (row < p.R && threadIdx.x % TEAM == 0) {
+      if (p.g0 > 0) dmax = fmaxf(dmax, p.row_max[row]);
+      p.row_max[row] = dmax;
+      p.row_scale[row] = scale_to_2_13(dmax);
+    }
+  }
 }
 
 template <int FMT, int SD, bool HAS_ZP>
