@@ -31,6 +31,7 @@
 // leaves, and the result is the identity as for any failed factorisation.
 #pragma once
 #include "chol_block.h"
+#include "split2.h"
 
 namespace cholregion {
 using namespace cholblk;
@@ -66,6 +67,11 @@ struct RegionArgs {
   int n, tiles;        // problems; sets of ROWS rows below the region
   uint32_t ticket0;    // tickets of the launches before
   uint32_t region;     // regions before this one, all of MAX_BLOCKS blocks
+  // where the rows below go as two f16 terms as well (split2.h), for the updates that read them, or NULL: row i of the
+  // matrix at i * split_ld, one set every split_stride words
+  uint32_t* split;
+  int64_t split_stride;
+  int split_ld;
 };
 
 struct CoreLds {
@@ -73,7 +79,7 @@ struct CoreLds {
   float S[NB][LDD];  // rows to be solved, then solved
 };
 struct RowsLds {
-  float R[MAX_BLOCKS - 1][ROWS][LDD];  // the solved block columns
+  float R[MAX_BLOCKS][ROWS][LDD];  // the solved block columns
   float S[ROWS][LDD];
 };
 struct RegionLds {
@@ -147,6 +153,8 @@ struct Region {
   HinvScalars* sc;
   int Kp, K, r0, nb;
   uint32_t done;  // hand-overs of one kind in the regions before
+  uint32_t* split;
+  int split_ld;
   __device__ uint32_t* word(int which) const { return sync + which * SYNC_LINE; }
   // count of SYNC_ROW + j once `blocks` blocks of this region have arrived
   __device__ uint32_t row_target(int j, int blocks) const { return (done * j + blocks) * 16u; }
@@ -367,7 +375,19 @@ __device__ __forceinline__ void rows_below(const Region& g, RegionLds& lds, int 
     v4f sol = {0.f, 0.f, 0.f, 0.f};
     sol = tile_mm<false>(sol, operand_load(&L.S[s][0], LDD, r), operand_load(g.Xs + j * BLOCK + 16 * tc * NB, NB, r));
     tile_store(sol, own + NB * j, ld, tc, r);
-    if (j + 1 < MAX_BLOCKS) tile_store(sol, &L.R[j < MAX_BLOCKS - 1 ? j : 0][s][0], LDD, tc, r);
+    tile_store(sol, &L.R[j][s][0], LDD, tc, r);
+    if (g.split) {  // this wave's tile once more, four neighbouring columns of a row per lane
+      float one = 1.f;
+      asm("" : "+s"(one));
+      const int row = s + (r >> 2), col = 16 * tc + 4 * (r & 3);
+      const float4 x = *(const float4*)&L.R[j][row][col];
+      uint2 p0, p1;
+      split2_unscaled(x.x, x.y, one, p0.x, p1.x);
+      split2_unscaled(x.z, x.w, one, p0.y, p1.y);
+      uint32_t* const out = g.split + (int64_t)(g.r0 + NB * g.nb + ROWS * tile + row) * g.split_ld + NB * j + (col & ~7) + (col & 4) / 2;
+      *(uint2*)out = p0;
+      *(uint2*)(out + 4) = p1;
+    }
     acc = ahead;
   }
 }
@@ -394,6 +414,8 @@ __global__ __launch_bounds__(REGION_NT) void chol_region_kernel(RegionArgs a) {
   g.sc = a.sc + problem;
   g.Kp = a.Kp; g.K = a.K; g.r0 = a.r0; g.nb = a.nb;
   g.done = a.region;
+  g.split = a.split ? a.split + problem * a.split_stride : nullptr;
+  g.split_ld = a.split_ld;
   if (task < all) {
     const int role = task - problem * cores;
     if (role == 0)

@@ -35,6 +35,8 @@ struct GemmF32 {
   // 0 or 1 = none
   int batch2;
   int64_t stride2_a, stride2_b, stride2_c;
+  // llmc_gemm_x2 only: A and B hold their elements split into two f16 terms already (split2.h)
+  int split;
   // llmc_gemm_x2 only, powers of two: C = alpha * diag(row_scale)^-1 (diag(row_scale) A) (diag(k_scale) B), one k_scale
   // per index of the contraction (of the whole one when it is cut into pieces); strides per problem of batch2
   const float* row_scale;
@@ -53,7 +55,7 @@ int llmc_gemm_x3(const GemmF32& g, hipStream_t st);
 void llmc_gemm_x3_set_mode(int mode);
 
 // The product of operands whose range is known, split into two f16 terms (gemm_x2.hip): |A| and |B| (scaled, where scales
-// are given) at most 2^15, at least one element of a row that matters near 2^13.  A B^T without scales, A B with them; takes
+// are given) at most 2^15, at least one element of a row that matters near 2^13.  A B^T of operands that are split, A B with scales; takes
 // what llmc_gemm_x2_fits.
 bool llmc_gemm_x2_fits(const GemmF32& g);
 int llmc_gemm_x2(const GemmF32& g, hipStream_t st);
