@@ -9,9 +9,11 @@
 //                    columns and to its diagonal block; then hands A[b, b-1] and the diagonal block to the spine
 //   rows below       32 rows to a workgroup, two independent sets of 16: each block column solved as its X arrives
 // One launch per step, with every workgroup factoring the block for itself, and one more for the rows below took 49.8 and
-// 10.2 us for a region of a 4096-wide matrix, 4.5 us of each launch being the launch; 45 us now.  What bounds the region is
-// the spine: the 64 x 64 factor-and-invert (one wave's instruction issue, chol_block.h) and two products per step, 8.6 us.
-// Whole chains: 4096 columns 1323 -> 1114 us, 14336 9.0 -> 8.1 ms, 128 of 2048 8.16 -> 7.95 ms.
+// 10.2 us for a region of a 4096-wide matrix, 4.5 us of each launch being the launch; 39 us now.  What bounds the region is
+// the spine, 9 us a step: the 64 x 64 factor-and-invert (one wave's instruction issue, chol_block.h; 6.2 us), the solve of
+// the next row block (0.9), its part of the next diagonal block (1.2).  The tiles of that one which the first slab needs are
+// formed in the registers that factor it, the others beside it.
+// Whole chains: 4096 columns 1323 -> 1022 us, 14336 9.0 -> 8.1 ms with this form of the launches alone.
 //
 // 512 threads and at most 80 KB of LDS to a workgroup: two fit a CU, and one fits beside a workgroup of the 128-wide
 // products.  With 1024 threads and 131 KB a launch needed CUs of its own, and beside another stream's products every third
@@ -49,8 +51,9 @@ constexpr int BLOCK = NB * NB;
 constexpr int SYNC_LINE = 32;
 constexpr int SYNC_X = 0;                                // + m: X_m, 16 per region
 constexpr int SYNC_ROW = SYNC_X + MAX_BLOCKS - 1;        // + j (1..3): solved blocks (j, i), i < j, 16 each
-constexpr int SYNC_NEXT = SYNC_ROW + MAX_BLOCKS - 2;     // + b (2, 3): A[b, b-1] and diagonal block b, 16 per region
-constexpr int SYNC_TICKET = SYNC_NEXT + MAX_BLOCKS;      // of problem 0: tickets of all launches
+constexpr int SYNC_NEXT = SYNC_ROW + MAX_BLOCKS - 2;     // + b (2, 3): A[b, b-1], 16 per region
+constexpr int SYNC_DIAG = SYNC_NEXT + MAX_BLOCKS - 2;    // + b (2, 3): diagonal block b, 16 per region
+constexpr int SYNC_TICKET = SYNC_DIAG + MAX_BLOCKS;      // of problem 0: tickets of all launches
 constexpr int SYNC_WORDS = (SYNC_TICKET + 1) * SYNC_LINE;
 // floats of a problem that hold what is handed over besides X: solved blocks (j, i), then A[b, b-1] and diagonal block b
 constexpr int SIDE_NEXT = 6 * BLOCK;
@@ -78,6 +81,9 @@ struct CoreLds {
   FactorScratch fs;
   float S[NB][LDD];  // rows to be solved, then solved
 };
+struct RowBlockLds {
+  float S[2][NB][LDD];  // row block b's rows and row block m + 1's
+};
 struct RowsLds {
   float R[MAX_BLOCKS][ROWS][LDD];  // the solved block columns
   float S[ROWS][LDD];
@@ -85,6 +91,7 @@ struct RowsLds {
 struct RegionLds {
   union {
     CoreLds core;
+    RowBlockLds block;
     RowsLds rows;
   };
   int word, gave_up;
@@ -161,136 +168,172 @@ struct Region {
   __device__ uint32_t target() const { return (done + 1) * 16u; }
 };
 
+// Tiles of a 64 x 64 block, two to a wave: row w / 2, columns p and 3 - p with p = w % 2 -- a product with X_m^T, whose
+// tile column c ends after c + 1 chunks, then has the same length in every wave.
+struct WaveTiles {
+  int row, col[2];
+  __device__ explicit WaveTiles(int w) : row(w >> 1), col{w & 1, 3 - (w & 1)} {}
+  __device__ int tile(int i) const { return row * 4 + col[i]; }
+};
+// rows x X^T, X in `inverse` (row stride ld)
+__device__ __forceinline__ void solve(v4f (&sol)[2], const WaveTiles& t, const Operand64& x, const float* inverse, int ld, int lane) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    sol[i] = tile_mm<false>(v4f{0.f, 0.f, 0.f, 0.f}, x, operand_load(inverse + 16 * t.col[i] * ld, ld, lane), t.col[i] + 1);
+}
+
 __device__ __forceinline__ void spine(const Region& g, RegionLds& lds, int thread) {
   CoreLds& L = lds.core;
   const int w = __builtin_amdgcn_readfirstlane(thread >> 6);
   const int64_t ld = g.Kp;
-  {
-    const int r = thread & 63;
-    const float* src = g.A + (int64_t)(g.r0 + r) * ld + g.r0 + 8 * w;
-    factor_block_put(L.fs, *(const float4*)src, *(const float4*)(src + 4), w, r);
-  }
+  const float* const corner = g.A + (int64_t)g.r0 * ld + g.r0;
   for (int m = 0; m < g.nb; ++m) {
     const int c0 = g.r0 + NB * m;
     const bool more = m + 1 < g.nb;
     int tid = thread;
     asm("" : "+v"(tid));  // the many addresses that follow from it are formed where they are used, not kept (and spilled)
     const int r = tid & 63;
-    // What waves 4 to 7 do beside the factorisation: the row block solved last goes out, the next one (A[m+1, m] into S,
-    // the tiles on and below the diagonal of block m + 1 into registers, three or two per wave) comes in.
+    // What waves 4 to 7 do beside the factorisation: the row block solved last goes out, the next one (A[m+1, m], to be S,
+    // and the tiles on and below the diagonal of block m + 1, three or two per wave, to be fs.M) comes in.
     const int t = (tid - NT / 2) & (NT / 2 - 1), row = t >> 4, c4 = (t & 15) * 4, q = w & 3;
     auto tile_row = [](int i) { return i < 1 ? 0 : i < 3 ? 1 : i < 6 ? 2 : 3; };
     auto tile_col = [&](int i) { return i - tile_row(i) * (tile_row(i) + 1) / 2; };
+    auto tile_at = [&](const float* block, int64_t sld, int i, int j) {
+      const float4 x = *(const float4*)(block + (int64_t)(16 * i + (r & 15)) * sld + 16 * j + 4 * (r >> 4));
+      return v4f{x.x, x.y, x.z, x.w};
+    };
     float4 in0, in1, in2, in3;  // (an array ends up in scratch memory)
-    v4f dg[3];
+    v4f dg0, dg1, dg2;
     enum { WANTED, COMING, THERE };
-    int state = more ? WANTED : THERE, turn = 0;
-    uint32_t* const ready = g.word(SYNC_NEXT + m + 1);
-    auto fetch = [&]() {
-      const float* const src = m == 0 ? g.A + (int64_t)(c0 + NB) * ld + c0 : g.side + next_block(m + 1);
-      const float* const dsrc = m == 0 ? src + NB : src + BLOCK;
+    int rows_state = more ? WANTED : THERE, diag_state = rows_state, turn = 0;
+    uint32_t *const rows_ready = g.word(SYNC_NEXT + m + 1), *const diag_ready = g.word(SYNC_DIAG + m + 1);
+    auto fetch_rows = [&]() {
       const int64_t sld = m == 0 ? ld : NB;
-      const float* const at = src + row * sld + c4;
+      const float* const at = (m == 0 ? corner + NB * ld : g.side + next_block(m + 1)) + row * sld + c4;
       in0 = *(const float4*)at;
       in1 = *(const float4*)(at + 16 * sld);
       in2 = *(const float4*)(at + 32 * sld);
       in3 = *(const float4*)(at + 48 * sld);
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        const int d = min(q + 4 * i, 9);
-        dg[i] = tile_load(dsrc, sld, tile_row(d) * 4 + tile_col(d), r);
-      }
-      state = COMING;
+      rows_state = COMING;
     };
-    auto put = [&]() {
+    auto fetch_diag = [&]() {
+      const int64_t sld = m == 0 ? ld : NB;
+      const float* const at = m == 0 ? corner + NB * ld + NB : g.side + next_block(m + 1) + BLOCK;
+      dg0 = tile_at(at, sld, tile_row(q), tile_col(q));
+      dg1 = tile_at(at, sld, tile_row(q + 4), tile_col(q + 4));
+      const int d = min(q + 8, 9);
+      dg2 = tile_at(at, sld, tile_row(d), tile_col(d));
+      diag_state = COMING;
+    };
+    auto put_rows = [&]() {
       *(float4*)&L.S[row][c4] = in0;
       *(float4*)&L.S[row + 16][c4] = in1;
       *(float4*)&L.S[row + 32][c4] = in2;
       *(float4*)&L.S[row + 48][c4] = in3;
-      state = THERE;
+      rows_state = THERE;
     };
-    if (w >= 4 && m == 0 && more) fetch();
-    const int bad = factor_invert_64(L.fs, tid, [&]() {
-      if (turn == 0 && m > 0) {
-        const __amdgpu_buffer_rsrc_t out = block_rsrc(g.side + solved_block(m, m - 1));
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float4 v = *(const float4*)&L.S[row + 16 * i][c4];
-          store4_through(out, (row + 16 * i) * NB + c4, v);
-          *(float4*)(g.A + (int64_t)(c0 + row + 16 * i) * ld + c0 - NB + c4) = v;
-        }
-        publish(g.word(SYNC_ROW + m), 4, r);
+    auto await = [&](const uint32_t* word) {
+      if (!poll(word, g.target()) && r == 0) {
+        atomicExch(&g.sc->info, -1);
+        lds.gave_up = 1;
       }
-      if (state == COMING)
-        put();
-      else if (state == WANTED && reached(ready, g.target()))
-        fetch();
+    };
+    // R R^T, the solved rows' part of tile (i, j) of this step's block
+    auto less_rrt = [&](v4f d, int i, int j) {
+      return tile_mm<true>(d, operand_load(&L.S[16 * j][0], LDD, r), operand_load(&L.S[16 * i][0], LDD, r));
+    };
+    auto first = [&](int i) {
+      return m == 0 ? tile_at(corner, ld, i, 0) : less_rrt(tile_get(L.fs.tile(i, 0), r), i, 0);
+    };
+    auto beside = [&]() {
+      if (turn == 0) {
+        // the tiles that the first slab does not need: (1, 1) and (2, 2), (2, 1) and (3, 3), (3, 1), (3, 2)
+        const int i0 = q < 2 ? q + 1 : 3, j0 = q < 3 ? 1 : 2;
+        if (m == 0) {
+          const v4f x = tile_at(corner, ld, i0, j0), y = tile_at(corner, ld, 2 + (q & 1), 2 + (q & 1));
+          if (more) {
+            fetch_rows();
+            fetch_diag();
+          }
+          tile_put(x, L.fs.tile(i0, j0), r);
+          if (q < 2) tile_put(y, L.fs.tile(2 + q, 2 + q), r);
+        } else {
+          tile_put(less_rrt(tile_get(L.fs.tile(i0, j0), r), i0, j0), L.fs.tile(i0, j0), r);
+          if (q < 2) tile_put(less_rrt(tile_get(L.fs.tile(2 + q, 2 + q), r), 2 + q, 2 + q), L.fs.tile(2 + q, 2 + q), r);
+          const __amdgpu_buffer_rsrc_t out = block_rsrc(g.side + solved_block(m, m - 1));
+          float* const home = g.A + (int64_t)c0 * ld + c0 - NB;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float4 v = *(const float4*)&L.S[row + 16 * i][c4];
+            store4_through(out, (row + 16 * i) * NB + c4, v);
+            // the row blocks read what was in the first one's place
+            if (m > 1 || g.nb < 3) *(float4*)(home + (row + 16 * i) * ld + c4) = v;
+          }
+        }
+      } else {
+        if (turn == 1 && m > 0) publish(g.word(SYNC_ROW + m), 4, r);
+        if (turn == 1 && m > 1 && !more) {  // they have by now
+          const float* const src = g.side + solved_block(1, 0);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            *(float4*)((float*)corner + (NB + row + 16 * i) * ld + c4) = *(const float4*)(src + (row + 16 * i) * NB + c4);
+        }
+        if (rows_state == COMING)
+          put_rows();
+        else if (rows_state == WANTED && reached(rows_ready, g.target()))
+          fetch_rows();
+        if (diag_state == WANTED && rows_state != WANTED && reached(diag_ready, g.target())) fetch_diag();
+      }
       ++turn;
-    });
+    };
+    const int bad = factor_invert_64(L.fs, tid, first, beside);
     // first failing pivot, 1-based index in the ORIGINAL (un-reversed) ordering
     if (tid == 0 && bad < NB && c0 + bad < g.K) atomicCAS(&g.sc->info, 0, g.K - (c0 + bad));
-    {
+    if (w >= 4) {
       const __amdgpu_buffer_rsrc_t xs = block_rsrc(g.Xs + m * BLOCK);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int idx = tid + NT * i, xr = idx >> 4, xc = (idx & 15) * 4;
-        store4_through(xs, xr * NB + xc, *(const float4*)&L.fs.X[xr][xc]);
-      }
+      for (int i = 0; i < 4; ++i) store4_through(xs, (row + 16 * i) * NB + c4, *(const float4*)&L.fs.X[row + 16 * i][c4]);
+      if (!more) publish(g.word(SYNC_X + m), 4, r);
     }
-    if (!more) {
-      publish(g.word(SYNC_X + m), 2, r);
-      return;
-    }
+    if (!more) return;
     if (w >= 4) {
-      if (state == WANTED) {
-        if (!poll(ready, g.target()) && r == 0) {
-          atomicExch(&g.sc->info, -1);
-          lds.gave_up = 1;
-        }
-        fetch();
+      if (rows_state == WANTED) {
+        await(rows_ready);
+        fetch_rows();
       }
-      if (state == COMING) put();
+      if (rows_state == COMING) put_rows();
     }
     __syncthreads();
     if (lds.gave_up) return;
-    // R = S X_m^T, two tiles per wave
-    v4f sol0 = {0.f, 0.f, 0.f, 0.f}, sol1 = sol0;
-    const int st = (w >> 1) * 4 + (w & 1) * 2;
-    {
-      const Operand64 x = operand_load(&L.S[16 * (w >> 1)][0], LDD, r);
-      sol0 = tile_mm<false>(sol0, x, operand_load(&L.fs.X[32 * (w & 1)][0], LDD, r));
-      sol1 = tile_mm<false>(sol1, x, operand_load(&L.fs.X[32 * (w & 1) + 16][0], LDD, r));
-    }
+    // R = S X_m^T
+    const WaveTiles mine(w);
+    v4f sol[2];
+    solve(sol, mine, operand_load(&L.S[16 * mine.row][0], LDD, r), &L.fs.X[0][0], LDD, r);
     __syncthreads();  // every wave has read S
-    tile_store(sol0, &L.S[0][0], LDD, st, r);
-    tile_store(sol1, &L.S[0][0], LDD, st + 1, r);
-    publish(g.word(SYNC_X + m), 2, r);
-    __syncthreads();
-    // the next block less R R^T, straight to where the factorisation takes it
+#pragma unroll
+    for (int i = 0; i < 2; ++i) tile_store(sol[i], &L.S[0][0], LDD, mine.tile(i), r);
     if (w >= 4) {
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        const int d = q + 4 * i;
-        if (d > 9) continue;
-        const int ti = tile_row(d), tj = tile_col(d);
-        const v4f v = tile_mm<true>(dg[i], operand_load(&L.S[16 * ti][0], LDD, r), operand_load(&L.S[16 * tj][0], LDD, r));
-        const int c = r & 15, k = 16 * ti + 4 * (r >> 4);
-        if (tj == 0) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) L.fs.P[k + e][c] = v[e];
-        } else {
-          *(float4*)L.fs.at(16 * tj + c, k) = make_float4(v[0], v[1], v[2], v[3]);
-        }
+      publish(g.word(SYNC_X + m), 4, r);
+      if (diag_state == WANTED) {
+        await(diag_ready);
+        fetch_diag();
       }
+      tile_put(dg0, L.fs.tile(tile_row(q), tile_col(q)), r);
+      tile_put(dg1, L.fs.tile(tile_row(q + 4), tile_col(q + 4)), r);
+      if (q < 2) tile_put(dg2, L.fs.tile(tile_row(q + 8), tile_col(q + 8)), r);
     }
+    __syncthreads();
+    if (lds.gave_up) return;
   }
 }
 
-// row block b >= 2 of the region, wave w: tiles (w / 2, 2 (w % 2)) and the one beside it of every block
+// Row block b >= 2 of the region.  What the spine waits for at step b - 1 is A[b, b-1] less R_{b,b-2} R_{b-1,b-2}^T and the
+// diagonal block; the spine's own R_{b-1,b-2} would arrive a hand-over later than X_{b-2}, so it is formed here once more
+// from the same numbers.
 __device__ __forceinline__ void row_block(const Region& g, RegionLds& lds, int b, int tid) {
-  CoreLds& L = lds.core;
+  RowBlockLds& L = lds.block;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6), r = tid & 63;
-  const int tr = 16 * (w >> 1), tc = 32 * (w & 1), t0 = (w >> 1) * 4 + (w & 1) * 2;
+  const WaveTiles mine(w);
   const int64_t ld = g.Kp;
   float* const own = g.A + (int64_t)(g.r0 + NB * b) * ld + g.r0;
   v4f acc[MAX_BLOCKS - 1][2], dg[2];
@@ -298,55 +341,62 @@ __device__ __forceinline__ void row_block(const Region& g, RegionLds& lds, int b
   for (int i = 0; i < 2; ++i) {
 #pragma unroll
     for (int c = 0; c < MAX_BLOCKS - 1; ++c) {
-      if (c < b) acc[c][i] = tile_load(own + NB * c, ld, t0 + i, r);
+      if (c < b) acc[c][i] = tile_load(own + NB * c, ld, mine.tile(i), r);
     }
-    dg[i] = tile_load(own + NB * b, ld, t0 + i, r);
+    dg[i] = tile_load(own + NB * b, ld, mine.tile(i), r);
   }
+  Operand64 z = operand_load(g.A + (int64_t)(g.r0 + NB + 16 * mine.row) * ld + g.r0, ld, r);  // of A[m+1, m]
 #pragma unroll
   for (int m = 0; m < MAX_BLOCKS - 2; ++m) {
     if (m + 1 >= b) break;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) tile_store(acc[m][i], &L.S[0][0], LDD, t0 + i, r);
-    if (!wait_for(lds, g.word(SYNC_X + m), g.target(), g.sc)) return;
-    v4f sol[2];
-    {
-      const Operand64 x = operand_load(&L.S[tr][0], LDD, r);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-        sol[i] = tile_mm<false>(v4f{0.f, 0.f, 0.f, 0.f}, x, operand_load(g.Xs + m * BLOCK + (tc + 16 * i) * NB, NB, r));
+    for (int i = 0; i < 2; ++i) tile_store(acc[m][i], &L.S[0][0][0], LDD, mine.tile(i), r);
+    if (m > 0) {
+      if (!wait_for(lds, g.word(SYNC_NEXT + m + 1), g.target(), g.sc)) return;
+      z = operand_load(g.side + next_block(m + 1) + 16 * mine.row * NB, NB, r);
     }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 2; ++i) tile_store(sol[i], &L.S[0][0], LDD, t0 + i, r);
+    if (!wait_for(lds, g.word(SYNC_X + m), g.target(), g.sc)) return;
+    v4f sol[2], near[2];
+    solve(sol, mine, operand_load(&L.S[0][16 * mine.row][0], LDD, r), g.Xs + m * BLOCK, NB, r);
+    solve(near, mine, z, g.Xs + m * BLOCK, NB, r);
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
+      tile_store(sol[i], &L.S[0][0][0], LDD, mine.tile(i), r);
+      tile_store(near[i], &L.S[1][0][0], LDD, mine.tile(i), r);
+    }
+    __syncthreads();
+    const Operand64 x = operand_load(&L.S[0][16 * mine.row][0], LDD, r);
+    const bool next = m + 2 == b;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      acc[m + 1][i] = tile_mm<true>(acc[m + 1][i], x, operand_load(&L.S[1][16 * mine.col[i]][0], LDD, r));
+      if (next) tile_store_through(acc[m + 1][i], block_rsrc(g.side + next_block(b)), mine.tile(i), r);
+    }
+    if (next) publish(g.word(SYNC_NEXT + b), 2, r);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      dg[i] = tile_mm<true>(dg[i], x, operand_load(&L.S[0][16 * mine.col[i]][0], LDD, r));
+      if (next) tile_store_through(dg[i], block_rsrc(g.side + next_block(b) + BLOCK), mine.tile(i), r);
+    }
+    if (next) publish(g.word(SYNC_DIAG + b), 2, r);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
       const int idx = tid + NT * i, row = idx >> 4, c4 = (idx & 15) * 4;
-      const float4 out = *(const float4*)&L.S[row][c4];
+      const float4 out = *(const float4*)&L.S[0][row][c4];
       store4_through(block_rsrc(g.side + solved_block(b, m)), row * NB + c4, out);
       *(float4*)(own + row * ld + NB * m + c4) = out;
     }
-    const Operand64 x = operand_load(&L.S[tr][0], LDD, r);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) dg[i] = tile_mm<true>(dg[i], x, operand_load(&L.S[tc + 16 * i][0], LDD, r));
     publish(g.word(SYNC_ROW + b), 2, r);
 #pragma unroll
-    for (int c = m + 1; c < MAX_BLOCKS - 1; ++c) {
+    for (int c = m + 2; c < MAX_BLOCKS - 1; ++c) {
       if (c >= b) break;
       if (!wait_for(lds, g.word(SYNC_ROW + c), g.row_target(c, m + 1), g.sc)) return;
 #pragma unroll
       for (int i = 0; i < 2; ++i)
-        acc[c][i] = tile_mm<true>(acc[c][i], x, operand_load(g.side + solved_block(c, m) + (tc + 16 * i) * NB, NB, r));
+        acc[c][i] = tile_mm<true>(acc[c][i], x, operand_load(g.side + solved_block(c, m) + 16 * mine.col[i] * NB, NB, r));
     }
-    // (S is written again only after the waits' barriers: every wave has its operands by then)
-    if (m + 2 == b) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        tile_store_through(acc[m + 1][i], block_rsrc(g.side + next_block(b)), t0 + i, r);
-        tile_store_through(dg[i], block_rsrc(g.side + next_block(b) + BLOCK), t0 + i, r);
-      }
-      publish(g.word(SYNC_NEXT + b), 2, r);
-    }
+    if (!next) __syncthreads();  // S is written again: every wave has its operands
   }
 }
 
@@ -373,7 +423,7 @@ __device__ __forceinline__ void rows_below(const Region& g, RegionLds& lds, int 
     tile_store(acc, &L.S[s][0], LDD, tc, r);
     if (!wait_for(lds, g.word(SYNC_X + j), g.target(), g.sc)) return;
     v4f sol = {0.f, 0.f, 0.f, 0.f};
-    sol = tile_mm<false>(sol, operand_load(&L.S[s][0], LDD, r), operand_load(g.Xs + j * BLOCK + 16 * tc * NB, NB, r));
+    sol = tile_mm<false>(sol, operand_load(&L.S[s][0], LDD, r), operand_load(g.Xs + j * BLOCK + 16 * tc * NB, NB, r), tc + 1);
     tile_store(sol, own + NB * j, ld, tc, r);
     tile_store(sol, &L.R[j][s][0], LDD, tc, r);
     if (g.split) {  // this wave's tile once more, four neighbouring columns of a row per lane
