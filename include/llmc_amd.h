@@ -122,6 +122,12 @@ int64_t llmc_minmax_workspace_bytes(void);
 int llmc_minmax_groups(const void* x, int32_t dtype, int64_t R, int64_t K, int64_t ldw,
                        int64_t group, void* min_out, void* max_out, void* workspace,
                        int64_t workspace_bytes, void* stream);
+/* llmc_minmax_groups for n contiguous [R, K] matrices in one launch per 64 of them (xs: HOST array of n device pointers, 16-byte
+ * aligned) -> [n, R, K/group]; takes the shapes that llmc_minmax_groups_many_fits answers with 1 (groups of a power of two
+ * of 16-byte vectors, at most 128 of them). */
+int32_t llmc_minmax_groups_many_fits(int32_t dtype, int64_t R, int64_t K, int64_t group);
+int llmc_minmax_groups_many(const void* const* xs, int32_t n, int32_t dtype, int64_t R, int64_t K, int64_t group,
+                            void* min_out, void* max_out, void* stream);
 int llmc_minmax_blocks(const void* x, int32_t dtype, int64_t R, int64_t K, int64_t ldw,
                        int32_t block_h, int32_t block_w, void* min_out, void* max_out,
                        void* stream);

@@ -67,6 +67,34 @@ __global__ __launch_bounds__(256) void minmax_flat_kernel(const void* __restrict
   }
 }
 
+// minmax_flat_kernel for several matrices of one shape (blockIdx.y), their statistics one after the other: the weights of an
+// MoE layer's experts, 3 MB each, whose launches take 4.3 us of which the reading is one.  32 of 768 x 2048 in bf16: 137 us of
+// launches -> 22 us, 4.6 TB/s.
+constexpr int MINMAX_MANY = 64;
+struct MinmaxMany {
+  const void* x[MINMAX_MANY];
+};
+template <int DT, int VPL>
+__global__ __launch_bounds__(256) void minmax_many_kernel(MinmaxMany args, int64_t units, int lshift, void* __restrict__ mn_out,
+                                                          void* __restrict__ mx_out) {
+  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (u >= units) return;  // (whole groups: units and the lanes of one are multiples of 1 << lshift)
+  const char* const x = (const char*)args.x[blockIdx.y];
+  float mn = INFINITY, mx = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < VPL; ++k) minmax16<DT>(x + (u * VPL + k) * 16, mn, mx);
+  const int L = 1 << lshift;
+  for (int o = L >> 1; o > 0; o >>= 1) {
+    mn = fminf(mn, __shfl_xor(mn, o, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+  }
+  if ((u & (L - 1)) == 0) {
+    const int64_t g = blockIdx.y * (units >> lshift) + (u >> lshift);
+    store_from_f32<DT>(mn_out, g, mn);
+    store_from_f32<DT>(mx_out, g, mx);
+  }
+}
+
 // Groups of g = L * VPL * N elements: one workgroup walks one row, L (power of two <= 64)
 // neighbouring lanes share a group and each lane loads VPL consecutive 16-byte vectors.
 template <int DT, int VPL>
@@ -326,6 +354,37 @@ __global__ __launch_bounds__(256) void qparams_kernel(const void* __restrict__ m
   if (scale_code_out) scale_code_out[i] = scale_mode == LLMC_SCALE_MXFP4 ? (uint8_t)e : e4m3_encode(s);
 }
 
+// lanes of a group on the flat walk: 16-byte vectors, a power of two of them (at most 128) to a group
+struct FlatWalk {
+  int vpl, lshift;  // vectors per lane; lanes per group
+  bool fits;
+};
+inline FlatWalk flat_walk(int64_t R, int64_t K, int64_t g, int N) {
+  const int64_t L = g / N;  // 16-byte vectors per group
+  FlatWalk w = {L >= 2 ? 2 : 1, 0, g % N == 0 && L >= 1 && L <= 128 && (L & (L - 1)) == 0 && R <= 0x7fffffffLL && K <= (1LL << 30)};
+  while ((1 << w.lshift) < L / w.vpl) ++w.lshift;
+  return w;
+}
+
+template <int DT>
+int observe_many(const void* const* xs, int n, int64_t R, int64_t K, int64_t g, void* mn, void* mx, hipStream_t st) {
+  const FlatWalk w = flat_walk(R, K, g, Vec<DT>::N);
+  const int64_t units = R * (K / (Vec<DT>::N * w.vpl)), stats = R * (K / g) * dtype_size(DT);
+  for (int first = 0; first < n; first += MINMAX_MANY) {
+    MinmaxMany args;
+    const int m = n - first < MINMAX_MANY ? n - first : MINMAX_MANY;
+    for (int b = 0; b < m; ++b) args.x[b] = xs[first + b];
+    const dim3 grid((unsigned)((units + 255) / 256), (unsigned)m);
+    char *const mn_at = (char*)mn + first * stats, *const mx_at = (char*)mx + first * stats;
+    if (w.vpl == 2)
+      hipLaunchKernelGGL((minmax_many_kernel<DT, 2>), grid, dim3(256), 0, st, args, units, w.lshift, mn_at, mx_at);
+    else
+      hipLaunchKernelGGL((minmax_many_kernel<DT, 1>), grid, dim3(256), 0, st, args, units, w.lshift, mn_at, mx_at);
+    LLMC_LAUNCH_STATUS();
+  }
+  return 0;
+}
+
 template <int DT>
 int observe_groups(const void* x, int64_t R, int64_t K, int64_t ldw, int64_t g, void* mn, void* mx,
                    float* ws, int64_t ws_bytes, hipStream_t st) {
@@ -334,12 +393,9 @@ int observe_groups(const void* x, int64_t R, int64_t K, int64_t ldw, int64_t g, 
   const int64_t ng = K / g;
   const int64_t total = R * ng;
   const bool aligned = (((uintptr_t)x) & 15) == 0 && (ldw % N) == 0 && (g % N) == 0;
-  const int64_t L = g / N;  // 16-byte vectors per group
-  if (aligned && L >= 1 && L <= 128 && (L & (L - 1)) == 0 && R <= 0x7fffffffLL && K <= (1LL << 30)) {
-    const int vpl = L >= 2 ? 2 : 1;
-    const int lanes = (int)(L / vpl);
-    int lshift = 0;
-    while ((1 << lshift) < lanes) ++lshift;
+  const FlatWalk walk = flat_walk(R, K, g, N);
+  if (aligned && walk.fits) {
+    const int vpl = walk.vpl, lshift = walk.lshift;
     const int upr = (int)(K / (N * vpl));
     if (ldw == K) {
       const int64_t units = R * upr;
@@ -403,6 +459,23 @@ extern "C" int llmc_minmax_groups(const void* x, int32_t dtype, int64_t R, int64
   if (dtype == LLMC_BF16) return observe_groups<LLMC_BF16>(x, R, K, ldw, group, min_out, max_out, ws, workspace_bytes, st);
   if (dtype == LLMC_F16) return observe_groups<LLMC_F16>(x, R, K, ldw, group, min_out, max_out, ws, workspace_bytes, st);
   return observe_groups<LLMC_F32>(x, R, K, ldw, group, min_out, max_out, ws, workspace_bytes, st);
+}
+
+extern "C" int32_t llmc_minmax_groups_many_fits(int32_t dtype, int64_t R, int64_t K, int64_t group) {
+  if (dtype < 0 || dtype > 2 || R <= 0 || K <= 0 || group <= 0 || K % group != 0) return 0;
+  return flat_walk(R, K, group, dtype == LLMC_F32 ? 4 : 8).fits && R <= (1LL << 32) / K;
+}
+
+extern "C" int llmc_minmax_groups_many(const void* const* xs, int32_t n, int32_t dtype, int64_t R, int64_t K, int64_t group,
+                                       void* min_out, void* max_out, void* stream) {
+  LLMC_CHECK_ARG(xs != nullptr && n >= 0, 1);
+  LLMC_CHECK_ARG(llmc_minmax_groups_many_fits(dtype, R, K, group), 6);
+  LLMC_CHECK_ARG(min_out && max_out, 7);
+  for (int b = 0; b < n; ++b) LLMC_CHECK_ARG(xs[b] != nullptr && ((uintptr_t)xs[b] & 15) == 0, 1);
+  hipStream_t st = (hipStream_t)stream;
+  if (dtype == LLMC_BF16) return observe_many<LLMC_BF16>(xs, n, R, K, group, min_out, max_out, st);
+  if (dtype == LLMC_F16) return observe_many<LLMC_F16>(xs, n, R, K, group, min_out, max_out, st);
+  return observe_many<LLMC_F32>(xs, n, R, K, group, min_out, max_out, st);
 }
 
 extern "C" int llmc_minmax_blocks(const void* x, int32_t dtype, int64_t R, int64_t K, int64_t ldw,

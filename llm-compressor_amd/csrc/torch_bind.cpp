@@ -13,6 +13,7 @@
 
 #include <cmath>
 #include <tuple>
+#include <vector>
 
 #include "llmc_amd.h"
 
@@ -134,6 +135,34 @@ Pair minmax_observe(const Tensor& W, int64_t group, const optional<Tensor>& work
   check(llmc_minmax_groups(W.const_data_ptr(), dt, R, K, W.stride(0), group, mn.data_ptr(), mx.data_ptr(),
                            ws.data_ptr(), nws, stream_of(W)),
         "llmc_minmax_groups");
+  return {mn, mx};
+}
+
+// the statistics of several contiguous, 16-byte aligned matrices of one shape as [n, R, K / group]
+Pair minmax_observe_many(at::TensorList Ws, int64_t group) {
+  TORCH_CHECK_VALUE(!Ws.empty(), "minmax_observe_many: no tensors");
+  const Tensor& W = Ws[0];
+  require_rows(W);
+  const int64_t R = W.size(0), K = W.size(1);
+  TORCH_CHECK_VALUE(group > 0 && K % group == 0, "minmax_observe_many: groups of ", group, " do not divide ", K, " columns");
+  const int dt = dtype_code(W);
+  std::vector<const void*> xs;
+  xs.reserve(Ws.size());
+  for (const Tensor& t : Ws) {
+    require_beside(W, t);
+    TORCH_CHECK_VALUE(t.dim() == 2 && t.size(0) == R && t.size(1) == K && t.scalar_type() == W.scalar_type(),
+                      "minmax_observe_many: the matrices differ in shape or dtype");
+    TORCH_CHECK_VALUE(t.is_contiguous() && ((uintptr_t)t.const_data_ptr() & 15) == 0,
+                      "minmax_observe_many: a matrix is not contiguous or not 16-byte aligned");
+    xs.push_back(t.const_data_ptr());
+  }
+  TORCH_CHECK_VALUE(llmc_minmax_groups_many_fits(dt, R, K, group), "minmax_observe_many: groups of ", group,
+                    " do not fit the flat walk");
+  Guard guard(W.device());
+  const int64_t n = (int64_t)xs.size();
+  Tensor mn = at::empty({n, R, K / group}, W.options()), mx = at::empty({n, R, K / group}, W.options());
+  check(llmc_minmax_groups_many(xs.data(), (int)n, dt, R, K, group, mn.data_ptr(), mx.data_ptr(), stream_of(W)),
+        "llmc_minmax_groups_many");
   return {mn, mx};
 }
 
@@ -451,6 +480,7 @@ TORCH_LIBRARY_IMPL(llmc, CUDA, m) {
   m.impl("hessian_accum_", hessian_accum_);
   m.impl("hessian_accum_counted_", hessian_accum_counted_);
   m.impl("minmax_observe", minmax_observe);
+  m.impl("minmax_observe_many", minmax_observe_many);
   m.impl("minmax_observe_blocks", minmax_observe_blocks);
   m.impl("minmax_observe_strided", minmax_observe_strided);
   m.impl("mse_observe", mse_observe);

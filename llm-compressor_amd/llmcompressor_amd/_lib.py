@@ -76,6 +76,8 @@ SIGNATURES = {
                              _I32, _I64, _P, _P],
     "llmc_hessian_accumulate": [_P, _I64, _P, _I64, _I64, _I64, _I32, _F32, _I32, _P, _I64, _P],
     "llmc_minmax_groups": [_P, _I32, _I64, _I64, _I64, _I64, _P, _P, _P, _I64, _P],
+    "llmc_minmax_groups_many_fits": [_I32, _I64, _I64, _I64],
+    "llmc_minmax_groups_many": [_P, _I32, _I32, _I64, _I64, _I64, _P, _P, _P],
     "llmc_minmax_blocks": [_P, _I32, _I64, _I64, _I64, _I32, _I32, _P, _P, _P],
     "llmc_minmax_strided": [_P, _I32, _I64, _I64, _I64, _I64, _I64, _P, _P, _P],
     "llmc_absmax_accumulate": [_P, _P, _I64, _I32, _P, _P],

@@ -14,6 +14,7 @@ import math
 import torch
 
 from ... import ops  # noqa: F401  (format constants)
+from ...observers import Observer
 from ...torch_ops import llmc
 from ...quantization import ActivationOrdering, QuantizationArgs, QuantizationStrategy
 from ...quantization.lifecycle import effective_scale, kernel_format
@@ -278,6 +279,7 @@ def finish_weight_group(ctx, blocksize: int = 128, max_bytes: int = GROUP_MAX_BY
                          f"for block size {ctx['blocksize']}")
     prep = []
     base_g_idx = {}
+    qps = Observer.get_qparams_of([m.weight_observer for m in mods])
     for j, m in enumerate(mods):
         quant_args = m.quantization_scheme.weights
         strategy, actorder = quant_args.strategy, quant_args.actorder
@@ -298,7 +300,7 @@ def finish_weight_group(ctx, blocksize: int = 128, max_bytes: int = GROUP_MAX_BY
                     g_idx = base_g_idx[("permuted", divisor)][j]
                 else:
                     g_idx = g_idx[perm]
-        qp = m.weight_observer.get_qparams()
+        qp = qps[j]
         prep.append(dict(args=quant_args, W=W, perm=perm, g_idx=g_idx, qp=qp, row_div=row_div, srow=srow,
                          zp=None if quant_args.symmetric else qp["zero_point"].to(torch.int8),
                          kscale=effective_scale(qp["scale"], quant_args, W.dtype)))

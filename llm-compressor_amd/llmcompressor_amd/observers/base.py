@@ -98,6 +98,34 @@ def _observed_layout(value: torch.Tensor, base_name: str, args: QuantizationArgs
     raise ValueError(f"Unknown quantization base name: {base_name}")
 
 
+def _run_length(observers: List["Observer"], at: int) -> int:
+    """How many observers from ``at`` on ``Observer.get_qparams_of`` can take in one launch."""
+
+    def asks(o):  # what the parameters depend on besides the statistics; None: not for sharing
+        if (type(o).get_qparams is not Observer.get_qparams or type(o).get_global_scale is not Observer.get_global_scale
+                or "get_qparams" in o.__dict__ or "get_global_scale" in o.__dict__ or not o.has_statistics
+                or o.args.strategy == QuantizationStrategy.TENSOR_GROUP or o.fusion_handler.is_fused):
+            return None
+        mn, mx = o.min_vals, o.max_vals
+        if not (mn.is_contiguous() and mx.is_contiguous() and mn.shape == mx.shape and mn.ndim == 2 and mn.numel()):
+            return None
+        a = o.args
+        return (a.strategy, kernel_format(a), a.symmetric, scale_mode(a, False), a.zp_dtype, mn.shape, mn.dtype, mx.dtype,
+                mn.untyped_storage().data_ptr(), mx.untyped_storage().data_ptr())
+
+    n, first = 1, observers[at]
+    key = asks(first) if at + 1 < len(observers) else None
+    if key is None:
+        return 1
+    while at + n < len(observers):
+        o = observers[at + n]
+        if (asks(o) != key or any(getattr(o, name).storage_offset() != getattr(first, name).storage_offset() + n * first.min_vals.numel()
+                                  for name in ("min_vals", "max_vals"))):
+            break
+        n += 1
+    return n
+
+
 class Observer(torch.nn.Module):
     """Computes quantization parameters from observations of weights, activations or attention states."""
 
@@ -203,6 +231,25 @@ class Observer(torch.nn.Module):
         )
         self.delete_statistics()
         return {"scale": scale, "zero_point": zero_point, "global_scale": global_scale}
+
+    @staticmethod
+    def get_qparams_of(observers: List["Observer"]) -> List[QParamsDict]:
+        """``get_qparams`` of each, one launch for every run of observers whose statistics lie one after the other in one
+        tensor (weights observed together) and ask for the same parameters; they are then slices of one tensor as well."""
+        out: List[QParamsDict] = []
+        while len(out) < len(observers):
+            n = _run_length(observers, len(out))
+            if n == 1:
+                out.append(observers[len(out)].get_qparams())
+                continue
+            run = observers[len(out) : len(out) + n]
+            first = run[0]
+            stacked = [t.detach().as_strided((n, *t.shape), (t.numel(), *t.stride())) for t in (first.min_vals, first.max_vals)]
+            scale, zero_point = calculate_qparams(*stacked, quantization_args=first.args, global_scale=None)
+            for observer in run:
+                observer.delete_statistics()
+            out += [{"scale": s, "zero_point": z, "global_scale": None} for s, z in zip(scale.unbind(0), zero_point.unbind(0))]
+        return out
 
     @_without_grad
     def qparams_into(self, scale: torch.Tensor, zero_point: Optional[torch.Tensor],

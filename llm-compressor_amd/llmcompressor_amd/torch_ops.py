@@ -149,6 +149,7 @@ _SEARCH = ("int fmt, int num_bits, bool symmetric, int scale_mode=0, float maxsh
 _ISEARCH = ("float maxshrink=0.95, int patience=5, float grid=20.0, float norm=3.0, float expand=1.0) "
             "-> (Tensor min, Tensor max)")
 _register("minmax_observe(Tensor W, int group, Tensor? workspace=None) -> (Tensor min, Tensor max)")
+_register("minmax_observe_many(Tensor[] Ws, int group) -> (Tensor min, Tensor max)")
 _register("minmax_observe_blocks(Tensor W, int block_h, int block_w) -> (Tensor min, Tensor max)")
 _register("minmax_observe_strided(Tensor x, int n0, int n1, int group, int stride0, int stride1) "
           "-> (Tensor min, Tensor max)")

@@ -1,0 +1,83 @@
+"""Weights that are observed together: their statistics and parameters are those of one call each, bit for bit, and what
+cannot share a launch still goes one by one."""
+import pytest
+import torch
+
+from llmcompressor_amd.modifiers.quantization.calibration import initialize_observer, observe
+from llmcompressor_amd.observers import Observer
+from llmcompressor_amd.quantization import initialize_module_for_quantization, preset_name_to_scheme
+
+pytestmark = pytest.mark.gpu
+
+
+def _linears(shapes, preset, dtype=torch.bfloat16, group=None, seed=0):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    out = []
+    for rows, cols in shapes:
+        lin = torch.nn.Linear(cols, rows, bias=False, dtype=dtype, device="cuda")
+        lin.weight.data = (torch.randn(rows, cols, device="cuda", generator=gen) * 0.02).to(dtype)
+        scheme = preset_name_to_scheme(preset, ["Linear"])
+        if group is not None:
+            scheme.weights.group_size = group
+        initialize_module_for_quantization(lin, scheme, force_zero_point=True)
+        initialize_observer(lin, "weight")
+        out.append(lin)
+    return out
+
+
+# group widths of 1, 2, 64 and 128 vectors of 16 bytes, 256 (too wide), 3 (no power of two); a set larger than one launch
+# takes; rows whose statistics are no multiple of 16; a workgroup and one unit more; single members between the others
+@pytest.mark.parametrize("shapes,preset,dtype,group", [
+    ([(16, 64)] * 2, "W4A16", torch.bfloat16, 8),
+    ([(48, 128)] * 3, "W4A16_ASYM", torch.float16, 16),
+    ([(32, 1024)] * 2, "W4A16", torch.bfloat16, 512),
+    ([(16, 1024)] * 2, "W8A16", torch.bfloat16, None),
+    ([(16, 2048)] * 2, "W8A16", torch.bfloat16, None),
+    ([(16, 512)] * 2, "W8A16", torch.float32, None),
+    ([(16, 192)] * 2, "W4A16", torch.bfloat16, 24),
+    ([(8, 256)] * 129, "W4A16_ASYM", torch.bfloat16, 32),
+    ([(17, 128)] * 2, "W4A16", torch.bfloat16, 128),
+    ([(272, 16)] * 2, "W4A16", torch.bfloat16, 16),
+    ([(64, 256), (32, 256), (64, 256), (96, 128), (64, 256)], "W4A16", torch.bfloat16, 128),
+    ([(64, 256)] * 3, "NVFP4A16", torch.bfloat16, None),
+    ([(64, 256)] * 3, "MXFP4A16", torch.bfloat16, None),
+])
+def test_together_is_one_by_one(shapes, preset, dtype, group):
+    together, alone = (_linears(shapes, preset, dtype, group) for _ in range(2))
+    with torch.no_grad():
+        together[0].weight[0, 0] = alone[0].weight[0, 0] = float("inf")
+        together[-1].weight[-1, -1] = alone[-1].weight[-1, -1] = float("nan")
+        observe(together, "weight")
+        for m in alone:
+            observe(m, "weight")
+        for a, b in zip(together, alone):
+            for name in ("min_vals", "max_vals"):
+                x, y = getattr(a.weight_observer, name), getattr(b.weight_observer, name)
+                assert x.shape == y.shape and x.dtype == y.dtype
+                torch.testing.assert_close(x, y, rtol=0, atol=0, equal_nan=True)
+        got = Observer.get_qparams_of([m.weight_observer for m in together])
+        assert not any(m.weight_observer.has_statistics for m in together)
+        for q, m in zip(got, alone):
+            want = m.weight_observer.get_qparams()
+            for key in ("scale", "zero_point", "global_scale"):
+                if want[key] is None:
+                    assert q[key] is None
+                    continue
+                assert q[key].shape == want[key].shape and q[key].dtype == want[key].dtype
+                assert torch.equal(q[key].contiguous().view(torch.uint8), want[key].contiguous().view(torch.uint8))
+
+
+def test_what_a_call_would_do_besides_still_happens():
+    hooked, held, plain, other, repeated = _linears([(64, 256)] * 5, "W4A16")
+    seen = []
+    hooked.weight_observer.register_forward_hook(lambda *a: seen.append("hook"))
+    with torch.no_grad():
+        observe(held, "weight")
+        before = held.weight_observer.min_vals.clone()
+        held.weight.zero_()  # a weight that is observed already keeps its statistics
+        observe([hooked, held, plain, repeated, other, repeated], "weight")
+    assert seen == ["hook"]
+    assert torch.equal(held.weight_observer.min_vals, before)
+    for m in (hooked, plain, other, repeated):
+        assert torch.equal(m.weight_observer.min_vals, m.weight.view(64, 2, 128).amin(-1))
+        assert torch.equal(m.weight_observer.max_vals, m.weight.view(64, 2, 128).amax(-1))
