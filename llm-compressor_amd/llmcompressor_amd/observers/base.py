@@ -114,7 +114,12 @@ def _run_length(observers: List["Observer"], at: int) -> int:
                 mn.untyped_storage().data_ptr(), mx.untyped_storage().data_ptr())
 
     n, first = 1, observers[at]
-    key = asks(first) if at + 1 < len(observers) else None
+    if at + 1 == len(observers):
+        return 1
+    mn, following = first.__dict__.get("min_vals"), observers[at + 1].__dict__.get("min_vals")
+    if mn is None or following is None or mn.untyped_storage().data_ptr() != following.untyped_storage().data_ptr():
+        return 1  # observed one by one: nothing more to look at
+    key = asks(first)
     if key is None:
         return 1
     while at + n < len(observers):
