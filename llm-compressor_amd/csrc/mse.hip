@@ -853,39 +853,61 @@ __global__ __launch_bounds__(256) void mse_generic_kernel(MseParams p, GenericLa
   }
 }
 
-// Per group its latest improvement at or before the stop step, which every thread finds by replaying the host loop's
-// patience rule on the per-step "any group improved" flags (uniform, a few dozen scalar operations).
+// Per group its latest improvement at or before the stop step, which every wave finds by replaying the host loop's
+// patience rule on the per-step "any group improved" flags (uniform, a few dozen scalar operations).  Reads and writes 16 bytes a
+// group.  Four groups a thread, so that the replay is one for 256 groups and its flags, the masks and the ranges are on their way at
+// once, and the step's factor from the table instead of a double division: 3.7 M groups 47 -> 24 us,
+// 59 MB.
+constexpr int SELECT_GROUPS = 4;
+template <int WORDS>
 __global__ __launch_bounds__(256) void mse_select_kernel(const uint64_t* __restrict__ masks, int64_t n,
-                                                         const uint64_t* __restrict__ flags, int steps, int patience,
-                                                         double grid, int dt,
+                                                         const uint64_t* __restrict__ flags, const float* __restrict__ factors,
+                                                         int steps, int patience, int dt,
                                                          const void* __restrict__ min0,
                                                          const void* __restrict__ max0,
                                                          void* __restrict__ min_out, void* __restrict__ max_out) {
-  int no_improve = 0, last = steps - 1;
-  for (int k = 0; k < steps; ++k) {
-    if ((flags[k >> 6] >> (k & 63)) & 1ull) {
-      no_improve = 0;
-    } else if (++no_improve >= patience) {
-      last = k;
-      break;
+  __shared__ float factor[WORDS * 64];
+  uint64_t any[WORDS], mask[SELECT_GROUPS][WORDS];
+  float mn[SELECT_GROUPS], mx[SELECT_GROUPS];
+  const int64_t first = (int64_t)blockIdx.x * (256 * SELECT_GROUPS) + threadIdx.x;
+#pragma unroll
+  for (int wd = 0; wd < WORDS; ++wd) any[wd] = flags[wd];
+#pragma unroll
+  for (int j = 0; j < SELECT_GROUPS; ++j) {
+    const int64_t i = first + 256 * j < n ? first + 256 * j : n - 1;
+#pragma unroll
+    for (int wd = 0; wd < WORDS; ++wd) mask[j][wd] = masks[i * WORDS + wd];
+    mn[j] = load_rt(min0, i, dt);
+    mx[j] = load_rt(max0, i, dt);
+  }
+  if (threadIdx.x < WORDS * 64) factor[threadIdx.x] = (int)threadIdx.x < steps ? factors[threadIdx.x] : 0.f;
+  int no_improve = 0, last = -1;
+#pragma unroll
+  for (int wd = 0; wd < WORDS; ++wd) {
+    const int end = steps - wd * 64 < 64 ? steps - wd * 64 : 64;
+    for (int k = 0; k < end && last < 0; ++k) {
+      no_improve = (any[wd] >> k) & 1ull ? 0 : no_improve + 1;
+      if (no_improve >= patience) last = wd * 64 + k;
     }
   }
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  int best = -1;
-  const int words = mask_words(steps);
-  for (int wd = words - 1; wd >= 0 && best < 0; --wd) {
-    const int lo = wd * 64;
-    if (last < lo) continue;
-    uint64_t m = masks[i * words + wd];
-    if (last - lo < 63) m &= (2ull << (last - lo)) - 1ull;
-    if (m) best = lo + 63 - __clzll((long long)m);
+  if (last < 0) last = steps - 1;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < SELECT_GROUPS; ++j) {
+    const int64_t i = first + 256 * j;
+    if (i >= n) break;
+    int best = -1;
+#pragma unroll
+    for (int wd = WORDS - 1; wd >= 0; --wd) {
+      const int upto = last - wd * 64;
+      const uint64_t m = upto < 0 ? 0 : upto < 63 ? mask[j][wd] & ((2ull << upto) - 1ull) : mask[j][wd];
+      if (best < 0 && m) best = wd * 64 + 63 - __clzll((long long)m);
+    }
+    // no recorded improvement (e.g. non-finite errors): the reference keeps the un-shrunk range
+    const float pb = best < 0 ? 1.0f : factor[best];
+    store_rt(min_out, i, best < 0 ? mn[j] : round_rt(product<LLMC_F16>(mn[j], pb), dt), dt);
+    store_rt(max_out, i, best < 0 ? mx[j] : round_rt(product<LLMC_F16>(mx[j], pb), dt), dt);
   }
-  const float mn = load_rt(min0, i, dt), mx = load_rt(max0, i, dt);
-  // no recorded improvement (e.g. non-finite errors): the reference keeps the un-shrunk range
-  const float pb = best < 0 ? 1.0f : step_factor(best, grid);
-  store_rt(min_out, i, best < 0 ? mn : round_rt(product<LLMC_F16>(mn, pb), dt), dt);
-  store_rt(max_out, i, best < 0 ? mx : round_rt(product<LLMC_F16>(mx, pb), dt), dt);
 }
 
 inline int64_t align256(int64_t b) { return (b + 255) / 256 * 256; }
@@ -928,8 +950,13 @@ Workspace carve(void* ws, int64_t n) {
 int finish(const MseParams& p, const Workspace& w, int64_t n, int patience, void* min_out, void* max_out,
            hipStream_t st) {
   LLMC_LAUNCH_STATUS();
-  hipLaunchKernelGGL(mse_select_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, w.masks, n, w.flags,
-                     p.steps, patience, p.grid, p.dt, w.min0, w.max0, min_out, max_out);
+  const dim3 blocks((unsigned)((n + 256 * SELECT_GROUPS - 1) / (256 * SELECT_GROUPS)));
+  if (mask_words(p.steps) == 1)
+    hipLaunchKernelGGL((mse_select_kernel<1>), blocks, dim3(256), 0, st, w.masks, n, w.flags, w.factors, p.steps, patience, p.dt,
+                       w.min0, w.max0, min_out, max_out);
+  else
+    hipLaunchKernelGGL((mse_select_kernel<MASK_WORDS>), blocks, dim3(256), 0, st, w.masks, n, w.flags, w.factors, p.steps, patience,
+                       p.dt, w.min0, w.max0, min_out, max_out);
   LLMC_LAUNCH_STATUS();
   return 0;
 }
