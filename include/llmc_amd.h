@@ -292,6 +292,7 @@ int llmc_dynamic_per_token_quantize(const void* x, int32_t x_dtype, int64_t N, i
  * *info_out (device int, may be NULL) = 0, or the 1-based index of the first
  * non-positive pivot; in that case H becomes the identity, which is the
  * reference's round-to-nearest fallback on _LinAlgError (gptq_quantize.py:157-164).
+ * -1, with the identity as well: a wait between workgroups did not end within 20 s.
  * perm may be NULL.  workspace must be 256-byte aligned.
  *
  * form selects what H holds afterwards.  LLMC_FACTOR_INVERSE: U as above.  LLMC_FACTOR_GROUPS (K a multiple of

@@ -24,9 +24,9 @@
 // A workgroup is four waves that run the chain, one per SIMD, and four that prepare the next block meanwhile: its slice
 // of U, its scales and the part of its tiles that does not wait for the current block.
 //   16 lanes per row (16 rows per workgroup): the shortest chain, for weights that the chip takes in one pass.
-//   A 4096-row group takes 48 us (as four block launches and three update launches: 124 us).
+//   A 4096-row group takes 48 us (as four block launches and three update launches: 124 us), 51 - 58 with P and D.
 //   8 lanes per row (32 rows per workgroup): a turn has a quarter more instructions for twice the rows.  24576 rows:
-//   210 us per group (before: 314 us).
+//   210 us per group (before: 314 us), 236 with P and D.
 // Both apply the same operations to every element in the same order, so they give the same bits.
 #pragma once
 #include "common.h"

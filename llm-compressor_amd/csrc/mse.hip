@@ -855,11 +855,12 @@ __global__ __launch_bounds__(256) void mse_generic_kernel(MseParams p, GenericLa
 
 // Per group its latest improvement at or before the stop step, which every wave finds by replaying the host loop's
 // patience rule on the per-step "any group improved" flags (uniform, a few dozen scalar operations).  Reads and writes 16 bytes a
-// group.  Four groups a thread, so that the replay is one for 256 groups and its flags, the masks and the ranges are on their way at
-// once, and the step's factor from the table instead of a double division: 3.7 M groups 47 -> 24 us,
-// 59 MB.
-constexpr int SELECT_GROUPS = 4;
-template <int WORDS>
+// group.  GROUPS of them a thread, whose loads are on their way at once; the step's factor comes from the table (it was a double
+// division).  Four where that leaves every CU two workgroups, so that one replay serves 256 groups of a wave: 3.7 M groups
+// 47 -> 24 us; one below, where the waves of a CU are few and four groups after the other take longer (a whole search of 0.3 M
+// MXFP4 groups 51.4 us with four, 49.3 with one).
+constexpr int64_t SELECT_FOUR_MIN_GROUPS = 1 << 19;
+template <int WORDS, int GROUPS>
 __global__ __launch_bounds__(256) void mse_select_kernel(const uint64_t* __restrict__ masks, int64_t n,
                                                          const uint64_t* __restrict__ flags, const float* __restrict__ factors,
                                                          int steps, int patience, int dt,
@@ -867,13 +868,13 @@ __global__ __launch_bounds__(256) void mse_select_kernel(const uint64_t* __restr
                                                          const void* __restrict__ max0,
                                                          void* __restrict__ min_out, void* __restrict__ max_out) {
   __shared__ float factor[WORDS * 64];
-  uint64_t any[WORDS], mask[SELECT_GROUPS][WORDS];
-  float mn[SELECT_GROUPS], mx[SELECT_GROUPS];
-  const int64_t first = (int64_t)blockIdx.x * (256 * SELECT_GROUPS) + threadIdx.x;
+  uint64_t any[WORDS], mask[GROUPS][WORDS];
+  float mn[GROUPS], mx[GROUPS];
+  const int64_t first = (int64_t)blockIdx.x * (256 * GROUPS) + threadIdx.x;
 #pragma unroll
   for (int wd = 0; wd < WORDS; ++wd) any[wd] = flags[wd];
 #pragma unroll
-  for (int j = 0; j < SELECT_GROUPS; ++j) {
+  for (int j = 0; j < GROUPS; ++j) {
     const int64_t i = first + 256 * j < n ? first + 256 * j : n - 1;
 #pragma unroll
     for (int wd = 0; wd < WORDS; ++wd) mask[j][wd] = masks[i * WORDS + wd];
@@ -893,7 +894,7 @@ __global__ __launch_bounds__(256) void mse_select_kernel(const uint64_t* __restr
   if (last < 0) last = steps - 1;
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < SELECT_GROUPS; ++j) {
+  for (int j = 0; j < GROUPS; ++j) {
     const int64_t i = first + 256 * j;
     if (i >= n) break;
     int best = -1;
@@ -950,13 +951,15 @@ Workspace carve(void* ws, int64_t n) {
 int finish(const MseParams& p, const Workspace& w, int64_t n, int patience, void* min_out, void* max_out,
            hipStream_t st) {
   LLMC_LAUNCH_STATUS();
-  const dim3 blocks((unsigned)((n + 256 * SELECT_GROUPS - 1) / (256 * SELECT_GROUPS)));
+  auto select = [&](auto kern, int groups) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)((n + 256 * groups - 1) / (256 * groups))), dim3(256), 0, st, w.masks, n, w.flags,
+                       w.factors, p.steps, patience, p.dt, w.min0, w.max0, min_out, max_out);
+  };
+  const bool four = n >= SELECT_FOUR_MIN_GROUPS;
   if (mask_words(p.steps) == 1)
-    hipLaunchKernelGGL((mse_select_kernel<1>), blocks, dim3(256), 0, st, w.masks, n, w.flags, w.factors, p.steps, patience, p.dt,
-                       w.min0, w.max0, min_out, max_out);
+    four ? select(mse_select_kernel<1, 4>, 4) : select(mse_select_kernel<1, 1>, 1);
   else
-    hipLaunchKernelGGL((mse_select_kernel<MASK_WORDS>), blocks, dim3(256), 0, st, w.masks, n, w.flags, w.factors, p.steps, patience,
-                       p.dt, w.min0, w.max0, min_out, max_out);
+    four ? select(mse_select_kernel<MASK_WORDS, 4>, 4) : select(mse_select_kernel<MASK_WORDS, 1>, 1);
   LLMC_LAUNCH_STATUS();
   return 0;
 }
