@@ -1,5 +1,5 @@
 // Internal fp32 GEMM on the matrix cores (v_mfma_f32_32x32x2_f32), used for the
-// trailing-matrix updates of the Cholesky chain and of the GPTQ block loop.
+// chain's triangular inverse and the updates of the GPTQ and SparseGPT loops.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

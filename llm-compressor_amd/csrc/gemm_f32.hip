@@ -1,4 +1,4 @@
-// fp32 GEMM on v_mfma_f32_32x32x2_f32 for the trailing-matrix updates (Cholesky chain, GPTQ).
+// fp32 GEMM on v_mfma_f32_32x32x2_f32 for the chain's triangular inverse and the updates of the GPTQ and SparseGPT loops.
 //
 // 256 threads = 2x2 waves; a BM x BN tile of C per workgroup; the A and B slabs
 // (BK = 16 deep) are staged k-major in LDS so the per-lane MFMA operands

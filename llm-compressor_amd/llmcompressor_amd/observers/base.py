@@ -102,8 +102,8 @@ def _run_length(observers: List["Observer"], at: int) -> int:
     """How many observers from ``at`` on ``Observer.get_qparams_of`` can take in one launch."""
 
     def asks(o):  # what the parameters depend on besides the statistics; None: not for sharing
-        if (type(o).get_qparams is not Observer.get_qparams or type(o).get_global_scale is not Observer.get_global_scale
-                or "get_qparams" in o.__dict__ or "get_global_scale" in o.__dict__ or not o.has_statistics
+        if (not isinstance(o, Observer) or type(o).get_qparams is not Observer.get_qparams
+                or type(o).get_global_scale is not Observer.get_global_scale or "get_qparams" in o.__dict__ or "get_global_scale" in o.__dict__ or not o.has_statistics
                 or o.args.strategy == QuantizationStrategy.TENSOR_GROUP or o.fusion_handler.is_fused):
             return None
         mn, mx = o.min_vals, o.max_vals
@@ -116,8 +116,9 @@ def _run_length(observers: List["Observer"], at: int) -> int:
     n, first = 1, observers[at]
     if at + 1 == len(observers):
         return 1
-    mn, following = first.__dict__.get("min_vals"), observers[at + 1].__dict__.get("min_vals")
-    if mn is None or following is None or mn.untyped_storage().data_ptr() != following.untyped_storage().data_ptr():
+    mn, following = (vars(o).get("min_vals") if isinstance(o, Observer) else None for o in observers[at : at + 2])
+    if (type(mn) is not torch.Tensor or type(following) is not torch.Tensor
+            or mn.untyped_storage().data_ptr() != following.untyped_storage().data_ptr()):
         return 1  # observed one by one: nothing more to look at
     key = asks(first)
     if key is None:
