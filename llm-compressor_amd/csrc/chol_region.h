@@ -20,11 +20,11 @@
 // launch waited for one to run out (280 us).
 //
 // Handing over.  The L2s of the eight XCDs do not see each other's writes within a launch.  A producer stores with sc1
-// (through its L2, to where every XCD reads), waits for its stores and counts up a word in memory; a consumer polls that
-// word and then loads.  Its loads may use the caches: nothing that is handed over lies in a line that was touched earlier
-// in the launch by anyone but its producer (side buffers of their own; the caches start the launch without them).  One
-// hand-over of 16 KB, store to loaded, takes 1.3 us; with agent-scope fences, which write back and invalidate whole caches,
-// 3.5, and 17 with 240 workgroups listening.
+// (through its L2, to where every XCD reads), waits for its stores and counts up a word in memory that nobody else counts
+// (chol_handover.h); a consumer polls that word and then loads.  Its loads may use the caches: nothing that is handed over
+// lies in a line that was touched earlier in the launch by anyone but its producer (side buffers of their own; the caches
+// start the launch without them).  One hand-over of 16 KB, store to loaded, takes 1.3 us; with agent-scope fences, which
+// write back and invalidate whole caches, 3.5, and 17 with 240 workgroups listening.
 //
 // Progress.  A workgroup takes its task by a ticket when it starts to run, so whoever waits, waits for tasks that already
 // run or come next: the core tasks (spine, row blocks) of all problems come first, a problem's next to each other, then the
@@ -33,6 +33,7 @@
 // leaves, and the result is the identity as for any failed factorisation.
 #pragma once
 #include "chol_block.h"
+#include "chol_handover.h"
 #include "split2.h"
 
 namespace cholregion {
@@ -45,16 +46,7 @@ struct HinvScalars {
 
 constexpr int REGION_NT = NT;
 constexpr int ROWS = 32;  // of a task below the region
-constexpr int MAX_BLOCKS = 4;
 constexpr int BLOCK = NB * NB;
-// words of a problem that count hand-overs, each in a line of its own; they grow over the whole factorisation
-constexpr int SYNC_LINE = 32;
-constexpr int SYNC_X = 0;                                // + m: X_m, 16 per region
-constexpr int SYNC_ROW = SYNC_X + MAX_BLOCKS - 1;        // + j (1..3): solved blocks (j, i), i < j, 16 each
-constexpr int SYNC_NEXT = SYNC_ROW + MAX_BLOCKS - 2;     // + b (2, 3): A[b, b-1], 16 per region
-constexpr int SYNC_DIAG = SYNC_NEXT + MAX_BLOCKS - 2;    // + b (2, 3): diagonal block b, 16 per region
-constexpr int SYNC_TICKET = SYNC_DIAG + MAX_BLOCKS;      // of problem 0: tickets of all launches
-constexpr int SYNC_WORDS = (SYNC_TICKET + 1) * SYNC_LINE;
 // floats of a problem that hold what is handed over besides X: solved blocks (j, i), then A[b, b-1] and diagonal block b
 constexpr int SIDE_NEXT = 6 * BLOCK;
 constexpr int SIDE_FLOATS = SIDE_NEXT + 4 * BLOCK;
@@ -139,17 +131,25 @@ __device__ __forceinline__ bool poll(const uint32_t* word, uint32_t target) {
   } while (__builtin_readsteadycounter() - start < 2000000000ull);
   return false;
 }
-// for the whole workgroup; a barrier on either side
-__device__ __forceinline__ bool wait_for(RegionLds& L, const uint32_t* word, uint32_t target, HinvScalars* sc) {
+// for the whole workgroup, until every one of the words is there (one to a lane of the first wave, their loads in flight
+// together); a barrier on either side
+struct Awaited {
+  const uint32_t* word;
+  uint32_t target;
+};
+__device__ __forceinline__ bool wait_for(RegionLds& L, HinvScalars* sc, Awaited a, Awaited b) {
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const bool ok = poll(word, target);
-    if (!ok) atomicExch(&sc->info, -1);
-    L.gave_up = !ok;
+  if (threadIdx.x < 2) {
+    const Awaited mine = threadIdx.x == 0 ? a : b;
+    if (!poll(mine.word, mine.target)) {
+      atomicExch(&sc->info, -1);
+      L.gave_up = 1;
+    }
   }
   __syncthreads();
   return !L.gave_up;
 }
+__device__ __forceinline__ bool wait_for(RegionLds& L, HinvScalars* sc, Awaited a) { return wait_for(L, sc, a, a); }
 
 // a problem's pointers
 struct Region {
@@ -163,9 +163,12 @@ struct Region {
   uint32_t* split;
   int split_ld;
   __device__ uint32_t* word(int which) const { return sync + which * SYNC_LINE; }
-  // count of SYNC_ROW + j once `blocks` blocks of this region have arrived
-  __device__ uint32_t row_target(int j, int blocks) const { return (done * j + blocks) * 16u; }
-  __device__ uint32_t target() const { return (done + 1) * 16u; }
+  __device__ uint32_t target() const { return target_one(done); }
+  __device__ Awaited x(int m) const { return {word(word_x(m)), target()}; }
+  __device__ Awaited spine_row(int j) const { return {word(word_spine_row(j)), target()}; }
+  __device__ Awaited row(int b, int blocks) const { return {word(word_row(b)), target_row(done, b, blocks)}; }
+  __device__ Awaited next(int b) const { return {word(word_next(b)), target()}; }
+  __device__ Awaited diag(int b) const { return {word(word_diag(b)), target()}; }
 };
 
 // Tiles of a 64 x 64 block, two to a wave: row w / 2, columns p and 3 - p with p = w % 2 -- a product with X_m^T, whose
@@ -206,7 +209,7 @@ __device__ __forceinline__ void spine(const Region& g, RegionLds& lds, int threa
     v4f dg0, dg1, dg2;
     enum { WANTED, COMING, THERE };
     int rows_state = more ? WANTED : THERE, diag_state = rows_state, turn = 0;
-    uint32_t *const rows_ready = g.word(SYNC_NEXT + m + 1), *const diag_ready = g.word(SYNC_DIAG + m + 1);
+    const Awaited rows_ready = g.next(m + 1), diag_ready = g.diag(m + 1);  // (waited for from the second step on)
     auto fetch_rows = [&]() {
       const int64_t sld = m == 0 ? ld : NB;
       const float* const at = (m == 0 ? corner + NB * ld : g.side + next_block(m + 1)) + row * sld + c4;
@@ -232,8 +235,8 @@ __device__ __forceinline__ void spine(const Region& g, RegionLds& lds, int threa
       *(float4*)&L.S[row + 48][c4] = in3;
       rows_state = THERE;
     };
-    auto await = [&](const uint32_t* word) {
-      if (!poll(word, g.target()) && r == 0) {
+    auto await = [&](const Awaited& a) {
+      if (!poll(a.word, a.target) && r == 0) {
         atomicExch(&g.sc->info, -1);
         lds.gave_up = 1;
       }
@@ -271,7 +274,7 @@ __device__ __forceinline__ void spine(const Region& g, RegionLds& lds, int threa
           }
         }
       } else {
-        if (turn == 1 && m > 0) publish(g.word(SYNC_ROW + m), 4, r);
+        if (turn == 1 && m > 0) publish(g.word(word_spine_row(m)), HAND_OVER / 4, r);
         if (turn == 1 && m > 1 && !more) {  // they have by now
           const float* const src = g.side + solved_block(1, 0);
 #pragma unroll
@@ -280,9 +283,9 @@ __device__ __forceinline__ void spine(const Region& g, RegionLds& lds, int threa
         }
         if (rows_state == COMING)
           put_rows();
-        else if (rows_state == WANTED && reached(rows_ready, g.target()))
+        else if (rows_state == WANTED && reached(rows_ready.word, rows_ready.target))
           fetch_rows();
-        if (diag_state == WANTED && rows_state != WANTED && reached(diag_ready, g.target())) fetch_diag();
+        if (diag_state == WANTED && rows_state != WANTED && reached(diag_ready.word, diag_ready.target)) fetch_diag();
       }
       ++turn;
     };
@@ -293,7 +296,7 @@ __device__ __forceinline__ void spine(const Region& g, RegionLds& lds, int threa
       const __amdgpu_buffer_rsrc_t xs = block_rsrc(g.Xs + m * BLOCK);
 #pragma unroll
       for (int i = 0; i < 4; ++i) store4_through(xs, (row + 16 * i) * NB + c4, *(const float4*)&L.fs.X[row + 16 * i][c4]);
-      if (!more) publish(g.word(SYNC_X + m), 4, r);
+      if (!more) publish(g.word(word_x(m)), HAND_OVER / 4, r);
     }
     if (!more) return;
     if (w >= 4) {
@@ -313,7 +316,7 @@ __device__ __forceinline__ void spine(const Region& g, RegionLds& lds, int threa
 #pragma unroll
     for (int i = 0; i < 2; ++i) tile_store(sol[i], &L.S[0][0], LDD, mine.tile(i), r);
     if (w >= 4) {
-      publish(g.word(SYNC_X + m), 4, r);
+      publish(g.word(word_x(m)), HAND_OVER / 4, r);
       if (diag_state == WANTED) {
         await(diag_ready);
         fetch_diag();
@@ -352,10 +355,10 @@ __device__ __forceinline__ void row_block(const Region& g, RegionLds& lds, int b
 #pragma unroll
     for (int i = 0; i < 2; ++i) tile_store(acc[m][i], &L.S[0][0][0], LDD, mine.tile(i), r);
     if (m > 0) {
-      if (!wait_for(lds, g.word(SYNC_NEXT + m + 1), g.target(), g.sc)) return;
+      if (!wait_for(lds, g.sc, g.next(m + 1))) return;
       z = operand_load(g.side + next_block(m + 1) + 16 * mine.row * NB, NB, r);
     }
-    if (!wait_for(lds, g.word(SYNC_X + m), g.target(), g.sc)) return;
+    if (!wait_for(lds, g.sc, g.x(m))) return;
     v4f sol[2], near[2];
     solve(sol, mine, operand_load(&L.S[0][16 * mine.row][0], LDD, r), g.Xs + m * BLOCK, NB, r);
     solve(near, mine, z, g.Xs + m * BLOCK, NB, r);
@@ -373,13 +376,13 @@ __device__ __forceinline__ void row_block(const Region& g, RegionLds& lds, int b
       acc[m + 1][i] = tile_mm<true>(acc[m + 1][i], x, operand_load(&L.S[1][16 * mine.col[i]][0], LDD, r));
       if (next) tile_store_through(acc[m + 1][i], block_rsrc(g.side + next_block(b)), mine.tile(i), r);
     }
-    if (next) publish(g.word(SYNC_NEXT + b), 2, r);
+    if (next) publish(g.word(word_next(b)), HAND_OVER / 8, r);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       dg[i] = tile_mm<true>(dg[i], x, operand_load(&L.S[0][16 * mine.col[i]][0], LDD, r));
       if (next) tile_store_through(dg[i], block_rsrc(g.side + next_block(b) + BLOCK), mine.tile(i), r);
     }
-    if (next) publish(g.word(SYNC_DIAG + b), 2, r);
+    if (next) publish(g.word(word_diag(b)), HAND_OVER / 8, r);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       const int idx = tid + NT * i, row = idx >> 4, c4 = (idx & 15) * 4;
@@ -387,11 +390,11 @@ __device__ __forceinline__ void row_block(const Region& g, RegionLds& lds, int b
       store4_through(block_rsrc(g.side + solved_block(b, m)), row * NB + c4, out);
       *(float4*)(own + row * ld + NB * m + c4) = out;
     }
-    publish(g.word(SYNC_ROW + b), 2, r);
+    publish(g.word(word_row(b)), HAND_OVER / 8, r);
 #pragma unroll
     for (int c = m + 2; c < MAX_BLOCKS - 1; ++c) {
       if (c >= b) break;
-      if (!wait_for(lds, g.word(SYNC_ROW + c), g.row_target(c, m + 1), g.sc)) return;
+      if (!wait_for(lds, g.sc, g.row(c, m + 1))) return;
 #pragma unroll
       for (int i = 0; i < 2; ++i)
         acc[c][i] = tile_mm<true>(acc[c][i], x, operand_load(g.side + solved_block(c, m) + 16 * mine.col[i] * NB, NB, r));
@@ -414,14 +417,15 @@ __device__ __forceinline__ void rows_below(const Region& g, RegionLds& lds, int 
     if (j + 1 < g.nb) ahead = tile_load(own + NB * (j + 1), ld, tc, r);
     if (j > 0) {
       // the solved blocks arrive before the inverse of the diagonal block does
-      if (!wait_for(lds, g.word(SYNC_ROW + j), g.row_target(j, j), g.sc)) return;
+      const Awaited last = g.spine_row(j);
+      if (!wait_for(lds, g.sc, last, j > 1 ? g.row(j, j - 1) : last)) return;
 #pragma unroll
       for (int i = 0; i < j; ++i)
         acc = tile_mm<true>(acc, operand_load(&L.R[i][s][0], LDD, r),
                             operand_load(g.side + solved_block(j, i) + 16 * tc * NB, NB, r));
     }
     tile_store(acc, &L.S[s][0], LDD, tc, r);
-    if (!wait_for(lds, g.word(SYNC_X + j), g.target(), g.sc)) return;
+    if (!wait_for(lds, g.sc, g.x(j))) return;
     v4f sol = {0.f, 0.f, 0.f, 0.f};
     sol = tile_mm<false>(sol, operand_load(&L.S[s][0], LDD, r), operand_load(g.Xs + j * BLOCK + 16 * tc * NB, NB, r), tc + 1);
     tile_store(sol, own + NB * j, ld, tc, r);
@@ -449,7 +453,7 @@ __global__ __launch_bounds__(REGION_NT) void chol_region_kernel(RegionArgs a) {
   const int cores = core_tasks(a.nb), all = a.n * cores;
   auto problem_of = [&](int task) { return task < all ? task / cores : (task - all) / a.tiles; };
   if (tid == 0) {
-    const int task = (int)(atomicAdd(a.sync + SYNC_TICKET * SYNC_LINE, 1u) - a.ticket0);
+    const int task = (int)(atomicAdd(a.sync + WORD_TICKET * SYNC_LINE, 1u) - a.ticket0);
     lds.word = task;
     lds.gave_up = a.sc[problem_of(task)].info < 0;  // in an earlier region
   }
