@@ -292,7 +292,8 @@ int llmc_dynamic_per_token_quantize(const void* x, int32_t x_dtype, int64_t N, i
  * *info_out (device int, may be NULL) = 0, or the 1-based index of the first
  * non-positive pivot; in that case H becomes the identity, which is the
  * reference's round-to-nearest fallback on _LinAlgError (gptq_quantize.py:157-164).
- * -1, with the identity as well: a wait between workgroups did not end within 20 s.
+ * -1, with the identity as well: a wait between workgroups did not end within 20 s (wait_us <= 20 s in the call that takes it).
+ * That is a fault of the machine or of this library, not of H: do not go on with the result.
  * perm may be NULL.  workspace must be 256-byte aligned.
  *
  * form selects what H holds afterwards.  LLMC_FACTOR_INVERSE: U as above.  LLMC_FACTOR_GROUPS (K a multiple of
@@ -318,6 +319,9 @@ int64_t llmc_gptq_hinv_workspace_bytes(int64_t K);
 int llmc_gptq_hinv(float* H, int64_t ldh, int64_t K, const int32_t* perm, float divisor,
                    float percdamp, int32_t form, uint8_t* dead_out, void* workspace,
                    int64_t workspace_bytes, int32_t* info_out, void* stream);
+int llmc_gptq_hinv_within(float* H, int64_t ldh, int64_t K, const int32_t* perm, float divisor,
+                          float percdamp, int32_t form, uint8_t* dead_out, void* workspace,
+                          int64_t workspace_bytes, int32_t* info_out, int64_t wait_us, void* stream);
 
 /* Column order of GPTQ's activation ordering (gptq_quantize.py:131-140: argsort of diag(H), descending): for each of
  * the n Hessians (HOST array of n device pointers, fp32 [K, K], row stride ldh) the column numbers ordered by

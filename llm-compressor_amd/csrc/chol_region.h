@@ -26,11 +26,13 @@
 // start the launch without them).  One hand-over of 16 KB, store to loaded, takes 1.3 us; with agent-scope fences, which
 // write back and invalidate whole caches, 3.5, and 17 with 240 workgroups listening.
 //
-// Progress.  A workgroup takes its task by a ticket when it starts to run, so whoever waits, waits for tasks that already
-// run or come next: the core tasks (spine, row blocks) of all problems come first, a problem's next to each other, then the
-// rows below.  A launch holds at most two workgroups whose partners have not started, whatever else occupies the chip.  A
-// wait that has not ended after 20 s (it cannot, short of a fault) gives up: info becomes -1, every task of the problem
-// leaves, and the result is the identity as for any failed factorisation.
+// Progress.  A workgroup takes its task by a ticket when it starts to run.  The core tasks of all problems come first, a
+// problem's next to each other: spine, row block 2, row block 3; then the rows below.  Row blocks and rows below wait for
+// smaller tickets of their problem, but the spine waits for the next one or two, which may not have started.  So of the chip's
+// 512 places a launch holds at most two (a spine's and a row block's, the last that started) that do not come free by
+// themselves, and the next workgroups find one as long as there are more places than two for each launch that runs beside
+// others.  A wait that lasts longer than its limit (20 s) gives up: info becomes -1, every task of the problem leaves, and the
+// result is the identity.  Callers raise then: it is no property of the matrix.
 #pragma once
 #include "chol_block.h"
 #include "chol_handover.h"
@@ -62,6 +64,7 @@ struct RegionArgs {
   int n, tiles;        // problems; sets of ROWS rows below the region
   uint32_t ticket0;    // tickets of the launches before
   uint32_t region;     // regions before this one, all of MAX_BLOCKS blocks
+  uint64_t wait_ticks; // how long a wait may last
   // where the rows below go as two f16 terms as well (split2.h), for the updates that read them, or NULL: row i of the
   // matrix at i * split_ld, one set every split_stride words
   uint32_t* split;
@@ -121,35 +124,21 @@ __device__ __forceinline__ bool reached(const uint32_t* word, uint32_t target) {
   asm volatile("" ::: "memory");  // what is loaded next is loaded after the word
   return there;
 }
+constexpr uint64_t TICKS_PER_US = 100;  // of the steady counter
 // false: gave up
-__device__ __forceinline__ bool poll(const uint32_t* word, uint32_t target) {
+__device__ __forceinline__ bool poll(const uint32_t* word, uint32_t target, uint64_t ticks) {
   if (reached(word, target)) return true;
-  const uint64_t start = __builtin_readsteadycounter();  // 100 MHz
+  const uint64_t start = __builtin_readsteadycounter();
   do {
     __builtin_amdgcn_s_sleep(2);
     if (reached(word, target)) return true;
-  } while (__builtin_readsteadycounter() - start < 2000000000ull);
+  } while (__builtin_readsteadycounter() - start < ticks);
   return false;
 }
-// for the whole workgroup, until every one of the words is there (one to a lane of the first wave, their loads in flight
-// together); a barrier on either side
 struct Awaited {
   const uint32_t* word;
   uint32_t target;
 };
-__device__ __forceinline__ bool wait_for(RegionLds& L, HinvScalars* sc, Awaited a, Awaited b) {
-  __syncthreads();
-  if (threadIdx.x < 2) {
-    const Awaited mine = threadIdx.x == 0 ? a : b;
-    if (!poll(mine.word, mine.target)) {
-      atomicExch(&sc->info, -1);
-      L.gave_up = 1;
-    }
-  }
-  __syncthreads();
-  return !L.gave_up;
-}
-__device__ __forceinline__ bool wait_for(RegionLds& L, HinvScalars* sc, Awaited a) { return wait_for(L, sc, a, a); }
 
 // a problem's pointers
 struct Region {
@@ -160,6 +149,7 @@ struct Region {
   HinvScalars* sc;
   int Kp, K, r0, nb;
   uint32_t done;  // hand-overs of one kind in the regions before
+  uint64_t wait_ticks;
   uint32_t* split;
   int split_ld;
   __device__ uint32_t* word(int which) const { return sync + which * SYNC_LINE; }
@@ -170,6 +160,22 @@ struct Region {
   __device__ Awaited next(int b) const { return {word(word_next(b)), target()}; }
   __device__ Awaited diag(int b) const { return {word(word_diag(b)), target()}; }
 };
+
+// for the whole workgroup, until both are there (one to a lane of the first wave, their loads in flight together); a barrier
+// on either side
+__device__ __forceinline__ bool wait_for(const Region& g, RegionLds& L, Awaited a, Awaited b) {
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    const Awaited mine = threadIdx.x == 0 ? a : b;
+    if (!poll(mine.word, mine.target, g.wait_ticks)) {
+      atomicExch(&g.sc->info, -1);
+      L.gave_up = 1;
+    }
+  }
+  __syncthreads();
+  return !L.gave_up;
+}
+__device__ __forceinline__ bool wait_for(const Region& g, RegionLds& L, Awaited a) { return wait_for(g, L, a, a); }
 
 // Tiles of a 64 x 64 block, two to a wave: row w / 2, columns p and 3 - p with p = w % 2 -- a product with X_m^T, whose
 // tile column c ends after c + 1 chunks, then has the same length in every wave.
@@ -236,7 +242,7 @@ __device__ __forceinline__ void spine(const Region& g, RegionLds& lds, int threa
       rows_state = THERE;
     };
     auto await = [&](const Awaited& a) {
-      if (!poll(a.word, a.target) && r == 0) {
+      if (!poll(a.word, a.target, g.wait_ticks) && r == 0) {
         atomicExch(&g.sc->info, -1);
         lds.gave_up = 1;
       }
@@ -355,10 +361,10 @@ __device__ __forceinline__ void row_block(const Region& g, RegionLds& lds, int b
 #pragma unroll
     for (int i = 0; i < 2; ++i) tile_store(acc[m][i], &L.S[0][0][0], LDD, mine.tile(i), r);
     if (m > 0) {
-      if (!wait_for(lds, g.sc, g.next(m + 1))) return;
+      if (!wait_for(g, lds, g.next(m + 1))) return;
       z = operand_load(g.side + next_block(m + 1) + 16 * mine.row * NB, NB, r);
     }
-    if (!wait_for(lds, g.sc, g.x(m))) return;
+    if (!wait_for(g, lds, g.x(m))) return;
     v4f sol[2], near[2];
     solve(sol, mine, operand_load(&L.S[0][16 * mine.row][0], LDD, r), g.Xs + m * BLOCK, NB, r);
     solve(near, mine, z, g.Xs + m * BLOCK, NB, r);
@@ -394,7 +400,7 @@ __device__ __forceinline__ void row_block(const Region& g, RegionLds& lds, int b
 #pragma unroll
     for (int c = m + 2; c < MAX_BLOCKS - 1; ++c) {
       if (c >= b) break;
-      if (!wait_for(lds, g.sc, g.row(c, m + 1))) return;
+      if (!wait_for(g, lds, g.row(c, m + 1))) return;
 #pragma unroll
       for (int i = 0; i < 2; ++i)
         acc[c][i] = tile_mm<true>(acc[c][i], x, operand_load(g.side + solved_block(c, m) + 16 * mine.col[i] * NB, NB, r));
@@ -418,14 +424,14 @@ __device__ __forceinline__ void rows_below(const Region& g, RegionLds& lds, int 
     if (j > 0) {
       // the solved blocks arrive before the inverse of the diagonal block does
       const Awaited last = g.spine_row(j);
-      if (!wait_for(lds, g.sc, last, j > 1 ? g.row(j, j - 1) : last)) return;
+      if (!wait_for(g, lds, last, j > 1 ? g.row(j, j - 1) : last)) return;
 #pragma unroll
       for (int i = 0; i < j; ++i)
         acc = tile_mm<true>(acc, operand_load(&L.R[i][s][0], LDD, r),
                             operand_load(g.side + solved_block(j, i) + 16 * tc * NB, NB, r));
     }
     tile_store(acc, &L.S[s][0], LDD, tc, r);
-    if (!wait_for(lds, g.sc, g.x(j))) return;
+    if (!wait_for(g, lds, g.x(j))) return;
     v4f sol = {0.f, 0.f, 0.f, 0.f};
     sol = tile_mm<false>(sol, operand_load(&L.S[s][0], LDD, r), operand_load(g.Xs + j * BLOCK + 16 * tc * NB, NB, r), tc + 1);
     tile_store(sol, own + NB * j, ld, tc, r);
@@ -468,6 +474,7 @@ __global__ __launch_bounds__(REGION_NT) void chol_region_kernel(RegionArgs a) {
   g.sc = a.sc + problem;
   g.Kp = a.Kp; g.K = a.K; g.r0 = a.r0; g.nb = a.nb;
   g.done = a.region;
+  g.wait_ticks = a.wait_ticks;
   g.split = a.split ? a.split + problem * a.split_stride : nullptr;
   g.split_ld = a.split_ld;
   if (task < all) {

@@ -90,6 +90,7 @@ SIGNATURES = {
 SIGNATURES.update({
     "llmc_gptq_hinv_workspace_bytes": [_I64],
     "llmc_gptq_hinv": [_P, _I64, _I64, _P, _F32, _F32, _I32, _P, _P, _I64, _P, _P],
+    "llmc_gptq_hinv_within": [_P, _I64, _I64, _P, _F32, _F32, _I32, _P, _P, _I64, _P, _I64, _P],
     "llmc_gptq_factor_form": [_I64, _I32],
     "llmc_gptq_quantize_form": [_I64, _I32],
     "llmc_gptq_quantize_form_rows": [_I64, _I64, _I32],

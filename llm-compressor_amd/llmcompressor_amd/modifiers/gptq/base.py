@@ -392,7 +392,8 @@ class GPTQModifier(Modifier, QuantizationMixin, HessianStagingMixin):
 
     def _finish_sets(self, launched, consumed_on=None):
         # one host wait for everything enqueued so far
-        failed = torch.cat([torch.stack([r[2] for r in results]) for _, _, results in launched]).tolist()
+        infos = torch.cat([torch.stack([r[2] for r in results]) for _, _, results in launched]).tolist()
+        failed = [ops.factorisation_failed(i) for i in infos]  # (raises before any module is changed)
         at = 0
         for part, names, results in launched:
             for m, name, (loss, q_param_dict, _) in zip(part, names, results):

@@ -139,7 +139,7 @@ def quantize_weight_tensors(weight: torch.Tensor, observer, quant_args: Quantiza
     kscale = effective_scale(scale, quant_args, final_dtype)
     Wq, loss = llmc.gptq_quantize(W2, U, kscale, zp, fmt, bits, row_div, srow, g_idx=g_idx, perm=perm, dead=dead,
                                   global_scale=global_scale, blocksize=blocksize, form=form)
-    if int(info.item()) != 0:
+    if ops.factorisation_failed(int(info.item())):
         logger.warning("Failed to invert hessian due to numerical instability. Consider increasing "
                        "GPTQModifier.dampening_frac, increasing the number of calibration samples, or shuffling "
                        "the calibration dataset. Falling back to round-to-nearest for this module.")
@@ -214,7 +214,7 @@ def quantize_weight_group(modules, hessians, hessian_divisors, blocksize: int = 
     and one lock-step column loop per set of equal shape and scheme, instead of a chain of small kernels per
     module.  Same results as calling ``quantize_weight`` on each.  ``max_bytes`` bounds the factors and the column loops'
     work buffers (those of one problem are never split).  Returns a list of
-    (loss tensor, q_param_dict, info tensor) in the order of ``modules``."""
+    (loss tensor, q_param_dict, info tensor) in the order of ``modules``; ``ops.factorisation_failed`` reads the last."""
     return finish_weight_group(begin_weight_group(modules, hessians, hessian_divisors, percdamp, blocksize),
                                blocksize, max_bytes)
 

@@ -88,7 +88,7 @@ def sparsify_weight(module: torch.nn.Module, hessians_dict: dict, sparsity: floa
         W = W.t()
     loss, Q, info = sparsify_weight_tensors(W, H, sparsity, prune_n, prune_m, block_size, dampening_frac,
                                             preserve_sparsity_mask, num_samples)
-    if int(info.item()) != 0:
+    if ops.factorisation_failed(int(info.item())):
         logger.warning("Failed to invert hessian due to numerical instability. Consider increasing "
                        "SparseGPTModifier.dampening_frac, increasing the number of calibration samples, or "
                        "shuffling the calibration dataset")

@@ -274,10 +274,20 @@ def gptq_quantize_form(K: int, blocksize: int = 128, rows: int = 0) -> int:
     return int(_lib.lib().llmc_gptq_quantize_form_rows(int(rows), int(K), int(blocksize)))
 
 
-def gptq_hinv_(H: torch.Tensor, perm=None, divisor: float = 1.0, percdamp: float = 0.01, form: int = FACTOR_INVERSE):
+def factorisation_failed(info: int) -> bool:
+    """What a caller does with the ``info`` of the calls below: True = a pivot was not positive and the factor is the identity.
+    A negative one says that the chain's workgroups lost each other, which is no property of the Hessian: raises."""
+    if info < 0:
+        raise RuntimeError(f"The Cholesky chain gave up waiting for one of its own workgroups (info = {info}); its factor is not "
+                           "valid. This is a fault of the GPU or of the library, not of the calibration data.")
+    return info > 0
+
+
+def gptq_hinv_(H: torch.Tensor, perm=None, divisor: float = 1.0, percdamp: float = 0.01, form: int = FACTOR_INVERSE,
+               wait_us: int = 20_000_000):
     """In place: H -> upper factor U of (H/divisor [permuted] + damping)^-1; with form = FACTOR_GROUPS only inside
     the 512-column diagonal blocks (aligned to the last column), the upper Cholesky factor of the damped H itself
-    outside them.
+    outside them.  ``wait_us`` bounds each wait between the chain's workgroups.
 
     Returns (U (= H), dead uint8 [K], info int32 [1] on device)."""
     _require_gpu(H, perm)
@@ -290,9 +300,9 @@ def gptq_hinv_(H: torch.Tensor, perm=None, divisor: float = 1.0, percdamp: float
     nbytes = _lib.lib().llmc_gptq_hinv_workspace_bytes(K)
     ws = _workspace(H.device, nbytes)
     with torch.cuda.device(H.device):
-        rc = _lib.lib().llmc_gptq_hinv(H.data_ptr(), H.stride(0), K, _ptr(perm), float(divisor), float(percdamp),
-                                       int(form), dead.data_ptr(), ws.data_ptr(), ws.numel(), info.data_ptr(),
-                                       _stream(H))
+        rc = _lib.lib().llmc_gptq_hinv_within(H.data_ptr(), H.stride(0), K, _ptr(perm), float(divisor), float(percdamp),
+                                              int(form), dead.data_ptr(), ws.data_ptr(), ws.numel(), info.data_ptr(),
+                                              int(wait_us), _stream(H))
     _lib.check(rc, "llmc_gptq_hinv")
     return H, dead, info
 

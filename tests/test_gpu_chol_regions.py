@@ -88,3 +88,19 @@ def test_replayed_from_a_graph():
         want = ops.gptq_hinv_(src.clone())[0]
         torch.cuda.synchronize()
         assert int(info) == 0 and torch.equal(U, want)
+
+
+# one region, whose row blocks wait; one with rows below it; regions after the one that gives up
+@pytest.mark.parametrize("K", [320, 256, 1088])
+def test_waits_that_give_up_end_the_call(K):
+    """With no time to wait every task leaves, the result is the identity and info -1; the next call is as ever."""
+    from llmcompressor_amd import ops
+
+    H = _hessian(K, K)
+    want = ops.gptq_hinv_(H.clone())[0]
+    U, _, info = ops.gptq_hinv_(H.clone(), wait_us=0)
+    assert int(info) == -1 and torch.equal(U, torch.eye(K, device="cuda"))
+    with pytest.raises(RuntimeError, match="gave up waiting"):
+        ops.factorisation_failed(int(info))
+    again, _, info = ops.gptq_hinv_(H.clone())
+    assert int(info) == 0 and torch.equal(again, want)
