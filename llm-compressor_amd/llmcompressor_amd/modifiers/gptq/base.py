@@ -13,7 +13,7 @@ import logging
 import torch
 from pydantic import PrivateAttr
 
-from ... import ops  # noqa: F401
+from ... import ops
 from ...torch_ops import llmc
 from ...core import Event, State
 from ...observers import ACTIVATION_OBS
@@ -351,8 +351,8 @@ class GPTQModifier(Modifier, QuantizationMixin, HessianStagingMixin):
             if len(members) < max(2, self.group_min_modules):
                 continue
             K = members[0].weight.shape[1]
-            # factors + the chain's work matrices: about 10 K^2 bytes per problem (finish_weight_group bounds the loops')
-            per_call = max(1, min(len(members), int(self.group_max_bytes // (10 * K * K))))
+            # what the chain allocates; no further problem takes more than one by itself (finish_weight_group bounds the loops')
+            per_call = max(1, min(len(members), int(self.group_max_bytes // ops.gptq_hinv_grouped_bytes(1, K))))
             for i in range(0, len(members), per_call):
                 part = members[i:i + per_call]
                 planned.append(part if len(part) > 1 else part[0])

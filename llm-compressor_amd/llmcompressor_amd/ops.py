@@ -341,6 +341,11 @@ def gptq_hinv_grouped(Hs, perms=None, divisors=None, percdamp: float = 0.01, for
     return U, dead, info
 
 
+def gptq_hinv_grouped_bytes(n: int, columns: int) -> int:
+    """What gptq_hinv_grouped allocates for n Hessians: the factors and the chain's workspace."""
+    return 4 * n * columns * columns + int(_lib.lib().llmc_gptq_hinv_grouped_workspace_bytes(int(n), int(columns)))
+
+
 def gptq_quantize(weight, U, scale, zero_point, fmt: int, bits: int, row_div: int, scale_row_stride: int,
                   g_idx=None, perm=None, dead=None, global_scale=None, blocksize: int = 128,
                   form: int = FACTOR_INVERSE):

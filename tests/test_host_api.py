@@ -567,9 +567,32 @@ def test_linearize_moe_keeps_the_function(transposed, bias):
     assert torch.allclose(got, want, atol=1e-4, rtol=1e-4)
 
 
+@pytest.mark.parametrize("K", [64, 100, 128, 256, 512, 2048, 8192, 14336])
+def test_gptq_chains_of_a_job_stay_within_their_memory(monkeypatch, K):
+    """A job's chain allocates no more than ``group_max_bytes``, counted by the library, whose hand-over blocks and split panels
+    weigh most in narrow problems (10 K^2 bytes, the sum of factor and work matrices, were 1/7 of it at 64 columns)."""
+    from llmcompressor_amd import ops
+    from llmcompressor_amd.modifiers.gptq import GPTQModifier
+
+    workspace = int(ops._lib.lib().llmc_gptq_hinv_grouped_workspace_bytes(1, K))
+    assert ops.gptq_hinv_grouped_bytes(1, K) == 4 * K * K + workspace
+    mod = GPTQModifier(targets="Linear", scheme="W4A16", group_min_modules=2)
+    members = [torch.nn.Linear(K, 8, bias=False, device="meta") for _ in range(40)]
+    for m in members:
+        m.quantization_scheme = preset_name_to_scheme("W8A16", ["Linear"])
+        mod._hessians[m] = None
+    monkeypatch.setattr("llmcompressor_amd.modifiers.gptq.base.width_key", lambda m, args, H: K)
+    for room in (1, 2, 7, 39.5):
+        mod.group_max_bytes = int(room * ops.gptq_hinv_grouped_bytes(1, K))
+        sizes = [len(j) if isinstance(j, list) else 1 for j in mod._plan_jobs(list(members))]
+        assert sum(sizes) == 40 and max(sizes) == int(room)
+        assert ops.gptq_hinv_grouped_bytes(max(sizes), K) <= mod.group_max_bytes
+
+
 def test_gptq_job_planning():
     """compress_module_list plans lock-step sets by input width: at least ``group_min_modules`` Linears of one width
     form a set (split so that a set's work buffers stay within ``group_max_bytes``), the rest go one by one."""
+    from llmcompressor_amd import ops
     from llmcompressor_amd.modifiers.gptq import GPTQModifier
     from llmcompressor_amd.quantization import QuantizationArgs, QuantizationScheme
 
@@ -599,7 +622,7 @@ def test_gptq_job_planning():
     mod.group_min_modules = 2
     plan = mod._plan_jobs(list(mods))
     assert [len(j) for j in plan if isinstance(j, list)] == [4, 2]
-    mod.group_max_bytes = 10 * 64 * 64 * 3                   # room for three width-64 problems per job
+    mod.group_max_bytes = 3 * ops.gptq_hinv_grouped_bytes(1, 64)   # room for three width-64 problems per job
     plan = mod._plan_jobs(list(mods))
     assert [len(j) if isinstance(j, list) else 1 for j in plan][:2] == [3, 1]
     mod.group_min_modules = 0
