@@ -13,13 +13,14 @@ pytestmark = pytest.mark.gpu
 def test_groups_against_the_inverse_factor(R, K, sym, n):
     from llmcompressor_amd import ops
 
+    whole = -(-R // 32) * 32  # the last workgroup filled up with other rows; R and this have the same padding and pieces
     g = torch.Generator(device="cuda").manual_seed(R + K)
     Hs, ws, scales, zps = [], [], [], []
     for _ in range(n):
         x = torch.randn(3 * K, K, device="cuda", generator=g) * torch.logspace(-0.5, 0.5, K, device="cuda").flip(0)
         Hs.append((x.T @ x) / (3 * K))
-        w = (torch.randn(R, K, device="cuda", generator=g) * 0.02).bfloat16()
-        blocks = w.float().view(R, K // 128, 128)
+        w = (torch.randn(whole, K, device="cuda", generator=g) * 0.02).bfloat16()
+        blocks = w.float().view(whole, K // 128, 128)
         if sym:
             scales.append((blocks.abs().amax(-1) / 7.5).bfloat16())
             zps.append(None)
@@ -29,21 +30,40 @@ def test_groups_against_the_inverse_factor(R, K, sym, n):
             zps.append((-8 - low / scales[-1].float()).round().clamp(-8, 7).to(torch.int8))
         ws.append(w)
     gi = torch.arange(K, dtype=torch.int32, device="cuda") // 128
-    out = {}
-    for form in (ops.FACTOR_INVERSE, ops.FACTOR_GROUPS):
-        U, dead, info = ops.gptq_hinv_grouped(Hs, None, [1.0] * n, form=form)
-        assert not info.any()
+
+    def quantize(form, first, last):
+        """The column loop on rows [first, last) of every weight -> codes' values, losses."""
+        w, s, z = ([None if t is None else t[first:last].contiguous() for t in ts] for ts in (ws, scales, zps))
         if n == 1:
-            q, loss = ops.gptq_quantize(ws[0], U[0], scales[0], zps[0], ops.FMT_INT, 4, 1, K // 128, g_idx=gi, dead=dead[0],
-                                        form=form)
-            out[form] = [q], loss
-        else:
-            out[form] = ops.gptq_quantize_grouped(ws, U, scales, None if sym else zps, ops.FMT_INT, 4, 1, K // 128,
-                                                  g_idxs=[gi] * n, dead=dead, form=form)
-    (a, la), (b, lb) = out.values()
+            q, loss = ops.gptq_quantize(w[0], U[0], s[0], z[0], ops.FMT_INT, 4, 1, K // 128, g_idx=gi, dead=dead[0], form=form)
+            return [q], loss
+        return ops.gptq_quantize_grouped(w, U, s, None if sym else z, ops.FMT_INT, 4, 1, K // 128, g_idxs=[gi] * n, dead=dead,
+                                         form=form)
+
+    U, dead, info = ops.gptq_hinv_grouped(Hs, None, [1.0] * n, form=ops.FACTOR_INVERSE)
+    assert not info.any()
+    # a row's loss is a sum of squared rounding errors, uniform ones, over the squared diagonal of U
+    weight = U.diagonal(dim1=1, dim2=2).double().pow(-2)
+    a, la = quantize(ops.FACTOR_INVERSE, 0, R)
+    U, dead, info = ops.gptq_hinv_grouped(Hs, None, [1.0] * n, form=ops.FACTOR_GROUPS)
+    assert not info.any()
+    b, lb = quantize(ops.FACTOR_GROUPS, 0, R)
     assert torch.allclose(la, lb, rtol=2e-3)
     # each form's codes are those of a 64-bit loop up to a share of 0.1 %, which is less than one row here: a row that
     # meets a rounding boundary differs in about a third of what follows
     for x, y in zip(a, b):
         differ = x != y
         assert differ.float().mean().item() <= 2e-3 or differ.any(1).sum().item() <= 1
+    # and every row's error is that of a row quantised well, also where the codes took another path: a mean of squares of uniform
+    # errors varies by sqrt(4 / 5 / (their effective number)), the difference of two by sqrt(2) that; 6 times it
+    for x, y, w, H, v in zip(a, b, ws, Hs, weight):
+        ex, ey = (((w[:R].double() - q.double()) @ H.double() * (w[:R].double() - q.double())).sum(1) for q in (x, y))
+        spread = (1.6 * v.square().sum().item()) ** 0.5 / v.sum().item()
+        assert ((ey / ex - 1).abs().max().item()) <= 6 * spread
+    # a row does not depend on its neighbours: the same bits as in a workgroup without empty rows, and its share of the loss
+    full, lfull = quantize(ops.FACTOR_GROUPS, 0, whole)
+    for x, y in zip(b, full):
+        assert torch.equal(x, y[:R])
+    if whole > R:
+        _, rest = quantize(ops.FACTOR_GROUPS, R, whole)
+        assert (((lfull - lb - rest) / lfull).abs() * whole).max().item() <= 0.5
