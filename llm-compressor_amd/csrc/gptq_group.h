@@ -498,7 +498,7 @@ __global__ __launch_bounds__(Q_THREADS) void gptq_group_kernel(GptqGroupParams p
   float* const Us = qsmem;                       // slice of U of this block
   float* const Ds = Us + Q_U;                    // its column constants
   float* const Es = Ds + Q_D;                    // P, then P plus the errors of the finished blocks
-  float* const Ws = Es + ROWS * Q_LDS_E;         // the block's values after the group's earlier errors
+  float* const Ws = Es + ROWS * Q_LDS_E;         // what the block's values owe to earlier columns, to be added to them
   float* const Ss = Ws + ROWS * Q_LDS_W;         // scales
   int8_t* const Zs = (int8_t*)(Ss + ROWS * Q_LDS_W);  // zero points (HAS_ZP only)
   if (p.items) {

@@ -663,6 +663,18 @@ def test_gptq_loops_of_a_group_stay_within_their_memory(count, rows, K):
             assert len(runs) == 1 or bytes_of(-(-count // (len(runs) - 1))) > budget
 
 
+@pytest.mark.parametrize("rows,K,pieces", [(1, 1024, 1), (300, 2048, 3), (4096, 4096, 7), (768, 14336, 16)])
+def test_gptq_loop_takes_the_work_buffers_of_its_form(rows, K, pieces):
+    """Per row and in floats: the work copy and, on the inverse factor, a group's 512 errors; on the factor in groups D and the
+    pieces of the far product instead.  The rest (losses, scales, alignment) is small."""
+    from llmcompressor_amd import ops
+
+    padded = -(-rows // 128) * 128
+    for form, floats in ((ops.FACTOR_INVERSE, K + 512), (ops.FACTOR_GROUPS, 2 * K + 512 * pieces)):
+        taken = ops.gptq_quantize_grouped_workspace_bytes(1, rows, K, form)
+        assert 0 <= taken - 4 * padded * floats <= 4 * (3 * padded + K) + 4096
+
+
 def test_observed_kv_cache_stand_in():
     """The stand-in for ``past_key_values`` shows keys and values to the module's observers and defers to the
     real cache when there is one."""
