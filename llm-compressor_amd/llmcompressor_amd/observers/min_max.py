@@ -40,24 +40,22 @@ def _group_of(observer, value):
 
 def observe_weights_together(observed):
     """``observer(value)`` for the pairs that can share a launch: weights of one shape and dtype in groups of one size (an MoE
-    layer's experts, q / k / v, gate / up), whose statistics become slices of one tensor.  Returns the others."""
-    sets, rest, seen = {}, [], set()
-    for observer, value in observed:
+    layer's experts, q / k / v, gate / up), whose statistics become slices of one tensor.  Returns the others, in their order."""
+    sets, seen, done = {}, set(), set()
+    for at, (observer, value) in enumerate(observed):
         group = 0 if observer in seen else _group_of(observer, value)
         seen.add(observer)
         # (slices of whole 16-byte vectors, int8 zero points' too: every kernel finds them as aligned as a tensor of their own)
         if group and value.shape[0] * (value.shape[1] // group) % 16 == 0:
-            sets.setdefault((value.shape, value.dtype, value.device, group), {})[observer] = value
-        else:
-            rest.append((observer, value))
+            sets.setdefault((value.shape, value.dtype, value.device, group), []).append(at)
     for (shape, dtype, _, group), members in sets.items():
         if len(members) < 2 or not _lib.lib().llmc_minmax_groups_many_fits(_DTYPE_CODES[dtype], *shape, group):
-            rest += members.items()
             continue
-        mins, maxs = llmc.minmax_observe_many([v.detach() for v in members.values()], group)
-        for observer, mn, mx in zip(members, mins.unbind(0), maxs.unbind(0)):
-            observer.update_statistics(mn, mx)
-    return rest
+        mins, maxs = llmc.minmax_observe_many([observed[at][1].detach() for at in members], group)
+        for at, mn, mx in zip(members, mins.unbind(0), maxs.unbind(0)):
+            observed[at][0].update_statistics(mn, mx)
+        done.update(members)
+    return [pair for at, pair in enumerate(observed) if at not in done]
 
 
 @Observer.register("static_minmax")

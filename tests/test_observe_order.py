@@ -1,7 +1,9 @@
-"""``observe`` of many modules: each weight is seen while its module is at hand (reference: modifiers/quantization/calibration.py observes module by module)."""
+"""``observe`` of many modules: each weight is seen while its module is at hand and in the order of the call, whatever shares
+a launch (reference: modifiers/quantization/calibration.py observes module by module)."""
 import torch
 
 from llmcompressor_amd.modifiers.quantization.calibration import observe
+from llmcompressor_amd.observers import min_max
 
 
 class _Recorder(torch.nn.Module):
@@ -41,3 +43,12 @@ def test_modules_of_an_iterator_are_observed_one_at_a_time():
     observe(mods, "weight")
     observe({m: None for m in mods}.keys(), "weight")
     assert [[int(s[0, 0]) for s in m.weight_observer.seen] for m in mods] == [[1, 4, 4], [2, 5, 5], [3, 6, 6]]
+
+
+def test_an_observer_of_two_modules_sees_the_first_one_first(monkeypatch):
+    """A weight's observer keeps the first value that it is shown; what could share a launch but finds no partner keeps its place."""
+    monkeypatch.setattr(min_max, "_group_of", lambda observer, value: 64)
+    first, second = _modules(2)
+    second.weight_observer = first.weight_observer
+    observe([first, second], "weight")
+    assert [int(s[0, 0]) for s in first.weight_observer.seen] == [1, 2]
