@@ -103,7 +103,8 @@ def _run_length(observers: List["Observer"], at: int) -> int:
 
     def asks(o):  # what the parameters depend on besides the statistics; None: not for sharing
         if (not isinstance(o, Observer) or type(o).get_qparams is not Observer.get_qparams
-                or type(o).get_global_scale is not Observer.get_global_scale or "get_qparams" in o.__dict__ or "get_global_scale" in o.__dict__ or not o.has_statistics
+                or type(o).get_global_scale is not Observer.get_global_scale or "get_qparams" in o.__dict__
+                or "get_global_scale" in o.__dict__ or not o.has_statistics
                 or o.args.strategy == QuantizationStrategy.TENSOR_GROUP or o.fusion_handler.is_fused):
             return None
         mn, mx = o.min_vals, o.max_vals
@@ -130,6 +131,14 @@ def _run_length(observers: List["Observer"], at: int) -> int:
             break
         n += 1
     return n
+
+
+def _apart(stacked: torch.Tensor) -> List[torch.Tensor]:
+    """The slices of a contiguous tensor as tensors of their own, copied in one launch."""
+    slices = list(stacked.unbind(0))
+    out = [torch.empty_like(s) for s in slices]
+    torch._foreach_copy_(out, slices)
+    return out
 
 
 class Observer(torch.nn.Module):
@@ -241,7 +250,8 @@ class Observer(torch.nn.Module):
     @staticmethod
     def get_qparams_of(observers: List["Observer"]) -> List[QParamsDict]:
         """``get_qparams`` of each, one launch for every run of observers whose statistics lie one after the other in one
-        tensor (weights observed together) and ask for the same parameters; they are then slices of one tensor as well."""
+        tensor (weights observed together) and ask for the same parameters.  Each parameter is a tensor of its own: a module
+        that keeps one keeps no other module's, and libraries that refuse to save part of a storage take it."""
         out: List[QParamsDict] = []
         while len(out) < len(observers):
             n = _run_length(observers, len(out))
@@ -254,7 +264,7 @@ class Observer(torch.nn.Module):
             scale, zero_point = calculate_qparams(*stacked, quantization_args=first.args, global_scale=None)
             for observer in run:
                 observer.delete_statistics()
-            out += [{"scale": s, "zero_point": z, "global_scale": None} for s, z in zip(scale.unbind(0), zero_point.unbind(0))]
+            out += [{"scale": s, "zero_point": z, "global_scale": None} for s, z in zip(_apart(scale), _apart(zero_point))]
         return out
 
     @_without_grad

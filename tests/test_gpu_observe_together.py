@@ -81,3 +81,21 @@ def test_what_a_call_would_do_besides_still_happens():
     for m in (hooked, plain, other, repeated):
         assert torch.equal(m.weight_observer.min_vals, m.weight.view(64, 2, 128).amin(-1))
         assert torch.equal(m.weight_observer.max_vals, m.weight.view(64, 2, 128).amax(-1))
+
+
+@pytest.mark.parametrize("preset", ["W4A16_ASYM", "MXFP4A16"])
+def test_parameters_found_together_are_tensors_of_their_own(preset, tmp_path):
+    """As those of one call each: nothing of the others is kept with one, and it can be saved with its module."""
+    from safetensors.torch import load_file, save_model
+
+    mods = _linears([(64, 256)] * 3, preset)
+    with torch.no_grad():
+        observe(mods, "weight")
+        found = Observer.get_qparams_of([m.weight_observer for m in mods])
+    for i, (m, q) in enumerate(zip(mods, found)):
+        for key in ("scale", "zero_point"):
+            assert q[key].untyped_storage().nbytes() == q[key].nbytes and q[key].data_ptr() % 16 == 0
+            m.register_parameter(f"found_{key}", torch.nn.Parameter(q[key], requires_grad=False))
+        save_model(m, str(tmp_path / f"{i}.safetensors"))
+        saved = load_file(str(tmp_path / f"{i}.safetensors"))
+        assert torch.equal(saved["found_scale"], q["scale"].cpu()) and torch.equal(saved["found_zero_point"], q["zero_point"].cpu())
