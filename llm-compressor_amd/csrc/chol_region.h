@@ -64,7 +64,7 @@ struct RegionArgs {
   int n, tiles;        // problems; sets of ROWS rows below the region
   uint32_t ticket0;    // tickets of the launches before
   uint32_t region;     // regions before this one, all of MAX_BLOCKS blocks
-  uint64_t wait_ticks; // how long a wait may last
+  uint32_t wait_ticks; // how long a wait may last, at most 2^31
   // where the rows below go as two f16 terms as well (split2.h), for the updates that read them, or NULL: row i of the
   // matrix at i * split_ld, one set every split_stride words
   uint32_t* split;
@@ -90,6 +90,7 @@ struct RegionLds {
     RowsLds rows;
   };
   int word, gave_up;
+  uint32_t wait_ticks;  // (here, not in a scalar register that the spine has other uses for)
 };
 static_assert(sizeof(RegionLds) <= 80 * 1024, "two workgroups to a CU");
 
@@ -124,15 +125,15 @@ __device__ __forceinline__ bool reached(const uint32_t* word, uint32_t target) {
   asm volatile("" ::: "memory");  // what is loaded next is loaded after the word
   return there;
 }
-constexpr uint64_t TICKS_PER_US = 100;  // of the steady counter
+constexpr int64_t TICKS_PER_US = 100;  // of the steady counter, of which a wait needs the low half
 // false: gave up
-__device__ __forceinline__ bool poll(const uint32_t* word, uint32_t target, uint64_t ticks) {
+__device__ __forceinline__ bool poll(const uint32_t* word, uint32_t target, const uint32_t& ticks) {
   if (reached(word, target)) return true;
-  const uint64_t start = __builtin_readsteadycounter();
+  const uint32_t start = (uint32_t)__builtin_readsteadycounter();
   do {
     __builtin_amdgcn_s_sleep(2);
     if (reached(word, target)) return true;
-  } while (__builtin_readsteadycounter() - start < ticks);
+  } while ((uint32_t)__builtin_readsteadycounter() - start < ticks);
   return false;
 }
 struct Awaited {
@@ -149,7 +150,6 @@ struct Region {
   HinvScalars* sc;
   int Kp, K, r0, nb;
   uint32_t done;  // hand-overs of one kind in the regions before
-  uint64_t wait_ticks;
   uint32_t* split;
   int split_ld;
   __device__ uint32_t* word(int which) const { return sync + which * SYNC_LINE; }
@@ -167,7 +167,7 @@ __device__ __forceinline__ bool wait_for(const Region& g, RegionLds& L, Awaited 
   __syncthreads();
   if (threadIdx.x < 2) {
     const Awaited mine = threadIdx.x == 0 ? a : b;
-    if (!poll(mine.word, mine.target, g.wait_ticks)) {
+    if (!poll(mine.word, mine.target, L.wait_ticks)) {
       atomicExch(&g.sc->info, -1);
       L.gave_up = 1;
     }
@@ -242,7 +242,7 @@ __device__ __forceinline__ void spine(const Region& g, RegionLds& lds, int threa
       rows_state = THERE;
     };
     auto await = [&](const Awaited& a) {
-      if (!poll(a.word, a.target, g.wait_ticks) && r == 0) {
+      if (!poll(a.word, a.target, lds.wait_ticks) && r == 0) {
         atomicExch(&g.sc->info, -1);
         lds.gave_up = 1;
       }
@@ -461,6 +461,7 @@ __global__ __launch_bounds__(REGION_NT) void chol_region_kernel(RegionArgs a) {
   if (tid == 0) {
     const int task = (int)(atomicAdd(a.sync + WORD_TICKET * SYNC_LINE, 1u) - a.ticket0);
     lds.word = task;
+    lds.wait_ticks = a.wait_ticks;
     lds.gave_up = a.sc[problem_of(task)].info < 0;  // in an earlier region
   }
   __syncthreads();
@@ -474,7 +475,6 @@ __global__ __launch_bounds__(REGION_NT) void chol_region_kernel(RegionArgs a) {
   g.sc = a.sc + problem;
   g.Kp = a.Kp; g.K = a.K; g.r0 = a.r0; g.nb = a.nb;
   g.done = a.region;
-  g.wait_ticks = a.wait_ticks;
   g.split = a.split ? a.split + problem * a.split_stride : nullptr;
   g.split_ld = a.split_ld;
   if (task < all) {
