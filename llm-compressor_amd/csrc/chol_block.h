@@ -4,16 +4,17 @@
 // form: the update of column c by pivot column j is x[c] -= x[j] * (x_c[j] / d_j)), so no square root is on the chain, and a
 // pivot that is not positive and finite is only recorded: what follows it is discarded by the caller.
 //
-// What bounds it is one wave's instruction issue, a vector instruction every 5.5 cycles and one with a cross-lane operand
-// every 9.  A slab of 16 columns is therefore factored in four blocks of four: the four pivots of a block on the vector
-// ALU, which touch only the block's own columns, and the rest of the slab by one matrix instruction for all four.  16 x 16
-// tiles lie in registers as v_mfma_f32_16x16x4_f32 holds its result: lane (g = lane / 16, r = lane % 16) has row r of the
-// tile, columns 4 g .. 4 g + 3, so that block b's columns are what the row b of lanes holds, a row of the matrix per lane,
-// and a pivot's multipliers are operands across lanes of that row (row_newbcast).  For the matrix instruction the four
-// columns of the block are moved to the four rows of lanes (three lane swaps).  Waves 0 to 3 each keep the slab's diagonal
-// tile -- the same arithmetic in each, so nothing crosses waves -- and one more tile that takes the same column operations:
-// wave u > 0 the rows of tile row K + u, wave 0 rows of the identity, which end up as the transposed inverse of the
-// unit-lower factor.  The tiles of the next slab are brought up to date in the registers that will factor them.
+// What bounds it is one wave's instruction issue: a vector instruction every 4.8 to 5.8 cycles (5.2 with a cross-lane operand),
+// one that takes the result of the one before every 9.  A slab of 16 columns is therefore factored in four blocks of four:
+// the four pivots of a block on the vector ALU, which touch only the block's own columns, and the rest of the slab by one
+// matrix instruction for all four.  16 x 16 tiles lie in registers as v_mfma_f32_16x16x4_f32 holds its result: lane
+// (g = lane / 16, r = lane % 16) has row r of the tile, columns 4 g .. 4 g + 3, so that block b's columns are what the row b
+// of lanes holds, a row of the matrix per lane, and a pivot's multipliers are operands across lanes of that row
+// (row_newbcast).  For the matrix instruction the four columns of the block are moved to the four rows of lanes (three lane
+// swaps).  Waves 0 to 3 each keep the slab's diagonal tile -- the same arithmetic in each, so nothing crosses waves -- and
+// one more tile that takes the same column operations: wave u > 0 the rows of tile row K + u, wave 0 rows of the identity,
+// which end up as the transposed inverse of the unit-lower factor.  The tiles of the next slab are brought up to date in the
+// registers that will factor them.
 // 2750 cycles for the last slab, 3150 for the ones before it with their tiles' update, 14.9k for the block.  Pivot by pivot,
 // one wave with all of a slab's rows and a cross-lane multiply-add per column: 3500 a slab, 17.3k the block.
 //

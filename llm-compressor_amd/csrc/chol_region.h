@@ -9,11 +9,12 @@
 //                    columns and to its diagonal block; then hands A[b, b-1] and the diagonal block to the spine
 //   rows below       32 rows to a workgroup, two independent sets of 16: each block column solved as its X arrives
 // One launch per step, with every workgroup factoring the block for itself, and one more for the rows below took 49.8 and
-// 10.2 us for a region of a 4096-wide matrix, 4.5 us of each launch being the launch; 39 us now.  What bounds the region is
+// 10.2 us for a region of a 4096-wide matrix, 4.5 us of each launch being the launch; 41 us now.  What bounds the region is
 // the spine, 9 us a step: the 64 x 64 factor-and-invert (one wave's instruction issue, chol_block.h; 6.2 us), the solve of
 // the next row block (0.9), its part of the next diagonal block (1.2).  The tiles of that one which the first slab needs are
 // formed in the registers that factor it, the others beside it.
-// Whole chains: 4096 columns 1323 -> 1022 us, 14336 9.0 -> 8.1 ms with this form of the launches alone.
+// Whole chains: 4096 columns 1323 -> 1114 us, 14336 9.0 -> 8.1 ms with this form of the launches alone; 1010 us and 7.4 ms with
+// split rows (chol.hip) and slabs in blocks of four pivots (chol_block.h) as well.
 //
 // 512 threads and at most 80 KB of LDS to a workgroup: two fit a CU, and one fits beside a workgroup of the 128-wide
 // products.  With 1024 threads and 131 KB a launch needed CUs of its own, and beside another stream's products every third

@@ -2,7 +2,7 @@
 // Launched once per group by gptq.hip, instantiated in gptq_group_int.hip and gptq_group_fp.hip.
 //
 // What bounds it: rows are independent, but every column of a row depends on the one before it, so a wave works
-// through 128 dependent steps per block.  A wave issues an independent vector instruction every 5.5 cycles here and a
+// through 128 dependent steps per block.  A wave issues an independent vector instruction every 4.8 to 5.8 cycles and a
 // dependent one every 9, and a SIMD completes one every 4 however many waves it holds.  Both kernels are therefore
 // laid out for few instructions on that chain:
 //   * a row belongs to a team of 16 or 8 lanes, each holding runs of 4 neighbouring columns in registers.  In every
@@ -18,8 +18,8 @@
 // W[:, b] - E U[:, b], as 16 x 16 tiles accumulated by v_mfma_f32_16x16x4_f32 in fp32.  In the left-looking form the same
 // products bring in what the group owes to all earlier columns, P U[group, group]: E starts out as P in LDS, a block's own
 // columns of it are multiplied ahead of the block before, and its errors are added to them.  As a pass over the pieces of P,
-// a 512-wide product and a pass that formed D this took three launches more per group: with them 4096 x 4096 2441 -> 2202
-// us (a whole call), 4096 x 14336 19.7 -> 19.1 ms, 32 of 768 x 2048 5341 -> 5000 us.
+// a 512-wide product and a pass that formed D this took three launches more per group: without them 4096 x 4096
+// 2441 -> 2181 us (a whole call), 4096 x 14336 19.7 -> 18.6 ms, 32 of 768 x 2048 5341 -> 4867 us.
 //
 // A workgroup is four waves that run the chain, one per SIMD, and four that prepare the next block meanwhile: its slice
 // of U, its scales and the part of its tiles that does not wait for the current block.
