@@ -16,15 +16,17 @@ class MemorylessMinMaxObserver(Observer):
     """min/max of the observed value."""
 
 
+# what a call goes through before the statistics are kept, as a caller may have set it on one observer
+_REPLACED = {"forward", "compute_min_max", "_min_max_kernel"}
 _DTYPE_CODES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
 
 def _group_of(observer, value):
     """Columns that share a scale, where calling ``observer`` on the weight ``value`` would do nothing but replace its
-    statistics by the min-max of such groups (no hooks, no fused partner, nothing observed before); else 0."""
+    statistics by the min-max of such groups (no hooks, no step replaced, no fused partner, nothing observed before); else 0."""
     if (type(observer) is not MemorylessMinMaxObserver or not observer.is_weight_obs or observer._forward_hooks
             or observer._forward_pre_hooks or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks
-            or "forward" in observer.__dict__ or observer.has_statistics or observer._buffers or observer._parameters
+            or not _REPLACED.isdisjoint(observer.__dict__) or observer.has_statistics or observer._buffers or observer._parameters
             or observer.fusion_handler.is_fused):
         return 0
     if not (type(value) in (torch.Tensor, torch.nn.Parameter) and value.is_cuda and value.ndim == 2 and value.numel()

@@ -99,3 +99,21 @@ def test_parameters_found_together_are_tensors_of_their_own(preset, tmp_path):
         save_model(m, str(tmp_path / f"{i}.safetensors"))
         saved = load_file(str(tmp_path / f"{i}.safetensors"))
         assert torch.equal(saved["found_scale"], q["scale"].cpu()) and torch.equal(saved["found_zero_point"], q["zero_point"].cpu())
+
+
+@pytest.mark.parametrize("step", ["forward", "compute_min_max", "_min_max_kernel"])
+def test_steps_replaced_on_one_observer_are_taken(step):
+    mods = _linears([(64, 256)] * 3, "W4A16")
+    observer, seen = mods[1].weight_observer, []
+    original = getattr(observer, step)
+
+    def replaced(value):
+        seen.append(value.shape)
+        return original(value)
+
+    setattr(observer, step, replaced)
+    with torch.no_grad():
+        observe(mods, "weight")
+    assert seen == [mods[1].weight.shape]
+    for m in mods:
+        assert torch.equal(m.weight_observer.min_vals, m.weight.view(64, 2, 128).amin(-1))
