@@ -1,5 +1,5 @@
 // Internal fp32 GEMM on the matrix cores (v_mfma_f32_32x32x2_f32), used for the
-// chain's triangular inverse and the updates of the GPTQ and SparseGPT loops.
+// chain's triangular inverse and the updates of the GPTQ and SparseGPT loops; B^T and lower triangles for llmc_sgemm.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
